@@ -319,7 +319,7 @@ def tolerance(case):
     if kind == "layer":  # int8 steps one apart early in the layer: rel 3.4e-3, max 0.10, caches differ in 2e-5
         return {"rel": 1.4e-2, "max": 0.4, "differ": 1e-4}
     if kind == "bmm_chain":  # rel 3.4e-4, 4.5e-8 of the probabilities one step apart (0 against 1)
-        return {"rel": 1.4e-3, "max": 1.0, "differ": 1e-6}
+        return {"rel": 1.4e-3, "max": 0.99, "differ": 1e-6}
     if kind in ("rows", "linear_set") or case.get("epilogue") == "gelu_q":  # rel 5.3e-5, 1.1e-6 one step apart
         return {"rel": 2e-4, "max": 0.2, "differ": 4e-6}
     return "exact"  # integer sums, with one rounding per fixed step before and after them
