@@ -348,7 +348,8 @@ int ti_kv_append_i8(const int8_t* k_src, int64_t k_src_row_stride, const int8_t*
  *     out    = q8(pv_alpha * (probs . v))                  (bmm_s8t_s8n_s8t again, b = V^T)
  * q [batch, S, D], k [batch, T, D], vt [batch, D, T] (V^T, as the P.V BMM takes it), out
  * [batch, S, D]; int8, unit stride along the last dimension, batch and row strides in elements
- * (all multiples of 16, like the pointers); D = 128; T a multiple of 16; 0 < score_scale <= 64.
+ * (all multiples of 16, like the pointers; those of vt may be anything, aligned rows are faster);
+ * D = 128; any T > 0; 0 < score_scale <= 64.
  * The scalars are host floats.  The int8 scores are the BMM's and the probabilities ti_softmax_q's
  * bit for bit (a row's exponentials are summed as integers, so the order in which the keys are
  * visited does not matter): the output equals the three-launch chain's exactly.
@@ -363,6 +364,18 @@ int ti_attention_i8(const int8_t* q, int64_t q_batch_stride, int64_t q_row_strid
                     int8_t* out, int64_t out_batch_stride, int64_t out_row_stride,
                     int batch, int S, int T, int D,
                     float qk_alpha, float score_scale, float pv_alpha, int causal_q_len, void* stream);
+
+/*
+ * The same for `seqs` sequences of `heads` heads each in one launch: every operand has a stride per
+ * sequence and a stride per head inside it (q [seqs, heads, S, D] may be a view of a [seqs, S, 3H]
+ * projection, out a view of [seqs, S, H]).
+ */
+int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int64_t q_head_stride, int64_t q_row_stride,
+                          const int8_t* k, int64_t k_seq_stride, int64_t k_head_stride, int64_t k_row_stride,
+                          const int8_t* vt, int64_t vt_seq_stride, int64_t vt_head_stride, int64_t vt_row_stride,
+                          int8_t* out, int64_t out_seq_stride, int64_t out_head_stride, int64_t out_row_stride,
+                          int seqs, int heads, int S, int T, int D,
+                          float qk_alpha, float score_scale, float pv_alpha, int causal_q_len, void* stream);
 
 /*
  * Dynamic per-token activation quantisation, dynamic_quantize_activation_per_token_absmax

@@ -1,0 +1,47 @@
+"""Kernels on sizes that are no multiple of anything: attention over any number of keys, several sequences in
+one launch."""
+import numpy as np
+import pytest
+import torch
+
+from tests.test_gpu_rowops import _attention_chain_checked
+from tests.util import gpu, rng
+
+pytestmark = pytest.mark.gpu
+
+
+# the last number: the pitch of V^T's rows (0: exactly T, so that rows start at any byte)
+@pytest.mark.parametrize("BH,S,T,q_len,pitch", [
+    (2, 1, 1, 1, 0), (3, 1, 15, 0, 16), (2, 16, 17, 16, 0), (2, 5, 63, 5, 64), (40, 1, 1531, 1, 2048), (3, 3, 1025, 3, 0),
+    (300, 1, 77, 1, 80), (2, 16, 2047, 0, 0), (2, 2, 2049, 2, 4096), (1, 1, 4093, 0, 0),     # few query rows
+    (2, 333, 333, 333, 336), (2, 333, 333, 333, 0), (3, 17, 65, 17, 0), (2, 130, 1007, 0, 1024), (1, 128, 129, 128, 0)])
+def test_attention_i8_over_any_number_of_keys(BH, S, T, q_len, pitch):
+    """Equal to the three-launch chain, bit for bit, whatever the length and the alignment of V^T's rows."""
+    from triton_int_amd.kernels import fused
+
+    g = rng(BH * 1000 + S * 7 + T)
+    q, k = (g.integers(-127, 128, size=(BH, n, 128), dtype=np.int8) for n in (S, T))
+    vt = g.integers(-127, 128, size=(BH, 128, T), dtype=np.int8)
+    room = torch.full((BH, 128, max(pitch, T)), 99, dtype=torch.int8, device="cuda")  # what lies past T must not matter
+    gvt = room[:, :, :T]
+    gvt.copy_(gpu(vt))
+    for qk_alpha, score_scale, pv_alpha in ((1e-3, 0.05, 1.0 / 127.0), (4e-3, 0.2, 0.03)):
+        want = _attention_chain_checked(q, k, vt, qk_alpha, score_scale, pv_alpha, q_len)
+        got = fused.attention_i8(gpu(q), gpu(k), gvt, qk_alpha, score_scale, pv_alpha, causal_q_len=q_len)
+        assert torch.equal(got, want), f"{int((got != want).sum())} values differ"
+
+
+@pytest.mark.parametrize("B,heads,S,T", [(3, 2, 1, 53), (2, 3, 150, 150), (16, 4, 1, 1007)])
+def test_attention_i8_of_several_sequences_in_one_launch(B, heads, S, T):
+    """4-D operands with a stride per sequence and per head: each sequence as if launched by itself."""
+    from triton_int_amd.kernels import fused
+
+    g = torch.Generator(device="cuda").manual_seed(B * 100 + T)
+    i8 = lambda *shape: torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda", generator=g)
+    q = i8(B, S, 3, heads, 128)[:, :, 0].transpose(1, 2)   # views of a [B, S, 3H] projection
+    k, vt = i8(B, heads, T + 3, 128)[:, :, :T], i8(B, heads, 128, T + 16)[:, :, :, :T]
+    out = torch.zeros((B, S, heads, 128), dtype=torch.int8, device="cuda")
+    fused.attention_i8(q, k, vt, 2e-3, 0.1, 0.02, causal_q_len=S, out=out.transpose(1, 2))
+    for b in range(B):
+        want = fused.attention_i8(q[b], k[b], vt[b], 2e-3, 0.1, 0.02, causal_q_len=S)
+        assert torch.equal(out[b].transpose(0, 1), want)

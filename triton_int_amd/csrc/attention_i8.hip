@@ -41,8 +41,10 @@ constexpr int AT_VBYTES = AT_D * AT_VP;
 
 struct AttnParams {
   const int8_t* q; const int8_t* k; const int8_t* vt; int8_t* out;
-  int64_t sQb, sQm, sKb, sKn, sVb, sVd, sOb, sOm;
-  int S, T, causal_q_len, nblk, batch;
+  // strides of a sequence, of a head inside it, of a row inside that
+  int64_t sQb, sQh, sQm, sKb, sKh, sKn, sVb, sVh, sVd, sOb, sOh, sOm;
+  int S, T, causal_q_len, nblk;
+  int batch, heads;  // batch = sequences * heads
   float qk_alpha, s2, pv_alpha;  // s2 = score_scale * log2(e)
 };
 
@@ -50,6 +52,34 @@ __device__ __forceinline__ int attn_limit(const AttnParams& p, int row) {
   return p.causal_q_len > 0 ? min(p.T, (row % p.causal_q_len) + (p.T - p.causal_q_len) + 1) : p.T;
 }
 
+// 16 keys of a V^T row whose address has no alignment (a row pitch that is not a multiple of 16: a cache
+// allocated at exactly its length).  Whole chunks are one unaligned 16-byte load; the chunk that crosses T
+// is put together from bytes, because an unaligned load there could leave the allocation.
+__device__ __forceinline__ v4i load_keys_any(const int8_t* row, int col, int T) {
+  v4i v = {0, 0, 0, 0};
+  if (col + 16 <= T) {
+    __builtin_memcpy(&v, row + col, 16);
+  } else {
+#pragma unroll 1
+    for (int i = T - 1 - col; i >= 0; --i) {  // shifts the bytes up one by one: no indexed register access
+      v[3] = (int)(((unsigned)v[3] << 8) | ((unsigned)v[2] >> 24));
+      v[2] = (int)(((unsigned)v[2] << 8) | ((unsigned)v[1] >> 24));
+      v[1] = (int)(((unsigned)v[1] << 8) | ((unsigned)v[0] >> 24));
+      v[0] = (int)(((unsigned)v[0] << 8) | (unsigned)(uint8_t)row[col + i]);
+    }
+  }
+  return v;
+}
+
+// Any number of keys, all sequences of a batch in one launch: what a length that is no multiple of 16 used to
+// cost was the three-launch chain with P.V through byte gathers, once per sequence.  Whole layer, before ->
+// after: two prompts of 333 tokens (4096 wide) 377 -> 239 us, sixteen sequences decoding at position 1007
+// 1105 -> 284 us.
+//
+// VANY: rows of V^T start anywhere (load_keys_any).  Otherwise they are 16-byte aligned, and a chunk that
+// crosses T is loaded whole: an aligned 16-byte chunk that holds at least one key of the row lies inside the
+// row's pitch, and the keys past T are multiplied by probabilities that are exactly 0.
+template <bool VANY>
 __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) char lds[2 * (AT_KBYTES + AT_VBYTES)];
   __shared__ int wg_lim[4];
@@ -67,9 +97,10 @@ __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
   const int pos = pass * 256 + ((pass & 1) ? cnt - 1 - c : c);
   const int bh = pos % p.batch;
   const int m0 = (p.nblk - 1 - pos / p.batch) * AT_ROWS + wave * 32;
-  const int8_t* qb = p.q + (int64_t)bh * p.sQb;
-  const int8_t* kb_ = p.k + (int64_t)bh * p.sKb;
-  const int8_t* vb = p.vt + (int64_t)bh * p.sVb;
+  const int seq = bh / p.heads, head = bh - seq * p.heads;
+  const int8_t* qb = p.q + (int64_t)seq * p.sQb + (int64_t)head * p.sQh;
+  const int8_t* kb_ = p.k + (int64_t)seq * p.sKb + (int64_t)head * p.sKh;
+  const int8_t* vb = p.vt + (int64_t)seq * p.sVb + (int64_t)head * p.sVh;
 
   // ---- per-lane row, visible-key limit; wave and workgroup bounds
   const int row = m0 + lrow;
@@ -111,8 +142,13 @@ __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
       for (int c = 0; c < 2; ++c) {
         const int q_ = c * 256 + tid;        // chunk index: 128 d x 4 chunks of 16 keys
         const int vr = q_ >> 2, vc = q_ & 3;
-        const bool in = key0 + vc * 16 < p.T;  // T % 16 == 0: a chunk is wholly inside or outside
-        vreg[c] = in ? *(const v4i*)(vb + (int64_t)vr * p.sVd + key0 + vc * 16) : (v4i){0, 0, 0, 0};
+        const int8_t* row = vb + (int64_t)vr * p.sVd;
+        if constexpr (VANY) {
+          vreg[c] = load_keys_any(row, key0 + vc * 16, p.T);
+        } else {
+          const bool in = key0 + vc * 16 < p.T;
+          vreg[c] = in ? *(const v4i*)(row + key0 + vc * 16) : (v4i){0, 0, 0, 0};
+        }
       }
     }
   };
@@ -324,7 +360,7 @@ __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
 
   // ---- context: o[db][r] is row lrow, d = 32*db + 8*(r/4) + 4*lhi + r%4 -> int8, 16 bytes per lane
   if (!wave_live) return;
-  int8_t* ob = p.out + (int64_t)bh * p.sOb;
+  int8_t* ob = p.out + (int64_t)seq * p.sOb + (int64_t)head * p.sOh;
 #pragma unroll
   for (int db = 0; db < 4; ++db) {
     unsigned X[4];
@@ -368,7 +404,8 @@ constexpr int AD_MAXT = 4096;
 // produces (8: the whole head; fewer: the head is spread over 8 / DBW workgroups, each of which
 // repeats the scores and the softmax and reads only its rows of V^T — a single CU fills its caches at
 // about 30 GB/s, so a head's 512 KB of K and V^T through one CU alone would take 17 us).
-template <int CPW, int DBW>
+// VANY: V^T rows without alignment, as in attention_i8_kernel.
+template <int CPW, int DBW, bool VANY>
 __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(AttnParams p) {
   constexpr int TMAX = 256 * CPW;
   constexpr int PP = TMAX + 16;             // LDS pitch of a query's probabilities
@@ -388,13 +425,20 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   const int dbase = (blockIdx.x / p.batch) * DBW;
   const int OOB = 0x7ffffff0;
   const float MAGIC = 12582912.0f;
-  const __amdgpu_buffer_rsrc_t rQ =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(p.q + (int64_t)bh * p.sQb), 0, (int)((p.S - 1) * p.sQm + AT_D), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rK =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(p.k + (int64_t)bh * p.sKb), 0, (int)((p.T - 1) * p.sKn + AT_D), 0x00020000);
+  const int seq = bh / p.heads, head = bh - seq * p.heads;
+  const int8_t* vb = p.vt + (int64_t)seq * p.sVb + (int64_t)head * p.sVh;
+  const __amdgpu_buffer_rsrc_t rQ = __builtin_amdgcn_make_buffer_rsrc((void*)(p.q + (int64_t)seq * p.sQb + (int64_t)head * p.sQh), 0,
+                                                                      (int)((p.S - 1) * p.sQm + AT_D), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)(p.k + (int64_t)seq * p.sKb + (int64_t)head * p.sKh), 0,
+                                                                      (int)((p.T - 1) * p.sKn + AT_D), 0x00020000);
+  // the last chunk of an aligned row may cross T (see attention_i8_kernel)
   const __amdgpu_buffer_rsrc_t rV =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(p.vt + (int64_t)bh * p.sVb), 0, (int)((AT_D - 1) * p.sVd + p.T), 0x00020000);
-  const int NCH = p.T >> 4;         // 16-key chunks
+      __builtin_amdgcn_make_buffer_rsrc((void*)vb, 0, (int)((AT_D - 1) * p.sVd + ((p.T + 15) & ~15)), 0x00020000);
+  auto load_v = [&](int d, int col) -> v4i {
+    if constexpr (VANY) return load_keys_any(vb + (int64_t)d * p.sVd, col, p.T);
+    else return __builtin_amdgcn_raw_buffer_load_b128(rV, col < p.T ? d * (int)p.sVd + col : OOB, 0, 0);
+  };
+  const int NCH = (p.T + 15) >> 4;  // 16-key chunks; rows of K past T read as zeros and are masked
   const int NG = (p.T + 63) >> 6;   // 64-key groups
   const int db = dbase + wave % DBW, kh = wave / DBW;
 
@@ -439,7 +483,7 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   for (int i = 0; i < HOIST; ++i) {
     const int g = kh + KPARTS * i;
     const int col = 64 * g + 16 * kq;
-    vf[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, col < p.T ? (16 * db + n) * (int)p.sVd + col : OOB, 0, 0);
+    vf[i] = load_v(16 * db + n, col);
   }
 
   // ---- row maximum (exact: integers), exponentials, row sum
@@ -495,16 +539,16 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   }
 #pragma unroll
   for (int i0 = HOIST; i0 < GPW; i0 += 4) {
-    v4i vb[4];
+    v4i vn[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int col = 64 * (kh + KPARTS * (i0 + i)) + 16 * kq;
-      vb[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, col < p.T ? (16 * db + n) * (int)p.sVd + col : OOB, 0, 0);
+      vn[i] = load_v(16 * db + n, col);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int g = kh + KPARTS * (i0 + i);
-      if (g < NG) o = __builtin_amdgcn_mfma_i32_16x16x64_i8(vb[i], *(const v4i*)(p_lds + n * PP + 64 * g + 16 * kq), o, 0, 0, 0);
+      if (g < NG) o = __builtin_amdgcn_mfma_i32_16x16x64_i8(vn[i], *(const v4i*)(p_lds + n * PP + 64 * g + 16 * kq), o, 0, 0, 0);
     }
   }
   if (kh > 0) ctx_red[wave][lane] = o;
@@ -519,50 +563,55 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
       v = __builtin_amdgcn_fmed3f(v, -128.0f, 127.0f);
       b[r] = __float_as_uint(v + MAGIC);
     }
-    *(unsigned*)(p.out + (int64_t)bh * p.sOb + (int64_t)n * p.sOm + 16 * db + 4 * kq) =
+    *(unsigned*)(p.out + (int64_t)seq * p.sOb + (int64_t)head * p.sOh + (int64_t)n * p.sOm + 16 * db + 4 * kq) =
         __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
   }
 }
 
 }  // namespace ti
 
-extern "C" int ti_attention_i8(const int8_t* q, int64_t q_batch_stride, int64_t q_row_stride, const int8_t* k,
-                               int64_t k_batch_stride, int64_t k_row_stride, const int8_t* vt,
-                               int64_t vt_batch_stride, int64_t vt_row_stride, int8_t* out, int64_t out_batch_stride,
-                               int64_t out_row_stride, int batch, int S, int T, int D, float qk_alpha,
-                               float score_scale, float pv_alpha, int causal_q_len, void* stream) {
+extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int64_t q_head_stride, int64_t q_row_stride,
+                                     const int8_t* k, int64_t k_seq_stride, int64_t k_head_stride, int64_t k_row_stride,
+                                     const int8_t* vt, int64_t vt_seq_stride, int64_t vt_head_stride, int64_t vt_row_stride,
+                                     int8_t* out, int64_t out_seq_stride, int64_t out_head_stride, int64_t out_row_stride,
+                                     int seqs, int heads, int S, int T, int D, float qk_alpha, float score_scale,
+                                     float pv_alpha, int causal_q_len, void* stream) {
   using namespace ti;
-  if (batch < 0 || S < 0 || T < 0 || causal_q_len < 0) return fail(TI_E_SHAPE, "negative size");
-  if (batch == 0 || S == 0) return TI_OK;
+  if (seqs < 0 || heads < 0 || S < 0 || T < 0 || causal_q_len < 0) return fail(TI_E_SHAPE, "negative size");
+  if (seqs == 0 || heads == 0 || S == 0) return TI_OK;
   if (!q || !k || !vt || !out) return fail(TI_E_NULL, "q, k, vt and out are required");
   if (D != AT_D) return fail(TI_E_SHAPE, "head dimension %d: this kernel is built for %d", D, AT_D);
-  if (T <= 0 || (T & 15)) return fail(TI_E_SHAPE, "T = %d must be a positive multiple of 16", T);
-  if (batch > 65535) return fail(TI_E_SHAPE, "batch %d > 65535", batch);
+  if (T <= 0) return fail(TI_E_SHAPE, "T = %d must be positive", T);
+  if ((int64_t)seqs * heads > 65535) return fail(TI_E_SHAPE, "%d x %d heads: more than 65535", seqs, heads);
   if (causal_q_len > T) return fail(TI_E_SHAPE, "causal_q_len %d > T %d", causal_q_len, T);
   if (causal_q_len > 0 && S % causal_q_len) return fail(TI_E_SHAPE, "S %d not a multiple of causal_q_len %d", S, causal_q_len);
   if (q_row_stride < D || k_row_stride < D || out_row_stride < D || vt_row_stride < T)
     return fail(TI_E_STRIDE, "row strides must cover a row");
-  const uintptr_t align = (uintptr_t)q | (uintptr_t)k | (uintptr_t)vt | (uintptr_t)out | (uintptr_t)q_batch_stride |
-                          (uintptr_t)q_row_stride | (uintptr_t)k_batch_stride | (uintptr_t)k_row_stride |
-                          (uintptr_t)vt_batch_stride | (uintptr_t)vt_row_stride | (uintptr_t)out_batch_stride |
-                          (uintptr_t)out_row_stride;
-  if (align & 15) return fail(TI_E_STRIDE, "pointers and strides must be multiples of 16 bytes");
+  const uintptr_t align = (uintptr_t)q | (uintptr_t)k | (uintptr_t)out | (uintptr_t)q_seq_stride | (uintptr_t)q_head_stride |
+                          (uintptr_t)q_row_stride | (uintptr_t)k_seq_stride | (uintptr_t)k_head_stride | (uintptr_t)k_row_stride |
+                          (uintptr_t)out_seq_stride | (uintptr_t)out_head_stride | (uintptr_t)out_row_stride;
+  if (align & 15) return fail(TI_E_STRIDE, "pointers and strides of q, k and out must be multiples of 16 bytes");
+  const bool vany = (((uintptr_t)vt | (uintptr_t)vt_seq_stride | (uintptr_t)vt_head_stride | (uintptr_t)vt_row_stride) & 15) != 0;
   const float s2 = score_scale * 1.44269504088896340736f;
   if (!(score_scale > 0.0f) || !(score_scale <= SM_MAX_SCALE))
     return fail(TI_E_COMBO, "score_scale %g outside (0, %g]: the quantised softmax is exact in that range only", (double)score_scale, (double)SM_MAX_SCALE);
   const int64_t lim32 = (int64_t)1 << 31;
-  const bool few_rows = S <= 16 && T <= AD_MAXT && (int64_t)T * k_row_stride < lim32 && (int64_t)AT_D * vt_row_stride < lim32 &&
+  const bool few_rows = S <= 16 && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 && (int64_t)AT_D * vt_row_stride < lim32 &&
                         (int64_t)S * q_row_stride < lim32;
   int rc = check_device();
   if (rc != TI_OK) return rc;
+  const int batch = seqs * heads;
   AttnParams p;
   p.q = q; p.k = k; p.vt = vt; p.out = out;
-  p.sQb = q_batch_stride; p.sQm = q_row_stride; p.sKb = k_batch_stride; p.sKn = k_row_stride;
-  p.sVb = vt_batch_stride; p.sVd = vt_row_stride; p.sOb = out_batch_stride; p.sOm = out_row_stride;
+  p.sQb = q_seq_stride; p.sQh = q_head_stride; p.sQm = q_row_stride;
+  p.sKb = k_seq_stride; p.sKh = k_head_stride; p.sKn = k_row_stride;
+  p.sVb = vt_seq_stride; p.sVh = vt_head_stride; p.sVd = vt_row_stride;
+  p.sOb = out_seq_stride; p.sOh = out_head_stride; p.sOm = out_row_stride;
   p.S = S; p.T = T; p.causal_q_len = causal_q_len;
   p.qk_alpha = qk_alpha; p.s2 = s2; p.pv_alpha = pv_alpha;
   p.nblk = (S + AT_ROWS - 1) / AT_ROWS;
-  p.batch = batch;
+  p.batch = batch; p.heads = heads;
+  const hipStream_t st = (hipStream_t)stream;
   if (few_rows) {
     // spread a head over as many workgroups as keep the launch within one round of the 256 CUs
     // (measured, 40 heads x 16 rows x 2048 keys: 18.9 / 15.3 / 13.6 us for 1 / 2 / 4 workgroups per head,
@@ -570,16 +619,27 @@ extern "C" int ti_attention_i8(const int8_t* q, int64_t q_batch_stride, int64_t 
     int dbw = 8;
     while (dbw > 1 && (int64_t)batch * (16 / dbw) <= 256) dbw /= 2;
     const dim3 grid((unsigned)(batch * (8 / dbw))), block(AD_WAVES * 64);
-    const hipStream_t st = (hipStream_t)stream;
-#define TI_AD_LAUNCH(C) \
-    (dbw == 8 ? attention_decode_i8_kernel<C, 8><<<grid, block, 0, st>>>(p) : dbw == 4 ? attention_decode_i8_kernel<C, 4><<<grid, block, 0, st>>>(p) \
-     : dbw == 2 ? attention_decode_i8_kernel<C, 2><<<grid, block, 0, st>>>(p) : attention_decode_i8_kernel<C, 1><<<grid, block, 0, st>>>(p))
-    if (T <= 1024) TI_AD_LAUNCH(4);
-    else if (T <= 2048) TI_AD_LAUNCH(8);
-    else TI_AD_LAUNCH(16);
+#define TI_AD_LAUNCH(C, V) \
+    (dbw == 8 ? attention_decode_i8_kernel<C, 8, V><<<grid, block, 0, st>>>(p) : dbw == 4 ? attention_decode_i8_kernel<C, 4, V><<<grid, block, 0, st>>>(p) \
+     : dbw == 2 ? attention_decode_i8_kernel<C, 2, V><<<grid, block, 0, st>>>(p) : attention_decode_i8_kernel<C, 1, V><<<grid, block, 0, st>>>(p))
+    if (T <= 1024) vany ? TI_AD_LAUNCH(4, true) : TI_AD_LAUNCH(4, false);
+    else if (T <= 2048) vany ? TI_AD_LAUNCH(8, true) : TI_AD_LAUNCH(8, false);
+    else vany ? TI_AD_LAUNCH(16, true) : TI_AD_LAUNCH(16, false);
 #undef TI_AD_LAUNCH
     return launch_status("attention_decode_i8_kernel");
   }
-  attention_i8_kernel<<<dim3((unsigned)(p.nblk * batch)), dim3(256), 0, (hipStream_t)stream>>>(p);
+  const dim3 grid((unsigned)(p.nblk * batch));
+  if (vany) attention_i8_kernel<true><<<grid, dim3(256), 0, st>>>(p);
+  else attention_i8_kernel<false><<<grid, dim3(256), 0, st>>>(p);
   return launch_status("attention_i8_kernel");
+}
+
+extern "C" int ti_attention_i8(const int8_t* q, int64_t q_batch_stride, int64_t q_row_stride, const int8_t* k,
+                               int64_t k_batch_stride, int64_t k_row_stride, const int8_t* vt,
+                               int64_t vt_batch_stride, int64_t vt_row_stride, int8_t* out, int64_t out_batch_stride,
+                               int64_t out_row_stride, int batch, int S, int T, int D, float qk_alpha,
+                               float score_scale, float pv_alpha, int causal_q_len, void* stream) {
+  return ti_attention_i8_heads(q, 0, q_batch_stride, q_row_stride, k, 0, k_batch_stride, k_row_stride, vt, 0, vt_batch_stride,
+                               vt_row_stride, out, 0, out_batch_stride, out_row_stride, batch == 0 ? 0 : 1, batch, S, T, D,
+                               qk_alpha, score_scale, pv_alpha, causal_q_len, stream);
 }

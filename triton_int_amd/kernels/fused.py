@@ -209,22 +209,30 @@ def attention_i8(q, k, vt, qk_alpha, score_scale, pv_alpha, causal_q_len=0, out=
     registers (reference: the same three steps are separate launches, kernels/bmm.py:576-612 twice
     plus the caller's softmax).  q [BH,S,128], k [BH,T,128], vt [BH,128,T] int8 with unit stride
     along the last dimension; `out` may be any int8 [BH,S,128] view with unit last stride (e.g. the
-    head-merged [S, heads, 128] layout).  Scalars are python floats."""
+    head-merged [S, heads, 128] layout).  All four may be 4-D instead, [B,heads,...] views with any
+    strides of the two leading dimensions: all sequences in one launch.  Scalars are python floats."""
     L.require_cuda(q, k, vt, out)
     assert q.dtype == torch.int8 and k.dtype == torch.int8 and vt.dtype == torch.int8, "operands must be int8"
-    assert q.dim() == 3 and k.dim() == 3 and vt.dim() == 3, "q, k, vt must be 3-D"
-    BH, S, D = q.shape
-    T = k.shape[1]
-    assert k.shape == (BH, T, D) and vt.shape == (BH, D, T), "Incompatible dimensions"
-    assert q.stride(2) == 1 and k.stride(2) == 1 and vt.stride(2) == 1, "unit stride along the last dimension"
+    assert q.dim() in (3, 4) and k.dim() == q.dim() and vt.dim() == q.dim(), "q, k, vt must be all 3-D or all 4-D"
+    lead = q.shape[:-2]
+    S, D = q.shape[-2:]
+    T = k.shape[-2]
+    assert k.shape == (*lead, T, D) and vt.shape == (*lead, D, T), "Incompatible dimensions"
+    # a T of 1 leaves the last stride of vt undefined
+    assert q.stride(-1) == 1 and k.stride(-1) == 1 and (vt.stride(-1) == 1 or T == 1), "unit stride along the last dimension"
     if out is None:
-        out = torch.empty((BH, S, D), dtype=torch.int8, device=q.device)
-    assert out.dtype == torch.int8 and tuple(out.shape) == (BH, S, D) and out.stride(2) == 1
+        out = torch.empty((*lead, S, D), dtype=torch.int8, device=q.device)
+    assert out.dtype == torch.int8 and out.shape == q.shape and out.stride(-1) == 1
+
+    def strides(t):
+        st = t.stride()
+        return (0, *st[:2]) if t.dim() == 3 else st[:3]
+
+    B, heads = (1, lead[0]) if q.dim() == 3 else lead
     with L.on_device(q.device):
-        rc = L.lib().ti_attention_i8(L.ptr(q), q.stride(0), q.stride(1), L.ptr(k), k.stride(0), k.stride(1),
-                                     L.ptr(vt), vt.stride(0), vt.stride(1), L.ptr(out), out.stride(0), out.stride(1),
-                                     BH, S, T, D, float(qk_alpha), float(score_scale), float(pv_alpha),
-                                     int(causal_q_len), L.current_stream(q.device))
+        rc = L.lib().ti_attention_i8_heads(q.data_ptr(), *strides(q), k.data_ptr(), *strides(k), vt.data_ptr(), *strides(vt),
+                                           out.data_ptr(), *strides(out), B, heads, S, T, D, float(qk_alpha),
+                                           float(score_scale), float(pv_alpha), int(causal_q_len), L.current_stream(q.device))
     L.check(rc, "ti_attention_i8")
     return out
 

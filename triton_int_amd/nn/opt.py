@@ -130,43 +130,46 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
             qkv = qkv.view(1, S, 3 * H)
         else:
             qkv = linear_group_a8_w8_b8_o8(h8, w3, b3, a3, s3, 3)                   # [B,S,3H] int8
-        q = self._heads(qkv[..., :H], B, S)
-        k_new = self._heads(qkv[..., H:2 * H], B, S)
+        heads, D = self.heads, self.head_dim
         v = qkv[..., 2 * H:]                                                       # [B,S,H] int8, row pitch 3H
         mark("qkv_3x_linear_o8")
+        T = S if kv_cache is None else kv_cache[0].shape[1]
+        # few query rows (decode) against up to 4096 keys run the attention kernel's one-pass form
+        fused = (self.fused_attention and (S >= self.fused_attention_min_queries or (S <= 16 and T <= 4096))
+                 and D == 128 and self.score_scale > 0.0)
         if kv_cache is None:
-            k_all = k_new
-            vt_all = torch.empty((B * self.heads, self.head_dim, S), dtype=torch.int8, device=hidden.device)
+            # rows of V^T padded to a multiple of 16 bytes: the attention kernel reads them in 16-byte pieces
+            vt_all = torch.empty((B * heads, D, (S + 15) // 16 * 16), dtype=torch.int8, device=hidden.device)[:, :, :S]
             # V^T of every head of a batch in one transpose: [S, heads*D] -> [heads*D, S]
             for b in range(B):
-                transpose_i8(v[b], out=vt_all[b * self.heads:(b + 1) * self.heads].view(H, S))
+                transpose_i8(v[b], out=vt_all[b * heads:(b + 1) * heads].view(H, S))
+            k_all = None
         else:
             # the new K rows and V^T columns go into the last S slots of the cache, one launch per batch
             k_all, vt_all = kv_cache
             if appended:
                 pass
-            elif k_all.is_contiguous() and vt_all.is_contiguous() and self.head_dim % 16 == 0:
+            elif k_all.is_contiguous() and vt_all.is_contiguous() and D % 16 == 0:
                 for b in range(B):
-                    hs = slice(b * self.heads, (b + 1) * self.heads)
+                    hs = slice(b * heads, (b + 1) * heads)
                     kv_append_i8(qkv[b, :, H:2 * H], v[b], k_all[hs], vt_all[hs])
             else:
-                T = k_all.shape[1]
-                k_all[:, T - S:, :] = k_new
+                k_all[:, T - S:, :] = self._heads(qkv[..., H:2 * H], B, S)
                 for b in range(B):
-                    transpose_i8(v[b], out=vt_all[b * self.heads:(b + 1) * self.heads].view(H, T)[:, T - S:])
+                    transpose_i8(v[b], out=vt_all[b * heads:(b + 1) * heads].view(H, T)[:, T - S:])
         mark("kv_append_v_transpose")
-        T = k_all.shape[1]
         ctx = torch.empty((B, S, H), dtype=torch.int8, device=hidden.device)
-        # 16 or fewer query rows (decode) against up to 4096 keys run the kernel's one-workgroup-per-head form
-        fused = (self.fused_attention and (S >= self.fused_attention_min_queries or (S <= 16 and T <= 4096))
-                 and self.head_dim == 128 and T % 16 == 0 and self.score_scale > 0.0)
-        scores = probs = None
+        q = scores = probs = None
+        if not fused or _trace is not None:
+            q = self._heads(qkv[..., :H], B, S)
+            if k_all is None:
+                k_all = self._heads(qkv[..., H:2 * H], B, S)
         if fused:
-            for b in range(B):
-                hs = slice(b * self.heads, (b + 1) * self.heads)
-                attention_i8(q[hs], k_all[hs], vt_all[hs], self.qk_alpha, self.score_scale, self.pv_alpha,
-                             causal_q_len=S if self.causal else 0,
-                             out=ctx[b].view(S, self.heads, self.head_dim).transpose(0, 1))
+            # every operand as [B, heads, rows, D] views: all sequences in one launch
+            by_head = lambda t: t.view(B, S, heads, D).transpose(1, 2)
+            attention_i8(by_head(qkv[..., :H]), by_head(qkv[..., H:2 * H]) if kv_cache is None else k_all.unflatten(0, (B, heads)),
+                         vt_all.unflatten(0, (B, heads)), self.qk_alpha, self.score_scale, self.pv_alpha,
+                         causal_q_len=S if self.causal else 0, out=by_head(ctx))
             mark("attention_i8_fused")
         else:
             scores = bmm_s8t_s8n_s8t(q, k_all, self.qk_alpha)                       # [B*heads, S, T] int8
@@ -176,8 +179,8 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
             # P.V with the head merge folded into the output strides: head h of batch b writes columns
             # h*D .. h*D+D of row (b, s) of a [B,S,H] tensor
             for b in range(B):
-                out_view = ctx[b].view(S, self.heads, self.head_dim).transpose(0, 1)   # [heads, S, D] strided
-                bmm_s8t_s8n_s8t(probs[b * self.heads:(b + 1) * self.heads], vt_all[b * self.heads:(b + 1) * self.heads],
+                out_view = ctx[b].view(S, heads, D).transpose(0, 1)                # [heads, S, D] strided
+                bmm_s8t_s8n_s8t(probs[b * heads:(b + 1) * heads], vt_all[b * heads:(b + 1) * heads],
                                 self.pv_alpha, out=out_view)
             mark("pv_bmm_o8")
         acc = self.out_proj(ctx)                                                    # int32 [B,S,H]
