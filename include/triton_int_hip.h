@@ -330,6 +330,17 @@ int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw,
                      void* stream);
 
 /*
+ * The same for the rows of `seqs` sequences (M / seqs rows each, one sequence after the other) and caches
+ * that may be views of longer ones: row m is position s = m % (M / seqs) of sequence q = m / (M / seqs);
+ * with h = q * heads + head, k goes to k_dst[h * k_head_stride + s * k_row_stride + d] and v to
+ * vt_dst[(h * D + d) * vt_row_stride + s].
+ */
+int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+                          const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
+                          int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst,
+                          int64_t vt_row_stride, int D, void* stream);
+
+/*
  * Appends S new positions to an int8 KV cache in one launch: K [S, heads*D] (row stride
  * k_src_row_stride) is copied to k_dst[h][s][d] = k_dst + h * k_head_stride + s * D + d (k_dst points at
  * the first new slot of head 0 in a [heads, T, D] cache, k_head_stride = T * D), and V [S, heads*D]
@@ -340,6 +351,14 @@ int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw,
 int ti_kv_append_i8(const int8_t* k_src, int64_t k_src_row_stride, const int8_t* v_src, int64_t v_src_row_stride,
                     int8_t* k_dst, int64_t k_head_stride, int8_t* vt_dst, int64_t vt_row_stride,
                     int S, int heads, int D, void* stream);
+
+/*
+ * The same for `seqs` sequences in one launch, source rows q * S + s, cache addresses as in
+ * ti_qkv_decode_i8_seqs.  k_dst = NULL: only V^T is written (a prompt without a cache).
+ */
+int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const int8_t* v_src, int64_t v_src_row_stride,
+                         int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
+                         int seqs, int S, int heads, int D, void* stream);
 
 /*
  * One attention block without the score round trip through memory:

@@ -45,3 +45,31 @@ def test_attention_i8_of_several_sequences_in_one_launch(B, heads, S, T):
     for b in range(B):
         want = fused.attention_i8(q[b], k[b], vt[b], 2e-3, 0.1, 0.02, causal_q_len=S)
         assert torch.equal(out[b].transpose(0, 1), want)
+
+
+@pytest.mark.parametrize("B,S,heads,D,K,T,room", [(16, 1, 2, 128, 1024, 53, 64), (3, 5, 5, 16, 1040, 37, 37), (1, 16, 3, 128, 2064, 100, 128)])
+def test_qkv_decode_of_several_sequences_into_views_of_longer_caches(B, S, heads, D, K, T, room):
+    """Projections equal to the grouped launch's; caches equal to torch indexing, the rest of them untouched.
+    The append kernel alone on the same projections: the same caches."""
+    from triton_int_amd.kernels import fused, linear
+
+    g = torch.Generator(device="cuda").manual_seed(B * 10 + T)
+    i8 = lambda *shape: torch.randint(-127, 128, shape, dtype=torch.int8, device="cuda", generator=g)
+    H = heads * D
+    a, w3, b3 = i8(B * S, K), i8(3 * H, K), i8(3 * H)
+    al = torch.full((3,), 40.0 / (73.0 * 73.0 * K ** 0.5), device="cuda")
+    be = torch.full((3,), 0.1, device="cuda")
+    k0, vt0 = i8(B * heads, room, D), i8(B * heads, D, room)
+    want = linear.linear_group_a8_w8_b8_o8(a, w3, b3, al, be, 3)
+    want_k, want_vt = k0.clone(), vt0.clone()
+    want_k[:, T - S:T] = want[:, H:2 * H].reshape(B, S, heads, D).transpose(1, 2).reshape(B * heads, S, D)
+    want_vt[:, :, T - S:T] = want[:, 2 * H:].reshape(B, S, heads, D).permute(0, 2, 3, 1).reshape(B * heads, D, S)
+    k, vt = k0.clone(), vt0.clone()
+    got = linear.linear_qkv_decode_a8_w8_b8_o8(a, w3, b3, al, be, k[:, :T], vt[:, :, :T], seqs=B)
+    assert torch.equal(got, want) and torch.equal(k, want_k) and torch.equal(vt, want_vt)
+    k, vt = k0.clone(), vt0.clone()
+    fused.kv_append_i8(want[:, H:2 * H], want[:, 2 * H:], k[:, :T], vt[:, :, :T], seqs=B)
+    assert torch.equal(k, want_k) and torch.equal(vt, want_vt)
+    vt = vt0.clone()
+    fused.kv_append_i8(None, want[:, 2 * H:], None, vt[:, :, :T], seqs=B)
+    assert torch.equal(vt, want_vt)

@@ -53,12 +53,13 @@ struct GemmParams {
   // fp32 outputs of gemm_rows4_kernel and of the persistent kernels' fp32 epilogue: C = epilogue value + resid[m * resid_rs + n]
   const float* resid;
   int64_t resid_rs;
-  // int8 outputs of a grouped q/k/v launch of gemm_rows4_kernel only: batch 1 (k) also goes to
-  // kv_k[head * kv_k_hs + m * kv_D + d], batch 2 (v) to kv_vt[(head * kv_D + d) * kv_vt_rs + m]
+  // int8 outputs of a grouped q/k/v launch of gemm_rows4_kernel only.  Row m is position s = m % kv_S of
+  // sequence q = m / kv_S, h = q * heads + head: batch 1 (k) also goes to kv_k[h * kv_k_hs + s * kv_k_rs + d],
+  // batch 2 (v) to kv_vt[(h * kv_D + d) * kv_vt_rs + s]
   int8_t* kv_k;
   int8_t* kv_vt;
-  int64_t kv_k_hs, kv_vt_rs;
-  int kv_D;
+  int64_t kv_k_hs, kv_k_rs, kv_vt_rs;
+  int kv_D, kv_S;
   // split K (gemm_mfma_ws_kernel, batch == 1): a tile's k-tiles are dealt to `splits` work items of
   // kt_split k-tiles each (the last takes what is left); the items leave their int32 sums in
   // sk_partial, and the item of a tile that finishes last adds them up and stores the tile.
@@ -1939,11 +1940,13 @@ __device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char*
       // the kernel passes it along)
       if (kp->kv_k) {
         const int D = kp->kv_D, head = n0 / D, d = n0 - head * D;
+        const int seq = row / kp->kv_S, pos = row - seq * kp->kv_S;
         if (bz == 1) {
-          *(unsigned*)(kp->kv_k + (int64_t)head * kp->kv_k_hs + (int64_t)row * D + d) = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
+          *(unsigned*)(kp->kv_k + ((int64_t)seq * (N / D) + head) * kp->kv_k_hs + (int64_t)pos * kp->kv_k_rs + d) =
+              b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
         } else if (bz == 2) {
 #pragma unroll
-          for (int i = 0; i < R4_RG; ++i) kp->kv_vt[(int64_t)(n0 + i) * kp->kv_vt_rs + row] = (int8_t)b[i];
+          for (int i = 0; i < R4_RG; ++i) kp->kv_vt[((int64_t)seq * N + n0 + i) * kp->kv_vt_rs + pos] = (int8_t)b[i];
         }
       }
     }
@@ -2819,7 +2822,7 @@ int ti_bmm_i8_config(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, con
   p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
   p.bias_bs = 0; p.scale_bs = 0;
   p.resid = nullptr; p.resid_rs = 0;
-  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_vt_rs = 0; p.kv_D = 1;
+  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   return ti::run(p, config, (hipStream_t)stream);
 }
@@ -2842,19 +2845,20 @@ int ti_bmm_i8_grouped(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, co
   p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
   p.bias_bs = bias_batch_stride; p.scale_bs = scale_batch_stride;
   p.resid = nullptr; p.resid_rs = 0;
-  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_vt_rs = 0; p.kv_D = 1;
+  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   return ti::run(p, config, (hipStream_t)stream);
 }
 
-int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
-                     const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int M, int N, int K,
-                     int8_t* k_dst, int64_t k_head_stride, int8_t* vt_dst, int64_t vt_row_stride, int D,
-                     void* stream) {
+int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+                          const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
+                          int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
+                          int D, void* stream) {
   using namespace ti;
+  if (seqs < 1 || M % seqs) return fail(TI_E_SHAPE, "%d rows are not %d sequences of one length", M, seqs);
   if (M > 16 || K < 1024 || D <= 0 || (D & 15) || N % D) return fail(TI_E_COMBO, "needs M <= 16, K >= 1024, D %% 16 == 0, N %% D == 0");
   if (!k_dst || !vt_dst) return fail(TI_E_NULL, "k_dst and vt_dst are required");
-  if (((uintptr_t)k_dst & 3) || (k_head_stride & 3)) return fail(TI_E_STRIDE, "k_dst and its head stride must be multiples of 4 bytes");
+  if (((uintptr_t)k_dst & 3) || (k_head_stride & 3) || (k_row_stride & 3)) return fail(TI_E_STRIDE, "k_dst and its strides must be multiples of 4 bytes");
   GemmParams p;
   p.A = A; p.B = W; p.C = C;
   p.sAb = 0; p.sAm = lda; p.sAk = 1;
@@ -2867,7 +2871,8 @@ int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw,
   p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
   p.bias_bs = N; p.scale_bs = 1;
   p.resid = nullptr; p.resid_rs = 0;
-  p.kv_k = k_dst; p.kv_vt = vt_dst; p.kv_k_hs = k_head_stride; p.kv_vt_rs = vt_row_stride; p.kv_D = D;
+  p.kv_k = k_dst; p.kv_vt = vt_dst; p.kv_k_hs = k_head_stride; p.kv_k_rs = k_row_stride; p.kv_vt_rs = vt_row_stride;
+  p.kv_D = D; p.kv_S = M > 0 ? M / seqs : 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   int rc = validate(p);
   if (rc != TI_OK) return rc;
@@ -2878,6 +2883,14 @@ int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw,
   const int cfg = pick_config(p, &splits);
   if (!g_configs[cfg].rows4) return fail(TI_E_COMBO, "operands not eligible for the decode kernel (16-byte aligned, K-contiguous)");
   return run(p, cfg, (hipStream_t)stream);
+}
+
+int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+                     const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int M, int N, int K,
+                     int8_t* k_dst, int64_t k_head_stride, int8_t* vt_dst, int64_t vt_row_stride, int D,
+                     void* stream) {
+  return ti_qkv_decode_i8_seqs(A, lda, W, ldw, bias, alpha3, beta3, C, ldc, 1, M, N, K, k_dst, k_head_stride, D, vt_dst,
+                               vt_row_stride, D, stream);
 }
 
 int ti_bmm_i8(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, const int8_t* B, int64_t sBb, int64_t sBn,
@@ -2904,7 +2917,7 @@ int ti_bmm_i8_static_scratch(const int8_t* A, int64_t sAb, int64_t sAm, int64_t 
   p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
   p.bias_bs = 0; p.scale_bs = 0;
   p.resid = nullptr; p.resid_rs = 0;
-  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_vt_rs = 0; p.kv_D = 1;
+  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   return ti::run(p, config, (hipStream_t)stream, true);
 }
@@ -2924,7 +2937,7 @@ int ti_linear_i8_residual_f32(const int8_t* A, int64_t lda, const int8_t* W, int
   p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
   p.bias_bs = 0; p.scale_bs = 0;
   p.resid = nullptr; p.resid_rs = 0;
-  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_vt_rs = 0; p.kv_D = 1;
+  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   return ti::run_with_residual(p, residual, ldr, (hipStream_t)stream);
 }
@@ -2947,7 +2960,7 @@ int ti_gemm_plan(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, const i
   p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
   p.bias_bs = 0; p.scale_bs = 0;
   p.resid = nullptr; p.resid_rs = 0;
-  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_vt_rs = 0; p.kv_D = 1;
+  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   ti::LaunchPlan lp;
   const int rc = ti::run(p, config, nullptr, static_scratch != 0, &lp);

@@ -259,19 +259,30 @@ def quantize_per_token_absmax(t):
     return q.view(t.shape), scale.view(*t.shape[:-1], 1)
 
 
-def kv_append_i8(k_new, v_new, k_cache, vt_cache):
-    """Write S new positions into the last S slots of an int8 KV cache with one launch.
-    k_new, v_new: int8 [S, heads*D] (unit column stride; e.g. column slices of a fused q/k/v
-    projection); k_cache int8 [heads, T, D]; vt_cache int8 [heads, D, T].  Replaces
+def kv_append_i8(k_new, v_new, k_cache, vt_cache, seqs=1):
+    """Write S new positions of each of `seqs` sequences into the last S slots of an int8 KV cache with one
+    launch.  k_new, v_new: int8 [seqs*S, heads*D] (unit column stride; e.g. column slices of a fused q/k/v
+    projection); k_cache int8 [seqs*heads, T, D]; vt_cache int8 [seqs*heads, D, T], both contiguous or views
+    of longer caches.  k_cache = None (k_new is then ignored) writes V^T only.  Replaces
     `k_cache[:, T-S:, :] = k_new.view(S, heads, D).transpose(0, 1)` and the V transpose."""
-    L.require_cuda(k_new, v_new, k_cache, vt_cache)
-    heads, T, D = k_cache.shape
-    S, H = k_new.shape
-    assert H == heads * D and tuple(v_new.shape) == (S, H) and tuple(vt_cache.shape) == (heads, D, T) and S <= T
-    assert k_new.dtype == v_new.dtype == k_cache.dtype == vt_cache.dtype == torch.int8
-    assert k_new.stride(1) == 1 and v_new.stride(1) == 1 and k_cache.is_contiguous() and vt_cache.is_contiguous()
-    with L.on_device(k_new.device):
-        rc = L.lib().ti_kv_append_i8(L.ptr(k_new), k_new.stride(0), L.ptr(v_new), v_new.stride(0),
-                                     k_cache.data_ptr() + (T - S) * D, T * D, vt_cache.data_ptr() + (T - S), T,
-                                     S, heads, D, L.current_stream(k_new.device))
+    L.require_cuda(v_new, k_cache, vt_cache)
+    BH, D, T = vt_cache.shape
+    M, H = v_new.shape
+    S, heads = M // seqs, BH // seqs
+    vs = vt_cache.stride()
+    assert H == heads * D and seqs * S == M and seqs * heads == BH and S <= T
+    assert v_new.dtype == vt_cache.dtype == torch.int8
+    assert v_new.stride(1) == 1 and (vs[2] == 1 or T == 1) and (vs[0] == D * vs[1] or BH == 1), "V^T rows one pitch apart across the heads"
+    k_ptr = k_rs = kc_ptr = k_hs = k_ps = 0
+    if k_cache is not None:
+        L.require_cuda(k_new)
+        ks = k_cache.stride()
+        assert k_new.shape == (M, H) and k_cache.shape == (BH, T, D) and k_new.dtype == k_cache.dtype == torch.int8
+        assert k_new.stride(1) == 1 and ks[2] == 1
+        k_ptr, k_rs = k_new.data_ptr(), k_new.stride(0) if M > 1 else H
+        kc_ptr, k_hs, k_ps = k_cache.data_ptr() + (T - S) * ks[1], ks[0], ks[1]
+    with L.on_device(v_new.device):
+        rc = L.lib().ti_kv_append_i8_seqs(k_ptr, k_rs, v_new.data_ptr(), v_new.stride(0) if M > 1 else H, kc_ptr, k_hs, k_ps,
+                                          vt_cache.data_ptr() + (T - S), vs[1], seqs, S, heads, D,
+                                          L.current_stream(v_new.device))
     L.check(rc, "ti_kv_append_i8")

@@ -108,6 +108,21 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
             return t.view(S, self.heads, self.head_dim).transpose(0, 1)
         return t.view(B, S, self.heads, self.head_dim).transpose(1, 2).reshape(B * self.heads, S, self.head_dim)
 
+    def _append(self, k_new, v_new, k_all, vt_all):
+        """k_new, v_new int8 [B,S,H] into the last S slots of K [B*heads,T,D] (unless None) and of V^T
+        [B*heads,D,T]: one launch for head dimensions that are multiples of 16 and caches whose rows have
+        unit stride and one pitch."""
+        B, S, H = v_new.shape
+        heads, D, T = self.heads, self.head_dim, vt_all.shape[2]
+        vs = vt_all.stride()
+        if D % 16 == 0 and (k_all is None or k_all.stride(2) == 1) and (vs[0] == D * vs[1] or B * heads == 1):
+            kv_append_i8(k_new.view(B * S, H), v_new.view(B * S, H), k_all, vt_all, seqs=B)
+            return
+        if k_all is not None:
+            k_all[:, T - S:, :] = self._heads(k_new, B, S)
+        for b in range(B):
+            transpose_i8(v_new[b], out=vt_all[b * heads:(b + 1) * heads].view(H, T)[:, T - S:])
+
     @torch.no_grad()
     def forward(self, hidden, kv_cache=None, _trace=None, _mark=None):
         """hidden fp32 [B,S,H].  kv_cache = (K int8 [B*heads, T, D], V^T int8 [B*heads, D, T]) holds the
@@ -122,12 +137,12 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         mark("ln1_layernorm_q")
         w3, b3, a3, s3 = self._qkv_pack()
         qkv = None
-        if kv_cache is not None and B == 1 and S <= 16:
+        if kv_cache is not None and B * S <= 16:
             # decode: projections and KV-cache append in one launch
-            qkv = linear_qkv_decode_a8_w8_b8_o8(h8.view(S, H), w3, b3, a3, s3, kv_cache[0], kv_cache[1])
+            qkv = linear_qkv_decode_a8_w8_b8_o8(h8.view(B * S, H), w3, b3, a3, s3, kv_cache[0], kv_cache[1], seqs=B)
         appended = qkv is not None
         if appended:
-            qkv = qkv.view(1, S, 3 * H)
+            qkv = qkv.view(B, S, 3 * H)
         else:
             qkv = linear_group_a8_w8_b8_o8(h8, w3, b3, a3, s3, 3)                   # [B,S,3H] int8
         heads, D = self.heads, self.head_dim
@@ -140,23 +155,12 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         if kv_cache is None:
             # rows of V^T padded to a multiple of 16 bytes: the attention kernel reads them in 16-byte pieces
             vt_all = torch.empty((B * heads, D, (S + 15) // 16 * 16), dtype=torch.int8, device=hidden.device)[:, :, :S]
-            # V^T of every head of a batch in one transpose: [S, heads*D] -> [heads*D, S]
-            for b in range(B):
-                transpose_i8(v[b], out=vt_all[b * heads:(b + 1) * heads].view(H, S))
             k_all = None
         else:
-            # the new K rows and V^T columns go into the last S slots of the cache, one launch per batch
             k_all, vt_all = kv_cache
-            if appended:
-                pass
-            elif k_all.is_contiguous() and vt_all.is_contiguous() and D % 16 == 0:
-                for b in range(B):
-                    hs = slice(b * heads, (b + 1) * heads)
-                    kv_append_i8(qkv[b, :, H:2 * H], v[b], k_all[hs], vt_all[hs])
-            else:
-                k_all[:, T - S:, :] = self._heads(qkv[..., H:2 * H], B, S)
-                for b in range(B):
-                    transpose_i8(v[b], out=vt_all[b * heads:(b + 1) * heads].view(H, T)[:, T - S:])
+        if not appended:
+            # the new K rows and V^T columns go into the last S slots of the cache
+            self._append(qkv[..., H:2 * H], v, k_all, vt_all)
         mark("kv_append_v_transpose")
         ctx = torch.empty((B, S, H), dtype=torch.int8, device=hidden.device)
         q = scores = probs = None
