@@ -372,8 +372,8 @@ int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const in
  * The scalars are host floats.  The int8 scores are the BMM's and the probabilities ti_softmax_q's
  * bit for bit (a row's exponentials are summed as integers, so the order in which the keys are
  * visited does not matter): the output equals the three-launch chain's exactly.
- * With S <= 16 and T <= 4096 (decode) a one-pass kernel runs instead, one to four workgroups per
- * batch entry.
+ * Launches of few query rows (batch * ceil(S / 16) <= 1024) against T <= 4096 keys run a one-pass kernel,
+ * one to eight workgroups per batch entry and 16 rows.
  * The reference has no fused form (its modules stop at the BMMs, nn/bmm.py:10-74); the
  * three-launch chain remains available and is what this is tested against.
  */

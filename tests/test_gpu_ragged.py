@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("BH,S,T,q_len,pitch", [
     (2, 1, 1, 1, 0), (3, 1, 15, 0, 16), (2, 16, 17, 16, 0), (2, 5, 63, 5, 64), (40, 1, 1531, 1, 2048), (3, 3, 1025, 3, 0),
     (300, 1, 77, 1, 80), (2, 16, 2047, 0, 0), (2, 2, 2049, 2, 4096), (1, 1, 4093, 0, 0),     # few query rows
-    (2, 333, 333, 333, 336), (2, 333, 333, 333, 0), (3, 17, 65, 17, 0), (2, 130, 1007, 0, 1024), (1, 128, 129, 128, 0)])
+    (3, 17, 65, 17, 0), (2, 47, 1000, 47, 0), (2, 130, 1007, 0, 1024), (2, 48, 333, 24, 336), (1, 129, 4096, 129, 4096),  # groups of 16
+    (49, 333, 333, 333, 336), (49, 333, 333, 333, 0), (70, 240, 257, 0, 0), (130, 128, 129, 128, 0), (2, 17, 4097, 17, 0)])  # blocks of 128
 def test_attention_i8_over_any_number_of_keys(BH, S, T, q_len, pitch):
     """Equal to the three-launch chain, bit for bit, whatever the length and the alignment of V^T's rows."""
     from triton_int_amd.kernels import fused

@@ -20,7 +20,7 @@
 // half-wave swaps put a row's keys in order) and feeds them to the P.V MFMAs, so P never goes
 // through memory.
 //
-// (Blocks of 16 or fewer query rows take attention_decode_i8_kernel further down instead.)
+// (Launches of few query rows take attention_decode_i8_kernel further down instead.)
 //
 // Workgroup = 4 waves = 128 query rows of one head; a wave owns 32 rows.  K and V^T are staged
 // through LDS in tiles of 64 keys, double-buffered, one barrier per tile.  Causal masking skips
@@ -386,17 +386,17 @@ __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
 }
 
 
-// ---- few query rows (decode): one workgroup per head ------------------------------------------------
+// ---- few query rows (decode, short chunks of a prompt): one workgroup per head and 16 rows ----------
 //
-// With 16 or fewer query rows per head a head's whole attention fits one workgroup: 16 waves, one
-// pass.  Wave w computes the scores of the 16-key chunks w, w + 16, ... with 16x16x64 MFMAs (K rows
+// 16 query rows of a head's attention fit one workgroup: 16 waves, one pass.  Wave w computes the scores
+// of the 16-key chunks w, w + 16, ... with 16x16x64 MFMAs (K rows
 // loaded from memory straight into the operand layout: 16 rows x 64 bytes per instruction) and keeps
 // them in registers; row maximum and sum go through LDS; the int8 probabilities are written to LDS in
 // key order ([16 queries][T]), from where every wave reads them back as MFMA operands for P.V: wave w
 // owns 16 of the 128 output columns (V^T rows, also loaded straight into the operand layout) and
 // one half of the 64-key groups; the two halves meet in LDS.  The arithmetic is that of the three
 // kernels (score quantisation, exponent against the row maximum, 127 / sum, context quantisation);
-// only the order of a row's sum differs.
+// only the order of a row's sum differs.  More rows are more workgroups, which share K and V^T in L2.
 constexpr int AD_WAVES = 16;
 constexpr int AD_MAXT = 4096;
 
@@ -422,7 +422,9 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   // the workgroups of a head are p.batch apart: with a batch that is a multiple of 8 they run on the
   // same XCD and share its L2 for K
   const int bh = blockIdx.x % p.batch;
-  const int dbase = (blockIdx.x / p.batch) * DBW;
+  const int part = blockIdx.x / p.batch, ngrp = (p.S + 15) >> 4;
+  const int row0 = (part % ngrp) * 16;  // this workgroup's 16 query rows
+  const int dbase = (part / ngrp) * DBW;
   const int OOB = 0x7ffffff0;
   const float MAGIC = 12582912.0f;
   const int seq = bh / p.heads, head = bh - seq * p.heads;
@@ -434,20 +436,23 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   // the last chunk of an aligned row may cross T (see attention_i8_kernel)
   const __amdgpu_buffer_rsrc_t rV =
       __builtin_amdgcn_make_buffer_rsrc((void*)vb, 0, (int)((AT_D - 1) * p.sVd + ((p.T + 15) & ~15)), 0x00020000);
+  // keys that any of the rows sees (under a causal mask the later ones are not even loaded)
+  const int rlast = min(row0 + 15, p.S - 1);
+  const int keys = p.causal_q_len > 0 && row0 / p.causal_q_len == rlast / p.causal_q_len ? attn_limit(p, rlast) : p.T;
   auto load_v = [&](int d, int col) -> v4i {
     if constexpr (VANY) return load_keys_any(vb + (int64_t)d * p.sVd, col, p.T);
-    else return __builtin_amdgcn_raw_buffer_load_b128(rV, col < p.T ? d * (int)p.sVd + col : OOB, 0, 0);
+    else return __builtin_amdgcn_raw_buffer_load_b128(rV, col < keys ? d * (int)p.sVd + col : OOB, 0, 0);
   };
-  const int NCH = (p.T + 15) >> 4;  // 16-key chunks; rows of K past T read as zeros and are masked
-  const int NG = (p.T + 63) >> 6;   // 64-key groups
+  const int NCH = (keys + 15) >> 4;  // 16-key chunks; rows of K past T read as zeros and are masked
+  const int NG = (keys + 63) >> 6;   // 64-key groups
   const int db = dbase + wave % DBW, kh = wave / DBW;
 
   // ---- scores: f = the int8 score as a float, -inf where masked or beyond T
   v4i qf[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks)
-    qf[ks] = __builtin_amdgcn_raw_buffer_load_b128(rQ, n < p.S ? n * (int)p.sQm + ks * 64 + kq * 16 : OOB, 0, 0);
-  const int limit = p.causal_q_len > 0 ? min(p.T, (n % p.causal_q_len) + (p.T - p.causal_q_len) + 1) : p.T;
+    qf[ks] = __builtin_amdgcn_raw_buffer_load_b128(rQ, row0 + n < p.S ? (row0 + n) * (int)p.sQm + ks * 64 + kq * 16 : OOB, 0, 0);
+  const int limit = attn_limit(p, row0 + n);
   const float NEG = -__builtin_inff();
   float f[CPW][4];
   constexpr int NB = CPW < 8 ? CPW : (CPW > 8 ? 4 : 8);  // chunks whose K operands are in flight together
@@ -553,7 +558,7 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   }
   if (kh > 0) ctx_red[wave][lane] = o;
   __syncthreads();
-  if (kh == 0 && n < p.S) {
+  if (kh == 0 && row0 + n < p.S) {
 #pragma unroll
     for (int k2 = 1; k2 < KPARTS; ++k2) o += ctx_red[wave + k2 * DBW][lane];
     unsigned b[4];
@@ -563,7 +568,7 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
       v = __builtin_amdgcn_fmed3f(v, -128.0f, 127.0f);
       b[r] = __float_as_uint(v + MAGIC);
     }
-    *(unsigned*)(p.out + (int64_t)seq * p.sOb + (int64_t)head * p.sOh + (int64_t)n * p.sOm + 16 * db + 4 * kq) =
+    *(unsigned*)(p.out + (int64_t)seq * p.sOb + (int64_t)head * p.sOh + (int64_t)(row0 + n) * p.sOm + 16 * db + 4 * kq) =
         __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
   }
 }
@@ -596,7 +601,14 @@ extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int6
   if (!(score_scale > 0.0f) || !(score_scale <= SM_MAX_SCALE))
     return fail(TI_E_COMBO, "score_scale %g outside (0, %g]: the quantised softmax is exact in that range only", (double)score_scale, (double)SM_MAX_SCALE);
   const int64_t lim32 = (int64_t)1 << 31;
-  const bool few_rows = S <= 16 && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 && (int64_t)AT_D * vt_row_stride < lim32 &&
+  // Groups of 16 query rows on attention_decode_i8_kernel as long as they are at most four rounds of the chip
+  // (256 workgroups each), 128-row blocks on attention_i8_kernel beyond.  A group walks the keys once on 16
+  // waves; a block walks them three times on 4 waves, 2.1 us per 64 keys however few blocks there are.
+  // Measured, causal (us, groups / blocks): 32 heads x 64 rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 /
+  // 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81, 64 x 256 x 1064 (1024) 48 / 46,
+  // 160 x 96 x 2048 (960) 83 / 81, 40 x 512 x 2048 (1280) 88 / 81, 160 x 128 x 2048 (1280) 103 / 82.
+  const int64_t groups = (int64_t)seqs * heads * ((S + 15) / 16);
+  const bool few_rows = groups <= 1024 && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 && (int64_t)AT_D * vt_row_stride < lim32 &&
                         (int64_t)S * q_row_stride < lim32;
   int rc = check_device();
   if (rc != TI_OK) return rc;
@@ -617,8 +629,8 @@ extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int6
     // (measured, 40 heads x 16 rows x 2048 keys: 18.9 / 15.3 / 13.6 us for 1 / 2 / 4 workgroups per head,
     // 24 us for 8, which no longer fit one round)
     int dbw = 8;
-    while (dbw > 1 && (int64_t)batch * (16 / dbw) <= 256) dbw /= 2;
-    const dim3 grid((unsigned)(batch * (8 / dbw))), block(AD_WAVES * 64);
+    while (dbw > 1 && groups * (16 / dbw) <= 256) dbw /= 2;
+    const dim3 grid((unsigned)(groups * (8 / dbw))), block(AD_WAVES * 64);
 #define TI_AD_LAUNCH(C, V) \
     (dbw == 8 ? attention_decode_i8_kernel<C, 8, V><<<grid, block, 0, st>>>(p) : dbw == 4 ? attention_decode_i8_kernel<C, 4, V><<<grid, block, 0, st>>>(p) \
      : dbw == 2 ? attention_decode_i8_kernel<C, 2, V><<<grid, block, 0, st>>>(p) : attention_decode_i8_kernel<C, 1, V><<<grid, block, 0, st>>>(p))

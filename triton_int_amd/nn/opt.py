@@ -11,8 +11,9 @@ end-to-end tests: every heavy step is one of the package's HIP kernels, torch on
       scores = BMM_S8T_S8N_S8T(q, k) -> int8                (bmm_s8t_s8n_s8t)
       probs  = softmax_q(scores, causal) -> int8 [0,127]    (ti_softmax_q)
       ctx    = BMM_S8T_S8N_S8T(probs, v^T) -> int8, written head-merged through output strides
-               (with `fused_attention`, the default for 128 or more query positions and for 16 or fewer,
-               these three run as one kernel, ti_attention_i8, and scores / probabilities never reach memory)
+               (with `fused_attention`, the default for 128 or more query positions and for any number of them
+               against up to 4096 keys, these three run as one kernel, ti_attention_i8, and scores / probabilities
+               never reach memory)
       acc    = W8A8B32O32LinearWithoutScaling(ctx) -> int32 (linear_a8_w8_b32_o32)   out_proj
       resid, h8 = DQ_Add_LayerNorm_Q(hidden, acc)           (ti_dq_add_layernorm_q)
       f8     = W8A8BFP32OFP32_GeLu_Q(h8) -> int8            (GEMM + GELU-quant epilogue)   fc1
@@ -48,8 +49,8 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         self.qk_alpha = 1e-3
         self.score_scale = 0.05
         self.pv_alpha = 1.0 / 127.0
-        # one-kernel attention for prefill-sized blocks of queries and for decode-sized ones (16 or fewer
-        # rows per head); the three-launch chain in between (too few workgroups for the block kernel)
+        # one-kernel attention for blocks of queries of this size against any number of keys, for shorter ones
+        # against up to 4096; the three-launch chain otherwise (too few workgroups for the block kernel)
         self.fused_attention = True
         self.fused_attention_min_queries = 128
         # fc2 and the residual add that follows it as one library call (a traced forward keeps them apart
@@ -149,9 +150,10 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         v = qkv[..., 2 * H:]                                                       # [B,S,H] int8, row pitch 3H
         mark("qkv_3x_linear_o8")
         T = S if kv_cache is None else kv_cache[0].shape[1]
-        # few query rows (decode) against up to 4096 keys run the attention kernel's one-pass form
-        fused = (self.fused_attention and (S >= self.fused_attention_min_queries or (S <= 16 and T <= 4096))
-                 and D == 128 and self.score_scale > 0.0)
+        # short blocks of queries against up to 4096 keys run the attention kernel's one-pass form; a traced
+        # forward keeps the three steps of blocks of 17 .. 127 apart so that they can be inspected
+        short = T <= 4096 and (S <= 16 or _trace is None)
+        fused = self.fused_attention and (S >= self.fused_attention_min_queries or short) and D == 128 and self.score_scale > 0.0
         if kv_cache is None:
             # rows of V^T padded to a multiple of 16 bytes: the attention kernel reads them in 16-byte pieces
             vt_all = torch.empty((B * heads, D, (S + 15) // 16 * 16), dtype=torch.int8, device=hidden.device)[:, :, :S]
