@@ -1628,19 +1628,34 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
       if (lane == 0) ticket = atomicAdd(p.sk_counter + rank * NWC + wave, 1);
       ticket = __builtin_amdgcn_readfirstlane(ticket);
       if (ticket != SPL - 1) continue;
-      for (int o = 0; o < SPL; ++o) {
-        if (o == sp) continue;
-        const int theirs = ((rank * SPL + o) * NWC + wave) * WAVE_BYTES + lane * 16;
+      // The other items' sums, 64 registers' worth of loads at a time (several items when an item's part is
+      // small) and all of them issued before the first add: left to itself the compiler waits for every
+      // 16-byte load before it issues the next, 2-byte and 4-byte outputs' kernels alike (64 x 4096 x 16384,
+      // 6 splits, fp32 out: 30.2 -> 21.3 us).
+      constexpr int NB = TM * TN, BPR = NB < 4 ? NB : 4, OPR = 4 / BPR;  // blocks of 32 x 32; blocks and items per round
+      for (int o = 0; o < SPL; o += OPR) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int b0 = 0; b0 < NB; b0 += BPR) {
+          v4i part[OPR][BPR][4];
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
+          for (int d = 0; d < OPR; ++d) {
+            // this item's own sums and items past the last: out of range, zeros
+            const int theirs = o + d == sp || o + d >= SPL ? (int)0x80000000 : ((rank * SPL + o + d) * NWC + wave) * WAVE_BYTES + lane * 16;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rP, theirs + ((i * TN + j) * 4 + q) * 1024, 0, SC1);
-              acc[i][j][4 * q] += (int)v[0]; acc[i][j][4 * q + 1] += (int)v[1];
-              acc[i][j][4 * q + 2] += (int)v[2]; acc[i][j][4 * q + 3] += (int)v[3];
-            }
+            for (int b = 0; b < BPR; ++b)
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                if (b0 + b < NB) part[d][b][q] = __builtin_amdgcn_raw_buffer_load_b128(rP, theirs + ((b0 + b) * 4 + q) * 1024, 0, SC1);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int d = 0; d < OPR; ++d)
+#pragma unroll
+            for (int b = 0; b < BPR; ++b)
+#pragma unroll
+              for (int r = 0; r < 16; ++r)
+                if (b0 + b < NB) acc[(b0 + b) / TN][(b0 + b) % TN][r] += part[d][b][r >> 2][r & 3];
+        }
       }
       if (lane == 0) atomicExch(p.sk_counter + rank * NWC + wave, 0);
     }
