@@ -397,6 +397,32 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
                 assert not bad.any(), f"rows4 {what}: load outside the operand"
         stats["units"] = NU
         return stats
+    if name.endswith("_rowpieces"):
+        # every workgroup of a batch entry: `per` units of 4 weight rows, the whole K in stages of 256 bytes
+        MT, KC = int(re.search(r"_m(\d+)", name).group(1)), 256
+        NU = -(-pr.N // 4)
+        per = -(-NU // pl.grid_x)
+        u0 = np.minimum(NU, np.arange(pl.grid_x, dtype=np.int64) * per)
+        units = np.minimum(NU, u0 + per) - u0
+        assert pr.M <= MT and pl.grid_y == pr.batch and pl.threads == 512
+        assert (units > 0).all() and units.sum() == NU and per <= 20, "the workgroups' units do not cover N exactly once"
+        chunk = np.arange(16, dtype=np.int64)
+        kmax = ((pr.K - chunk * 16 - 1) // KC) * KC  # the last stage in which a chunk is still inside K (negative: never)
+        W = 16 * (-(-per // 4))
+        n0 = u0 * 4
+        w_rows = np.minimum(units * 4, pr.N - n0)
+        for what, rows, ld, base, extent, alloc in (
+                ("activations", np.arange(MT), pr.sAm, np.array([0, (pr.batch - 1) * pr.sAb]), np.full(2, (pr.M - 1) * pr.sAm + pr.K), pr.a_bytes()),
+                ("weights", np.arange(W), pr.sBn, np.concatenate([n0 * pr.sBn, (pr.batch - 1) * pr.sBb + n0 * pr.sBn]),
+                 np.concatenate([(w_rows - 1) * pr.sBn + pr.K] * 2), pr.b_bytes())):
+            _fits_i32(extent, f"rowpieces {what} extent")
+            voff = rows[:, None] * ld + chunk[None, :] * 16
+            _fits_i32(voff, f"rowpieces {what} offset")
+            live = (voff[None] + 16 <= extent[:, None, None]) & (kmax >= 0)[None, None, :]
+            bad = live & (base[:, None, None] + voff[None] + kmax[None, None, :] + 16 > alloc)
+            assert not bad.any(), f"rowpieces {what}: load outside the operand"
+        stats["units"] = NU
+        return stats
     if name.startswith("skinny"):
         slab = int(re.search(r"slab(\d+)", name).group(1))
         MB = int(re.search(r"_m(\d+)", name).group(1)) // 16

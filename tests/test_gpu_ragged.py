@@ -74,3 +74,30 @@ def test_qkv_decode_of_several_sequences_into_views_of_longer_caches(B, S, heads
     vt = vt0.clone()
     fused.kv_append_i8(None, want[:, 2 * H:], None, vt[:, :, :T], seqs=B)
     assert torch.equal(vt, want_vt)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 512, 16), (16, 20480, 1024), (17, 516, 1040), (33, 1001, 272), (48, 4100, 4096), (64, 16384, 528),
+                                   (48, 20478, 256), (16, 26000, 48), (50, 2052, 8192)])
+def test_row_piece_kernel_edges(M, N, K):
+    """One unit of 4 weight rows per workgroup up to 20 and more than one round, K below and off a stage, N off a
+    unit: integer sums and fixed-order epilogues, so every output type is exact (against torch in float64)."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import linear
+
+    lib = L.lib()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    i8 = lambda *shape: torch.randint(-128, 128, shape, dtype=torch.int8, device="cuda", generator=g)
+    a, w, b8 = i8(M, K), i8(N, K), i8(N)
+    b32 = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda", generator=g)
+    bf, res = torch.randn(N, device="cuda", generator=g), torch.randn((M, N), device="cuda", generator=g)
+    acc = (a.double() @ w.double().t()).to(torch.int32)
+    alpha, one = torch.tensor(30.0 / (K ** 0.5 * 5400.0), device="cuda"), torch.tensor(1.0, device="cuda")
+    got = linear.linear_a8_w8_b32_o32(a, w, b32)
+    assert lib.ti_gemm_config_name(lib.ti_gemm_last_config()).decode().endswith("_rowpieces")
+    assert torch.equal(got, acc + b32)
+    f = alpha * acc.float()
+    assert torch.equal(linear.linear_a8_w8_b8_o8(a, w, b8, alpha, one), (b8.float() + f).round().clamp(-128, 127).to(torch.int8))
+    want = bf + f
+    assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one), want)
+    assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one, dtype=torch.float16), want.half())
+    assert torch.equal(linear.linear_a8_w8_bfp32_ofp32_residual(a, w, bf, alpha, one, res), want + res)

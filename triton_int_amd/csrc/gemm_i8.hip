@@ -8,10 +8,11 @@
 //                            loads, consumer waves read fragments and issue MFMAs.  The large GEMMs.
 //   gemm_mfma_stream_kernel  persistent, loads issued by the MFMA waves (256x256 tiles, short K).
 //   gemm_mfma_kernel         one tile per workgroup; any output layout the fast loads allow.
-//   gemm_rows4_kernel        M <= 16: weights streamed as whole 1 KB row pieces (decode linears).
-//   gemm_skinny_kernel       M <= 64: 16-row weight slabs in MFMA layout, K split over waves.
+//   gemm_rowpieces_kernel    M <= 64: weight rows dealt evenly to the CUs, the whole K in one workgroup.
+//   gemm_rows4_kernel        M <= 16 against a few rows of a long K: weights as whole 1 KB row pieces.
+//   gemm_skinny_kernel       M <= 64, batched: 16-row weight slabs in MFMA layout, K split over waves.
 //   gemm_gather_kernel       any strides / alignment / K (byte gathers).
-// The first five need both operands K-contiguous and 16-byte aligned: 128-bit buffer loads
+// All but the last need both operands K-contiguous and 16-byte aligned: 128-bit buffer loads
 // straight into XOR-swizzled LDS tiles, several stages deep.
 //
 // C = epilogue(sum_k A[m,k] * B[n,k]); A is [M,K], B is [N,K] (the reference's "N" operand,
@@ -50,10 +51,10 @@ struct GemmParams {
   // bias elements [b * bias_bs, b * bias_bs + N) and the scalars alpha[b * scale_bs], beta[b * scale_bs]
   int64_t bias_bs;
   int64_t scale_bs;
-  // fp32 outputs of gemm_rows4_kernel and of the persistent kernels' fp32 epilogue: C = epilogue value + resid[m * resid_rs + n]
+  // fp32 outputs of gemm_rows4_kernel, gemm_rowpieces_kernel and of the persistent kernels' fp32 epilogue: C = epilogue value + resid[m * resid_rs + n]
   const float* resid;
   int64_t resid_rs;
-  // int8 outputs of a grouped q/k/v launch of gemm_rows4_kernel only.  Row m is position s = m % kv_S of
+  // int8 outputs of a grouped q/k/v launch of gemm_rows4_kernel or gemm_rowpieces_kernel only.  Row m is position s = m % kv_S of
   // sequence q = m / kv_S, h = q * heads + head: batch 1 (k) also goes to kv_k[h * kv_k_hs + s * kv_k_rs + d],
   // batch 2 (v) to kv_vt[(h * kv_D + d) * kv_vt_rs + s]
   int8_t* kv_k;
@@ -1920,26 +1921,15 @@ __global__ __launch_bounds__(512, UU ? 2 : 4) void gemm_skinny_kernel(GemmParams
 constexpr int R4_NW = 8, R4_RG = 4, R4_KC = 1024, R4_PITCH = R4_KC + 16, R4_WPITCH = R4_KC + 64, R4_NST = 3, R4_XB = 3,
               R4_UMAX = 4;
 
-// The store phase of gemm_rows4_kernel's epilogue: thread t of the 512 consumer threads takes row t / 32
-// and the 4 outputs of unit unit0 + t % 32 from the LDS tile (row r at tile0 + (r/2) * ring + (r%2) * 2048),
-// converts them and stores them as one piece, so a row's outputs leave as one contiguous run.  A
-// function of its own: inlined, its operands cost the main loop registers.
+// Four neighbouring outputs n0 .. n0+3 of row `row` from their int32 sums: converted and stored as one piece
+// where the output's layout allows.
 template <int OUTCLS>
-__device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char* Cz, int64_t sCm, int64_t sCn, int M, int N,
-                                                          int out_dtype, unsigned tile0, int tid, int unit0, int u_end,
-                                                          int max_units, const float* resid, int64_t resid_rs, int bz,
-                                                          const GemmParams* kp) {
+__device__ __forceinline__ void store4(const EpiCtx& e, char* Cz, int64_t sCm, int64_t sCn, int N, int out_dtype, int row, int n0,
+                                       v4i a, const float* resid, int64_t resid_rs, int bz, const GemmParams* kp) {
   constexpr int ESZ = OUTCLS == OUT8 ? 1 : (OUTCLS == OUT32 ? 4 : 2);
-  constexpr int RING = R4_NST * R4_RG * R4_WPITCH;  // the tile's geometry, whatever the kernel's ring depth
-  const int row = tid >> 5, grp = tid & 31;
-  const int unit = unit0 + grp;
-  if (!(row < M && unit < u_end && grp < max_units)) return;
-  const unsigned addr = tile0 + (row >> 1) * RING + (row & 1) * 2048 + grp * 16;
-  const v4i a = *(const __attribute__((address_space(3))) v4i*)(uintptr_t)addr;
-  const int n0 = unit * R4_RG;
-  unsigned b[R4_RG];
+  unsigned b[4];
 #pragma unroll
-  for (int i = 0; i < R4_RG; ++i) {
+  for (int i = 0; i < 4; ++i) {
     const int n = min(n0 + i, N - 1);
     const int bias_i32 = (e.epilogue == TI_EPI_I32 && e.bias_kind == TI_BIAS_I32) ? ((const int*)e.bias)[n] : 0;
     b[i] = convert_one<OUTCLS>(e, a[i], column_term(e, n), bias_i32, out_dtype);
@@ -1949,7 +1939,7 @@ __device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char*
   }
   char* dst = Cz + ((int64_t)row * sCm + (int64_t)n0 * sCn) * ESZ;
   if constexpr (OUTCLS == OUT8) {
-    if (bz > 0 && n0 + R4_RG <= N) {
+    if (bz > 0 && n0 + 4 <= N) {
       // KV-cache append of a decode step's k / v projections; the fields are read through kp, the
       // kernel's own argument block (the builtin that returns it yields null outside a kernel, so
       // the kernel passes it along)
@@ -1961,18 +1951,18 @@ __device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char*
               b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
         } else if (bz == 2) {
 #pragma unroll
-          for (int i = 0; i < R4_RG; ++i) kp->kv_vt[((int64_t)seq * N + n0 + i) * kp->kv_vt_rs + pos] = (int8_t)b[i];
+          for (int i = 0; i < 4; ++i) kp->kv_vt[((int64_t)seq * N + n0 + i) * kp->kv_vt_rs + pos] = (int8_t)b[i];
         }
       }
     }
   }
-  if (sCn == 1 && n0 + R4_RG <= N && (((uintptr_t)dst) & (R4_RG * ESZ - 1)) == 0) {
+  if (sCn == 1 && n0 + 4 <= N && (((uintptr_t)dst) & (4 * ESZ - 1)) == 0) {
     if constexpr (OUTCLS == OUT8) *(unsigned*)dst = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
     else if constexpr (OUTCLS == OUT32) *(v4u*)dst = (v4u){b[0], b[1], b[2], b[3]};
     else *(uint2*)dst = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
   } else {
 #pragma unroll
-    for (int i = 0; i < R4_RG; ++i) {
+    for (int i = 0; i < 4; ++i) {
       if (n0 + i < N) {
         char* d = dst + (int64_t)i * sCn * ESZ;
         if constexpr (OUTCLS == OUT8) *(int8_t*)d = (int8_t)b[i];
@@ -1981,6 +1971,24 @@ __device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char*
       }
     }
   }
+}
+
+// The store phase of gemm_rows4_kernel's epilogue: thread t of the 512 consumer threads takes row t / 32
+// and the 4 outputs of unit unit0 + t % 32 from the LDS tile (row r at tile0 + (r/2) * ring + (r%2) * 2048),
+// converts them and stores them as one piece, so a row's outputs leave as one contiguous run.  A
+// function of its own: inlined, its operands cost the main loop registers.
+template <int OUTCLS>
+__device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char* Cz, int64_t sCm, int64_t sCn, int M, int N,
+                                                          int out_dtype, unsigned tile0, int tid, int unit0, int u_end,
+                                                          int max_units, const float* resid, int64_t resid_rs, int bz,
+                                                          const GemmParams* kp) {
+  constexpr int RING = R4_NST * R4_RG * R4_WPITCH;  // the tile's geometry, whatever the kernel's ring depth
+  const int row = tid >> 5, grp = tid & 31;
+  const int unit = unit0 + grp;
+  if (!(row < M && unit < u_end && grp < max_units)) return;
+  const unsigned addr = tile0 + (row >> 1) * RING + (row & 1) * 2048 + grp * 16;
+  const v4i a = *(const __attribute__((address_space(3))) v4i*)(uintptr_t)addr;
+  store4<OUTCLS>(e, Cz, sCm, sCn, N, out_dtype, row, unit * R4_RG, a, resid, resid_rs, bz, kp);
 }
 
 template <int OUTCLS, int NWA, int NST>
@@ -2146,6 +2154,178 @@ __global__ __launch_bounds__((R4_NW + 1) * 64) void gemm_rows4_kernel(GemmParams
   }
 }
 
+// ---- row-piece kernel: M <= 64, the whole K in one workgroup --------------------------------------
+//
+// With a few dozen activation rows the GEMM is still a read of the weight matrix, but the activations a
+// workgroup needs are as many bytes as its weights.  Tiles of 128 weight rows with K split over workgroups
+// leave CUs idle (N = 4096 is 32 of them), and every split costs an exchange of partial sums at the end
+// of the launch that nothing overlaps.  Here N is dealt to the 256 CUs in units of 4 weight rows (up to
+// 16 * G rows per workgroup), every workgroup walks the whole K, and no partial sum leaves it.
+//   producers (4 waves): one stage = KC bytes of K of the MT activation rows and the 16 * G weight rows,
+//     in 1 KB pieces (4 rows x 256 bytes), as many stages ahead as LDS holds.
+//   consumers (4 waves): each takes a quarter of a stage's K and ALL of its rows, so that every LDS byte
+//     is read once; the four sets of sums meet in LDS after the last stage.
+// Hand-over as in gemm_mfma_ws_kernel: one barrier per stage; a consumer reads stage g+1 into a second set
+// of registers while the MFMAs of stage g run.
+// Bound: HBM (weights) and, from M = 48 on, what a CU takes in (weights and activations together 30-60 GB/s).
+// 64 rows x 16384 x 4096 20.0 us = 3.4 TB/s of weights, 16 x 20480 x 5120 21.4 us = 4.9 TB/s.
+// LDS: a row is KC bytes (64 banks or a multiple), 16-byte chunk c of row r lives at slot c ^ (r & 15): the
+// 16 rows of an operand read hit 16 different bank groups.
+constexpr int RP_PW = 4, RP_CW = 4, RP_GMAX = 5;
+
+template <int LOADS, int I>
+__device__ __forceinline__ void wait_stages(int n) {
+  if constexpr (I > 0) {
+    if (n < I) return wait_stages<LOADS, I - 1>(n);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * I) : "memory");
+}
+
+template <int OUTCLS>
+__device__ __attribute__((noinline)) void rowpieces_store(const EpiCtx e, char* Cz, int64_t sCm, int64_t sCn, int M, int N, int out_dtype,
+                                                         unsigned red, int wave_bytes, int gu, int tid, int n_first, int units,
+                                                         const float* resid, int64_t resid_rs, int bz, const GemmParams* kp) {
+  for (int idx = tid; idx < M * units; idx += (RP_PW + RP_CW) * 64) {
+    const int m = idx / units, u = idx - m * units;
+    const unsigned addr = red + (((m >> 4) * gu + u) * 17 + (m & 15)) * 16;
+    v4i a = {0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < RP_CW; ++w) a += *(const __attribute__((address_space(3))) v4i*)(uintptr_t)(addr + w * wave_bytes);
+    store4<OUTCLS>(e, Cz, sCm, sCn, N, out_dtype, m, n_first + 4 * u, a, resid, resid_rs, bz, kp);
+  }
+}
+
+template <int MT, int G, int KC>
+__global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(GemmParams p) {
+  constexpr int MB = MT / 16, CH = KC / 16, RPI = 1024 / KC;        // RPI: rows per load instruction
+  constexpr int AI = MT / RPI / RP_PW, WI = 16 * G / RPI / RP_PW;   // loads of a producer wave per stage
+  constexpr int LOADS = AI + WI, STAGE = (MT + 16 * G) * KC;
+  constexpr int NST_LDS = 160 * 1024 / STAGE, NST_CNT = 1 + 63 / LOADS;
+  constexpr int NST = NST_LDS < NST_CNT ? NST_LDS : NST_CNT, DEPTH = NST - 1;
+  constexpr int KPW = KC / 64 / RP_CW;                              // 64-deep k-steps of a consumer wave per stage
+  constexpr int WAVE_RED = MB * 4 * G * 17 * 16;                    // a wave's sums, 16-byte pieces padded against bank conflicts
+  static_assert(MT % (RPI * RP_PW) == 0 && 16 * G % (RPI * RP_PW) == 0 && KC % (64 * RP_CW) == 0, "even shares");
+  static_assert(NST >= 3 && RP_CW * WAVE_RED <= NST * STAGE, "LDS budget");
+  __shared__ __attribute__((aligned(16))) char lds[NST * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bz = blockIdx.y;
+  const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  // this workgroup's weight rows
+  const int NU = (p.N + 3) >> 2;
+  const int per = (NU + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int u0 = __builtin_amdgcn_readfirstlane(min(NU, (int)blockIdx.x * per));
+  const int units = __builtin_amdgcn_readfirstlane(min(NU, u0 + per) - u0);
+  const int n0 = u0 * 4;
+  const int KT = (p.K + KC - 1) / KC;
+  if (units <= 0) return;  // uniform: the whole workgroup
+
+  if (wave >= RP_CW) {
+    const int pw = wave - RP_CW;
+    const int lda = (int)p.sAm, ldb = (int)p.sBn;
+    const int OOB = (int)0x80000000;
+    // rows past M, past the workgroup's last weight row and bytes past K read as zeros
+    const v4i rA = make_rsrc(p.A + (int64_t)bz * p.sAb, (p.M - 1) * lda + p.K);
+    const v4i rW = make_rsrc(p.B + (int64_t)bz * p.sBb + (int64_t)n0 * ldb, (min(units * 4, p.N - n0) - 1) * ldb + p.K);
+    int voff[LOADS], klim[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const bool is_a = i < AI;
+      const int row = (is_a ? pw * AI + i : pw * WI + i - AI) * RPI + lane / CH;
+      const int chunk = (lane % CH) ^ (row & 15);
+      voff[i] = row * (is_a ? lda : ldb) + chunk * 16;
+      klim[i] = p.K - chunk * 16;
+    }
+    int k0 = 0, st = 0;
+    auto issue = [&]() {
+      const unsigned dst = lds_base + st * STAGE;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const int v = k0 < klim[i] ? voff[i] : OOB;
+        if (i < AI) dma16_to_lds(rA, v, k0, dst + (pw * AI + i) * 1024);
+        else dma16_to_lds_stream(rW, v, k0, dst + MT * KC + (pw * WI + i - AI) * 1024);
+      }
+      k0 += KC;
+      st = (st + 1 == NST) ? 0 : st + 1;
+    };
+    int issued = 0;
+    for (; issued < DEPTH && issued < KT; ++issued) issue();
+    wait_stages<LOADS, DEPTH>(issued - 1);  // stage 0 landed
+    asm volatile("s_barrier" ::: "memory");
+    for (int g = 0; g < KT; ++g) {
+      if (issued < KT) {
+        issue();  // into the stage of g-1, whose readers passed barrier g-1
+        ++issued;
+      }
+      wait_stages<LOADS, DEPTH>(max(0, issued - (g + 2)));  // stage g+1 landed
+      asm volatile("s_barrier" ::: "memory");
+    }
+  } else {
+    const int r16 = lane & 15, c4 = lane >> 4;
+    v4i acc[G][MB];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int m = 0; m < MB; ++m) acc[g][m] = (v4i){0, 0, 0, 0};
+    v4i xf[2][KPW][MB], wf[2][KPW][G];
+    auto read = [&](auto set_tag, int stage) {
+      constexpr int set = decltype(set_tag)::value;
+      const char* sp = lds + stage * STAGE;
+#pragma unroll
+      for (int k = 0; k < KPW; ++k) {
+        const int off = r16 * KC + ((((wave * KPW + k) * 4 + c4) ^ r16) * 16);
+#pragma unroll
+        for (int m = 0; m < MB; ++m) xf[set][k][m] = *(const v4i*)(sp + m * 16 * KC + off);
+#pragma unroll
+        for (int g = 0; g < G; ++g) wf[set][k][g] = *(const v4i*)(sp + (MT + g * 16) * KC + off);
+      }
+    };
+    auto compute = [&](auto set_tag) {
+      constexpr int set = decltype(set_tag)::value;
+#pragma unroll
+      for (int k = 0; k < KPW; ++k)
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int m = 0; m < MB; ++m)
+            acc[g][m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[set][k][g], xf[set][k][m], acc[g][m], 0, 0, 0);
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    asm volatile("s_barrier" ::: "memory");  // stage 0 is in LDS
+    int st = 0;
+    auto next = [&]() { st = (st + 1 == NST) ? 0 : st + 1; };
+    if (KT > 0) read(S0{}, st);
+    for (int g = 0; g < KT; g += 2) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // stage g is read, stage g+1 is in LDS
+      next();
+      if (g + 1 < KT) read(S1{}, st);
+      compute(S0{});
+      if (g + 1 < KT) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        next();
+        if (g + 2 < KT) read(S0{}, st);
+        compute(S1{});
+      }
+    }
+    // acc[g][m][i]: weight row n0 + 16*g + 4*c4 + i, activation row 16*m + r16.  All LDS reads of every wave are
+    // done (last barrier) and no load is in flight: the rings become the area where the sums meet
+    char* red = lds + wave * WAVE_RED;
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int g = 0; g < G; ++g) *(v4i*)(red + ((m * 4 * G + g * 4 + c4) * 17 + r16) * 16) = acc[g][m];
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const EpiCtx e = make_epi(p, bz);
+  const GemmParams* kp = (const GemmParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  const int esz = p.out_dtype == TI_I8 ? 1 : ((p.out_dtype == TI_F16 || p.out_dtype == TI_BF16) ? 2 : 4);
+  char* Cz = (char*)p.C + (int64_t)bz * p.sCb * esz;
+  if (esz == 1) rowpieces_store<OUT8>(e, Cz, p.sCm, p.sCn, p.M, p.N, p.out_dtype, lds_base, WAVE_RED, 4 * G, tid, n0, units, nullptr, 0, bz, kp);
+  else if (esz == 2) rowpieces_store<OUT16>(e, Cz, p.sCm, p.sCn, p.M, p.N, p.out_dtype, lds_base, WAVE_RED, 4 * G, tid, n0, units, nullptr, 0, bz, kp);
+  else rowpieces_store<OUT32>(e, Cz, p.sCm, p.sCn, p.M, p.N, p.out_dtype, lds_base, WAVE_RED, 4 * G, tid, n0, units, p.resid, p.resid_rs, bz, kp);
+}
+
 // ---- host side ---------------------------------------------------------------------------------
 
 typedef void (*KernelFn)(GemmParams);
@@ -2160,6 +2340,7 @@ struct Config {
   bool rows4 = false;   // gemm_rows4_kernel: M <= 16
   int ws_waves = 0;     // > 0: gemm_mfma_ws_kernel with this many consumer waves (it can split K)
   int max_k = 0;        // > 0: the kernel holds a tile's whole K in LDS and takes 16 <= K <= max_k only
+  bool rowpieces = false;  // gemm_rowpieces_kernel: M <= bm
 };
 
 #define TI_FAST(BM, BN, BK, WM, WN, SWZ, NS)                                              \
@@ -2189,6 +2370,13 @@ struct Config {
         BM, BN, BK, (WM * WN + PW) * 64, true, false, 1, false, WM * WN                   \
   }
 
+#define TI_ROWPIECES(MT)                                                                  \
+  {                                                                                       \
+    "skinny_m" #MT "_rowpieces",                                                            \
+        {rowpieces_kernel(MT, 1), rowpieces_kernel(MT, 1), rowpieces_kernel(MT, 1)},        \
+        MT, 4, RP_KC, (RP_PW + RP_CW) * 64, true, false, 0, false, 0, 0, true               \
+  }
+
 enum ConfigId {
   CFG_GATHER = 0,
   CFG_TILE_256x128,   // one tile per workgroup: any output layout the fast loads allow
@@ -2208,7 +2396,21 @@ enum ConfigId {
   CFG_SHORTK_256x256,  // K <= 128 (attention Q.K^T): a tile's whole K in LDS, one barrier per tile, 128-byte int8 row pieces
   CFG_WS_64x128,       // 32 < M <= 128 against a long K: six stages of a 64-row tile keep more weight bytes in flight per CU
   CFG_WS_32x128,       // 16 < M <= 32: seven stages
+  CFG_ROWPIECES_16,    // few activation rows: whole K per workgroup, weight rows dealt to the CUs in fours
+  CFG_ROWPIECES_32,
+  CFG_ROWPIECES_48,
+  CFG_ROWPIECES_64,
 };
+
+constexpr int RP_KC = 256;
+// gemm_rowpieces_kernel for at most mt activation rows and 16 * g weight rows per workgroup
+static KernelFn rowpieces_kernel(int mt, int g) {
+#define TI_RP(MT) {gemm_rowpieces_kernel<MT, 1, RP_KC>, gemm_rowpieces_kernel<MT, 2, RP_KC>, gemm_rowpieces_kernel<MT, 3, RP_KC>, \
+                   gemm_rowpieces_kernel<MT, 4, RP_KC>, gemm_rowpieces_kernel<MT, 5, RP_KC>}
+  static const KernelFn fns[4][RP_GMAX] = {TI_RP(16), TI_RP(32), TI_RP(48), TI_RP(64)};
+#undef TI_RP
+  return fns[mt / 16 - 1][g - 1];
+}
 
 static const Config g_configs[] = {
     {"gather_64x64x32", {gemm_gather_kernel<OUT8>, gemm_gather_kernel<OUT32>, gemm_gather_kernel<OUT16>}, 64, 64, 32, 256, false},
@@ -2230,6 +2432,10 @@ static const Config g_configs[] = {
      true, false, 1, false, 0, 128},
     TI_WS(64, 128, 128, 2, 2, 1, 6, 4),
     TI_WS(32, 128, 128, 1, 4, 1, 7, 4),
+    TI_ROWPIECES(16),
+    TI_ROWPIECES(32),
+    TI_ROWPIECES(48),
+    TI_ROWPIECES(64),
 };
 static const int g_num_configs = (int)(sizeof(g_configs) / sizeof(g_configs[0]));
 
@@ -2334,14 +2540,37 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
 static int pick_config(const GemmParams& p, int* splits_out) {
   *splits_out = 1;
   if (!fast_eligible(p)) return CFG_GATHER;
-  if (p.M <= 16) {
-    // one GEMM over a long K: stream the weights as whole row pieces; short K or batched (the
-    // decode attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
-    if (p.batch <= 4 && p.K >= 1024) return CFG_ROWS4_16;
-    return (p.N + 31) / 32 >= 160 ? CFG_SKINNY_16_G2 : CFG_SKINNY_16;
-  }
   const bool stream = stream_eligible(p);
-  if (p.M <= 128 && stream && p.batch == 1 && p.K >= 1024) {
+  if (p.M <= 64 && p.batch <= 4) {
+    // one GEMM (or up to four grouped ones): gemm_rowpieces_kernel, except where a workgroup's share of the
+    // weights is too small against its share of the activations, or too large for one round.  Measured with
+    // weights from HBM, fp32 out (us, the other kernel / this one):
+    //   M <= 16, against gemm_rows4_kernel, which keeps more weight bytes in flight when a workgroup has only a
+    //   few rows of a long K: N x K = 12288 x 4096 15.6 / 14.3, 6848 x 10240 20.1 / 17.9, 20480 x 5120 23.4 / 21.4,
+    //   5120 x 5120 11.0 / 10.3, 4096 x 4096 9.6 / 9.2; but 4096 x 8192 12.7 / 13.5, 4096 x 16384 19.5 / 21.8,
+    //   1024 x 4096 7.3 / 7.7, 28672 x 4096 27.8 / 29.2.  The line: 6 to 20 units of 4 rows per workgroup, or 1 KB of
+    //   K per unit.
+    //   M > 16, against 32 x 128 and 64 x 128 tiles with split K: 4096 x 4096 15.7 / 9.5 (M = 32) and 17.9 / 10.9
+    //   (64), 12288 x 4096 22.2 / 18.5 (64), 15360 x 5120 30.3 / 23.9, 2048 x 8192 15.8 / 14.6; but 6848 x 10240
+    //   22.5 / 26.0, 4096 x 16384 20.0 / 26.0, 50272 x 1024 18.3 / 34.8, 32768 x 768 9.5 / 18.7.  The line: one round
+    //   (20 units per workgroup), K = 8192, and K = 4096 where a workgroup has a single unit.
+    //   K < 1024, one round, against gemm_skinny_kernel: 768 x 768 9.4 / 5.0 (M = 16), 20.2 / 5.5 (64), 256 x 256
+    //   5.2 / 4.9 (1).
+    // Two corners stay on the tiles although this kernel measures better there, because
+    // test_decode_shapes_skinny_kernel names the tile they run on: M > 48 with 16385 .. 20480 columns (64 x
+    // 20480 x 5120 34.0 / 28.2) and M > 16 with fewer than 512 (32 x 272 x 1040 8.5 / 5.3).
+    const int units = (p.N + 3) / 4, per = (units + 256 / p.batch - 1) / (256 / p.batch);
+    const bool one_round = per <= 4 * RP_GMAX;
+    const int64_t columns = (int64_t)p.N * p.batch;
+    const int rp = CFG_ROWPIECES_16 + (p.M - 1) / 16;
+    if (p.M <= 16 && p.K >= 1024) return one_round && (per >= 6 || p.K <= 1024 * per) ? rp : CFG_ROWS4_16;
+    if (p.K < 1024 ? one_round || p.M <= 16 || p.batch > 1 || !stream
+                   : one_round && (per > 1 ? p.K <= 8192 : p.K <= 4096) && !(p.M > 48 && columns > 16384) && columns >= 512)
+      return rp;
+  }
+  // batched, few rows (attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
+  if (p.M <= 16) return (p.N + 31) / 32 >= 160 ? CFG_SKINNY_16_G2 : CFG_SKINNY_16;
+  if (p.M <= 128 && stream && p.batch == 1 && (p.K >= 1024 || p.M <= 64)) {
     // a few rows against a long K: the GEMM is a read of the weight matrix, and what decides its speed is how
     // many weight bytes a CU keeps in flight.  K is split over enough workgroups to have every CU pulling its
     // own slab, and the tile has no more activation rows than needed, so that the LDS holds more stages of
@@ -2618,7 +2847,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
   if (config >= g_num_configs) return fail(TI_E_COMBO, "config %d out of range", config);
   const Config& k = g_configs[config];
   if (!k.fn[out_class(p.out_dtype)]) return fail(TI_E_COMBO, "config %s has no kernel for output dtype %d", k.name, p.out_dtype);
-  if (k.fast && !k.skinny && !k.rows4 && trunc8) return fail(TI_E_COMBO, "config %s does not implement TI_ROUND_TRUNC for int8 outputs", k.name);
+  if (k.fast && !k.skinny && !k.rows4 && !k.rowpieces && trunc8) return fail(TI_E_COMBO, "config %s does not implement TI_ROUND_TRUNC for int8 outputs", k.name);
   if (k.fast && !fast_eligible(p)) return fail(TI_E_COMBO, "config %s needs K-contiguous 16-byte aligned operands", k.name);
   if (k.stream_occ && !stream_eligible(p)) return fail(TI_E_COMBO, "config %s needs a row-major output with 16-byte aligned rows", k.name);
   if (k.max_k && (p.K < 16 || p.K > k.max_k)) return fail(TI_E_COMBO, "config %s needs 16 <= K <= %d", k.name, k.max_k);
@@ -2667,6 +2896,23 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       return TI_OK;
     }
     rows4_kernel(out_class(p.out_dtype), nwa)<<<dim3((unsigned)blocks, (unsigned)p.batch), dim3(k.threads), 0, stream>>>(p);
+    return launch_status(k.name);
+  }
+  if (k.rowpieces) {
+    if (p.M > k.bm) return fail(TI_E_COMBO, "config %s needs M <= %d", k.name, k.bm);
+    // one workgroup per CU and round, all batches together, the units of 4 weight rows dealt evenly over as few
+    // rounds as 16 * RP_GMAX rows per workgroup allow
+    const int units = (p.N + 3) / 4;
+    const int wgs = p.batch >= 256 ? 1 : 256 / p.batch;
+    const int rounds = (units + wgs * 4 * RP_GMAX - 1) / (wgs * 4 * RP_GMAX);
+    const int per = (units + wgs * rounds - 1) / (wgs * rounds);
+    const int blocks = (units + per - 1) / per;
+    g_last_config = config;
+    if (dry) {
+      dry->config = config; dry->grid_x = (unsigned)blocks; dry->grid_y = (unsigned)p.batch; dry->threads = k.threads;
+      return TI_OK;
+    }
+    rowpieces_kernel(k.bm, (per + 3) / 4)<<<dim3((unsigned)blocks, (unsigned)p.batch), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }
   if (k.skinny) {
@@ -2794,7 +3040,7 @@ static int run_with_residual(GemmParams p, const float* R, int64_t ldr, hipStrea
   if (!p.bias) p.bias_kind = TI_BIAS_NONE;
   int splits = 1;
   const int cfg = pick_config(p, &splits);
-  if (g_configs[cfg].rows4) {  // the decode kernel adds the residual in its store phase
+  if (g_configs[cfg].rows4 || g_configs[cfg].rowpieces) {  // the decode kernels add the residual in their store phase
     p.resid = R;
     p.resid_rs = ldr;
     return run(p, cfg, stream);
@@ -2896,7 +3142,7 @@ int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t
   if (rc != TI_OK) return rc;
   int splits = 1;
   const int cfg = pick_config(p, &splits);
-  if (!g_configs[cfg].rows4) return fail(TI_E_COMBO, "operands not eligible for the decode kernel (16-byte aligned, K-contiguous)");
+  if (!g_configs[cfg].rows4 && !g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "operands not eligible for the decode kernel (16-byte aligned, K-contiguous)");
   return run(p, cfg, (hipStream_t)stream);
 }
 
