@@ -99,6 +99,23 @@ def _declare(lib):
     lib.ti_gelu_q.argtypes = [_vp, _vp, _vp, _i64, _int, _vp]
 
 
+class _MissingHost:
+    """Stands in for the extension module until it is built: there is no fallback path."""
+
+    def __init__(self, error):
+        self._error = error
+
+    def __getattr__(self, name):
+        raise RuntimeError(f"triton_int_amd._host cannot be loaded ({self._error}): build it with "
+                           "`python -m triton_int_amd.build` (g++, hipcc, gfx950)")
+
+
+try:
+    from . import _host as host  # the launchers' host path; its functions return None for what is not the ordinary case
+except ImportError as e:
+    host = _MissingHost(e)
+
+
 def lib() -> ctypes.CDLL:
     """The loaded library.  Raises if it has not been built: there is no fallback path."""
     global _lib

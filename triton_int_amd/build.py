@@ -1,4 +1,5 @@
-"""Builds libtriton_int_hip.so (gfx950 only) from triton_int_amd/csrc/*.hip with hipcc.
+"""Builds libtriton_int_hip.so (gfx950 only) from triton_int_amd/csrc/*.hip with hipcc, and the extension
+module _host.so (the launchers' host path, csrc/host.cpp, against torch's headers) with g++.
 
     python -m triton_int_amd.build
 
@@ -12,12 +13,16 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "_obj")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libtriton_int_hip.so")
+
+HOST_SRC = os.path.join(CSRC, "host.cpp")
+HOST_PATH = os.path.join(HERE, "_host.so")
 
 SOURCES = ["lib.hip", "gemm_i8.hip", "rowops.hip", "attention_i8.hip", "quant.hip", "layernorm_fp.hip"]
 
@@ -41,6 +46,26 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_host() -> None:
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    if not os.path.isdir(os.path.join(rocm, "include", "hip")):
+        rocm = "/opt/rocm"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{d}" for d in (os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                                      os.path.join(rocm, "include"), sysconfig.get_paths()["include"])),
+           HOST_SRC, "-o", HOST_PATH, f"-L{os.path.join(root, 'lib')}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu",
+           "-lc10_hip", "-lc10", f"-L{LIB_DIR}", "-l:libtriton_int_hip.so", "-Wl,-rpath,$ORIGIN/lib"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{r.stderr}")
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr + "\n")
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -51,6 +76,7 @@ def build(verbose: bool = True) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
+    _build_host()
     if verbose:
         print(f"built {LIB_PATH} ({os.path.getsize(LIB_PATH) // 1024} KiB)")
     return LIB_PATH

@@ -1,0 +1,495 @@
+// host.cpp — the launchers' host path as a CPython extension (triton_int_amd._host).
+//
+// A launch of libtriton_int_hip.so through ctypes costs about as much again as the launch itself, and the
+// argument checks, views and allocations around it in Python three times as much: 15.9 us for a 512 x 768 x 768
+// linear module whose kernel runs 5 us.  These functions take the tensors as they are, check what the Python
+// launchers check, allocate the output and call the C ABI.
+//
+// Every function returns None, having done nothing, when an argument is anything but the ordinary case (a
+// tensor subclass, another device than the current one, a layout that needs a copy, a python-float scale, a
+// wrong dtype or size, a status from the library).  The Python launcher then takes its own path, which
+// converts or raises: there is one definition of every conversion and every error message.
+#include <Python.h>
+
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include "../../include/triton_int_hip.h"
+
+namespace {
+
+using at::ScalarType;
+using at::Tensor;
+
+struct NotOrdinary {};  // thrown by the argument readers, turned into None
+
+void need(bool ok) {
+  if (!ok) throw NotOrdinary{};
+}
+
+// A call's device and stream: those of its first tensor, which has to be on the current device.
+struct Call {
+  c10::DeviceIndex dev;
+  void* stream;
+  explicit Call(const Tensor& t) : dev(t.get_device()) {
+    need(dev == c10::hip::current_device());
+    stream = (void*)c10::hip::getCurrentHIPStream(dev).stream();
+  }
+  Tensor empty(at::IntArrayRef sizes, ScalarType type) const {
+    return Tensor(at::detail::empty_cuda(sizes, type, c10::Device(c10::kCUDA, dev), std::nullopt));
+  }
+};
+
+// A plain tensor on a GPU; `dev` < 0: on any.
+const Tensor& tensor(PyObject* o, int dev = -1) {
+  need(THPVariable_CheckExact(o));
+  const Tensor& t = THPVariable_Unpack(o);
+  need(t.is_cuda() && (dev < 0 || t.get_device() == dev));
+  return t;
+}
+
+const Tensor& tensor(PyObject* o, int dev, ScalarType type) {
+  const Tensor& t = tensor(o, dev);
+  need(t.scalar_type() == type);
+  return t;
+}
+
+const void* ptr(const Tensor& t) { return t.const_data_ptr(); }
+void* mptr(const Tensor& t) { return t.mutable_data_ptr(); }
+
+// an optional contiguous vector of `n` elements of `type`
+const void* vector(PyObject* o, int dev, ScalarType type, int64_t n) {
+  if (o == Py_None) return nullptr;
+  const Tensor& t = tensor(o, dev, type);
+  need(t.numel() == n && t.is_contiguous());
+  return ptr(t);
+}
+
+const float* scale(PyObject* o, int dev) {
+  if (o == Py_None) return nullptr;
+  return (const float*)ptr(tensor(o, dev, ScalarType::Float));
+}
+
+int64_t integer(PyObject* o) {
+  const int64_t v = PyLong_AsLongLong(o);
+  need(!(v == -1 && PyErr_Occurred()));
+  return v;
+}
+
+double number(PyObject* o) {
+  need(PyFloat_Check(o) || PyLong_Check(o));
+  return PyFloat_AsDouble(o);
+}
+
+int bias_kind(ScalarType t) {
+  switch (t) {
+    case ScalarType::Char: return TI_BIAS_I8;
+    case ScalarType::Int: return TI_BIAS_I32;
+    case ScalarType::Float: return TI_BIAS_F32;
+    case ScalarType::Half: return TI_BIAS_F16;
+    case ScalarType::BFloat16: return TI_BIAS_BF16;
+    default: throw NotOrdinary{};
+  }
+}
+
+ScalarType out_type(int dt) {
+  switch (dt) {
+    case TI_I8: return ScalarType::Char;
+    case TI_I32: return ScalarType::Int;
+    case TI_F32: return ScalarType::Float;
+    case TI_F16: return ScalarType::Half;
+    case TI_BF16: return ScalarType::BFloat16;
+    default: throw NotOrdinary{};
+  }
+}
+
+int dtype_code(ScalarType t) {
+  switch (t) {
+    case ScalarType::Float: return TI_F32;
+    case ScalarType::Half: return TI_F16;
+    case ScalarType::BFloat16: return TI_BF16;
+    default: throw NotOrdinary{};
+  }
+}
+
+int int32_size(int64_t v) {
+  need(v >= 0 && v <= 0x7fffffff);
+  return (int)v;
+}
+
+// activations [..., K] as M rows of one pitch
+struct Rows {
+  int M, K;
+  int64_t pitch;
+  Rows(const Tensor& a, int64_t k) {
+    need(a.dim() >= 2 && a.size(-1) == k && k > 0);
+    need(a.dim() == 2 ? a.stride(1) == 1 : a.is_contiguous());
+    K = int32_size(k);
+    M = int32_size(a.numel() / k);
+    pitch = a.dim() == 2 ? a.stride(0) : k;
+  }
+};
+
+c10::SmallVector<int64_t, 6> with_last(const Tensor& a, int64_t n) {
+  c10::SmallVector<int64_t, 6> s(a.sizes().begin(), a.sizes().end());
+  s.back() = n;
+  return s;
+}
+
+template <class F>
+PyObject* guarded(Py_ssize_t n, Py_ssize_t want, F f) {
+  if (n != want) {
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
+    return nullptr;
+  }
+  try {
+    return f();
+  } catch (const NotOrdinary&) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+// linear(a, w, bias, alpha, beta, out, epilogue, out_dtype, round_mode, config, groups): kernels/_gemm.py linear and,
+// with groups > 0, linear_group
+PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 11, [&]() -> PyObject* {
+    const Tensor& a = tensor(v[0], -1, ScalarType::Char);
+    const Call c(a);
+    const Tensor& w = tensor(v[1], c.dev, ScalarType::Char);
+    need(w.dim() == 2);
+    const int64_t groups = integer(v[10]), N = w.size(0), per = groups ? N / groups : N;
+    need(!groups || N % groups == 0);
+    const Rows r(a, w.size(1));
+    int bk = TI_BIAS_NONE;
+    const void* bias = nullptr;
+    if (v[2] != Py_None) {
+      const Tensor& b = tensor(v[2], c.dev);
+      bk = bias_kind(b.scalar_type());
+      need(b.numel() == N && b.is_contiguous());
+      bias = ptr(b);
+    }
+    const float *alpha = scale(v[3], c.dev), *beta = scale(v[4], c.dev);
+    const int dt = (int)integer(v[7]);
+    const ScalarType type = out_type(dt);
+    const auto sizes = with_last(a, N);
+    Tensor out;
+    if (v[5] == Py_None) {
+      out = c.empty(sizes, type);
+    } else {
+      const Tensor& o = tensor(v[5], c.dev, type);
+      need(o.numel() == (int64_t)r.M * N && o.is_contiguous());
+      out = o.view(sizes);
+    }
+    int rc;
+    if (groups) {
+      for (int i = 3; i < 5; ++i)
+        if (v[i] != Py_None) need(THPVariable_Unpack(v[i]).numel() == groups && THPVariable_Unpack(v[i]).is_contiguous());
+      rc = ti_bmm_i8_grouped((const int8_t*)ptr(a), 0, r.pitch, 1, (const int8_t*)ptr(w), per * w.stride(0), w.stride(0), w.stride(1),
+                             mptr(out), per, N, 1, (int)groups, r.M, int32_size(per), r.K, bias, bk, per, alpha, beta, 1,
+                             (int)integer(v[6]), dt, (int)integer(v[8]), (int)integer(v[9]), c.stream);
+    } else {
+      rc = ti_bmm_i8_config((const int8_t*)ptr(a), 0, r.pitch, 1, (const int8_t*)ptr(w), 0, w.stride(0), w.stride(1), mptr(out), 0, N, 1, 1,
+                            r.M, int32_size(N), r.K, bias, bk, alpha, beta, (int)integer(v[6]), dt, (int)integer(v[8]),
+                            (int)integer(v[9]), c.stream);
+    }
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// bmm(a, b, b_is_kn, alpha, out, epilogue, out_dtype, round_mode, config): kernels/_gemm.py bmm
+PyObject* bmm(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 9, [&]() -> PyObject* {
+    const Tensor& a = tensor(v[0], -1, ScalarType::Char);
+    const Call c(a);
+    const Tensor& b = tensor(v[1], c.dev, ScalarType::Char);
+    need(a.dim() == 3 && b.dim() == 3 && a.size(0) == b.size(0));
+    const int kn = v[2] == Py_True;  // b is [B, K, N]
+    need(a.size(2) == b.size(kn ? 1 : 2));
+    const int64_t B = a.size(0), M = a.size(1), K = a.size(2), N = b.size(kn ? 2 : 1);
+    const int dt = (int)integer(v[6]);
+    Tensor out;
+    if (v[4] == Py_None) {
+      out = c.empty({B, M, N}, out_type(dt));
+    } else {
+      out = tensor(v[4], c.dev, out_type(dt));
+      need(out.dim() == 3 && out.size(0) == B && out.size(1) == M && out.size(2) == N);
+    }
+    const int rc = ti_bmm_i8_config((const int8_t*)ptr(a), a.stride(0), a.stride(1), a.stride(2), (const int8_t*)ptr(b), b.stride(0),
+                                    b.stride(kn ? 2 : 1), b.stride(kn ? 1 : 2), mptr(out), out.stride(0), out.stride(1), out.stride(2),
+                                    int32_size(B), int32_size(M), int32_size(N), int32_size(K), nullptr, TI_BIAS_NONE,
+                                    scale(v[3], c.dev), nullptr, (int)integer(v[5]), dt, (int)integer(v[7]), (int)integer(v[8]), c.stream);
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// linear_residual(a, w, bias, alpha, beta, residual): linear_a8_w8_bfp32_ofp32_residual without `out`
+PyObject* linear_residual(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* {
+    const Tensor& a = tensor(v[0], -1, ScalarType::Char);
+    const Call c(a);
+    const Tensor& w = tensor(v[1], c.dev, ScalarType::Char);
+    need(w.dim() == 2 && w.stride(1) == 1);
+    const int64_t N = w.size(0);
+    const Rows r(a, w.size(1));
+    const float *bias = (const float*)vector(v[2], c.dev, ScalarType::Float, N), *alpha = scale(v[3], c.dev), *beta = scale(v[4], c.dev);
+    need(alpha && beta);
+    const float* res = (const float*)vector(v[5], c.dev, ScalarType::Float, (int64_t)r.M * N);
+    need(res);
+    Tensor out = c.empty(with_last(a, N), ScalarType::Float);
+    const int rc = ti_linear_i8_residual_f32((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), w.stride(0), bias, alpha, beta, res, N,
+                                             (float*)mptr(out), N, r.M, int32_size(N), r.K, c.stream);
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// layernorm_q(x, weight, bias, eps, rms, round_mode)
+PyObject* layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* {
+    const Tensor& x = tensor(v[0], -1, ScalarType::Float);
+    const Call c(x);
+    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
+    const int64_t N = x.size(-1);
+    const float *g = (const float*)vector(v[1], c.dev, ScalarType::Float, N), *b = (const float*)vector(v[2], c.dev, ScalarType::Float, N);
+    need(g);
+    Tensor out = c.empty(x.sizes(), ScalarType::Char);
+    const int rc = ti_layernorm_q((const float*)ptr(x), N, g, b, (float)number(v[3]), (int8_t*)mptr(out), N, int32_size(x.numel() / N),
+                                  int32_size(N), v[4] == Py_True, (int)integer(v[5]), nullptr, nullptr, c.stream);
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// dq_add_layernorm_q(acc, scale, residual, gamma, beta, eps, round_mode) -> (residual_out, int8)
+PyObject* dq_add_layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 7, [&]() -> PyObject* {
+    const Tensor& acc = tensor(v[0], -1, ScalarType::Int);
+    const Call c(acc);
+    const Tensor& res = tensor(v[2], c.dev, ScalarType::Float);
+    need(acc.dim() >= 1 && acc.is_contiguous() && res.is_contiguous() && acc.sizes() == res.sizes() && acc.size(-1) > 0);
+    const int64_t H = acc.size(-1);
+    const float *g = (const float*)vector(v[3], c.dev, ScalarType::Float, H), *b = (const float*)vector(v[4], c.dev, ScalarType::Float, H);
+    need(g);
+    const float s = (float)number(v[1]);
+    Tensor rout = c.empty(acc.sizes(), ScalarType::Float), y = c.empty(acc.sizes(), ScalarType::Char);
+    const int rc = ti_dq_add_layernorm_q((const int32_t*)ptr(acc), H, s, nullptr, (const float*)ptr(res), H, g, b, (float)number(v[5]),
+                                         (float*)mptr(rout), H, (int8_t*)mptr(y), H, nullptr, H, int32_size(acc.numel() / H), int32_size(H),
+                                         (int)integer(v[6]), nullptr, nullptr, c.stream);
+    need(rc == TI_OK);
+    PyObject* pair = PyTuple_New(2);
+    PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(rout));
+    PyTuple_SET_ITEM(pair, 1, THPVariable_Wrap(y));
+    return pair;
+  });
+}
+
+// layernorm_fp(x, skip, weight, bias, eps, rms, want_out, want_skip_out) -> (out or None, skip_out or None)
+PyObject* layernorm_fp(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 8, [&]() -> PyObject* {
+    const Tensor& x = tensor(v[0]);
+    const Call c(x);
+    const ScalarType type = x.scalar_type();
+    const int dt = dtype_code(type);
+    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
+    const int64_t N = x.size(-1);
+    const void *g = vector(v[2], c.dev, type, N), *b = vector(v[3], c.dev, type, N), *skip = nullptr;
+    need(g);
+    if (v[1] != Py_None) {
+      const Tensor& s = tensor(v[1], c.dev, type);
+      need(s.is_contiguous() && s.numel() == x.numel() && s.size(-1) == N);
+      skip = ptr(s);
+    }
+    Tensor out, sout;
+    if (v[6] == Py_True) out = c.empty(x.sizes(), type);
+    if (v[7] == Py_True) sout = c.empty(x.sizes(), type);
+    const int rc = ti_layernorm_fp(ptr(x), N, skip, skip ? N : 0, dt, g, b, (float)number(v[4]), v[5] == Py_True,
+                                   out.defined() ? mptr(out) : nullptr, N, sout.defined() ? mptr(sout) : nullptr, N,
+                                   int32_size(x.numel() / N), int32_size(N), c.stream);
+    need(rc == TI_OK);
+    PyObject* pair = PyTuple_New(2);
+    const Tensor* both[2] = {&out, &sout};
+    for (int i = 0; i < 2; ++i) {
+      PyObject* o = both[i]->defined() ? THPVariable_Wrap(*both[i]) : (Py_INCREF(Py_None), Py_None);
+      PyTuple_SET_ITEM(pair, i, o);
+    }
+    return pair;
+  });
+}
+
+// gelu_q(x, scale, round_mode)
+PyObject* gelu_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 3, [&]() -> PyObject* {
+    const Tensor& x = tensor(v[0], -1, ScalarType::Float);
+    const Call c(x);
+    need(x.is_contiguous());
+    const float* s = scale(v[1], c.dev);
+    need(s);
+    Tensor out = c.empty(x.sizes(), ScalarType::Char);
+    need(ti_gelu_q((const float*)ptr(x), s, (int8_t*)mptr(out), x.numel(), (int)integer(v[2]), c.stream) == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// softmax_q(x, scale, causal_q_len)
+PyObject* softmax_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 3, [&]() -> PyObject* {
+    const Tensor& x = tensor(v[0], -1, ScalarType::Char);
+    const Call c(x);
+    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
+    const int64_t cols = x.size(-1);
+    Tensor out = c.empty(x.sizes(), ScalarType::Char);
+    const int rc = ti_softmax_q((const int8_t*)ptr(x), cols, (float)number(v[1]), (int8_t*)mptr(out), cols, int32_size(x.numel() / cols),
+                                int32_size(cols), (int)integer(v[2]), c.stream);
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// quantize_per_token(x) -> (int8, scale)
+PyObject* quantize_per_token(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 1, [&]() -> PyObject* {
+    const Tensor& x = tensor(v[0]);
+    const Call c(x);
+    need(x.scalar_type() == ScalarType::Float || x.scalar_type() == ScalarType::Half);
+    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
+    const int64_t cols = x.size(-1);
+    Tensor q = c.empty(x.sizes(), ScalarType::Char), s = c.empty(with_last(x, 1), x.scalar_type());
+    const int rc = ti_quantize_per_token_absmax(ptr(x), dtype_code(x.scalar_type()), cols, (int8_t*)mptr(q), cols, mptr(s),
+                                                int32_size(x.numel() / cols), int32_size(cols), c.stream);
+    need(rc == TI_OK);
+    PyObject* pair = PyTuple_New(2);
+    PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(q));
+    PyTuple_SET_ITEM(pair, 1, THPVariable_Wrap(s));
+    return pair;
+  });
+}
+
+// strides of [seqs, heads, rows, D] or [heads, rows, D] with unit last stride
+struct Heads {
+  int64_t ss, hs, rs;
+  int seqs, heads;
+  explicit Heads(const Tensor& t) {
+    const int64_t d = t.dim();
+    need(d == 3 || d == 4);
+    need(t.stride(d - 1) == 1 || t.size(d - 1) == 1);
+    ss = d == 4 ? t.stride(0) : 0;
+    hs = t.stride(d - 3);
+    rs = t.stride(d - 2);
+    seqs = d == 4 ? int32_size(t.size(0)) : 1;
+    heads = int32_size(t.size(d - 3));
+  }
+};
+
+// attention(q, k, vt, qk_alpha, score_scale, pv_alpha, causal_q_len, out)
+PyObject* attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 8, [&]() -> PyObject* {
+    const Tensor& q = tensor(v[0], -1, ScalarType::Char);
+    const Call c(q);
+    const Tensor &k = tensor(v[1], c.dev, ScalarType::Char), &vt = tensor(v[2], c.dev, ScalarType::Char);
+    const Heads hq(q), hk(k), hv(vt);
+    const int64_t S = q.size(-2), D = q.size(-1), T = k.size(-2);
+    need(k.dim() == q.dim() && vt.dim() == q.dim() && hk.seqs == hq.seqs && hv.seqs == hq.seqs && hk.heads == hq.heads && hv.heads == hq.heads);
+    need(k.size(-1) == D && vt.size(-2) == D && vt.size(-1) == T);
+    Tensor out;
+    if (v[7] == Py_None) {
+      out = c.empty(q.sizes(), ScalarType::Char);
+    } else {
+      out = tensor(v[7], c.dev, ScalarType::Char);
+      need(out.sizes() == q.sizes());
+    }
+    const Heads ho(out);
+    const int rc = ti_attention_i8_heads((const int8_t*)ptr(q), hq.ss, hq.hs, hq.rs, (const int8_t*)ptr(k), hk.ss, hk.hs, hk.rs,
+                                         (const int8_t*)ptr(vt), hv.ss, hv.hs, hv.rs, (int8_t*)mptr(out), ho.ss, ho.hs, ho.rs, hq.seqs,
+                                         hq.heads, int32_size(S), int32_size(T), int32_size(D), (float)number(v[3]), (float)number(v[4]),
+                                         (float)number(v[5]), (int)integer(v[6]), c.stream);
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// A K cache [seqs*heads, T, D] and a V^T cache [seqs*heads, D, T]: addresses of the last S positions
+struct Caches {
+  int64_t BH, T, D;
+  int8_t *k = nullptr, *vt;
+  int64_t k_hs = 0, k_rs = 0, vt_rs;
+  Caches(PyObject* ko, PyObject* vo, int dev, int64_t S) {
+    const Tensor& v = tensor(vo, dev, ScalarType::Char);
+    need(v.dim() == 3);
+    BH = v.size(0), D = v.size(1), T = v.size(2);
+    need(D % 16 == 0 && S <= T && (v.stride(2) == 1 || T == 1) && (v.stride(0) == D * v.stride(1) || BH == 1));
+    vt_rs = v.stride(1);
+    vt = (int8_t*)mptr(v) + (T - S);
+    if (ko == Py_None) return;
+    const Tensor& kc = tensor(ko, dev, ScalarType::Char);
+    need(kc.dim() == 3 && kc.size(0) == BH && kc.size(1) == T && kc.size(2) == D && kc.stride(2) == 1);
+    k_hs = kc.stride(0), k_rs = kc.stride(1);
+    k = (int8_t*)mptr(kc) + (T - S) * k_rs;
+  }
+};
+
+// qkv_decode(a, w3, bias3, alpha3, beta3, k_cache, vt_cache, seqs)
+PyObject* qkv_decode(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 8, [&]() -> PyObject* {
+    const Tensor& a = tensor(v[0], -1, ScalarType::Char);
+    const Call c(a);
+    const Tensor& w = tensor(v[1], c.dev, ScalarType::Char);
+    const int64_t seqs = integer(v[7]);
+    need(a.dim() == 2 && w.dim() == 2 && w.is_contiguous() && w.size(0) % 3 == 0 && seqs > 0 && a.size(0) % seqs == 0 && a.size(0) <= 16);
+    const Rows r(a, w.size(1));
+    const int64_t N = w.size(0) / 3;
+    const Caches kv(v[5], v[6], c.dev, r.M / seqs);
+    need(kv.k && kv.BH * kv.D == seqs * N && r.K >= 1024);
+    const int8_t* bias = (const int8_t*)vector(v[2], c.dev, ScalarType::Char, 3 * N);
+    const float *al = (const float*)vector(v[3], c.dev, ScalarType::Float, 3), *be = (const float*)vector(v[4], c.dev, ScalarType::Float, 3);
+    need(bias && al && be);
+    Tensor out = c.empty({r.M, 3 * N}, ScalarType::Char);
+    const int rc = ti_qkv_decode_i8_seqs((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), r.K, bias, al, be, (int8_t*)mptr(out), 3 * N,
+                                         (int)seqs, r.M, int32_size(N), r.K, kv.k, kv.k_hs, kv.k_rs, kv.vt, kv.vt_rs, (int)kv.D, c.stream);
+    need(rc == TI_OK);
+    return THPVariable_Wrap(out);
+  });
+}
+
+// kv_append(k_new, v_new, k_cache, vt_cache, seqs) -> True
+PyObject* kv_append(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 5, [&]() -> PyObject* {
+    const Tensor& vn = tensor(v[1], -1, ScalarType::Char);
+    const Call c(vn);
+    const int64_t seqs = integer(v[4]);
+    need(vn.dim() == 2 && vn.stride(1) == 1 && seqs > 0 && vn.size(0) % seqs == 0);
+    const int64_t S = vn.size(0) / seqs;
+    const Caches kv(v[2], v[3], c.dev, S);
+    need(kv.BH % seqs == 0 && kv.BH / seqs * kv.D == vn.size(1));
+    const int8_t* ksrc = nullptr;
+    int64_t k_rs = 0;
+    if (kv.k) {
+      const Tensor& kn = tensor(v[0], c.dev, ScalarType::Char);
+      need(kn.sizes() == vn.sizes() && kn.stride(1) == 1);
+      ksrc = (const int8_t*)ptr(kn);
+      k_rs = kn.stride(0);
+    }
+    const int rc = ti_kv_append_i8_seqs(ksrc, k_rs, (const int8_t*)ptr(vn), vn.stride(0), kv.k, kv.k_hs, kv.k_rs, kv.vt, kv.vt_rs, (int)seqs,
+                                        int32_size(S), (int)(kv.BH / seqs), (int)kv.D, c.stream);
+    need(rc == TI_OK);
+    Py_RETURN_TRUE;
+  });
+}
+
+#define TI_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    TI_METHOD(linear), TI_METHOD(bmm), TI_METHOD(linear_residual), TI_METHOD(layernorm_q), TI_METHOD(dq_add_layernorm_q),
+    TI_METHOD(layernorm_fp), TI_METHOD(gelu_q), TI_METHOD(softmax_q), TI_METHOD(quantize_per_token), TI_METHOD(attention),
+    TI_METHOD(qkv_decode), TI_METHOD(kv_append), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host path of the launchers (see csrc/host.cpp).", -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }

@@ -62,7 +62,11 @@ def launch_bmm(a3, b3, c3, *, epilogue, bias=None, alpha=None, beta=None, round_
 
 def linear(a, w, *, epilogue, out_dtype, bias=None, alpha=None, beta=None, out=None,
            round_mode=L.ROUND_RNE_CLAMP, config=-1):
-    """Common body of the linear_* launchers (reference: kernels/linear.py:257-288 and siblings)."""
+    """Common body of the linear_* launchers (reference: kernels/linear.py:257-288 and siblings).  The ordinary
+    call is one function of the extension module; what it declines is converted or refused here."""
+    y = L.host.linear(a, w, bias, alpha, beta, out, epilogue, L.TORCH_TO_DT[out_dtype], round_mode, config, 0)
+    if y is not None:
+        return y
     tmp_shape = a.shape[:-1]
     assert len(w.shape) == 2
     assert a.shape[-1] == w.shape[1], "Incompatible dimensions"
@@ -82,7 +86,10 @@ def linear(a, w, *, epilogue, out_dtype, bias=None, alpha=None, beta=None, out=N
 
 
 def bmm(a, b, *, b_is_kn, epilogue, out_dtype, alpha=None, out=None, round_mode=L.ROUND_RNE_CLAMP, config=-1):
-    """Common body of the bmm_* launchers (reference: kernels/bmm.py:577-612 and siblings)."""
+    """Common body of the bmm_* launchers (reference: kernels/bmm.py:577-612 and siblings); as in `linear`."""
+    y = L.host.bmm(a, b, b_is_kn, alpha, out, epilogue, L.TORCH_TO_DT[out_dtype], round_mode, config)
+    if y is not None:
+        return y
     tmp_shape = a.shape[:-1]
     assert len(a.shape) == 3 and len(b.shape) == 3
     assert a.shape[0] == b.shape[0]
@@ -108,6 +115,9 @@ def linear_group(a, w, groups, *, epilogue, out_dtype, bias=None, alpha=None, be
     [groups*N, K], bias [groups*N], alpha / beta fp32 device tensors [groups].  Returns
     [*, groups*N]: projection g is columns g*N .. g*N+N.  Same arithmetic per projection as
     `linear` (reference: kernels/linear.py:257-288 launched once per projection)."""
+    y = L.host.linear(a, w, bias, alpha, beta, out, epilogue, L.TORCH_TO_DT[out_dtype], round_mode, config, groups)
+    if y is not None:
+        return y
     tmp_shape = a.shape[:-1]
     assert len(w.shape) == 2 and w.shape[0] % groups == 0
     assert a.shape[-1] == w.shape[1], "Incompatible dimensions"

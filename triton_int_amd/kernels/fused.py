@@ -25,6 +25,10 @@ def layer_norm_fwd_fused_single_pass_q(x, weight, bias, eps, use_rms_norm=False,
                                        _return_stats=False):
     """LayerNorm (or RMSNorm) over the last dim, output quantised to int8
     (reference: kernels/fused.py:336-382)."""
+    if not _return_stats:
+        y = L.host.layernorm_q(x, weight, bias, eps, use_rms_norm, _round_mode)
+        if y is not None:
+            return y
     assert x.dtype == weight.dtype, f"input and weight bias must have the same dtype: {x.dtype}, {weight.dtype}"
     if bias is not None:
         assert x.dtype == bias.dtype, f"input and bias must have the same dtype: {x.dtype}, {bias.dtype}"
@@ -53,12 +57,16 @@ def layer_norm_fwd_fused_single_pass_q(x, weight, bias, eps, use_rms_norm=False,
 
 
 def _layernorm_fp(x, skip, weight, bias, eps, use_rms_norm, want_out, want_skip_out):
+    # catch eps being too small if the tensors are fp16 (kernels/fused.py:501-503)
+    y = L.host.layernorm_fp(x, skip, weight, bias, max(eps, 1.6e-5) if x.dtype == torch.float16 else eps, use_rms_norm, want_out,
+                            want_skip_out)
+    if y is not None:
+        return y
     assert x.dtype == weight.dtype, f"input and weight bias must have the same dtype: {x.dtype}, {weight.dtype}"
     if bias is not None:
         assert x.dtype == bias.dtype, f"input and bias must have the same dtype: {x.dtype}, {bias.dtype}"
     assert x.dtype in (torch.float32, torch.float16, torch.bfloat16), f"floating-point LayerNorm takes fp32 / fp16 / bf16, got {x.dtype}"
     L.require_cuda(x, weight, bias, skip)
-    # catch eps being too small if the tensors are fp16 (kernels/fused.py:501-503)
     if x.dtype == torch.float16:
         eps = max(eps, 1.6e-5)
     N = x.shape[-1]
@@ -110,6 +118,10 @@ def dq_add_layernorm_q(input_int32, input_scale_fp, residual_input_fp, gamma, be
     int8) — or the fp32 LayerNorm output when quantize=False.  Semantics of
     functional/fused.py:6-24; the argument order is that of the intended native op,
     functional/fused.py:27-32."""
+    if quantize and not _return_stats:
+        y = L.host.dq_add_layernorm_q(input_int32, input_scale_fp, residual_input_fp, gamma, beta, eps, _round_mode)
+        if y is not None:
+            return y
     L.require_cuda(input_int32, residual_input_fp, gamma, beta)
     assert input_int32.dtype == torch.int32, "input_int32 must be int32"
     assert input_int32.shape == residual_input_fp.shape, "Incompatible dimensions"
@@ -155,6 +167,9 @@ def dq_add_layernorm_q(input_int32, input_scale_fp, residual_input_fp, gamma, be
 
 def gelu_q(x, scale, *, _round_mode=L.ROUND_RNE_CLAMP):
     """q8(gelu_tanh(x) * scale) element-wise, x fp32 -> int8 (math of kernels/fused.py:76-79)."""
+    y = L.host.gelu_q(x, scale, _round_mode)
+    if y is not None:
+        return y
     L.require_cuda(x)
     x = x.to(torch.float32).contiguous()
     y = torch.empty(x.shape, dtype=torch.int8, device=x.device)
@@ -170,6 +185,9 @@ def softmax_q(x, scale, causal_q_len=0):
     The reference has no kernel for this step (callers of its BMM modules do it in fp32 torch between
     bmm_s8t_s8n_s8t and the P.V BMM).  `scale` is a python float; causal_q_len > 0 masks position i of
     every group of causal_q_len rows to columns 0 .. i + (cols - causal_q_len)."""
+    y = L.host.softmax_q(x, scale, causal_q_len)
+    if y is not None:
+        return y
     L.require_cuda(x)
     assert x.dtype == torch.int8, "scores must be int8"
     cols = x.shape[-1]
@@ -211,6 +229,9 @@ def attention_i8(q, k, vt, qk_alpha, score_scale, pv_alpha, causal_q_len=0, out=
     along the last dimension; `out` may be any int8 [BH,S,128] view with unit last stride (e.g. the
     head-merged [S, heads, 128] layout).  All four may be 4-D instead, [B,heads,...] views with any
     strides of the two leading dimensions: all sequences in one launch.  Scalars are python floats."""
+    y = L.host.attention(q, k, vt, qk_alpha, score_scale, pv_alpha, causal_q_len, out)
+    if y is not None:
+        return y
     L.require_cuda(q, k, vt, out)
     assert q.dtype == torch.int8 and k.dtype == torch.int8 and vt.dtype == torch.int8, "operands must be int8"
     assert q.dim() in (3, 4) and k.dim() == q.dim() and vt.dim() == q.dim(), "q, k, vt must be all 3-D or all 4-D"
@@ -243,6 +264,9 @@ def quantize_per_token_absmax(t):
     and q = clamp(round(t / max_val), -128, 127), bit-identical to
     dynamic_quantize_activation_per_token_absmax (reference: functional/quantization.py:61-67).
     Unlike that helper it leaves `t` untouched."""
+    y = L.host.quantize_per_token(t)
+    if y is not None:
+        return y
     L.require_cuda(t)
     assert t.dtype in (torch.float32, torch.float16), "activations must be fp32 or fp16"
     cols = t.shape[-1]
@@ -265,6 +289,8 @@ def kv_append_i8(k_new, v_new, k_cache, vt_cache, seqs=1):
     projection); k_cache int8 [seqs*heads, T, D]; vt_cache int8 [seqs*heads, D, T], both contiguous or views
     of longer caches.  k_cache = None (k_new is then ignored) writes V^T only.  Replaces
     `k_cache[:, T-S:, :] = k_new.view(S, heads, D).transpose(0, 1)` and the V transpose."""
+    if L.host.kv_append(k_new, v_new, k_cache, vt_cache, seqs):
+        return
     L.require_cuda(v_new, k_cache, vt_cache)
     BH, D, T = vt_cache.shape
     M, H = v_new.shape

@@ -73,6 +73,10 @@ def linear_a8_w8_bfp32_ofp32_residual(a, b, bias, scale_a, scale_b, residual, ou
     decode kernel adds the residual while it stores, the persistent kernels that serve large outputs add it in
     their epilogue, otherwise an add kernel follows the GEMM.
     `out` must not overlap `residual`."""
+    if out is None:
+        y = L.host.linear_residual(a, b, bias, scale_a, scale_b, residual)
+        if y is not None:
+            return y
     L.require_cuda(a, b, bias, residual, out)
     assert a.dtype == torch.int8 and b.dtype == torch.int8, "operands must be int8"
     assert len(b.shape) == 2 and a.shape[-1] == b.shape[1], "Incompatible dimensions"
@@ -115,6 +119,10 @@ def linear_qkv_decode_a8_w8_b8_o8(a, w3, bias3, scale_a3, scale_b3, k_cache, vt_
     of every sequence in their last S slots.  Returns the [seqs*S, 3N] int8 projections, or None when the
     shapes do not fit the decode kernel (the caller then uses `linear_group_a8_w8_b8_o8` and
     `kv_append_i8`)."""
+    if out is None:
+        y = L.host.qkv_decode(a, w3, bias3, scale_a3, scale_b3, k_cache, vt_cache, seqs)
+        if y is not None:
+            return y
     L.require_cuda(a, w3, bias3, scale_a3, scale_b3, k_cache, vt_cache, out)
     M, K = a.shape
     N = w3.shape[0] // 3

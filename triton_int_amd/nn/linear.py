@@ -2,7 +2,7 @@
 
 Same class names, constructor arguments, buffer names (`weight` int8 [out,in], `bias`, 0-dim fp32
 scales `a`, `b`) and `from_float` algebra as the reference, so state_dicts interchange.  `forward`
-flattens the leading dims, calls the HIP launcher and restores the shape.
+calls the HIP launcher, which takes any leading dims.
 """
 from __future__ import annotations
 
@@ -45,14 +45,12 @@ class _Int8Linear(torch.nn.Module):
                 setattr(self, name, t.to(torch.float32))
         return self
 
-    def _launch(self, x2d):
+    def _launch(self, x):
         raise NotImplementedError
 
-    @torch.no_grad()
     def forward(self, x):
-        lead = x.shape[:-1]
-        y = self._launch(x.view(-1, x.shape[-1]))
-        return y.view(*lead, -1)
+        # the launchers take any leading dimensions, and their outputs are never part of an autograd graph
+        return self._launch(x)
 
 
 def _scale_tensor(v):
@@ -131,10 +129,7 @@ class W8A8BFP32OFP32Linear(_Int8Linear):
     @torch.no_grad()
     def forward_add(self, x, residual):
         """forward(x) + residual (fp32, same shape as the output) as one library call."""
-        lead = x.shape[:-1]
-        y = linear_a8_w8_bfp32_ofp32_residual(x.view(-1, x.shape[-1]), self.weight, self.bias, self.a, self.b,
-                                              residual.reshape(-1, self.out_features))
-        return y.view(*lead, -1)
+        return linear_a8_w8_bfp32_ofp32_residual(x, self.weight, self.bias, self.a, self.b, residual)
 
     @classmethod
     def from_float(cls, module: torch.nn.Linear, input_scale):
