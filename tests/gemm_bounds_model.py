@@ -446,5 +446,15 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
                 lo = row_off + tail[None, :]
                 assert (lo >= 0).all() and (lo + 16 <= alloc).all(), f"skinny {what}: K-tail load outside the operand"
         return stats
+    if name.startswith("ragged"):
+        # rows are clamped to the last one and no load leaves a row (a chunk across a row's end is loaded as the row's
+        # last 16 bytes): what can go wrong is the grid and a row that is not inside the operand
+        BM, BN = (int(x) for x in re.match(r"ragged_(\d+)x(\d+)x64", name).groups())
+        assert pl.tiles_m == -(-pr.M // BM) and pl.tiles_n == -(-pr.N // BN) and pl.threads == 256
+        assert pl.grid_x == pl.tiles_m * pl.tiles_n and pl.grid_y == pr.batch
+        assert (pr.batch - 1) * pr.sAb + (pr.M - 1) * pr.sAm + pr.K <= pr.a_bytes()
+        b_rows, b_len, ld = (pr.N, pr.K, pr.sBn) if pr.sBk == 1 else (pr.K, pr.N, pr.sBk)
+        assert (pr.batch - 1) * pr.sBb + (b_rows - 1) * ld + b_len <= pr.b_bytes()
+        return stats
     assert name.startswith("gather"), name
     return stats

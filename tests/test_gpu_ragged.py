@@ -101,3 +101,37 @@ def test_row_piece_kernel_edges(M, N, K):
     assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one), want)
     assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one, dtype=torch.float16), want.half())
     assert torch.equal(linear.linear_a8_w8_bfp32_ofp32_residual(a, w, bf, alpha, one, res), want + res)
+
+
+@pytest.mark.parametrize("B,M,N,K", [(1, 1, 1, 1), (2, 65, 63, 15), (3, 130, 129, 17), (40, 128, 128, 333), (2, 64, 16, 64), (1, 300, 1000, 1001),
+                                     (70, 129, 200, 31), (1, 17, 8, 130), (5, 1, 128, 777)])
+def test_ragged_kernel_any_alignment_and_layout(B, M, N, K):
+    """Rows that start anywhere (views of a padded buffer at an odd offset), any K, b as [B,N,K] and as [B,K,N],
+    both tile sizes: exact against torch in float64; what surrounds the operands must not matter."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import bmm
+
+    lib = L.lib()
+    g = torch.Generator(device="cuda").manual_seed(B + M + N + K)
+
+    def view(rows, cols):  # [B, rows, cols] at an odd offset of rows of cols + 3
+        buf = torch.randint(-128, 128, (B, rows, cols + 3), dtype=torch.int8, device="cuda", generator=g)
+        return buf[:, :, 1:cols + 1]
+
+    a, b_nk, b_kn = view(M, K), view(N, K), view(K, N)
+    alpha = torch.tensor(30.0 / (K ** 0.5 * 5400.0), device="cuda")
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    for b, kn in ((b_nk, False), (b_kn, True)):
+        acc = (a.double() @ (b if kn else b.transpose(1, 2).contiguous()).double()).to(torch.int32)
+        for cfg in [-1] + [i for i, nm in enumerate(names) if nm.startswith("ragged")]:
+            got = (bmm.bmm_s8t_s8t_s32t if kn else bmm.bmm_s8t_s8n_s32t)(a, b, _config=cfg)
+            assert torch.equal(got, acc), (kn, cfg)
+            if not (M == N == K == 1):
+                assert lib.ti_gemm_config_name(lib.ti_gemm_last_config()).decode().startswith("ragged")
+            got8 = (bmm.bmm_s8t_s8t_s8t if kn else bmm.bmm_s8t_s8n_s8t)(a, b, alpha, _config=cfg)
+            assert torch.equal(got8, (alpha * acc.float()).round().clamp(-128, 127).to(torch.int8)), (kn, cfg)
+    # fp32 output, and an int8 output whose rows start anywhere
+    assert torch.equal(bmm.bmm_s8t_s8n_f32t(a, b_nk, alpha), alpha * (a.double() @ b_nk.double().transpose(1, 2).contiguous()).float())
+    out = torch.full((B, M, N + 5), 77, dtype=torch.int8, device="cuda")
+    bmm.bmm_s8t_s8t_s8t(a, b_kn, alpha, out=out[:, :, 3:N + 3])
+    assert torch.equal(out[:, :, 3:N + 3], bmm.bmm_s8t_s8t_s8t(a, b_kn, alpha)) and bool((out[:, :, :3] == 77).all() and (out[:, :, N + 3:] == 77).all())

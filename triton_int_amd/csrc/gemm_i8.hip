@@ -11,8 +11,9 @@
 //   gemm_rowpieces_kernel    M <= 64: weight rows dealt evenly to the CUs, the whole K in one workgroup.
 //   gemm_rows4_kernel        M <= 16 against a few rows of a long K: weights as whole 1 KB row pieces.
 //   gemm_skinny_kernel       M <= 64, batched: 16-row weight slabs in MFMA layout, K split over waves.
-//   gemm_gather_kernel       any strides / alignment / K (byte gathers).
-// All but the last need both operands K-contiguous and 16-byte aligned: 128-bit buffer loads
+//   gemm_ragged_kernel       rows that start at any byte, any K, [K,N] operands (unaligned loads through registers).
+//   gemm_gather_kernel       any strides (byte gathers).
+// All but the last two need both operands K-contiguous and 16-byte aligned: 128-bit buffer loads
 // straight into XOR-swizzled LDS tiles, several stages deep.
 //
 // C = epilogue(sum_k A[m,k] * B[n,k]); A is [M,K], B is [N,K] (the reference's "N" operand,
@@ -323,6 +324,133 @@ __device__ __forceinline__ void wait_loads_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// ---- epilogue of the one-tile kernels: one wave's (TM*32) x (TN*32) block at (mw, nw), any output layout (int8:
+// unit column stride) ------------------------------------------------------------------------------
+template <int TM, int TN, int OUTCLS>
+__device__ __forceinline__ void tile_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz, int mw, int nw, int lane) {
+  // The per-element code below is fully unrolled over the accumulator registers, so everything
+  // that depends on the epilogue kind is decided once, outside the unrolled part: one uniform
+  // branch selects a specialised body, and the remaining run-time options (rounding mode, ReLU,
+  // bias present) are folded into branch-free selects.
+  char* Cb = (char*)p.C;
+  const int lrow = lane & 31, lhi = lane >> 5;
+  const bool has_bias = e.bias_kind != TI_BIAS_NONE;
+
+  if constexpr (OUTCLS == OUT8) {
+    // acc[i][j][r]: m = mw + i*32 + lrow;  n = nw + j*32 + 8*(r/4) + 4*lhi + r%4.
+    // Quantise and pack 4 consecutive n into a dword X[g] (g = r/4).  Lanes l and l+32 hold the two
+    // halves of every 8-byte group of a row, so two half-wave swaps, (X0, X2) and (X1, X3), leave
+    // lane l with bytes 0..15 and lane l+32 with bytes 16..31 of the row's 32-byte segment: one
+    // 16-byte store per 32x32 block and lane, no trip through LDS.
+    // Per element: cvt, mul, (add), clamp in fp32 (v_med3_f32), then one add of 1.5*2^23: that
+    // add rounds to the nearest integer, ties to even, and leaves the two's-complement int8 in the
+    // low byte of the float's bit pattern.  Clamping first keeps the sum in the exact range; since
+    // the bounds are integers, clamp-then-round equals round-then-clamp.  ReLU is a lower bound of 0.
+    // (Truncation, the test-time rounding switch, is served by the gather kernel instead.)
+    const float q_floor = e.epilogue == TI_EPI_SCALE_RELU_I8 ? 0.0f : -128.0f;
+    int8_t* Cz = (int8_t*)Cb + (int64_t)bz * p.sCb;
+    auto body = [&](auto gelu_tag, auto bias_tag) {
+      constexpr bool GELU = decltype(gelu_tag)::value;
+      constexpr bool BIAS = decltype(bias_tag)::value;
+      auto one = [&](int a, float col) -> float {
+        float v = (float)a * e.alpha;
+        if constexpr (BIAS) v = col + v;
+        if constexpr (GELU) v = gelu_tanh_scaled(v, e.beta);
+        return __builtin_amdgcn_fmed3f(v, q_floor, 127.0f);
+      };
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int nj = nw + j * 32;
+        float col[4][4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            if constexpr (BIAS)
+              col[g][t] = column_term_t<GELU ? TI_BIAS_F32 : TI_BIAS_I8>(e, min(nj + 8 * g + 4 * lhi + t, p.N - 1), GELU);
+            else
+              col[g][t] = 0.0f;
+          }
+        const int n = nj + 16 * lhi;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          unsigned X[4];
+          float f[4][4];
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) f[g][t] = one(acc[i][j][4 * g + t], col[g][t]);
+          pack16_q8(f, X);
+          const auto s02 = __builtin_amdgcn_permlane32_swap(X[0], X[2], false, false);
+          const auto s13 = __builtin_amdgcn_permlane32_swap(X[1], X[3], false, false);
+          v4u v;
+          v[0] = s02[0]; v[1] = s02[1]; v[2] = s13[0]; v[3] = s13[1];
+          const int m = mw + i * 32 + lrow;
+          if (m >= p.M || n >= p.N) continue;
+          int8_t* dst = Cz + (int64_t)m * p.sCm + n;
+          if (n + 16 <= p.N) {
+            // one 16-byte store whatever the row's alignment (160 heads of 1001 x 1001 int8 scores from K = 128: byte stores 473 us, this 98 us)
+            __builtin_memcpy(dst, &v, 16);
+          } else {
+            const int cnt = min(16, p.N - n);
+            for (int t = 0; t < cnt; ++t) dst[t] = (int8_t)(v[t >> 2] >> ((t & 3) * 8));
+          }
+        }
+      }
+    };
+    const bool gelu = e.epilogue == TI_EPI_GELU_I8;
+    if (gelu && has_bias) body(std::true_type{}, std::true_type{});
+    else if (gelu) body(std::true_type{}, std::false_type{});
+    else if (has_bias) body(std::false_type{}, std::true_type{});
+    else body(std::false_type{}, std::false_type{});
+  } else {
+    // acc[i][j][r]: m = mw + i*32 + 8*(r/4) + 4*lhi + r%4;  n = nw + j*32 + lrow.
+    constexpr int ESZ = OUTCLS == OUT32 ? 4 : 2;
+    char* Cz = Cb + (int64_t)bz * p.sCb * ESZ;
+    // KIND: 0 raw int32 (+ int32 bias), 1 scaled -> int32, 2 scaled -> fp32, 3 -> fp16, 4 -> bf16
+    auto body = [&](auto kind_tag) {
+      constexpr int KIND = decltype(kind_tag)::value;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int n = nw + j * 32 + lrow;
+        const int nc = min(n, p.N - 1);
+        const float col = KIND == 0 ? 0.0f : column_term_t<KIND == 1 ? TI_BIAS_I32 : TI_BIAS_F32>(e, nc, false);
+        const int bias_i32 = (KIND == 0 && e.bias_kind == TI_BIAS_I32) ? ((const int*)e.bias)[nc] : 0;
+        const bool n_ok = n < p.N;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int m = mw + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
+            if (!(n_ok && m < p.M)) continue;
+            const int64_t off = (int64_t)m * p.sCm + (int64_t)n * p.sCn;
+            const int a = acc[i][j][r];
+            if constexpr (KIND == 0) {
+              ((int*)Cz)[off] = (int)((unsigned)a + (unsigned)bias_i32);
+            } else {
+              float v = (float)a * e.alpha;
+              const float vb = col + v;
+              v = has_bias ? vb : v;
+              if constexpr (KIND == 1) ((int*)Cz)[off] = q32(v, e.round_mode);
+              else if constexpr (KIND == 2) ((float*)Cz)[off] = v;
+              else if constexpr (KIND == 3) ((uint16_t*)Cz)[off] = f32_to_f16_bits(v);
+              else ((uint16_t*)Cz)[off] = f32_to_bf16_bits(v);
+            }
+          }
+        }
+      }
+    };
+    if constexpr (OUTCLS == OUT32) {
+      if (e.epilogue == TI_EPI_I32) body(std::integral_constant<int, 0>{});
+      else if (e.epilogue == TI_EPI_SCALE_I32) body(std::integral_constant<int, 1>{});
+      else body(std::integral_constant<int, 2>{});
+    } else {
+      if (p.out_dtype == TI_F16) body(std::integral_constant<int, 3>{});
+      else body(std::integral_constant<int, 4>{});
+    }
+  }
+}
+
 // OCC = workgroups the register allocation must allow per CU (short-K batched shapes want two or
 // three co-resident workgroups so that one's epilogue overlaps another's loads).
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int OCC = 1>
@@ -492,129 +620,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (WAVES_M * WAVES_N * OCC + 3
   // the trailing (out-of-bounds) loads still write zeros into LDS: drain before re-using it
   wait_loads_and_barrier<0>();
 
-  // ---- epilogue ----
-  // The per-element code below is fully unrolled over the accumulator registers, so everything
-  // that depends on the epilogue kind is decided once, outside the unrolled part: one uniform
-  // branch selects a specialised body, and the remaining run-time options (rounding mode, ReLU,
-  // bias present) are folded into branch-free selects.
   const EpiCtx e = make_epi(p, bz);
-  char* Cb = (char*)p.C;
-  const int lrow = lane & 31, lhi = lane >> 5;
-  const bool has_bias = e.bias_kind != TI_BIAS_NONE;
-
-  if constexpr (OUTCLS == OUT8) {
-    // acc[i][j][r]: m = m0 + wm*WTM + i*32 + lrow;  n = n0 + wn*WTN + j*32 + 8*(r/4) + 4*lhi + r%4.
-    // Quantise and pack 4 consecutive n into a dword X[g] (g = r/4).  Lanes l and l+32 hold the two
-    // halves of every 8-byte group of a row, so two half-wave swaps, (X0, X2) and (X1, X3), leave
-    // lane l with bytes 0..15 and lane l+32 with bytes 16..31 of the row's 32-byte segment: one
-    // 16-byte store per 32x32 block and lane, no trip through LDS.
-    // Per element: cvt, mul, (add), clamp in fp32 (v_med3_f32), then one add of 1.5*2^23: that
-    // add rounds to the nearest integer, ties to even, and leaves the two's-complement int8 in the
-    // low byte of the float's bit pattern.  Clamping first keeps the sum in the exact range; since
-    // the bounds are integers, clamp-then-round equals round-then-clamp.  ReLU is a lower bound of 0.
-    // (Truncation, the test-time rounding switch, is served by the gather kernel instead.)
-    const float q_floor = e.epilogue == TI_EPI_SCALE_RELU_I8 ? 0.0f : -128.0f;
-    int8_t* Cz = (int8_t*)Cb + (int64_t)bz * p.sCb;
-    const bool vec_ok = ((p.sCm & 15) == 0) && ((((uintptr_t)Cz) & 15) == 0);
-    auto body = [&](auto gelu_tag, auto bias_tag) {
-      constexpr bool GELU = decltype(gelu_tag)::value;
-      constexpr bool BIAS = decltype(bias_tag)::value;
-      auto one = [&](int a, float col) -> float {
-        float v = (float)a * e.alpha;
-        if constexpr (BIAS) v = col + v;
-        if constexpr (GELU) v = gelu_tanh_scaled(v, e.beta);
-        return __builtin_amdgcn_fmed3f(v, q_floor, 127.0f);
-      };
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int nj = n0 + wn * WTN + j * 32;
-        float col[4][4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            if constexpr (BIAS)
-              col[g][t] = column_term_t<GELU ? TI_BIAS_F32 : TI_BIAS_I8>(e, min(nj + 8 * g + 4 * lhi + t, p.N - 1), GELU);
-            else
-              col[g][t] = 0.0f;
-          }
-        const int n = nj + 16 * lhi;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          unsigned X[4];
-          float f[4][4];
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) f[g][t] = one(acc[i][j][4 * g + t], col[g][t]);
-          pack16_q8(f, X);
-          const auto s02 = __builtin_amdgcn_permlane32_swap(X[0], X[2], false, false);
-          const auto s13 = __builtin_amdgcn_permlane32_swap(X[1], X[3], false, false);
-          v4u v;
-          v[0] = s02[0]; v[1] = s02[1]; v[2] = s13[0]; v[3] = s13[1];
-          const int m = m0 + wm * WTM + i * 32 + lrow;
-          if (m >= p.M || n >= p.N) continue;
-          int8_t* dst = Cz + (int64_t)m * p.sCm + n;
-          if (vec_ok && n + 16 <= p.N) {
-            *(v4u*)dst = v;
-          } else {
-            const int cnt = min(16, p.N - n);
-            for (int t = 0; t < cnt; ++t) dst[t] = (int8_t)(v[t >> 2] >> ((t & 3) * 8));
-          }
-        }
-      }
-    };
-    const bool gelu = e.epilogue == TI_EPI_GELU_I8;
-    if (gelu && has_bias) body(std::true_type{}, std::true_type{});
-    else if (gelu) body(std::true_type{}, std::false_type{});
-    else if (has_bias) body(std::false_type{}, std::true_type{});
-    else body(std::false_type{}, std::false_type{});
-  } else {
-    // acc[i][j][r]: m = m0 + wm*WTM + i*32 + 8*(r/4) + 4*lhi + r%4;  n = n0 + wn*WTN + j*32 + lrow.
-    constexpr int ESZ = OUTCLS == OUT32 ? 4 : 2;
-    char* Cz = Cb + (int64_t)bz * p.sCb * ESZ;
-    // KIND: 0 raw int32 (+ int32 bias), 1 scaled -> int32, 2 scaled -> fp32, 3 -> fp16, 4 -> bf16
-    auto body = [&](auto kind_tag) {
-      constexpr int KIND = decltype(kind_tag)::value;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = n0 + wn * WTN + j * 32 + lrow;
-        const int nc = min(n, p.N - 1);
-        const float col = KIND == 0 ? 0.0f : column_term_t<KIND == 1 ? TI_BIAS_I32 : TI_BIAS_F32>(e, nc, false);
-        const int bias_i32 = (KIND == 0 && e.bias_kind == TI_BIAS_I32) ? ((const int*)e.bias)[nc] : 0;
-        const bool n_ok = n < p.N;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int m = m0 + wm * WTM + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-            if (!(n_ok && m < p.M)) continue;
-            const int64_t off = (int64_t)m * p.sCm + (int64_t)n * p.sCn;
-            const int a = acc[i][j][r];
-            if constexpr (KIND == 0) {
-              ((int*)Cz)[off] = (int)((unsigned)a + (unsigned)bias_i32);
-            } else {
-              float v = (float)a * e.alpha;
-              const float vb = col + v;
-              v = has_bias ? vb : v;
-              if constexpr (KIND == 1) ((int*)Cz)[off] = q32(v, e.round_mode);
-              else if constexpr (KIND == 2) ((float*)Cz)[off] = v;
-              else if constexpr (KIND == 3) ((uint16_t*)Cz)[off] = f32_to_f16_bits(v);
-              else ((uint16_t*)Cz)[off] = f32_to_bf16_bits(v);
-            }
-          }
-        }
-      }
-    };
-    if constexpr (OUTCLS == OUT32) {
-      if (e.epilogue == TI_EPI_I32) body(std::integral_constant<int, 0>{});
-      else if (e.epilogue == TI_EPI_SCALE_I32) body(std::integral_constant<int, 1>{});
-      else body(std::integral_constant<int, 2>{});
-    } else {
-      if (p.out_dtype == TI_F16) body(std::integral_constant<int, 3>{});
-      else body(std::integral_constant<int, 4>{});
-    }
-  }
+  tile_epilogue<TM, TN, OUTCLS>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN, lane);
 }
 
 // ---- epilogue of the persistent kernels ----------------------------------------------------------
@@ -1668,6 +1675,178 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
   if (wave == 0) TI_TL(4);
 }
 
+// ---- ragged family -------------------------------------------------------------------------------
+//
+// Operands the global -> LDS loads cannot take: rows that start at any byte or whose length is no multiple of
+// 16 (P.V over an odd number of keys), and a [K,N] operand (BKN: V as it comes out of its projection).  Global
+// loads go through registers, 16 unaligned bytes per lane, one k-tile ahead of the MFMAs, into two LDS
+// stages; two or three workgroups per CU hide what one cannot.
+//   K-contiguous rows: LDS [row][64 k], 16-byte chunk c of row r at slot c ^ ((r >> 2) & 3).
+//   [K,N] rows:        LDS [k][BN n] as they are, chunk c of row k at c ^ (k & 7) (BN = 64: c ^ (k >> 2 & 1) * 2),
+//                      read with the transposing ds_read_b64_tr_b8: 16 lanes fetch an 8 x 16 block and each
+//                      gets one column's 8 k.  The swizzles keep both kinds of reads free of bank conflicts.
+// Measured, byte gathers -> this kernel: P.V with V as [K,N], int8 out: 40 x 1024 x 128 x 1024 155 -> 17 us, 160 x 2048 x 128 x
+// 2048 2900 -> 197 us (3.6 TB/s of probabilities; the aligned V^T form on the persistent kernel: 137 us); P.V fp32 out with an
+// odd key count: 160 x 1001 x 128 x 1001 649 -> 83 us, 40 x 2047 x 128 x 2047 531 -> 88 us.
+// No byte outside an operand's rows is touched: a chunk that crosses the end of a row is loaded as the row's
+// last 16 bytes and shifted (load16_tail).
+
+// 16 bytes of `row` (of `len` bytes) from byte `at`, zeros from `len` on
+__device__ __forceinline__ v4i load16_tail(const int8_t* row, int at, int len) {
+  v4i v = {0, 0, 0, 0};
+  if (at + 16 <= len) {
+    __builtin_memcpy(&v, row + at, 16);
+  } else if (at < len) {
+    if (len >= 16) {
+      __builtin_memcpy(&v, row + len - 16, 16);
+      const int bits = (at + 16 - len) * 8;  // 8 .. 120
+      unsigned long long lo = ((unsigned long long)(unsigned)v[1] << 32) | (unsigned)v[0], hi = ((unsigned long long)(unsigned)v[3] << 32) | (unsigned)v[2];
+      lo = bits >= 64 ? hi >> (bits - 64) : (lo >> bits) | (hi << (64 - bits));
+      hi = bits >= 64 ? 0ull : hi >> bits;
+      v = (v4i){(int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32)};
+    } else {
+#pragma unroll 1
+      for (int i = len - 1; i >= at; --i) {  // shifts the bytes up one by one: no indexed register access
+        v[3] = (int)(((unsigned)v[3] << 8) | ((unsigned)v[2] >> 24));
+        v[2] = (int)(((unsigned)v[2] << 8) | ((unsigned)v[1] >> 24));
+        v[1] = (int)(((unsigned)v[1] << 8) | ((unsigned)v[0] >> 24));
+        v[0] = (int)(((unsigned)v[0] << 8) | (unsigned)(uint8_t)row[i]);
+      }
+    }
+  }
+  return v;
+}
+
+template <int BM, int BN, bool BKN, int OUTCLS>
+__global__ __launch_bounds__(256) void gemm_ragged_kernel(GemmParams p) {
+  constexpr int BK = 64, WTM = BM / 2, WTN = BN / 2, TM = WTM / 32, TN = WTN / 32;
+  constexpr int A_BYTES = BM * BK, STAGE = A_BYTES + BN * BK;
+  constexpr int A_IT = BM * 4 / 256, B_IT = BN * 4 / 256, CHN = BN / 16;
+  typedef int v2i __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) v2i lds_v2i;
+  __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  int tile_m, tile_n, bz = 0;
+  if (gridDim.y == 1) tile_coords(p, blockIdx.x, tile_m, tile_n);
+  else batch_tile_coords(p, blockIdx.x, blockIdx.y, gridDim.y, bz, tile_m, tile_n);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int8_t* Ab = p.A + (int64_t)bz * p.sAb;
+  const int8_t* Bb = p.B + (int64_t)bz * p.sBb;
+  const int KT = (p.K + BK - 1) / BK;
+
+  // this thread's chunks: rows past the last one repeat it (their products are dropped, or multiplied by the
+  // zeros that A holds past K)
+  const int8_t* arow[A_IT];
+  const int8_t* brow[B_IT];
+#pragma unroll
+  for (int i = 0; i < A_IT; ++i) arow[i] = Ab + (int64_t)min(m0 + ((i * 256 + tid) >> 2), p.M - 1) * p.sAm;
+  if constexpr (!BKN) {
+#pragma unroll
+    for (int i = 0; i < B_IT; ++i) brow[i] = Bb + (int64_t)min(n0 + ((i * 256 + tid) >> 2), p.N - 1) * p.sBn;
+  }
+  v4i ar[A_IT], br[B_IT];
+  auto fetch = [&](int kt) {
+    const int k0 = kt * BK, ka = k0 + (tid & 3) * 16;
+    const bool whole = k0 + BK <= p.K;  // uniform
+#pragma unroll
+    for (int i = 0; i < A_IT; ++i) {
+      if (whole) __builtin_memcpy(&ar[i], arow[i] + ka, 16);
+      else ar[i] = load16_tail(arow[i], ka, p.K);
+    }
+    if constexpr (BKN) {
+      const bool wide = n0 + BN <= p.N;
+#pragma unroll
+      for (int i = 0; i < B_IT; ++i) {
+        const int q = i * 256 + tid, n = n0 + (q % CHN) * 16;
+        const int8_t* row = Bb + (int64_t)min(k0 + q / CHN, p.K - 1) * p.sBk;
+        if (wide) __builtin_memcpy(&br[i], row + n, 16);
+        else br[i] = load16_tail(row, n, p.N);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < B_IT; ++i) {
+        if (whole) __builtin_memcpy(&br[i], brow[i] + ka, 16);
+        else br[i] = load16_tail(brow[i], ka, p.K);
+      }
+    }
+  };
+  auto kn_slot = [](int k, int c) { return CHN == 8 ? c ^ (k & 7) : c ^ (((k >> 2) & 1) * 2); };
+  auto stash = [&](char* st) {
+#pragma unroll
+    for (int i = 0; i < A_IT; ++i) {
+      const int q = i * 256 + tid, row = q >> 2;
+      *(v4i*)(st + row * BK + (((q & 3) ^ ((row >> 2) & 3)) * 16)) = ar[i];
+    }
+#pragma unroll
+    for (int i = 0; i < B_IT; ++i) {
+      const int q = i * 256 + tid;
+      if constexpr (BKN) {
+        const int k = q / CHN;
+        *(v4i*)(st + A_BYTES + k * BN + kn_slot(k, q % CHN) * 16) = br[i];
+      } else {
+        const int row = q >> 2;
+        *(v4i*)(st + A_BYTES + row * BK + (((q & 3) ^ ((row >> 2) & 3)) * 16)) = br[i];
+      }
+    }
+  };
+
+  v16i acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+  const int frow = lane & 31, fhalf = lane >> 5, fsw = (frow >> 2) & 3;
+  // transposed reads: 16-lane group = 16 columns x 8 k; the lane's address is half of a row of the block
+  const int tk = fhalf * 16 + ((lane & 15) >> 1), tcol = (lane >> 4) & 1, thalf = (lane & 1) * 8;
+  auto compute = [&](const char* st) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      v4i fa[TM], fb[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[i] = *(const v4i*)(st + (wm * WTM + i * 32 + frow) * BK + (((ks * 2 + fhalf) ^ fsw) * 16));
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if constexpr (BKN) {
+          const int c = (wn * WTN + j * 32) / 16 + tcol;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int k = ks * 32 + tk + h * 8;
+            const v2i t = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(st + A_BYTES + k * BN + kn_slot(k, c) * 16 + thalf));
+            fb[j][2 * h] = t[0];
+            fb[j][2 * h + 1] = t[1];
+          }
+        } else {
+          fb[j] = *(const v4i*)(st + A_BYTES + (wn * WTN + j * 32 + frow) * BK + (((ks * 2 + fhalf) ^ fsw) * 16));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          if constexpr (OUTCLS == OUT8) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
+          else acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        }
+    }
+  };
+
+  if (KT > 0) {
+    fetch(0);
+    stash(lds);
+    __syncthreads();
+    for (int kt = 0; kt < KT; ++kt) {
+      if (kt + 1 < KT) fetch(kt + 1);
+      compute(lds + (kt & 1) * STAGE);
+      if (kt + 1 < KT) stash(lds + ((kt + 1) & 1) * STAGE);  // its readers passed the barrier of k-tile kt-1
+      __syncthreads();
+    }
+  }
+  const EpiCtx e = make_epi(p, bz);
+  tile_epilogue<TM, TN, OUTCLS>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN, lane);
+}
+
 // ---- gather family -----------------------------------------------------------------------------
 // 64x64 tile, BK = 32, 4 waves each owning one 32x32 MFMA block.  Every byte is fetched on its
 // own with 64-bit addressing, so any stride pattern, alignment and K works.
@@ -2341,6 +2520,7 @@ struct Config {
   int ws_waves = 0;     // > 0: gemm_mfma_ws_kernel with this many consumer waves (it can split K)
   int max_k = 0;        // > 0: the kernel holds a tile's whole K in LDS and takes 16 <= K <= max_k only
   bool rowpieces = false;  // gemm_rowpieces_kernel: M <= bm
+  bool ragged = false;     // gemm_ragged_kernel: any alignment and K; B K-contiguous or N-contiguous
 };
 
 #define TI_FAST(BM, BN, BK, WM, WN, SWZ, NS)                                              \
@@ -2377,6 +2557,14 @@ struct Config {
         MT, 4, RP_KC, (RP_PW + RP_CW) * 64, true, false, 0, false, 0, 0, true               \
   }
 
+#define TI_RAGGED(BM, BN, BKN) \
+  {gemm_ragged_kernel<BM, BN, BKN, OUT8>, gemm_ragged_kernel<BM, BN, BKN, OUT32>, gemm_ragged_kernel<BM, BN, BKN, OUT16>}
+// gemm_ragged_kernel of a tile size for a [K,N] operand
+static KernelFn ragged_kn_kernel(int bm, int oc) {
+  static const KernelFn fns[2][3] = {TI_RAGGED(64, 64, true), TI_RAGGED(128, 128, true)};
+  return fns[bm > 64][oc];
+}
+
 enum ConfigId {
   CFG_GATHER = 0,
   CFG_TILE_256x128,   // one tile per workgroup: any output layout the fast loads allow
@@ -2400,6 +2588,8 @@ enum ConfigId {
   CFG_ROWPIECES_32,
   CFG_ROWPIECES_48,
   CFG_ROWPIECES_64,
+  CFG_RAGGED_128,      // rows at any byte, any K, [K,N] operands
+  CFG_RAGGED_64,
 };
 
 constexpr int RP_KC = 256;
@@ -2436,6 +2626,8 @@ static const Config g_configs[] = {
     TI_ROWPIECES(32),
     TI_ROWPIECES(48),
     TI_ROWPIECES(64),
+    {"ragged_128x128x64", TI_RAGGED(128, 128, false), 128, 128, 64, 256, false, false, 0, false, 0, 0, false, true},
+    {"ragged_64x64x64", TI_RAGGED(64, 64, false), 64, 64, 64, 256, false, false, 0, false, 0, 0, false, true},
 };
 static const int g_num_configs = (int)(sizeof(g_configs) / sizeof(g_configs[0]));
 
@@ -2460,6 +2652,14 @@ static bool fast_eligible(const GemmParams& p) {
   if (((int64_t)p.M + 512) * p.sAm + p.K >= lim) return false;
   if (((int64_t)p.N + 512) * p.sBn + p.K >= lim) return false;
   return true;
+}
+
+// gemm_ragged_kernel: A K-contiguous, B K- or N-contiguous, rows that do not overlap
+static bool ragged_eligible(const GemmParams& p) {
+  if (p.K <= 0 || p.sAk != 1 || (p.M > 1 && p.sAm < p.K)) return false;
+  if (out_class(p.out_dtype) == OUT8 && p.sCn != 1) return false;
+  if (p.sBk == 1) return p.N == 1 || p.sBn >= p.K;
+  return p.sBn == 1 && (p.K == 1 || p.sBk >= p.N);
 }
 
 // The stream kernels store through range-checked buffer descriptors with 32-bit offsets and, for
@@ -2539,7 +2739,12 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
 // store (row-major, aligned) go to them; the rest to the one-tile kernels.
 static int pick_config(const GemmParams& p, int* splits_out) {
   *splits_out = 1;
-  if (!fast_eligible(p)) return CFG_GATHER;
+  if (!fast_eligible(p)) {
+    if (!ragged_eligible(p)) return CFG_GATHER;
+    // small tiles where large ones would not give every CU one
+    const int64_t tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+    return tiles >= 256 ? CFG_RAGGED_128 : CFG_RAGGED_64;
+  }
   const bool stream = stream_eligible(p);
   if (p.M <= 64 && p.batch <= 4) {
     // one GEMM (or up to four grouped ones): gemm_rowpieces_kernel, except where a workgroup's share of the
@@ -2847,7 +3052,8 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
   if (config >= g_num_configs) return fail(TI_E_COMBO, "config %d out of range", config);
   const Config& k = g_configs[config];
   if (!k.fn[out_class(p.out_dtype)]) return fail(TI_E_COMBO, "config %s has no kernel for output dtype %d", k.name, p.out_dtype);
-  if (k.fast && !k.skinny && !k.rows4 && !k.rowpieces && trunc8) return fail(TI_E_COMBO, "config %s does not implement TI_ROUND_TRUNC for int8 outputs", k.name);
+  if ((k.fast || k.ragged) && !k.skinny && !k.rows4 && !k.rowpieces && trunc8) return fail(TI_E_COMBO, "config %s does not implement TI_ROUND_TRUNC for int8 outputs", k.name);
+  if (k.ragged && !ragged_eligible(p)) return fail(TI_E_COMBO, "config %s needs unit strides along K (B: along K or N) and rows that do not overlap", k.name);
   if (k.fast && !fast_eligible(p)) return fail(TI_E_COMBO, "config %s needs K-contiguous 16-byte aligned operands", k.name);
   if (k.stream_occ && !stream_eligible(p)) return fail(TI_E_COMBO, "config %s needs a row-major output with 16-byte aligned rows", k.name);
   if (k.max_k && (p.K < 16 || p.K > k.max_k)) return fail(TI_E_COMBO, "config %s needs 16 <= K <= %d", k.name, k.max_k);
@@ -3004,7 +3210,8 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
     dry->grid_x = grid.x; dry->grid_y = grid.y;
     return TI_OK;
   }
-  k.fn[out_class(p.out_dtype)]<<<grid, dim3(k.threads), 0, stream>>>(p);
+  const KernelFn fn = k.ragged && p.sBk != 1 ? ragged_kn_kernel(k.bm, out_class(p.out_dtype)) : k.fn[out_class(p.out_dtype)];
+  fn<<<grid, dim3(k.threads), 0, stream>>>(p);
   return launch_status(k.name);
 }
 
