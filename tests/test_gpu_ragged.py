@@ -135,3 +135,27 @@ def test_ragged_kernel_any_alignment_and_layout(B, M, N, K):
     out = torch.full((B, M, N + 5), 77, dtype=torch.int8, device="cuda")
     bmm.bmm_s8t_s8t_s8t(a, b_kn, alpha, out=out[:, :, 3:N + 3])
     assert torch.equal(out[:, :, 3:N + 3], bmm.bmm_s8t_s8t_s8t(a, b_kn, alpha)) and bool((out[:, :, :3] == 77).all() and (out[:, :, N + 3:] == 77).all())
+
+
+@pytest.mark.parametrize("rows,cols,q_len", [(3, 1, 0), (4, 7, 0), (6, 15, 3), (5, 17, 5), (8, 333, 8), (6, 1001, 0), (3, 1024 + 9, 3), (2, 2047, 2), (2, 8191, 0)])
+@pytest.mark.parametrize("scale", [0.0, 0.1])
+def test_softmax_q_rows_at_any_byte(rows, cols, q_len, scale):
+    """Rows of an odd pitch at an odd offset, in and out: within the oracle's stated step, equal to the contiguous call,
+    and nothing written beside the rows."""
+    import oracle as O
+    from tests.util import cpu, mismatch_report
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import fused
+
+    g = rng(rows * 10 + cols)
+    x = g.integers(-128, 128, size=(rows, cols), dtype=np.int8)
+    wide = torch.full((rows, cols + 6), 99, dtype=torch.int8, device="cuda")
+    wide[:, 3:cols + 3] = gpu(x)
+    out = torch.full((rows, cols + 4), 77, dtype=torch.int8, device="cuda")
+    rc = L.lib().ti_softmax_q(wide.data_ptr() + 3, cols + 6, scale, out.data_ptr() + 1, cols + 4, rows, cols, q_len, L.current_stream(out.device))
+    assert rc == 0
+    got = out[:, 1:cols + 1]
+    assert bool((out[:, 0] == 77).all() and (out[:, cols + 1:] == 77).all())
+    mx, rate = mismatch_report(cpu(got), O.softmax_q(x, scale, causal_q_len=q_len))
+    assert mx <= 1 and rate <= max(2e-3, 1.5 / got.numel())
+    assert torch.equal(got, fused.softmax_q(gpu(x), scale, causal_q_len=q_len))

@@ -52,31 +52,13 @@ __device__ __forceinline__ int attn_limit(const AttnParams& p, int row) {
   return p.causal_q_len > 0 ? min(p.T, (row % p.causal_q_len) + (p.T - p.causal_q_len) + 1) : p.T;
 }
 
-// 16 keys of a V^T row whose address has no alignment (a row pitch that is not a multiple of 16: a cache
-// allocated at exactly its length).  Whole chunks are one unaligned 16-byte load; the chunk that crosses T
-// is put together from bytes, because an unaligned load there could leave the allocation.
-__device__ __forceinline__ v4i load_keys_any(const int8_t* row, int col, int T) {
-  v4i v = {0, 0, 0, 0};
-  if (col + 16 <= T) {
-    __builtin_memcpy(&v, row + col, 16);
-  } else {
-#pragma unroll 1
-    for (int i = T - 1 - col; i >= 0; --i) {  // shifts the bytes up one by one: no indexed register access
-      v[3] = (int)(((unsigned)v[3] << 8) | ((unsigned)v[2] >> 24));
-      v[2] = (int)(((unsigned)v[2] << 8) | ((unsigned)v[1] >> 24));
-      v[1] = (int)(((unsigned)v[1] << 8) | ((unsigned)v[0] >> 24));
-      v[0] = (int)(((unsigned)v[0] << 8) | (unsigned)(uint8_t)row[col + i]);
-    }
-  }
-  return v;
-}
-
 // Any number of keys, all sequences of a batch in one launch: what a length that is no multiple of 16 used to
 // cost was the three-launch chain with P.V through byte gathers, once per sequence.  Whole layer, before ->
 // after: two prompts of 333 tokens (4096 wide) 377 -> 239 us, sixteen sequences decoding at position 1007
 // 1105 -> 284 us.
 //
-// VANY: rows of V^T start anywhere (load_keys_any).  Otherwise they are 16-byte aligned, and a chunk that
+// VANY: rows of V^T start anywhere (a row pitch that is no multiple of 16: a cache allocated at exactly its
+// length; load16_tail).  Otherwise they are 16-byte aligned, and a chunk that
 // crosses T is loaded whole: an aligned 16-byte chunk that holds at least one key of the row lies inside the
 // row's pitch, and the keys past T are multiplied by probabilities that are exactly 0.
 template <bool VANY>
@@ -144,7 +126,7 @@ __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
         const int vr = q_ >> 2, vc = q_ & 3;
         const int8_t* row = vb + (int64_t)vr * p.sVd;
         if constexpr (VANY) {
-          vreg[c] = load_keys_any(row, key0 + vc * 16, p.T);
+          vreg[c] = load16_tail(row, key0 + vc * 16, p.T);
         } else {
           const bool in = key0 + vc * 16 < p.T;
           vreg[c] = in ? *(const v4i*)(row + key0 + vc * 16) : (v4i){0, 0, 0, 0};
@@ -440,7 +422,7 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   const int rlast = min(row0 + 15, p.S - 1);
   const int keys = p.causal_q_len > 0 && row0 / p.causal_q_len == rlast / p.causal_q_len ? attn_limit(p, rlast) : p.T;
   auto load_v = [&](int d, int col) -> v4i {
-    if constexpr (VANY) return load_keys_any(vb + (int64_t)d * p.sVd, col, p.T);
+    if constexpr (VANY) return load16_tail(vb + (int64_t)d * p.sVd, col, p.T);
     else return __builtin_amdgcn_raw_buffer_load_b128(rV, col < keys ? d * (int)p.sVd + col : OOB, 0, 0);
   };
   const int NCH = (keys + 15) >> 4;  // 16-key chunks; rows of K past T read as zeros and are masked

@@ -1690,33 +1690,6 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
 // odd key count: 160 x 1001 x 128 x 1001 649 -> 83 us, 40 x 2047 x 128 x 2047 531 -> 88 us.
 // No byte outside an operand's rows is touched: a chunk that crosses the end of a row is loaded as the row's
 // last 16 bytes and shifted (load16_tail).
-
-// 16 bytes of `row` (of `len` bytes) from byte `at`, zeros from `len` on
-__device__ __forceinline__ v4i load16_tail(const int8_t* row, int at, int len) {
-  v4i v = {0, 0, 0, 0};
-  if (at + 16 <= len) {
-    __builtin_memcpy(&v, row + at, 16);
-  } else if (at < len) {
-    if (len >= 16) {
-      __builtin_memcpy(&v, row + len - 16, 16);
-      const int bits = (at + 16 - len) * 8;  // 8 .. 120
-      unsigned long long lo = ((unsigned long long)(unsigned)v[1] << 32) | (unsigned)v[0], hi = ((unsigned long long)(unsigned)v[3] << 32) | (unsigned)v[2];
-      lo = bits >= 64 ? hi >> (bits - 64) : (lo >> bits) | (hi << (64 - bits));
-      hi = bits >= 64 ? 0ull : hi >> bits;
-      v = (v4i){(int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32)};
-    } else {
-#pragma unroll 1
-      for (int i = len - 1; i >= at; --i) {  // shifts the bytes up one by one: no indexed register access
-        v[3] = (int)(((unsigned)v[3] << 8) | ((unsigned)v[2] >> 24));
-        v[2] = (int)(((unsigned)v[2] << 8) | ((unsigned)v[1] >> 24));
-        v[1] = (int)(((unsigned)v[1] << 8) | ((unsigned)v[0] >> 24));
-        v[0] = (int)(((unsigned)v[0] << 8) | (unsigned)(uint8_t)row[i]);
-      }
-    }
-  }
-  return v;
-}
-
 template <int BM, int BN, bool BKN, int OUTCLS>
 __global__ __launch_bounds__(256) void gemm_ragged_kernel(GemmParams p) {
   constexpr int BK = 64, WTM = BM / 2, WTN = BN / 2, TM = WTM / 32, TN = WTN / 32;

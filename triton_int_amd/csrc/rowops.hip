@@ -391,6 +391,10 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_kernel(const int8_t* 
     __builtin_amdgcn_raw_buffer_store_b128(o, ry, c0, 0, 2);  // dropped beyond the row's end
   }
 }
+// Any alignment, length and scale >= 0: 16 unaligned bytes per lane.  160 x 1001 rows of 1001 columns 311 (byte loads
+// and stores) -> 84 us, 40 x 2047 rows of 2047 341 -> 61 us (aligned rows of 2048: 54 us).
+typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(1)));
+
 template <int VPT>
 __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8_t* __restrict__ x, int64_t x_rs,
                                                                   float scale, int8_t* __restrict__ y, int64_t y_rs,
@@ -401,9 +405,20 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8
   const int limit = causal_q_len > 0 ? min(cols, (row % causal_q_len) + (cols - causal_q_len) + 1) : cols;
   const int8_t* xr = x + (int64_t)row * x_rs;
   int8_t* yr = y + (int64_t)row * y_rs;
-  const bool vec = ((((uintptr_t)xr) | ((uintptr_t)yr)) & 15) == 0;
   const float NEG = -__builtin_inff();  // drops out of the maximum; its exponential is 0 (scale > 0) or masked below
 
+  // All of a row's loads first.  A lane past the row's last whole chunk loads the row's last 16 bytes (no byte
+  // outside the row is touched) and the one that holds the row's end shifts them into place.
+  v4i w[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int c0 = (j * 64 + lane) * 16;
+    if (cols >= 16) {
+      __builtin_memcpy(&w[j], xr + min(c0, cols - 16), 16);
+    } else {
+      w[j] = load16_tail(xr, c0, cols);
+    }
+  }
   // f[j][t] = the score as a float, or NEG for masked / out-of-row elements
   float f[VPT][16];
   float mx = NEG;
@@ -413,16 +428,14 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8
     if (c0 >= limit) {
 #pragma unroll
       for (int t = 0; t < 16; ++t) f[j][t] = NEG;
-    } else if (vec && c0 + 16 <= cols) {
-      // a chunk that straddles the causal limit is still inside the row: load it whole and mask
-      // in registers, so that no wave waits for a second, dependent round of byte loads
-      v4u w = __builtin_nontemporal_load((const v4u*)(xr + c0));
+    } else {
+      if (cols >= 16 && c0 + 16 > cols) w[j] = shift_down_bytes(w[j], c0 + 16 - cols);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        f[j][4 * g + 0] = sbyte_to_float<0>(w[g]);
-        f[j][4 * g + 1] = sbyte_to_float<1>(w[g]);
-        f[j][4 * g + 2] = sbyte_to_float<2>(w[g]);
-        f[j][4 * g + 3] = sbyte_to_float<3>(w[g]);
+        f[j][4 * g + 0] = sbyte_to_float<0>((unsigned)w[j][g]);
+        f[j][4 * g + 1] = sbyte_to_float<1>((unsigned)w[j][g]);
+        f[j][4 * g + 2] = sbyte_to_float<2>((unsigned)w[j][g]);
+        f[j][4 * g + 3] = sbyte_to_float<3>((unsigned)w[j][g]);
       }
       if (c0 + 16 > limit) {
 #pragma unroll
@@ -430,12 +443,6 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8
       }
 #pragma unroll
       for (int t = 0; t < 16; t += 2) mx = fmaxf(fmaxf(mx, f[j][t]), f[j][t + 1]);  // v_max3_f32
-    } else {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        f[j][t] = c0 + t < limit ? (float)(int)xr[c0 + t] : NEG;
-        mx = fmaxf(mx, f[j][t]);
-      }
     }
   }
   mx = wave_max(mx);
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8
   for (int j = 0; j < VPT; ++j) {
     const int c0 = (j * 64 + lane) * 16;
     if (c0 >= cols) continue;
-    v4u w = {0u, 0u, 0u, 0u};
+    v4u o = {0u, 0u, 0u, 0u};
     if (c0 < limit) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -469,15 +476,30 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8
         const unsigned b1 = __float_as_uint(__builtin_fmaf(f[j][4 * g + 1], r, 12582912.0f));
         const unsigned b2 = __float_as_uint(__builtin_fmaf(f[j][4 * g + 2], r, 12582912.0f));
         const unsigned b3 = __float_as_uint(__builtin_fmaf(f[j][4 * g + 3], r, 12582912.0f));
-        w[g] = __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) | __builtin_amdgcn_perm(b3, b2, 0x04000c0cu);
+        o[g] = __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) | __builtin_amdgcn_perm(b3, b2, 0x04000c0cu);
       }
     }
-    if (vec && c0 + 16 <= cols) {
-      __builtin_nontemporal_store(w, (v4u*)(yr + c0));
-    } else {
-#pragma unroll
-      for (int t = 0; t < 16; ++t)
-        if (c0 + t < cols) yr[c0 + t] = (int8_t)(w[t >> 2] >> ((t & 3) * 8));
+    const int left = cols - c0;
+    if (left >= 16) {
+      __builtin_nontemporal_store(o, (v4u_any*)(yr + c0));
+    } else {  // the lane with the row's end: 8, 4, 2 and 1 bytes
+      int8_t* d = yr + c0;
+      if (left & 8) {
+        __builtin_memcpy(d, &o, 8);
+        d += 8;
+        o[0] = o[2]; o[1] = o[3];
+      }
+      if (left & 4) {
+        __builtin_memcpy(d, &o, 4);
+        d += 4;
+        o[0] = o[1];
+      }
+      if (left & 2) {
+        d[0] = (int8_t)o[0]; d[1] = (int8_t)(o[0] >> 8);
+        d += 2;
+        o[0] >>= 16;
+      }
+      if (left & 1) d[0] = (int8_t)o[0];
     }
   }
 }

@@ -50,6 +50,39 @@ __device__ __forceinline__ unsigned pack4(int a, int b, int c, int d) {
          ((unsigned)d << 24);
 }
 
+// ---- device: rows that start at any byte ------------------------------------------------------------
+// v shifted down by n bytes (0 .. 15), zeros from above
+__device__ __forceinline__ v4i shift_down_bytes(v4i v, int n) {
+  unsigned long long lo = ((unsigned long long)(unsigned)v[1] << 32) | (unsigned)v[0], hi = ((unsigned long long)(unsigned)v[3] << 32) | (unsigned)v[2];
+  const int bits = n * 8;
+  lo = bits >= 64 ? hi >> (bits - 64) : (bits ? (lo >> bits) | (hi << (64 - bits)) : lo);
+  hi = bits >= 64 ? 0ull : hi >> bits;
+  return (v4i){(int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32)};
+}
+
+// 16 bytes of `row` (of `len` bytes) from byte `at`, zeros from `len` on.  No byte outside the row is touched: a
+// piece that crosses its end is loaded as the row's last 16 bytes and shifted.
+__device__ __forceinline__ v4i load16_tail(const int8_t* row, int at, int len) {
+  v4i v = {0, 0, 0, 0};
+  if (at + 16 <= len) {
+    __builtin_memcpy(&v, row + at, 16);
+  } else if (at < len) {
+    if (len >= 16) {
+      __builtin_memcpy(&v, row + len - 16, 16);
+      v = shift_down_bytes(v, at + 16 - len);
+    } else {
+#pragma unroll 1
+      for (int i = len - 1; i >= at; --i) {  // shifts the bytes up one by one: no indexed register access
+        v[3] = (int)(((unsigned)v[3] << 8) | ((unsigned)v[2] >> 24));
+        v[2] = (int)(((unsigned)v[2] << 8) | ((unsigned)v[1] >> 24));
+        v[1] = (int)(((unsigned)v[1] << 8) | ((unsigned)v[0] >> 24));
+        v[0] = (int)(((unsigned)v[0] << 8) | (unsigned)(uint8_t)row[i]);
+      }
+    }
+  }
+  return v;
+}
+
 // tanh-GELU times scale, 0.5 * x * (1 + tanh(k * (x + 0.044715 * x^3))) * scale
 // (kernels/fused.py:79), evaluated as (x * scale) / (1 + e^(-2u)) with
 // -2u * log2(e) = x * (c0 + c1 * x^2), c0 = -2 k log2 e, c1 = 0.044715 * c0: 6 plain operations, one
