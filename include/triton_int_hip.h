@@ -410,6 +410,18 @@ int ti_quantize_per_token_absmax(const void* x, int x_dtype, int64_t x_row_strid
                                  int rows, int cols, void* stream);
 
 /*
+ * Dynamic per-tensor activation quantisation, quantize_per_tensor_absmax (functional/quantization.py:5-14) on n
+ * contiguous elements of x (TI_F32 / TI_F16), bit for bit what torch's steps give on the GPU:
+ *     scale = max |x| / 127                       (x's dtype; scale_out, may be NULL)
+ *     q[i]  = int8(round_half_even(x[i] / scale))
+ *     alpha = float(scale) * weight_scale         (alpha_out fp32, may be NULL; weight_scale NULL: 1)
+ * x is not modified.  workspace: TI_QUANT_TENSOR_WORKSPACE bytes of device memory, contents irrelevant.
+ */
+#define TI_QUANT_TENSOR_WORKSPACE 4096
+int ti_quantize_per_tensor_absmax(const void* x, int x_dtype, int64_t n, int8_t* q, void* scale_out,
+                                  const float* weight_scale, float* alpha_out, void* workspace, void* stream);
+
+/*
  * Floating-point LayerNorm / RMSNorm over the rows of x [rows, cols], with the optional skip
  * (residual) add: layer_norm_fwd_fused_single_pass (kernels/fused.py:385-532),
  * skip_layer_norm_fwd_fused_single_pass (kernels/fused.py:535-693) and

@@ -159,3 +159,21 @@ def test_softmax_q_rows_at_any_byte(rows, cols, q_len, scale):
     mx, rate = mismatch_report(cpu(got), O.softmax_q(x, scale, causal_q_len=q_len))
     assert mx <= 1 and rate <= max(2e-3, 1.5 / got.numel())
     assert torch.equal(got, fused.softmax_q(gpu(x), scale, causal_q_len=q_len))
+
+
+@pytest.mark.parametrize("shape", [(1,), (7,), (8, 1024), (3, 1001), (2000, 640), (1, 3)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_quantize_per_tensor_is_the_torch_steps_bit_for_bit(shape, dtype):
+    """Against torch's own steps on the GPU, unaligned views and a tensor of zeros included."""
+    from triton_int_amd.kernels import fused
+
+    g = torch.Generator(device="cuda").manual_seed(sum(shape))
+    base = (torch.randn((int(np.prod(shape)) + 1,), device="cuda", generator=g) * 3).to(dtype)
+    ws = torch.tensor(0.0123, device="cuda")
+    for x in (base[:-1].view(shape), base[1:].view(shape), base[1:].view(shape) * 1e-3, torch.zeros(shape, dtype=dtype, device="cuda")):
+        kept = x.clone()
+        q, s, alpha = fused.quantize_per_tensor_absmax(x, ws)
+        want_s = x.abs().max() / 127
+        assert q.dtype == torch.int8 and q.shape == x.shape and torch.equal(x, kept)
+        assert torch.equal(s, want_s) and torch.equal(alpha, want_s.float() * ws)
+        assert torch.equal(q, (x / want_s).round_().to(torch.int8))

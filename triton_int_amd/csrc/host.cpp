@@ -372,6 +372,27 @@ PyObject* quantize_per_token(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
+// quantize_per_tensor(x, weight_scale) -> (int8, scale, alpha)
+PyObject* quantize_per_tensor(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 2, [&]() -> PyObject* {
+    const Tensor& x = tensor(v[0]);
+    const Call c(x);
+    need(x.scalar_type() == ScalarType::Float || x.scalar_type() == ScalarType::Half);
+    need(x.is_contiguous() && x.numel() > 0);
+    const float* ws = scale(v[1], c.dev);
+    Tensor q = c.empty(x.sizes(), ScalarType::Char), s = c.empty({}, x.scalar_type()), al = c.empty({}, ScalarType::Float);
+    Tensor work = c.empty({TI_QUANT_TENSOR_WORKSPACE}, ScalarType::Byte);
+    const int rc = ti_quantize_per_tensor_absmax(ptr(x), dtype_code(x.scalar_type()), x.numel(), (int8_t*)mptr(q), mptr(s), ws,
+                                                 (float*)mptr(al), mptr(work), c.stream);
+    need(rc == TI_OK);
+    PyObject* triple = PyTuple_New(3);
+    PyTuple_SET_ITEM(triple, 0, THPVariable_Wrap(q));
+    PyTuple_SET_ITEM(triple, 1, THPVariable_Wrap(s));
+    PyTuple_SET_ITEM(triple, 2, THPVariable_Wrap(al));
+    return triple;
+  });
+}
+
 // strides of [seqs, heads, rows, D] or [heads, rows, D] with unit last stride
 struct Heads {
   int64_t ss, hs, rs;
@@ -486,7 +507,7 @@ PyObject* kv_append(PyObject*, PyObject* const* v, Py_ssize_t n) {
 #define TI_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     TI_METHOD(linear), TI_METHOD(bmm), TI_METHOD(linear_residual), TI_METHOD(layernorm_q), TI_METHOD(dq_add_layernorm_q),
-    TI_METHOD(layernorm_fp), TI_METHOD(gelu_q), TI_METHOD(softmax_q), TI_METHOD(quantize_per_token), TI_METHOD(attention),
+    TI_METHOD(layernorm_fp), TI_METHOD(gelu_q), TI_METHOD(softmax_q), TI_METHOD(quantize_per_token), TI_METHOD(quantize_per_tensor), TI_METHOD(attention),
     TI_METHOD(qkv_decode), TI_METHOD(kv_append), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host path of the launchers (see csrc/host.cpp).", -1, methods};
 

@@ -1,4 +1,5 @@
-// quant.hip — dynamic per-token activation quantisation (functional/quantization.py:61-67):
+// quant.hip — dynamic activation quantisation, per token (functional/quantization.py:61-67) and, further down,
+// per tensor (:5-14).  Per token:
 //     max_val = clamp(max_j |t[r, j]|, min = 1e-8) / 127        (in t's dtype)
 //     q[r, j] = clamp(round_half_even(t[r, j] / max_val[r]), -128, 127) -> int8
 // for fp32 and fp16 activations.  Every step is rounded to the tensor's dtype as torch's elementwise
@@ -199,7 +200,137 @@ static int launch_quant(const void* x, int64_t x_rs, int8_t* q, int64_t q_rs, vo
   return launch_status("quant_per_token_kernel");
 }
 
+// ---- per tensor ------------------------------------------------------------------------------------
+//     scale = max |t| / 127                        (in t's dtype)
+//     q     = int8(round_half_even(t / scale))     (no clamp: functional/quantization.py:5-14)
+//     alpha = float(scale) * weight_scale
+// as torch computes them on the GPU, bit for bit: t.abs().max() / 127 multiplies by the reciprocal (a scalar
+// divisor), the quotient by the 0-dim scale tensor is a true division rounded to t's dtype, and the int8 cast
+// takes the low byte of the saturating int32 conversion.  Two launches: one maximum per workgroup, then every
+// workgroup of the second reduces those (4 KB from L2) before it quantises, so there is nothing to clear and no
+// grid-wide wait.  Bound: memory; 2000 x 5120 fp16: the torch steps (abs, max, div, div, round, cast, mul) 64 us,
+// these two 14 us (2, 4, 8, 16 and 32 workgroups per CU in the second: 13.9 / 13.4 / 13.8 / 14.5 / 15.0; fp32 8192 x 5120
+// 78 / 68 / 67 / 68 / 70).
+constexpr int QX_BLOCKS = TI_QUANT_TENSOR_WORKSPACE / 4;
+
+// |t| as an unsigned integer: larger magnitude, larger integer, and NaN above everything, so it propagates
+template <typename T>
+__device__ __forceinline__ unsigned abs_bits(T v) {
+  if constexpr (sizeof(T) == 2) return (unsigned)__builtin_bit_cast(unsigned short, v) & 0x7fffu;
+  else return __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
+}
+template <typename T>
+__device__ __forceinline__ T from_abs_bits(unsigned b) {
+  if constexpr (sizeof(T) == 2) return __builtin_bit_cast(T, (unsigned short)b);
+  else return __builtin_bit_cast(T, b);
+}
+
+__device__ __forceinline__ unsigned block_max_u32(unsigned v, unsigned* red, int tid) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, off, 64));
+  if ((tid & 63) == 0) red[tid >> 6] = v;
+  __syncthreads();
+  return max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
+template <typename T>
+__global__ __launch_bounds__(QT_THREADS) void absmax_partial_kernel(const T* __restrict__ x, int64_t n, int vec, unsigned* __restrict__ partial) {
+  constexpr int E = 16 / sizeof(T);
+  typedef T VE __attribute__((ext_vector_type(E)));
+  __shared__ unsigned red[QT_THREADS / 64];
+  const int64_t first = (int64_t)blockIdx.x * QT_THREADS + threadIdx.x, step = (int64_t)gridDim.x * QT_THREADS;
+  unsigned m = 0;
+  const int64_t nv = vec ? n / E : 0;
+  const VE* xv = (const VE*)x;
+  int64_t i = first;
+  for (; i + 3 * step < nv; i += 4 * step) {  // four loads in flight per thread
+    VE v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = xv[i + u * step];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) m = max(m, abs_bits<T>(v[u][e]));
+  }
+  for (; i < nv; i += step) {
+    const VE v = xv[i];
+#pragma unroll
+    for (int e = 0; e < E; ++e) m = max(m, abs_bits<T>(v[e]));
+  }
+  for (int64_t k = nv * E + first; k < n; k += step) m = max(m, abs_bits<T>(x[k]));
+  m = block_max_u32(m, red, threadIdx.x);
+  if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+
+template <typename T>
+__global__ __launch_bounds__(QT_THREADS) void quant_per_tensor_kernel(const T* __restrict__ x, int64_t n, int vec, const unsigned* __restrict__ partial,
+                                                                      int np, int8_t* __restrict__ q, T* __restrict__ scale_out,
+                                                                      const float* __restrict__ weight_scale, float* __restrict__ alpha_out) {
+  constexpr int E = 16 / sizeof(T);
+  typedef T VE __attribute__((ext_vector_type(E)));
+  __shared__ unsigned red[QT_THREADS / 64];
+  const int tid = threadIdx.x;
+  unsigned m = 0;
+  for (int i = tid; i < np; i += QT_THREADS) m = max(m, partial[i]);
+  m = block_max_u32(m, red, tid);
+  const T scale = (T)((float)from_abs_bits<T>(m) * (1.0f / 127.0f));
+  if (blockIdx.x == 0 && tid == 0) {
+    if (scale_out) *scale_out = scale;
+    if (alpha_out) *alpha_out = (float)scale * (weight_scale ? *weight_scale : 1.0f);
+  }
+  const RowDivisor by_scale((float)scale);
+  auto run = [&](auto direct_tag) {
+    constexpr bool DIRECT = decltype(direct_tag)::value;
+    auto one = [&](T v) -> unsigned {
+      const T d = (T)by_scale.template divide<DIRECT>((float)v);
+      return (unsigned)(int)__builtin_rintf((float)d) & 0xffu;
+    };
+    const int64_t first = (int64_t)blockIdx.x * QT_THREADS + tid, step = (int64_t)gridDim.x * QT_THREADS;
+    const int64_t nv = vec ? n / E : 0;
+    for (int64_t i = first; i < nv; i += step) {
+      const VE v = ((const VE*)x)[i];
+      unsigned w[E / 4];
+#pragma unroll
+      for (int g = 0; g < E / 4; ++g) w[g] = one(v[4 * g]) | (one(v[4 * g + 1]) << 8) | (one(v[4 * g + 2]) << 16) | (one(v[4 * g + 3]) << 24);
+      if constexpr (E == 8) *(uint2*)(q + i * E) = make_uint2(w[0], w[1]);
+      else *(unsigned*)(q + i * E) = w[0];
+    }
+    for (int64_t k = nv * E + first; k < n; k += step) q[k] = (int8_t)one(x[k]);
+  };
+  if (by_scale.direct) run(std::true_type{});
+  else run(std::false_type{});
+}
+
+template <typename T>
+static int launch_quant_tensor(const T* x, int64_t n, int8_t* q, T* scale_out, const float* weight_scale, float* alpha_out, unsigned* partial,
+                               hipStream_t stream) {
+  constexpr int E = 16 / (int)sizeof(T);
+  const int vec = (((uintptr_t)x) & 15) == 0 && (((uintptr_t)q) & (E - 1)) == 0;
+  const int64_t groups = (n + (int64_t)QT_THREADS * E - 1) / ((int64_t)QT_THREADS * E);
+  const unsigned np = (unsigned)(groups < QX_BLOCKS ? groups : QX_BLOCKS);
+  absmax_partial_kernel<T><<<dim3(np), dim3(QT_THREADS), 0, stream>>>(x, n, vec, partial);
+  int rc = launch_status("absmax_partial_kernel");
+  if (rc != TI_OK) return rc;
+  const unsigned grid = (unsigned)(groups < 256 * 8 ? groups : 256 * 8);
+  quant_per_tensor_kernel<T><<<dim3(grid), dim3(QT_THREADS), 0, stream>>>(x, n, vec, partial, (int)np, q, scale_out, weight_scale, alpha_out);
+  return launch_status("quant_per_tensor_kernel");
+}
+
 }  // namespace ti
+
+extern "C" int ti_quantize_per_tensor_absmax(const void* x, int x_dtype, int64_t n, int8_t* q, void* scale_out, const float* weight_scale,
+                                             float* alpha_out, void* workspace, void* stream) {
+  using namespace ti;
+  if (n < 0) return fail(TI_E_SHAPE, "negative size");
+  if (n == 0) return fail(TI_E_SHAPE, "an empty tensor has no largest element");
+  if (!x || !q || !workspace) return fail(TI_E_NULL, "x, q and the workspace are required");
+  if (x_dtype != TI_F32 && x_dtype != TI_F16) return fail(TI_E_COMBO, "activation dtype %d: fp32 or fp16", x_dtype);
+  int rc = check_device();
+  if (rc != TI_OK) return rc;
+  if (x_dtype == TI_F32)
+    return launch_quant_tensor<float>((const float*)x, n, q, (float*)scale_out, weight_scale, alpha_out, (unsigned*)workspace, (hipStream_t)stream);
+  return launch_quant_tensor<_Float16>((const _Float16*)x, n, q, (_Float16*)scale_out, weight_scale, alpha_out, (unsigned*)workspace, (hipStream_t)stream);
+}
 
 extern "C" int ti_quantize_per_token_absmax(const void* x, int x_dtype, int64_t x_row_stride, int8_t* q,
                                             int64_t q_row_stride, void* scale_out, int rows, int cols, void* stream) {

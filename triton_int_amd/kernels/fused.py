@@ -283,6 +283,30 @@ def quantize_per_token_absmax(t):
     return q.view(t.shape), scale.view(*t.shape[:-1], 1)
 
 
+def quantize_per_tensor_absmax(t, weight_scale=None):
+    """Dynamic per-tensor quantisation of fp32 / fp16 activations: returns (q int8 like t, scale 0-dim in t's dtype,
+    alpha 0-dim fp32) with scale = max|t| / 127, q = round(t / scale) and alpha = scale * weight_scale (an fp32 device
+    tensor; None: 1).  The first two are bit-identical to quantize_per_tensor_absmax on the GPU (reference:
+    functional/quantization.py:5-14), but `t` is left untouched and nothing synchronises."""
+    y = L.host.quantize_per_tensor(t, weight_scale)
+    if y is not None:
+        return y
+    L.require_cuda(t, weight_scale)
+    assert t.dtype in (torch.float32, torch.float16), "activations must be fp32 or fp16"
+    t = t.contiguous()
+    dev = t.device
+    ws = None if weight_scale is None else L.scale_tensor(weight_scale, dev)
+    q = torch.empty(t.shape, dtype=torch.int8, device=dev)
+    scale = torch.empty((), dtype=t.dtype, device=dev)
+    alpha = torch.empty((), dtype=torch.float32, device=dev)
+    work = torch.empty(4096, dtype=torch.uint8, device=dev)
+    with L.on_device(dev):
+        rc = L.lib().ti_quantize_per_tensor_absmax(L.ptr(t), L.TORCH_TO_DT[t.dtype], t.numel(), L.ptr(q), L.ptr(scale), L.ptr(ws),
+                                                   L.ptr(alpha), L.ptr(work), L.current_stream(dev))
+    L.check(rc, "ti_quantize_per_tensor_absmax")
+    return q, scale, alpha
+
+
 def kv_append_i8(k_new, v_new, k_cache, vt_cache, seqs=1):
     """Write S new positions of each of `seqs` sequences into the last S slots of an int8 KV cache with one
     launch.  k_new, v_new: int8 [seqs*S, heads*D] (unit column stride; e.g. column slices of a fused q/k/v

@@ -9,6 +9,7 @@ from __future__ import annotations
 import torch
 
 from ..functional.quantization import quantize_per_tensor_absmax
+from ..kernels.fused import quantize_per_tensor_absmax as quantize_per_tensor_absmax_kernel
 from ..kernels.linear import (
     linear_a8_w8_b8_o8,
     linear_a8_w8_b32_o32,
@@ -169,9 +170,12 @@ class DynamicW8A8BFP32OFP32Linear(torch.nn.Module):
     def forward(self, x):
         lead = x.shape[:-1]
         x2 = x.reshape(-1, x.shape[-1])
-        scale = x2.abs().max() / 127                        # quantize_per_tensor_absmax (functional/quantization.py:5-14)
-        x8 = (x2 / scale).round_().to(torch.int8)
-        alpha = (scale.to(torch.float32) * self.weight_scale).to(torch.float32)
+        if x2.dtype in (torch.float32, torch.float16) and x2.numel():
+            x8, _, alpha = quantize_per_tensor_absmax_kernel(x2, self.weight_scale)
+        else:
+            scale = x2.abs().max() / 127                    # quantize_per_tensor_absmax (functional/quantization.py:5-14)
+            x8 = (x2 / scale).round_().to(torch.int8)
+            alpha = (scale.to(torch.float32) * self.weight_scale).to(torch.float32)
         y = linear_a8_w8_bfp32_ofp32(x8, self.weight, self.bias, alpha, self.b)
         return y.view(*lead, -1)
 
