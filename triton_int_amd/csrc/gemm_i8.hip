@@ -3225,14 +3225,14 @@ static int run_with_residual(GemmParams p, const float* R, int64_t ldr, hipStrea
     p.resid_rs = ldr;
     return run(p, cfg, stream);
   }
-  // the persistent kernels add it in their fp32 epilogue (unsplit K only: partial sums carry no residual);
-  // 32-bit offsets into the residual, like the stores
+  // the persistent kernels add it in their fp32 epilogue (with split K: in that of a tile's last item, where the
+  // sums are whole); 32-bit offsets into the residual, like the stores
   const bool persistent = g_configs[cfg].stream_occ > 0 || g_configs[cfg].ws_waves > 0 || g_configs[cfg].max_k > 0;
-  if (persistent && splits == 1 && p.batch == 1 && p.out_dtype == TI_F32 && p.epilogue == TI_EPI_SCALE_F &&
+  if (persistent && p.batch == 1 && p.out_dtype == TI_F32 && p.epilogue == TI_EPI_SCALE_F &&
       ((int64_t)(p.M + 512) * ldr + p.N) * 4 < ((int64_t)1 << 31)) {
     p.resid = R;
     p.resid_rs = ldr;
-    return run(p, cfg | (1 << 8), stream);
+    return run(p, cfg | (splits << 8), stream);
   }
   rc = run(p, cfg | (splits << 8), stream);
   if (rc != TI_OK) return rc;
