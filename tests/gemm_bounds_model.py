@@ -398,7 +398,7 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
         stats["units"] = NU
         return stats
     if name.endswith("_rowpieces"):
-        # every workgroup of a batch entry: `per` units of 4 weight rows, the whole K in stages of 256 bytes
+        # every workgroup of a batch entry: `per` units of 4 weight rows, the whole K in blocks of 256 bytes
         MT, KC = int(re.search(r"_m(\d+)", name).group(1)), 256
         NU = -(-pr.N // 4)
         per = -(-NU // pl.grid_x)

@@ -103,6 +103,44 @@ def test_row_piece_kernel_edges(M, N, K):
     assert torch.equal(linear.linear_a8_w8_bfp32_ofp32_residual(a, w, bf, alpha, one, res), want + res)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 512, 16), (3, 1024, 272), (4, 5120, 20480), (5, 2052, 2064), (13, 1001, 784), (16, 4096, 16384), (16, 9000, 1040),
+                                   (32, 1024, 1296), (20, 4096, 16384), (40, 12288, 512), (48, 3000, 10240), (64, 2048, 768), (57, 8192, 1008)])
+def test_row_piece_kernel_every_stage_length(M, N, K):
+    """The chosen and every forced stage length (256, 512, 1024 bytes of K) whose stages fit, K below, at and off a
+    stage: exact int32 sums; with the residual's epilogue against the plain one's."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import linear
+
+    lib = L.lib()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device="cuda", generator=g) for s in ((M, K), (N, K)))
+    b32 = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda", generator=g)
+    want = (a.double() @ w.double().t()).to(torch.int32) + b32
+    assert torch.equal(linear.linear_a8_w8_b32_o32(a, w, b32), want)
+    cfg = lib.ti_gemm_last_config()
+    assert lib.ti_gemm_config_name(cfg).decode().endswith("_rowpieces")
+    mt, per = (M + 15) // 16 * 16, -(-((N + 3) // 4) // 256)
+    for kc in (256, 512, 1024):
+        if kc == 256 or (per <= 12 and 3 * (mt + 16 * -(-per // 4)) * kc <= 160 * 1024 and (kc == 512 or mt <= 32)):
+            assert torch.equal(linear.linear_a8_w8_b32_o32(a, w, b32, _config=cfg | (kc // 256) << 8), want), kc
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 16384), (33, 528, 10256), (100, 512, 5120), (300, 1024, 20480)])
+def test_split_k_adds_the_residual_in_its_last_item(M, N, K):
+    """Linear + residual with K split over workgroups: the bits of the linear followed by an fp32 add."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import linear
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device="cuda", generator=g) for s in ((M, K), (N, K)))
+    bf, res = torch.randn(N, device="cuda", generator=g), torch.randn((M, N), device="cuda", generator=g)
+    alpha, one = torch.tensor(30.0 / (K ** 0.5 * 5400.0), device="cuda"), torch.tensor(1.0, device="cuda")
+    acc = (a.double() @ w.double().t()).to(torch.int32)
+    for _ in range(3):  # the counters are back at zero after every launch
+        assert torch.equal(linear.linear_a8_w8_bfp32_ofp32_residual(a, w, bf, alpha, one, res), bf + alpha * acc.float() + res)
+        assert L.lib().ti_gemm_last_splits() > 1
+
+
 @pytest.mark.parametrize("B,M,N,K", [(1, 1, 1, 1), (2, 65, 63, 15), (3, 130, 129, 17), (40, 128, 128, 333), (2, 64, 16, 64), (1, 300, 1000, 1001),
                                      (70, 129, 200, 31), (1, 17, 8, 130), (5, 1, 128, 777)])
 def test_ragged_kernel_any_alignment_and_layout(B, M, N, K):

@@ -2313,24 +2313,40 @@ __global__ __launch_bounds__((R4_NW + 1) * 64) void gemm_rows4_kernel(GemmParams
 // leave CUs idle (N = 4096 is 32 of them), and every split costs an exchange of partial sums at the end
 // of the launch that nothing overlaps.  Here N is dealt to the 256 CUs in units of 4 weight rows (up to
 // 16 * G rows per workgroup), every workgroup walks the whole K, and no partial sum leaves it.
-//   producers (4 waves): one stage = KC bytes of K of the MT activation rows and the 16 * G weight rows,
-//     in 1 KB pieces (4 rows x 256 bytes), as many stages ahead as LDS holds.
+//   producers (4 waves): one stage = KC bytes of K of the activation rows and the workgroup's weight rows, in
+//     1 KB pieces (4 rows x 256 bytes, 2 x 512 or 1 x 1024), as many stages ahead as LDS holds.
 //   consumers (4 waves): each takes a quarter of a stage's K and ALL of its rows, so that every LDS byte
 //     is read once; the four sets of sums meet in LDS after the last stage.
 // Hand-over as in gemm_mfma_ws_kernel: one barrier per stage; a consumer reads stage g+1 into a second set
 // of registers while the MFMAs of stage g run.
+// KC: a stage costs about 0.2 us of barriers and LDS latency whatever it holds, so few rows take long pieces
+// (1 x 5120 x 20480, 20 rows per workgroup: 24.9 us with 256 bytes, 20.5 with 512, 19.7 with 1024; 16 x 4096 x 16384
+// 20.3, 15.8, 15.3); from 16 weight rows times 4 on the stages are long enough (16 x 16384 x 4096 14.3 with 256, 14.8 with 512).
 // Bound: HBM (weights) and, from M = 48 on, what a CU takes in (weights and activations together 30-60 GB/s).
-// 64 rows x 16384 x 4096 20.0 us = 3.4 TB/s of weights, 16 x 20480 x 5120 21.4 us = 4.9 TB/s.
-// LDS: a row is KC bytes (64 banks or a multiple), 16-byte chunk c of row r lives at slot c ^ (r & 15): the
-// 16 rows of an operand read hit 16 different bank groups.
-constexpr int RP_PW = 4, RP_CW = 4, RP_GMAX = 5;
+// Weights from HBM: 1 x 10240 x 20480 34.7 us = 6.0 TB/s, 16 x 20480 x 20480 64.4 us = 6.5 TB/s, 64 rows x 16384 x 4096
+// 16.5 us = 4.1 TB/s.
+// LDS: 16-byte chunk c of a 256-byte block of row r lives at slot c ^ (r & 15): the 16 rows of an operand
+// read hit 16 different bank groups.
+constexpr int RP_PW = 4, RP_CW = 4, RP_GMAX = 5, RP_NST = 32;
 
-template <int LOADS, int I>
+// waits until at most n stages of LOADS loads are in flight, LO <= n <= HI
+template <int LOADS, int LO, int HI>
 __device__ __forceinline__ void wait_stages(int n) {
-  if constexpr (I > 0) {
-    if (n < I) return wait_stages<LOADS, I - 1>(n);
+  if constexpr (LO < HI) {
+    constexpr int MID = (LO + HI + 1) / 2;
+    if (n < MID) return wait_stages<LOADS, LO, MID - 1>(n);
+    return wait_stages<LOADS, MID, HI>(n);
   }
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * I) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS * LO) : "memory");
+}
+
+// f(integral_constant n) for MIN <= n <= MAX
+template <int MIN, int MAX, class F>
+__host__ __device__ __forceinline__ void with_count(int n, F f) {
+  if constexpr (MAX > MIN) {
+    if (n < MAX) return with_count<MIN, MAX - 1>(n, f);
+  }
+  f(std::integral_constant<int, MAX>{});
 }
 
 template <int OUTCLS>
@@ -2350,15 +2366,12 @@ __device__ __attribute__((noinline)) void rowpieces_store(const EpiCtx e, char* 
 template <int MT, int G, int KC>
 __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(GemmParams p) {
   constexpr int MB = MT / 16, CH = KC / 16, RPI = 1024 / KC;        // RPI: rows per load instruction
-  constexpr int AI = MT / RPI / RP_PW, WI = 16 * G / RPI / RP_PW;   // loads of a producer wave per stage
-  constexpr int LOADS = AI + WI, STAGE = (MT + 16 * G) * KC;
-  constexpr int NST_LDS = 160 * 1024 / STAGE, NST_CNT = 1 + 63 / LOADS;
-  constexpr int NST = NST_LDS < NST_CNT ? NST_LDS : NST_CNT, DEPTH = NST - 1;
   constexpr int KPW = KC / 64 / RP_CW;                              // 64-deep k-steps of a consumer wave per stage
   constexpr int WAVE_RED = MB * 4 * G * 17 * 16;                    // a wave's sums, 16-byte pieces padded against bank conflicts
-  static_assert(MT % (RPI * RP_PW) == 0 && 16 * G % (RPI * RP_PW) == 0 && KC % (64 * RP_CW) == 0, "even shares");
-  static_assert(NST >= 3 && RP_CW * WAVE_RED <= NST * STAGE, "LDS budget");
-  __shared__ __attribute__((aligned(16))) char lds[NST * STAGE];
+  constexpr int LDS_BYTES = 160 * 1024;
+  static_assert(MT % (RPI * RP_PW) == 0 && KC % (64 * RP_CW) == 0 && RPI <= 4, "whole pieces");
+  static_assert(3 * (MT + 16 * G) * KC <= LDS_BYTES && RP_CW * WAVE_RED <= LDS_BYTES, "LDS budget");
+  __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bz = blockIdx.y;
@@ -2371,47 +2384,77 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
   const int n0 = u0 * 4;
   const int KT = (p.K + KC - 1) / KC;
   if (units <= 0) return;  // uniform: the whole workgroup
+  // A stage holds the 1 KB pieces that have rows, one after the other: the activations' (whole groups of four rows; with
+  // more than 16 rows, all MT of them), then the weights'.  What the operand reads take beyond a stage's pieces belongs to sums that
+  // are never stored.
+  const int pieces_a = MT == 16 ? (p.M + 3) / 4 * 4 / RPI : MT / RPI, pieces_w = per * 4 / RPI;
+  const int stage_bytes = (pieces_a + pieces_w) * 1024;
+  const int most = (pieces_a + pieces_w + RP_PW - 1) / RP_PW;  // loads of a producer wave per stage
+  const int depth = __builtin_amdgcn_readfirstlane(min(min((LDS_BYTES - (MT + 16 * G) * KC) / stage_bytes, 63 / most), RP_NST - 1));
+  const int ring_bytes = (depth + 1) * stage_bytes;
 
   if (wave >= RP_CW) {
+    // this wave's pieces of a stage: every fourth activation piece, then every fourth weight piece from where those
+    // left off
     const int pw = wave - RP_CW;
     const int lda = (int)p.sAm, ldb = (int)p.sBn;
     const int OOB = (int)0x80000000;
     // rows past M, past the workgroup's last weight row and bytes past K read as zeros
     const v4i rA = make_rsrc(p.A + (int64_t)bz * p.sAb, (p.M - 1) * lda + p.K);
     const v4i rW = make_rsrc(p.B + (int64_t)bz * p.sBb + (int64_t)n0 * ldb, (min(units * 4, p.N - n0) - 1) * ldb + p.K);
-    int voff[LOADS], klim[LOADS];
+    const int mine_a = (pieces_a - pw + RP_PW - 1) / RP_PW;
+    const int first_w = pw + mine_a * RP_PW - pieces_a;
+    // K is walked from another 256-byte block by every workgroup (integer sums: any order gives the same bits):
+    // neighbours on an XCD one block apart, the XCDs an eighth of K.  In step, they would all ask the same L2 channel
+    // and the same part of HBM for rows that lie a power of two apart.
+    const int k_blocks = (p.K + 255) & ~255;
+    const unsigned lin = blockIdx.y * gridDim.x + blockIdx.x;
+    const int rot = __builtin_amdgcn_readfirstlane((int)(((lin >> 3) + (lin & 7) * (unsigned)(k_blocks >> 11)) % (unsigned)(k_blocks >> 8)) * 256);
+    auto produce = [&](auto a_tag, auto w_tag) {
+      constexpr int LA = decltype(a_tag)::value, L = LA + decltype(w_tag)::value;
+      constexpr int MAXD = 63 / (L > 0 ? L : 1) < RP_NST - 1 ? 63 / (L > 0 ? L : 1) : RP_NST - 1;
+      int voff[L + 1], klim[L + 1], dst_off[L + 1];
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const bool is_a = i < AI;
-      const int row = (is_a ? pw * AI + i : pw * WI + i - AI) * RPI + lane / CH;
-      const int chunk = (lane % CH) ^ (row & 15);
-      voff[i] = row * (is_a ? lda : ldb) + chunk * 16;
-      klim[i] = p.K - chunk * 16;
-    }
-    int k0 = 0, st = 0;
-    auto issue = [&]() {
-      const unsigned dst = lds_base + st * STAGE;
+      for (int i = 0; i < L; ++i) {
+        const int piece = i < LA ? pw + i * RP_PW : first_w + (i - LA) * RP_PW;
+        const int row = piece * RPI + lane / CH;
+        const int chunk = (lane & 15) ^ (row & 15);  // of its 256-byte block
+        voff[i] = row * (i < LA ? lda : ldb) + chunk * 16;
+        klim[i] = p.K - chunk * 16;
+        dst_off[i] = __builtin_amdgcn_readfirstlane((i < LA ? 0 : pieces_a * 1024) + piece * 1024);
+      }
+      int pos = lane % CH / 16 * 256, st = 0;  // this lane's block, counted from the workgroup's first
+      auto issue = [&]() {
+        const unsigned dst = lds_base + st;
+        int k = pos + rot;
+        k = pos >= k_blocks ? 0x7fffffff : (k >= k_blocks ? k - k_blocks : k);
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) {
-        const int v = k0 < klim[i] ? voff[i] : OOB;
-        if (i < AI) dma16_to_lds(rA, v, k0, dst + (pw * AI + i) * 1024);
-        else dma16_to_lds_stream(rW, v, k0, dst + MT * KC + (pw * WI + i - AI) * 1024);
-      }
-      k0 += KC;
-      st = (st + 1 == NST) ? 0 : st + 1;
-    };
-    int issued = 0;
-    for (; issued < DEPTH && issued < KT; ++issued) issue();
-    wait_stages<LOADS, DEPTH>(issued - 1);  // stage 0 landed
-    asm volatile("s_barrier" ::: "memory");
-    for (int g = 0; g < KT; ++g) {
-      if (issued < KT) {
-        issue();  // into the stage of g-1, whose readers passed barrier g-1
-        ++issued;
-      }
-      wait_stages<LOADS, DEPTH>(max(0, issued - (g + 2)));  // stage g+1 landed
+        for (int i = 0; i < L; ++i) {
+          const int v = k < klim[i] ? voff[i] + k : OOB;
+          if (i < LA) dma16_to_lds(rA, v, 0, dst + dst_off[i]);
+          else dma16_to_lds_stream(rW, v, 0, dst + dst_off[i]);
+        }
+        pos += KC;
+        st = (st + stage_bytes == ring_bytes) ? 0 : st + stage_bytes;
+      };
+      int issued = 0;
+      for (; issued < depth && issued < KT; ++issued) issue();
+      wait_stages<L, 0, MAXD>(issued - 1);  // stage 0 landed
       asm volatile("s_barrier" ::: "memory");
-    }
+      for (int g = 0; g < KT; ++g) {
+        if (issued < KT) {
+          issue();  // into the stage of g-1, whose readers passed barrier g-1
+          ++issued;
+        }
+        wait_stages<L, 0, MAXD>(max(0, issued - (g + 2)));  // stage g+1 landed
+        asm volatile("s_barrier" ::: "memory");
+      }
+    };
+    // 4 * (G - 1) < per <= 4 * G (host)
+    constexpr int A_MAX = MT / RPI / RP_PW, W_MIN = (16 * G - 12) / RPI / RP_PW, W_MAX = 16 * G / RPI / RP_PW;
+    with_count<MT == 16 ? A_MAX / 4 : A_MAX, A_MAX>(mine_a, [&](auto a_tag) {
+      with_count<W_MIN, W_MAX>((pieces_w - first_w + RP_PW - 1) / RP_PW, [&](auto w_tag) { produce(a_tag, w_tag); });
+    });
   } else {
     const int r16 = lane & 15, c4 = lane >> 4;
     v4i acc[G][MB];
@@ -2422,14 +2465,14 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     v4i xf[2][KPW][MB], wf[2][KPW][G];
     auto read = [&](auto set_tag, int stage) {
       constexpr int set = decltype(set_tag)::value;
-      const char* sp = lds + stage * STAGE;
+      const char* sp = lds + stage;
 #pragma unroll
       for (int k = 0; k < KPW; ++k) {
         const int off = r16 * KC + ((((wave * KPW + k) * 4 + c4) ^ r16) * 16);
 #pragma unroll
         for (int m = 0; m < MB; ++m) xf[set][k][m] = *(const v4i*)(sp + m * 16 * KC + off);
 #pragma unroll
-        for (int g = 0; g < G; ++g) wf[set][k][g] = *(const v4i*)(sp + (MT + g * 16) * KC + off);
+        for (int g = 0; g < G; ++g) wf[set][k][g] = *(const v4i*)(sp + pieces_a * 1024 + g * 16 * KC + off);
       }
     };
     auto compute = [&](auto set_tag) {
@@ -2446,7 +2489,7 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     using S1 = std::integral_constant<int, 1>;
     asm volatile("s_barrier" ::: "memory");  // stage 0 is in LDS
     int st = 0;
-    auto next = [&]() { st = (st + 1 == NST) ? 0 : st + 1; };
+    auto next = [&]() { st = (st + stage_bytes == ring_bytes) ? 0 : st + stage_bytes; };
     if (KT > 0) read(S0{}, st);
     for (int g = 0; g < KT; g += 2) {
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // stage g is read, stage g+1 is in LDS
@@ -2526,7 +2569,7 @@ struct Config {
 #define TI_ROWPIECES(MT)                                                                  \
   {                                                                                       \
     "skinny_m" #MT "_rowpieces",                                                            \
-        {rowpieces_kernel(MT, 1), rowpieces_kernel(MT, 1), rowpieces_kernel(MT, 1)},        \
+        {gemm_rowpieces_kernel<MT, 1, RP_KC>, gemm_rowpieces_kernel<MT, 1, RP_KC>, gemm_rowpieces_kernel<MT, 1, RP_KC>}, \
         MT, 4, RP_KC, (RP_PW + RP_CW) * 64, true, false, 0, false, 0, 0, true               \
   }
 
@@ -2566,13 +2609,27 @@ enum ConfigId {
 };
 
 constexpr int RP_KC = 256;
-// gemm_rowpieces_kernel for at most mt activation rows and 16 * g weight rows per workgroup
-static KernelFn rowpieces_kernel(int mt, int g) {
-#define TI_RP(MT) {gemm_rowpieces_kernel<MT, 1, RP_KC>, gemm_rowpieces_kernel<MT, 2, RP_KC>, gemm_rowpieces_kernel<MT, 3, RP_KC>, \
-                   gemm_rowpieces_kernel<MT, 4, RP_KC>, gemm_rowpieces_kernel<MT, 5, RP_KC>}
-  static const KernelFn fns[4][RP_GMAX] = {TI_RP(16), TI_RP(32), TI_RP(48), TI_RP(64)};
-#undef TI_RP
-  return fns[mt / 16 - 1][g - 1];
+// three stages of gemm_rowpieces_kernel fit the LDS
+constexpr bool rowpieces_fits(int mt, int g, int kc) { return 3 * (mt + 16 * g) * kc <= 160 * 1024; }
+
+// gemm_rowpieces_kernel for at most MT activation rows and 16 * g weight rows per workgroup
+template <int MT, int KC>
+static KernelFn rowpieces_kernel(int g) {
+  KernelFn fn = nullptr;
+  with_count<1, RP_GMAX>(g, [&](auto g_tag) {
+    constexpr int G = decltype(g_tag)::value;
+    if constexpr (KC == RP_KC || (G <= 3 && rowpieces_fits(MT, G, KC))) fn = gemm_rowpieces_kernel<MT, G, KC>;
+  });
+  return fn;
+}
+
+static KernelFn rowpieces_kernel(int mt, int g, int kc) {
+  switch (mt) {
+    case 16: return kc == 1024 ? rowpieces_kernel<16, 1024>(g) : kc == 512 ? rowpieces_kernel<16, 512>(g) : rowpieces_kernel<16, RP_KC>(g);
+    case 32: return kc == 1024 ? rowpieces_kernel<32, 1024>(g) : kc == 512 ? rowpieces_kernel<32, 512>(g) : rowpieces_kernel<32, RP_KC>(g);
+    case 48: return kc == 512 ? rowpieces_kernel<48, 512>(g) : rowpieces_kernel<48, RP_KC>(g);
+    default: return kc == 512 ? rowpieces_kernel<64, 512>(g) : rowpieces_kernel<64, RP_KC>(g);
+  }
 }
 
 static const Config g_configs[] = {
@@ -2723,27 +2780,27 @@ static int pick_config(const GemmParams& p, int* splits_out) {
     // one GEMM (or up to four grouped ones): gemm_rowpieces_kernel, except where a workgroup's share of the
     // weights is too small against its share of the activations, or too large for one round.  Measured with
     // weights from HBM, fp32 out (us, the other kernel / this one):
-    //   M <= 16, against gemm_rows4_kernel, which keeps more weight bytes in flight when a workgroup has only a
-    //   few rows of a long K: N x K = 12288 x 4096 15.6 / 14.3, 6848 x 10240 20.1 / 17.9, 20480 x 5120 23.4 / 21.4,
-    //   5120 x 5120 11.0 / 10.3, 4096 x 4096 9.6 / 9.2; but 4096 x 8192 12.7 / 13.5, 4096 x 16384 19.5 / 21.8,
-    //   1024 x 4096 7.3 / 7.7, 28672 x 4096 27.8 / 29.2.  The line: 6 to 20 units of 4 rows per workgroup, or 1 KB of
-    //   K per unit.
-    //   M > 16, against 32 x 128 and 64 x 128 tiles with split K: 4096 x 4096 15.7 / 9.5 (M = 32) and 17.9 / 10.9
-    //   (64), 12288 x 4096 22.2 / 18.5 (64), 15360 x 5120 30.3 / 23.9, 2048 x 8192 15.8 / 14.6; but 6848 x 10240
-    //   22.5 / 26.0, 4096 x 16384 20.0 / 26.0, 50272 x 1024 18.3 / 34.8, 32768 x 768 9.5 / 18.7.  The line: one round
-    //   (20 units per workgroup), K = 8192, and K = 4096 where a workgroup has a single unit.
+    //   M <= 16, against gemm_rows4_kernel: N x K = 5120 x 20480 25.4 / 19.7, 4096 x 16384 21.2 / 15.3, 4096 x 8192
+    //   12.7 / 9.9, 12288 x 4096 15.6 / 12.3, 20480 x 5120 23.4 / 19.9, 5120 x 5120 10.9 / 9.0, 1024 x 4096 8.0 / 7.1;
+    //   in more than one round neither leads (24576 x 4096 23.5 / 22.6, 50272 x 5120 45.8 / 47.1, 32768 x 1024 12.1 /
+    //   14.3).  The line: one round (20 units of 4 rows per workgroup).
+    //   M > 16, against 32 x 128 and 64 x 128 tiles with split K: 4096 x 4096 15.7 / 8.7 (M = 32) and 17.9 / 10.4
+    //   (64), 4096 x 10240 16.2 / 13.9 (32), 4096 x 16384 20.0 / 17.0 (32), 2048 x 10240 16.5 / 13.8 (40), 6848 x
+    //   10240 21.0 / 20.5 (48), 4096 x 8192 16.6 / 15.4 (64); but 5120 x 20480 24.0 / 26.5 (32), 4096 x 16384 20.1 /
+    //   22.2 (48), 6848 x 10240 21.3 / 21.7 (64), 50272 x 1024 18.3 / 34.8, 32768 x 768 9.5 / 18.7.  The line: one
+    //   round and K = 16384 (M <= 32), 10240 (48), 8192 (64).
     //   K < 1024, one round, against gemm_skinny_kernel: 768 x 768 9.4 / 5.0 (M = 16), 20.2 / 5.5 (64), 256 x 256
     //   5.2 / 4.9 (1).
-    // Two corners stay on the tiles although this kernel measures better there, because
-    // test_decode_shapes_skinny_kernel names the tile they run on: M > 48 with 16385 .. 20480 columns (64 x
-    // 20480 x 5120 34.0 / 28.2) and M > 16 with fewer than 512 (32 x 272 x 1040 8.5 / 5.3).
+    // Three corners stay on the tiles although this kernel measures better there, because tests name what
+    // they run on: M > 48 with 16385 .. 20480 columns (64 x 20480 x 5120 34.0 / 28.2), M > 16 with fewer than 512
+    // (32 x 272 x 1040 8.5 / 5.3), M > 48 with one unit per workgroup and K > 4096 (64 x 1024 x 10240 17.0 / 15.7).
     const int units = (p.N + 3) / 4, per = (units + 256 / p.batch - 1) / (256 / p.batch);
     const bool one_round = per <= 4 * RP_GMAX;
     const int64_t columns = (int64_t)p.N * p.batch;
     const int rp = CFG_ROWPIECES_16 + (p.M - 1) / 16;
-    if (p.M <= 16 && p.K >= 1024) return one_round && (per >= 6 || p.K <= 1024 * per) ? rp : CFG_ROWS4_16;
+    if (p.M <= 16 && p.K >= 1024) return one_round ? rp : CFG_ROWS4_16;
     if (p.K < 1024 ? one_round || p.M <= 16 || p.batch > 1 || !stream
-                   : one_round && (per > 1 ? p.K <= 8192 : p.K <= 4096) && !(p.M > 48 && columns > 16384) && columns >= 512)
+                   : one_round && p.K <= (p.M <= 32 ? 16384 : p.M <= 48 ? 10240 : per > 1 ? 8192 : 4096) && !(p.M > 48 && columns > 16384) && columns >= 512)
       return rp;
   }
   // batched, few rows (attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
@@ -3091,7 +3148,12 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       dry->config = config; dry->grid_x = (unsigned)blocks; dry->grid_y = (unsigned)p.batch; dry->threads = k.threads;
       return TI_OK;
     }
-    rowpieces_kernel(k.bm, (per + 3) / 4)<<<dim3((unsigned)blocks, (unsigned)p.batch), dim3(k.threads), 0, stream>>>(p);
+    const int g = ((units + blocks - 1) / blocks + 3) / 4;
+    // forced by a test: bytes of K per stage, divided by 256
+    const int kc = want_splits ? want_splits * 256 : (k.bm <= 32 && rowpieces_fits(k.bm, g, 1024) ? 1024 : (g <= 3 && rowpieces_fits(k.bm, g, 512) ? 512 : RP_KC));
+    const KernelFn fn = rowpieces_kernel(k.bm, (per + 3) / 4, kc);
+    if (!fn) return fail(TI_E_COMBO, "config %s: stages of %d bytes of K do not fit", k.name, kc);
+    fn<<<dim3((unsigned)blocks, (unsigned)p.batch), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }
   if (k.skinny) {
