@@ -252,6 +252,24 @@ def _check_stream_stores(pr: Problem, bz, mw, nw, TM, TN, covered):
         commit(np.where(R < rows_left, base, oob), R * pitch, esz, mw + R + 4 * lhi, n, 1)
 
 
+def _check_kn_loads(what, pr, bz, n0, k_lo, k_hi, BN, BK):
+    """A [K,N] operand's k-tiles: descriptor at (k, n0) of the k-tile, chunks past N switched off, rows past K past its end."""
+    items = np.unique(np.stack([bz, n0, k_lo, k_hi], 1), axis=0)
+    row = np.arange(BK, dtype=np.int64)[:, None]
+    chunk = np.arange(BN // 16, dtype=np.int64)[None, :]
+    voff = row * pr.sBk + chunk * 16
+    _fits_i32(voff, f"{what} offset")
+    for b, n, lo, hi in items:
+        for k in {int(lo), int(lo + (hi - lo - 1) // BK * BK)}:
+            extent = (pr.K - 1 - k) * pr.sBk + pr.N - n
+            _fits_i32(extent, f"{what} extent")
+            assert extent > 0
+            base = b * pr.sBb + k * pr.sBk + n
+            live = (voff + 16 <= extent) & (n + chunk * 16 < pr.N)
+            assert not (live & ((row + k >= pr.K) | (base + voff + 16 > pr.b_bytes()))).any(), f"{what}: load outside the operand"
+            assert (live | (row + k >= pr.K) | (n + chunk * 16 >= pr.N)).all(), f"{what}: an operand chunk is not loaded"
+
+
 # ---- the kernels --------------------------------------------------------------------------------
 
 _TILED = re.compile(r"(ws|stream|mfma|shortk)_(\d+)x(\d+)x(\d+)_w(\d+)x(\d+)")
@@ -321,8 +339,11 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
             if persistent:  # origin in the descriptor, offsets relative to the tile
                 _check_tile_loads(f"{name} A", bz * pr.sAb + m0 * pr.sAm, _i32((pr.M - 1 - m0) * pr.sAm + pr.K), np.zeros_like(m0), pr.sAm, BM, BK, SWZ,
                                   pr.K, k_lo, k_hi, pr.a_bytes())
-                _check_tile_loads(f"{name} B", bz * pr.sBb + n0 * pr.sBn, _i32((pr.N - 1 - n0) * pr.sBn + pr.K), np.zeros_like(n0), pr.sBn, BN, BK, SWZ,
-                                  pr.K, k_lo, k_hi, pr.b_bytes())
+                if pr.sBk != 1:
+                    _check_kn_loads(f"{name} B", pr, bz, n0, k_lo, k_hi, BN, BK)
+                else:
+                    _check_tile_loads(f"{name} B", bz * pr.sBb + n0 * pr.sBn, _i32((pr.N - 1 - n0) * pr.sBn + pr.K), np.zeros_like(n0), pr.sBn, BN, BK, SWZ,
+                                      pr.K, k_lo, k_hi, pr.b_bytes())
             else:
                 _check_tile_loads(f"{name} A", bz * pr.sAb, np.full_like(m0, _i32((pr.M - 1) * pr.sAm + pr.K)), m0, pr.sAm, BM, BK, SWZ, pr.K, k_lo, k_hi,
                                   pr.a_bytes())

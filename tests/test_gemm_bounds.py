@@ -139,3 +139,16 @@ def test_static_scratch_falls_back_to_the_unsplit_launch_when_an_automatic_split
     rc = lib.ti_gemm_plan(pr.a_base, pr.sAb, pr.sAm, 1, pr.b_base, pr.sBb, pr.sBn, 1, pr.c_base, pr.sCb, pr.sCm, 1, 1, pr.M, pr.N, pr.K,
                           1 << 12, B_F32, 1 << 12, 1 << 12, EPI_SCALE_F, F32, 0, pl.config | (3 << 8), 1, out)
     assert rc == -2 and "static scratch" in lib.ti_last_error().decode()
+
+
+@pytest.mark.parametrize("B,M,N,K,pad", [(1, 65, 80, 16, 48), (3, 130, 128, 144, 0), (70, 129, 208, 304, 0), (2, 257, 144, 128, 32), (40, 700, 128, 1040, 16),
+                                         (1, 100, 512, 8192, 0), (2, 1, 16, 2064, 0)])
+def test_kn_operands_stay_inside(lib, B, M, N, K, pad):
+    """[K,N] operands on the wave-specialised kernels, forced and chosen, with K split where the batch allows it."""
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    forced = [i for i, nm in enumerate(names) if nm.startswith(("ws_256x128", "ws_128x128"))]
+    for cfg in [-1] + forced + ([i | (3 << 8) for i in forced] if B == 1 else []):
+        for epi, dt in ((EPI_SCALE_I8, I8), (EPI_SCALE_F, F32)):
+            ld = N + pad
+            pr = G.Problem(B, M, N, K, M * K, K, K * ld, 1, M * N, N, dt, sBk=ld)
+            G.check_launch(pr, G.plan_for(lib, pr, epi, B_NONE, cfg), store_sample=12)

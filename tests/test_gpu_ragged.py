@@ -125,6 +125,29 @@ def test_row_piece_kernel_every_stage_length(M, N, K):
             assert torch.equal(linear.linear_a8_w8_b32_o32(a, w, b32, _config=cfg | (kc // 256) << 8), want), kc
 
 
+@pytest.mark.parametrize("B,M,N,K,pad", [(1, 65, 80, 16, 48), (3, 130, 128, 144, 0), (1, 256, 1024, 4112, 16), (70, 129, 208, 304, 0), (2, 257, 144, 128, 32),
+                                         (1, 100, 512, 8192, 0), (40, 700, 128, 1040, 0), (2, 1, 16, 2064, 0)])
+def test_kn_operand_on_the_wave_specialised_kernels(B, M, N, K, pad):
+    """[K,N] operands with whole 16-byte pieces, both tile sizes and the chosen configuration: K below, at and off a
+    k-tile, N and M off a tile, rows at a pitch, split K: exact against torch in float64."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels._gemm import bmm
+
+    lib = L.lib()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randint(-128, 128, (B, M, K + pad), dtype=torch.int8, device="cuda", generator=g)[:, :, :K]
+    b = torch.randint(-128, 128, (B, K, N + pad), dtype=torch.int8, device="cuda", generator=g)[:, :, :N]
+    alpha = torch.tensor(40.0 / (K ** 0.5 * 5400.0), device="cuda")
+    acc = torch.stack([x.double() @ y.double() for x, y in zip(a, b)]).to(torch.int32)
+    f = acc.float() * alpha
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    for cfg in [-1] + [i for i, nm in enumerate(names) if nm.startswith(("ws_256x128", "ws_128x128"))]:
+        for dt, ep, want in ((torch.int8, L.EPI_SCALE_I8, f.round().clamp(-128, 127).to(torch.int8)), (torch.float32, L.EPI_SCALE_F, f),
+                             (torch.float16, L.EPI_SCALE_F, f.half())):
+            got = bmm(a, b, b_is_kn=True, epilogue=ep, out_dtype=dt, alpha=alpha, config=cfg)
+            assert torch.equal(got, want), (cfg, dt)
+
+
 @pytest.mark.parametrize("M,N,K", [(64, 4096, 16384), (33, 528, 10256), (100, 512, 5120), (300, 1024, 20480)])
 def test_split_k_adds_the_residual_in_its_last_item(M, N, K):
     """Linear + residual with K split over workgroups: the bits of the linear followed by an fp32 add."""

@@ -1372,7 +1372,11 @@ __global__ __launch_bounds__(512) void gemm_mfma_shortk_kernel(GemmParams p) {
 //             barrier g; last k-step, reading the first fragments of k-tile g+1 meanwhile.
 // The consumers issue no loads, so their stores (and bias loads) interfere with no counter; the
 // producers run ahead during an epilogue until the next barrier holds them.
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int PW>
+//
+// BKN: B is [K,N] (V as it comes out of its projection).  A stage holds it as [k][128 n] and the consumers read it
+// with the transposing LDS read.  40 x 1024 x 128 x 1024 14.5 us: 160 of the 256 CUs have a tile, and each takes in its
+// 384 KB at about 33 GB/s.
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int PW, bool BKN = false>
 __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_kernel(GemmParams p) {
   constexpr int NWC = WAVES_M * WAVES_N;  // consumer waves
   constexpr int NTP = PW * 64;            // producer threads
@@ -1388,6 +1392,7 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
   constexpr int DEPTH = NSTAGE - 1;
   static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BK % 64 == 0, "tile shape");
   static_assert(NSTAGE >= 3 && LDS_BYTES <= 160 * 1024, "LDS budget");
+  static_assert(!BKN || (BN == 128 && BK * BN / 16 % NTP == 0), "eight chunks per [k][n] row");
 
   __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
 
@@ -1446,18 +1451,20 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
   if (wave >= NWC) {
     // ================================ producer ================================
     const int ptid = tid - NWC * 64;
-    const int lda = (int)p.sAm, ldb = (int)p.sBn;
+    const int lda = (int)p.sAm, ldb = (int)(BKN ? p.sBk : p.sBn);
     const unsigned wave_slot = __builtin_amdgcn_readfirstlane(lds_base + (wave - NWC) * 1024);
     TileLoader<BM, BK, NTP, SWZ> la;
-    TileLoader<BN, BK, NTP, SWZ> lb;
+    std::conditional_t<BKN, TileLoader<BK, BN, NTP, 0>, TileLoader<BN, BK, NTP, SWZ>> lb;
     la.init(ptid, 0, lda, p.K);
-    lb.init(ptid, 0, ldb, p.K);
+    lb.init(ptid, 0, ldb, BKN ? p.N : p.K);
     constexpr int A_IT = decltype(la)::IT, B_IT = decltype(lb)::IT;
     constexpr int LOADS = A_IT + B_IT;
     static_assert(LOADS * DEPTH <= 63, "loads in flight must fit the counter");
     const int OOB = (int)0x80000000;
     v4i rA, rB;
     int i_issue = 0, k_issue = 0, st_issue = 0, kt_left = 0;
+    const int8_t* b_kn = p.B;  // BKN: the next k-tile's first byte, what the operand holds from there, the tile's first column
+    int b_extent = 0, b_n0 = 0;
     // one column of tiles: every byte of A is read exactly once, so it need not stay in the caches
     const bool a_once = p.tiles_n == 1;
     auto aim = [&](int i) {
@@ -1470,12 +1477,19 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
         k_issue = kt0 * BK;
         // rows at or past M (N) and bytes past K of the last row read as zero
         rA = make_rsrc(p.A + (int64_t)bz * p.sAb + (int64_t)m0 * lda, (p.M - 1 - m0) * lda + p.K);
-        rB = make_rsrc(p.B + (int64_t)bz * p.sBb + (int64_t)n0 * ldb, (p.N - 1 - n0) * ldb + p.K);
+        if constexpr (BKN) {
+          b_kn = p.B + (int64_t)bz * p.sBb + (int64_t)k_issue * ldb + n0;
+          b_extent = (p.K - 1 - k_issue) * ldb + p.N - n0;
+          b_n0 = n0;
+        } else {
+          rB = make_rsrc(p.B + (int64_t)bz * p.sBb + (int64_t)n0 * ldb, (p.N - 1 - n0) * ldb + p.K);
+        }
       } else {
         // past the last item: empty buffers, zeros into stages nobody reads; the number of loads
         // in flight, and so the count to wait for, stays constant
         rA = make_rsrc(p.A, 0);
-        rB = make_rsrc(p.B, 0);
+        if constexpr (BKN) b_extent = 0;
+        else rB = make_rsrc(p.B, 0);
       }
     };
     auto issue_ktile = [&]() {
@@ -1488,10 +1502,23 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
         for (int d = 0; d < A_IT; ++d)
           dma16_to_lds(rA, (k_issue < la.klim[d]) ? la.voff[d] : OOB, k_issue, wave_slot + st_issue * STAGE + d * NTP * 16);
       }
+      if constexpr (BKN) {
+        // the k-tile's rows: past the last one they are out of the descriptor's range, so it moves along
+        const uint64_t at = (uint64_t)b_kn;
+        rB = make_rsrc((const void*)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
+                                     (unsigned)__builtin_amdgcn_readfirstlane((int)at)),
+                       __builtin_amdgcn_readfirstlane(b_extent));
 #pragma unroll
-      for (int d = 0; d < B_IT; ++d)
-        dma16_to_lds(rB, (k_issue < lb.klim[d]) ? lb.voff[d] : OOB, k_issue,
-                     wave_slot + st_issue * STAGE + A_BYTES + d * NTP * 16);
+        for (int d = 0; d < B_IT; ++d)
+          dma16_to_lds(rB, b_n0 < lb.klim[d] ? lb.voff[d] : OOB, 0, wave_slot + st_issue * STAGE + A_BYTES + d * NTP * 16);
+        b_kn += (int64_t)BK * ldb;
+        b_extent = max(b_extent - BK * ldb, 0);
+      } else {
+#pragma unroll
+        for (int d = 0; d < B_IT; ++d)
+          dma16_to_lds(rB, (k_issue < lb.klim[d]) ? lb.voff[d] : OOB, k_issue,
+                       wave_slot + st_issue * STAGE + A_BYTES + d * NTP * 16);
+      }
       k_issue += BK;
       st_issue = (st_issue + 1 == NSTAGE) ? 0 : st_issue + 1;
       if (--kt_left == 0) {
@@ -1532,10 +1559,24 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
   const int fhalf = lane >> 5;
   const int a_lane = (wm * WTM + frow) * BK;
   const int b_lane = A_BYTES + (wn * WTN + frow) * BK;
+  // BKN: transposed reads of the [k][n] stage.  16 lanes fetch an 8 x 16 block (the lane's address is half of one of its
+  // rows) and each gets one column's 8 k; row k's chunk c lies at c ^ (k & 7)
+  typedef int v2i __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) v2i lds_v2i;
+  const int t_row = (lane & 15) >> 1, t_lane = A_BYTES + (fhalf * 16 + t_row) * BN + (lane & 1) * 8;
   v4i fa[2][TM], fb[2][TN];
   auto load_frag = [&](const char* stage, int ks, int buf, int r) {
     const int coff = ((ks * 2 + fhalf) ^ fsw) * 16;
     if (r < TM) fa[buf][r] = *(const v4i*)(stage + a_lane + r * 32 * BK + coff);
+    else if constexpr (BKN) {
+      const int c = ((wn * WTN + (r - TM) * 32) / 16 + ((lane >> 4) & 1)) ^ t_row;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const v2i t = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(stage + t_lane + (ks * 32 + h * 8) * BN + c * 16));
+        fb[buf][r - TM][2 * h] = t[0];
+        fb[buf][r - TM][2 * h + 1] = t[1];
+      }
+    }
     else fb[buf][r - TM] = *(const v4i*)(stage + b_lane + (r - TM) * 32 * BK + coff);
   };
   // first: the tile's first k-step starts from a zero C operand (an inline constant of the
@@ -2581,6 +2622,15 @@ static KernelFn ragged_kn_kernel(int bm, int oc) {
   return fns[bm > 64][oc];
 }
 
+// gemm_mfma_ws_kernel for a [K,N] operand: 256 x 128 and 128 x 128 tiles
+static KernelFn ws_kn_kernel(int bm, int oc) {
+#define TI_WS_KN(BM, NS) {gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT8, 4, true>, \
+                          gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT32, 4, true>, gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT16, 4, true>}
+  static const KernelFn fns[2][3] = {TI_WS_KN(128, 4), TI_WS_KN(256, 3)};
+#undef TI_WS_KN
+  return fns[bm > 128][oc];
+}
+
 enum ConfigId {
   CFG_GATHER = 0,
   CFG_TILE_256x128,   // one tile per workgroup: any output layout the fast loads allow
@@ -2694,8 +2744,7 @@ static bool ragged_eligible(const GemmParams& p) {
 
 // The stream kernels store through range-checked buffer descriptors with 32-bit offsets and, for
 // int8, whole 16-byte segments only.
-static bool stream_eligible(const GemmParams& p) {
-  if (!fast_eligible(p)) return false;
+static bool stream_stores(const GemmParams& p) {
   if (p.sCn != 1 || p.sCm < p.N || p.sCb < 0) return false;
   const int oc = out_class(p.out_dtype);
   const int esz = oc == OUT8 ? 1 : (oc == OUT32 ? 4 : 2);
@@ -2705,6 +2754,21 @@ static bool stream_eligible(const GemmParams& p) {
   if ((uintptr_t)p.C % esz) return false;
   if (oc == OUT8 && ((p.N & 15) || (p.sCm & 15) || (p.sCb & 15) || ((uintptr_t)p.C & 15))) return false;
   return true;
+}
+
+static bool stream_eligible(const GemmParams& p) { return fast_eligible(p) && stream_stores(p); }
+
+// A [K,N] operand on the wave-specialised kernels: as fast_eligible and stream_eligible, with B's rows along k, whole
+// 16-byte chunks of n
+static bool kn_eligible(const GemmParams& p) {
+  if (p.sAk != 1 || p.sBn != 1 || p.K <= 0 || ((p.K | p.N) & 15)) return false;
+  if ((p.sAm & 15) || (p.sBk & 15) || (p.sAb & 15) || (p.sBb & 15)) return false;
+  if (((uintptr_t)p.A & 15) || ((uintptr_t)p.B & 15)) return false;
+  if (p.sAm < p.K || p.sBk < p.N) return false;
+  const int64_t lim = (int64_t)1 << 31;
+  if (((int64_t)p.M + 512) * p.sAm + p.K >= lim) return false;
+  if (((int64_t)p.K + 512) * p.sBk + p.N >= lim) return false;
+  return stream_stores(p);
 }
 
 // k-tiles per split and the number of non-empty splits for `want` splits of a K of `kt` k-tiles
@@ -2771,9 +2835,19 @@ static int pick_config(const GemmParams& p, int* splits_out) {
   *splits_out = 1;
   if (!fast_eligible(p)) {
     if (!ragged_eligible(p)) return CFG_GATHER;
+    // P.V with V as [keys, head_dim] and whole 16-byte pieces: the wave-specialised kernel once the k-loop is long
+    // enough (us, gemm_ragged_kernel / this one, int8 out, 128 columns: 40 x 1024 x 1024 17.1 / 14.5, 80 x 2048 x 2048 109 /
+    // 76, 24 x 1024 x 1024 11.8 / 9.9, 4 x 2048 x 2048 15.0 / 13.9; but 10 x 1024 x 1024 10.1 / 10.9, 80 x 304 x 304 7.1 /
+    // 8.0, and with 64 columns 40 x 2048 x 2048 33.6 / 46.9)
+    const int64_t tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+    if (kn_eligible(p) && p.N > 64 && p.M > 64 && (p.K >= 1536 || (p.K >= 1024 && tiles >= 192))) {
+      double wide, narrow;
+      const int sw = pick_splits(p, g_configs[CFG_WS_256x128], 1.0, &wide), sn = pick_splits(p, g_configs[CFG_WS_128x128], 0.8, &narrow);
+      *splits_out = wide <= narrow ? sw : sn;
+      return wide <= narrow ? CFG_WS_256x128 : CFG_WS_128x128;
+    }
     // small tiles where large ones would not give every CU one, or would be half padding (P.V with 64 columns, V as [K,N],
     // 80 x 1024 x 64 x 1024: 46.7 us on the large ones, 19.1 us on the small)
-    const int64_t tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
     return tiles >= 256 && p.N > 64 ? CFG_RAGGED_128 : CFG_RAGGED_64;
   }
   const bool stream = stream_eligible(p);
@@ -3085,8 +3159,9 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
   if (!k.fn[out_class(p.out_dtype)]) return fail(TI_E_COMBO, "config %s has no kernel for output dtype %d", k.name, p.out_dtype);
   if ((k.fast || k.ragged) && !k.skinny && !k.rows4 && !k.rowpieces && trunc8) return fail(TI_E_COMBO, "config %s does not implement TI_ROUND_TRUNC for int8 outputs", k.name);
   if (k.ragged && !ragged_eligible(p)) return fail(TI_E_COMBO, "config %s needs unit strides along K (B: along K or N) and rows that do not overlap", k.name);
-  if (k.fast && !fast_eligible(p)) return fail(TI_E_COMBO, "config %s needs K-contiguous 16-byte aligned operands", k.name);
-  if (k.stream_occ && !stream_eligible(p)) return fail(TI_E_COMBO, "config %s needs a row-major output with 16-byte aligned rows", k.name);
+  const bool kn = (config == CFG_WS_256x128 || config == CFG_WS_128x128) && kn_eligible(p);
+  if (k.fast && !kn && !fast_eligible(p)) return fail(TI_E_COMBO, "config %s needs K-contiguous 16-byte aligned operands", k.name);
+  if (k.stream_occ && !kn && !stream_eligible(p)) return fail(TI_E_COMBO, "config %s needs a row-major output with 16-byte aligned rows", k.name);
   if (k.max_k && (p.K < 16 || p.K > k.max_k)) return fail(TI_E_COMBO, "config %s needs 16 <= K <= %d", k.name, k.max_k);
   if (k.max_k && out_class(p.out_dtype) == OUT8 && (p.bias_kind != TI_BIAS_NONE || p.epilogue == TI_EPI_GELU_I8))
     return fail(TI_E_COMBO, "config %s has no int8 epilogue with a bias or GELU", k.name);
@@ -3238,7 +3313,8 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       dry->grid_x = (unsigned)g; dry->grid_y = 1;
       return TI_OK;
     }
-    k.fn[out_class(p.out_dtype)]<<<dim3((unsigned)g), dim3(k.threads), 0, stream>>>(p);
+    const KernelFn fn = kn ? ws_kn_kernel(k.bm, out_class(p.out_dtype)) : k.fn[out_class(p.out_dtype)];
+    fn<<<dim3((unsigned)g), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.batch, 1);
