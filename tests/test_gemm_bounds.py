@@ -152,3 +152,15 @@ def test_kn_operands_stay_inside(lib, B, M, N, K, pad):
             ld = N + pad
             pr = G.Problem(B, M, N, K, M * K, K, K * ld, 1, M * N, N, dt, sBk=ld)
             G.check_launch(pr, G.plan_for(lib, pr, epi, B_NONE, cfg), store_sample=12)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 65])
+@pytest.mark.parametrize("kn", [False, True])
+def test_truncating_int8_outputs_are_planned_for_every_operand_layout(lib, M, kn):
+    """TI_ROUND_TRUNC on operands the fast path does not take: any K, [K,N] rows."""
+    for B, N, K in ((1, 80, 77), (1, 128, 2048), (6, 128, 1040)):
+        pr = G.Problem(B, M, N, K, M * K, K, N * K, 1 if kn else K, M * N, N, I8, sBk=N if kn else 1)
+        if kn or K % 16:
+            assert G.plan_for(lib, pr, EPI_SCALE_I8, B_NONE, round_mode=1).name.startswith("gather")
+        else:
+            G.plan_for(lib, pr, EPI_SCALE_I8, B_NONE, round_mode=1)

@@ -3150,7 +3150,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
   int auto_splits = 1;
   if (config < 0) {
     // int8 truncation (a test-time switch) is implemented by the gather kernel and the M <= 64 kernels
-    if (trunc8 && p.M > 16) config = (p.M <= 64 && fast_eligible(p)) ? CFG_SKINNY_16 + 1 + (p.M > 32) : CFG_GATHER;
+    if (trunc8 && (p.M > 16 || !fast_eligible(p))) config = (p.M <= 64 && fast_eligible(p)) ? CFG_SKINNY_16 + 1 + (p.M > 32) : CFG_GATHER;
     else config = pick_config(p, &auto_splits);
   }
   else if (config < g_num_configs && !want_splits && g_configs[config].ws_waves) auto_splits = pick_splits(p, g_configs[config], 1.0, nullptr);
