@@ -472,7 +472,11 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
         # last 16 bytes): what can go wrong is the grid and a row that is not inside the operand
         BM, BN = (int(x) for x in re.match(r"ragged_(\d+)x(\d+)x64", name).groups())
         assert pl.tiles_m == -(-pr.M // BM) and pl.tiles_n == -(-pr.N // BN) and pl.threads == 256
-        assert pl.grid_x == pl.tiles_m * pl.tiles_n and pl.grid_y == pr.batch
+        T, KT = pl.tiles_m * pl.tiles_n, -(-pr.K // 64)
+        assert pl.grid_x == T * pl.splits and pl.grid_y == pr.batch
+        if pl.splits > 1:
+            assert pr.batch == 1 and (pl.splits - 1) * pl.kt_split < KT <= pl.splits * pl.kt_split, "the splits do not cover K once"
+            assert T * pl.splits * BM * BN * 4 <= pl.partial_bytes <= 0x7FFFFFF0 and T * 4 <= (1 << 14)
         assert (pr.batch - 1) * pr.sAb + (pr.M - 1) * pr.sAm + pr.K <= pr.a_bytes()
         b_rows, b_len, ld = (pr.N, pr.K, pr.sBn) if pr.sBk == 1 else (pr.K, pr.N, pr.sBk)
         assert (pr.batch - 1) * pr.sBb + (b_rows - 1) * ld + b_len <= pr.b_bytes()

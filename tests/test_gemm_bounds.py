@@ -164,3 +164,15 @@ def test_truncating_int8_outputs_are_planned_for_every_operand_layout(lib, M, kn
             assert G.plan_for(lib, pr, EPI_SCALE_I8, B_NONE, round_mode=1).name.startswith("gather")
         else:
             G.plan_for(lib, pr, EPI_SCALE_I8, B_NONE, round_mode=1)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1025), (1, 4097, 4097), (62, 304, 19542), (117, 1495, 8671), (65, 64, 1024 + 17), (300, 8200, 5001), (2048, 5120, 5119)])
+def test_split_k_of_the_ragged_kernel_covers_k_once(lib, M, N, K):
+    """The chosen split and forced ones, into the allocated workspace and the fixed scratch."""
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    forced = [i | (s << 8) for i, nm in enumerate(names) if nm.startswith("ragged") for s in (1, 2, 7)] if M <= 128 else []
+    for cfg in [-1] + forced:
+        for static in (0, 1):
+            for epi, dt in ((EPI_SCALE_I8, I8), (EPI_SCALE_F, F32)):
+                pr = G.contiguous(1, M, N, K, dt)
+                G.check_launch(pr, G.plan_for(lib, pr, epi, B_NONE, cfg, static))

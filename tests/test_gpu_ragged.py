@@ -198,6 +198,35 @@ def test_ragged_kernel_any_alignment_and_layout(B, M, N, K):
     assert torch.equal(out[:, :, 3:N + 3], bmm.bmm_s8t_s8t_s8t(a, b_kn, alpha)) and bool((out[:, :, :3] == 77).all() and (out[:, :, N + 3:] == 77).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1025), (17, 63, 1024), (62, 304, 9542), (65, 130, 4097), (129, 128, 2111)])
+def test_ragged_kernel_with_k_split(M, N, K):
+    """Exact for every split, chosen and forced, both tile sizes and operand layouts, every output class; repeated, since
+    the tickets have to be back at zero after each launch."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import bmm, linear
+
+    lib = L.lib()
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w, wt = (torch.randint(-128, 128, (1, r, c + 3), dtype=torch.int8, device="cuda", generator=g)[:, :, 1:c + 1] for r, c in ((M, K), (N, K), (K, N)))
+    acc = (a.double() @ w.double().transpose(1, 2).contiguous()).to(torch.int32)
+    acc_kn = (a.double() @ wt.double()).to(torch.int32)
+    alpha, one = torch.tensor(30.0 / (K ** 0.5 * 5400.0), device="cuda"), torch.tensor(1.0, device="cuda")
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    chosen = {}
+    for cfg in [-1] + [i | (s << 8) for i, nm in enumerate(names) if nm.startswith("ragged") for s in (1, 2, 3, 5, 16)]:
+        for _ in range(2):
+            assert torch.equal(bmm.bmm_s8t_s8n_s32t(a, w, _config=cfg), acc), cfg
+            chosen.setdefault(cfg, lib.ti_gemm_last_splits())
+            assert torch.equal(bmm.bmm_s8t_s8t_s32t(a, wt, _config=cfg), acc_kn), cfg
+            assert torch.equal(bmm.bmm_s8t_s8n_s8t(a, w, alpha, _config=cfg), (alpha * acc.float()).round().clamp(-128, 127).to(torch.int8)), cfg
+    assert chosen[-1] > 1
+    bf = torch.randn(N, device="cuda", generator=g)
+    half = linear.linear_a8_w8_bfp32_ofp32(a[0], w[0], bf.half(), alpha, one)
+    assert half.dtype == torch.float16 and torch.equal(half, (bf.half().float() + alpha * acc[0].float()).half())
+    res = torch.randn(M, N, device="cuda", generator=g)
+    assert torch.equal(linear.linear_a8_w8_bfp32_ofp32_residual(a[0], w[0], bf, alpha, one, res), bf + alpha * acc[0].float() + res)
+
+
 @pytest.mark.parametrize("rows,cols,q_len", [(3, 1, 0), (4, 7, 0), (6, 15, 3), (5, 17, 5), (8, 333, 8), (6, 1001, 0), (3, 1024 + 9, 3), (2, 2047, 2), (2, 8191, 0)])
 @pytest.mark.parametrize("scale", [0.0, 0.1])
 def test_softmax_q_rows_at_any_byte(rows, cols, q_len, scale):

@@ -62,7 +62,7 @@ struct GemmParams {
   int8_t* kv_vt;
   int64_t kv_k_hs, kv_k_rs, kv_vt_rs;
   int kv_D, kv_S;
-  // split K (gemm_mfma_ws_kernel, batch == 1): a tile's k-tiles are dealt to `splits` work items of
+  // split K (gemm_mfma_ws_kernel and gemm_ragged_kernel, batch == 1): a tile's k-tiles are dealt to `splits` work items of
   // kt_split k-tiles each (the last takes what is left); the items leave their int32 sums in
   // sk_partial, and the item of a tile that finishes last adds them up and stores the tile.
   int splits, kt_split;
@@ -1354,6 +1354,68 @@ __global__ __launch_bounds__(512) void gemm_mfma_shortk_kernel(GemmParams p) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// True: acc holds the tile's whole sums and this wave stores its part; false: another item's wave will.
+template <int TM, int TN, int NWC>
+__device__ __forceinline__ bool split_k_settle(const GemmParams& p, v16i (&acc)[TM][TN], int rank, int sp, int SPL, int wave, int lane) {
+  // Split K.  Each consumer wave settles its own part of the tile with the same wave of the
+  // tile's other items, no workgroup barrier involved: it stores its sums (every instruction
+  // 64 lanes x 16 consecutive bytes), waits until they are written and takes a ticket from the
+  // part's counter.  The wave that draws the last ticket knows that all the others' sums are
+  // in memory: it adds them to its own (integer sums: any order gives the same bits), puts the
+  // counter back to zero for the next launch and stores the tile.  Nobody waits for anybody.
+  // The sums travel with device-scope cache policy (sc1: written through to, and read from,
+  // the memory side that all XCDs share), so no cache-wide write-back or invalidation is needed.
+  constexpr int WAVE_BYTES = TM * TN * 16 * 64 * 4;
+  constexpr int SC1 = 16;
+  const __amdgpu_buffer_rsrc_t rP = __builtin_amdgcn_make_buffer_rsrc(p.sk_partial, 0, 0x7ffffff0, 0x00020000);
+  const int mine = ((rank * SPL + sp) * NWC + wave) * WAVE_BYTES + lane * 16;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        __builtin_amdgcn_raw_buffer_store_b128(
+            (v4u){(unsigned)acc[i][j][4 * q], (unsigned)acc[i][j][4 * q + 1], (unsigned)acc[i][j][4 * q + 2], (unsigned)acc[i][j][4 * q + 3]},
+            rP, mine + ((i * TN + j) * 4 + q) * 1024, 0, SC1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  int ticket = 0;
+  if (lane == 0) ticket = atomicAdd(p.sk_counter + rank * NWC + wave, 1);
+  ticket = __builtin_amdgcn_readfirstlane(ticket);
+  if (ticket != SPL - 1) return false;
+  // The other items' sums, 64 registers' worth of loads at a time (several items when an item's part is
+  // small) and all of them issued before the first add: left to itself the compiler waits for every
+  // 16-byte load before it issues the next, 2-byte and 4-byte outputs' kernels alike (64 x 4096 x 16384,
+  // 6 splits, fp32 out: 30.2 -> 21.3 us).
+  constexpr int NB = TM * TN, BPR = NB < 4 ? NB : 4, OPR = 4 / BPR;  // blocks of 32 x 32; blocks and items per round
+  for (int o = 0; o < SPL; o += OPR) {
+#pragma unroll
+    for (int b0 = 0; b0 < NB; b0 += BPR) {
+      v4i part[OPR][BPR][4];
+#pragma unroll
+      for (int d = 0; d < OPR; ++d) {
+        // this item's own sums and items past the last: out of range, zeros
+        const int theirs = o + d == sp || o + d >= SPL ? (int)0x80000000 : ((rank * SPL + o + d) * NWC + wave) * WAVE_BYTES + lane * 16;
+#pragma unroll
+        for (int b = 0; b < BPR; ++b)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (b0 + b < NB) part[d][b][q] = __builtin_amdgcn_raw_buffer_load_b128(rP, theirs + ((b0 + b) * 4 + q) * 1024, 0, SC1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < OPR; ++d)
+#pragma unroll
+        for (int b = 0; b < BPR; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (b0 + b < NB) acc[(b0 + b) / TN][(b0 + b) % TN][r] += part[d][b][r >> 2][r & 3];
+    }
+  }
+  if (lane == 0) atomicExch(p.sk_counter + rank * NWC + wave, 0);
+  return true;
+}
+
 // ---- wave-specialised persistent kernel -------------------------------------------------------
 //
 // A wave that issues a 16-byte-per-lane load is held for about 64 cycles by the address path, and
@@ -1651,62 +1713,7 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
       kstep((KS - 1) & 1, lds + st * STAGE, 0, Rpm1{}, std::false_type{});
     }
     if (SPL > 1) {
-      // Split K.  Each consumer wave settles its own quarter of the tile with the same wave of the
-      // tile's other items, no workgroup barrier involved: it stores its sums (every instruction
-      // 64 lanes x 16 consecutive bytes), waits until they are written and takes a ticket from the
-      // quarter's counter.  The wave that draws the last ticket knows that all the others' sums are
-      // in memory: it adds them to its own (integer sums: any order gives the same bits), puts the
-      // counter back to zero for the next launch and stores the tile.  Nobody waits for anybody.
-      // The sums travel with device-scope cache policy (sc1: written through to, and read from,
-      // the memory side that all XCDs share), so no cache-wide write-back or invalidation is needed.
-      constexpr int WAVE_BYTES = TM * TN * 16 * 64 * 4;
-      constexpr int SC1 = 16;
-      const __amdgpu_buffer_rsrc_t rP = __builtin_amdgcn_make_buffer_rsrc(p.sk_partial, 0, 0x7ffffff0, 0x00020000);
-      const int mine = ((rank * SPL + sp) * NWC + wave) * WAVE_BYTES + lane * 16;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            __builtin_amdgcn_raw_buffer_store_b128(
-                (v4u){(unsigned)acc[i][j][4 * q], (unsigned)acc[i][j][4 * q + 1], (unsigned)acc[i][j][4 * q + 2], (unsigned)acc[i][j][4 * q + 3]},
-                rP, mine + ((i * TN + j) * 4 + q) * 1024, 0, SC1);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      int ticket = 0;
-      if (lane == 0) ticket = atomicAdd(p.sk_counter + rank * NWC + wave, 1);
-      ticket = __builtin_amdgcn_readfirstlane(ticket);
-      if (ticket != SPL - 1) continue;
-      // The other items' sums, 64 registers' worth of loads at a time (several items when an item's part is
-      // small) and all of them issued before the first add: left to itself the compiler waits for every
-      // 16-byte load before it issues the next, 2-byte and 4-byte outputs' kernels alike (64 x 4096 x 16384,
-      // 6 splits, fp32 out: 30.2 -> 21.3 us).
-      constexpr int NB = TM * TN, BPR = NB < 4 ? NB : 4, OPR = 4 / BPR;  // blocks of 32 x 32; blocks and items per round
-      for (int o = 0; o < SPL; o += OPR) {
-#pragma unroll
-        for (int b0 = 0; b0 < NB; b0 += BPR) {
-          v4i part[OPR][BPR][4];
-#pragma unroll
-          for (int d = 0; d < OPR; ++d) {
-            // this item's own sums and items past the last: out of range, zeros
-            const int theirs = o + d == sp || o + d >= SPL ? (int)0x80000000 : ((rank * SPL + o + d) * NWC + wave) * WAVE_BYTES + lane * 16;
-#pragma unroll
-            for (int b = 0; b < BPR; ++b)
-#pragma unroll
-              for (int q = 0; q < 4; ++q)
-                if (b0 + b < NB) part[d][b][q] = __builtin_amdgcn_raw_buffer_load_b128(rP, theirs + ((b0 + b) * 4 + q) * 1024, 0, SC1);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int d = 0; d < OPR; ++d)
-#pragma unroll
-            for (int b = 0; b < BPR; ++b)
-#pragma unroll
-              for (int r = 0; r < 16; ++r)
-                if (b0 + b < NB) acc[(b0 + b) / TN][(b0 + b) % TN][r] += part[d][b][r >> 2][r & 3];
-        }
-      }
-      if (lane == 0) atomicExch(p.sk_counter + rank * NWC + wave, 0);
+      if (!split_k_settle<TM, TN, NWC>(p, acc, rank, sp, SPL, wave, lane)) continue;
     }
     if (wave == 0 && it == 0) TI_TL(2);
     stream_epilogue<TM, TN, OUTCLS>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN,
@@ -1729,6 +1736,7 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
 // Measured, byte gathers -> this kernel: P.V with V as [K,N], int8 out: 40 x 1024 x 128 x 1024 155 -> 17 us, 160 x 2048 x 128 x
 // 2048 2900 -> 197 us (3.6 TB/s of probabilities; the aligned V^T form on the persistent kernel: 137 us); P.V fp32 out with an
 // odd key count: 160 x 1001 x 128 x 1001 649 -> 83 us, 40 x 2047 x 128 x 2047 531 -> 88 us.
+// One GEMM of few tiles and a long K is split (pick_ragged), settled as in gemm_mfma_ws_kernel.
 // No byte outside an operand's rows is touched: a chunk that crosses the end of a row is loaded as the row's
 // last 16 bytes and shifted (load16_tail).
 template <int BM, int BN, bool BKN, int OUTCLS>
@@ -1741,13 +1749,16 @@ __global__ __launch_bounds__(256) void gemm_ragged_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
+  // split K (one GEMM): block sp * tiles + t is tile t's run sp of k-tiles
+  const int SPL = p.splits, tiles = p.tiles_m * p.tiles_n;
+  const int sp = SPL > 1 ? blockIdx.x / tiles : 0, rank = blockIdx.x - sp * tiles;
   int tile_m, tile_n, bz = 0;
-  if (gridDim.y == 1) tile_coords(p, blockIdx.x, tile_m, tile_n);
+  if (gridDim.y == 1) tile_coords(p, rank, tile_m, tile_n);
   else batch_tile_coords(p, blockIdx.x, blockIdx.y, gridDim.y, bz, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int8_t* Ab = p.A + (int64_t)bz * p.sAb;
   const int8_t* Bb = p.B + (int64_t)bz * p.sBb;
-  const int KT = (p.K + BK - 1) / BK;
+  const int kt0 = sp * p.kt_split, kt1 = SPL > 1 ? min((p.K + BK - 1) / BK, kt0 + p.kt_split) : (p.K + BK - 1) / BK;
 
   // this thread's chunks: rows past the last one repeat it (their products are dropped, or multiplied by the
   // zeros that A holds past K)
@@ -1846,17 +1857,18 @@ __global__ __launch_bounds__(256) void gemm_ragged_kernel(GemmParams p) {
     }
   };
 
-  if (KT > 0) {
-    fetch(0);
-    stash(lds);
+  if (kt1 > kt0) {
+    fetch(kt0);
+    stash(lds + (kt0 & 1) * STAGE);
     __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      if (kt + 1 < KT) fetch(kt + 1);
+    for (int kt = kt0; kt < kt1; ++kt) {
+      if (kt + 1 < kt1) fetch(kt + 1);
       compute(lds + (kt & 1) * STAGE);
-      if (kt + 1 < KT) stash(lds + ((kt + 1) & 1) * STAGE);  // its readers passed the barrier of k-tile kt-1
+      if (kt + 1 < kt1) stash(lds + ((kt + 1) & 1) * STAGE);  // its readers passed the barrier of k-tile kt-1
       __syncthreads();
     }
   }
+  if (SPL > 1 && !split_k_settle<TM, TN, 4>(p, acc, rank, sp, SPL, wave, lane)) return;
   const EpiCtx e = make_epi(p, bz);
   tile_epilogue<TM, TN, OUTCLS>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN, lane);
 }
@@ -2805,6 +2817,9 @@ static double config_cost(const GemmParams& p, const Config& k, double eff, int 
   return rounds_eff * k_len * (double)(k.bm * k.bn) * occ / eff / (1.0 + 0.1 / (double)rounds);
 }
 
+// Waves of a workgroup that settle their parts of a tile when K is split; 0: the configuration cannot
+static int sk_waves(const Config& k) { return k.ragged ? 4 : k.ws_waves; }
+
 // Number of K splits for a wave-specialised configuration: as many as fill the chip's 256 workgroup
 // slots once, but no split shorter than 2560 bytes of K (K = 4096 is faster whole, K = 5120 in two
 // parts) and no more than 8 (the last item of a tile reads the other splits' sums one after the other).
@@ -2828,6 +2843,35 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
   return used;
 }
 
+// Tile and K splits of gemm_ragged_kernel.  A k-tile costs a workgroup 0.5-0.8 us of load latency whatever else the chip
+// does, so a few tiles of a long K are bound by that chain.  Measured for one GEMM, weights from HBM, int32 out, us:
+//   64 x 64 tiles, whole K / 2 / 4 / 8 / 16 / 24 / 48 splits: 62 x 304 x 19542 179 / 92 / 49 / 27.8 / 19.7 / 18.7 / 22.3, 117 x
+//   1495 x 8671 83 / 44.7 / 26.2 / 20.0 / 20.7 / 24.2, 16 x 4096 x 4097 40.6 / 23.4 / 14.6 / 12.9 / 15.2, 64 x 5120 x 5121 52 /
+//   30.2 / 21.1 / 18.4 / 21.4, 256 x 1000 x 5001 49 / 27.9 / 16.7 / 14.8 / 16.5, 64 x 1000 x 1001 10.0 / 8.2 / (3) 7.2; with 128
+//   x 128 tiles slower at every one of them.  The line: two workgroups per CU, splits of 5 k-tiles and more, 24 of them.
+//   128 tiles and more fill the four workgroups that a CU holds (whole K / 2 / 3 / 4 splits): 256 x 4096 x 4097 39.9 / 29.5 /
+//   24.2 / 23.3, 256 x 4096 x 2001 22.0 / 18.5 / 15.3 / 16.0, 512 x 2048 x 2049 22.1 / 17.6 / 15.4 / 15.6, 512 x 4096 x 2049
+//   28.5 / 23.4 / 28.9, 65 x 8200 x 4097 42.1 / 31.0 / 24.6 / 30.9 (4: one more than the chip holds).
+//   128 x 128 tiles, 64 and more of them, split to two workgroups per CU, lead where each still has many k-tiles (64 x 64 at
+//   its best split / 128 x 128): 256 x 4096 x 10241 60 / 54, 512 x 4096 x 4097 38.9 / 34.8, 1000 x 2000 x 16383 116 / 86, 333 x
+//   4096 x 4001 31.7 / 31.5; but 256 x 4096 x 4097 23.3 / 28.3, 512 x 4096 x 2049 23.4 / 26.2.  The line: tiles x K of 384000.
+//   From 256 tiles on whole K: 785 x 5680 x 1082 26.3 (2 splits 39.5), 1500 x 4096 x 8191 150 (166).
+// Small tiles where the large ones would be half padding, split or not: P.V with 64 columns, V as [K,N], 80 x 1024 x 64 x
+// 1024: 46.7 us on the large ones, 19.1 us on the small.
+static int pick_ragged(const GemmParams& p, int64_t tiles128, int* splits_out) {
+  if (tiles128 >= 256 && p.N > 64) return CFG_RAGGED_128;
+  if (p.batch != 1) return CFG_RAGGED_64;
+  if (tiles128 >= 64 && p.N > 64 && p.M > 64 && tiles128 * p.K >= 384000) {
+    const int64_t fill = 512 / tiles128, by_k = p.K / 900;
+    *splits_out = (int)(fill < by_k ? fill : by_k);  // 1 or more: K is 1506 at least
+    return CFG_RAGGED_128;
+  }
+  const int64_t tiles = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64);
+  const int64_t fill = (tiles < 128 ? 512 : 1024) / tiles, by_k = p.K / 320, want = fill < by_k ? fill : by_k;
+  *splits_out = want < 1 ? 1 : (want > 24 ? 24 : (int)want);
+  return CFG_RAGGED_64;
+}
+
 // Tile choice: the configuration (and K split) with the lowest estimated run time.  The class
 // efficiencies were measured with weights streamed from HBM.  Outputs the persistent kernels can
 // store (row-major, aligned) go to them; the rest to the one-tile kernels.
@@ -2846,9 +2890,7 @@ static int pick_config(const GemmParams& p, int* splits_out) {
       *splits_out = wide <= narrow ? sw : sn;
       return wide <= narrow ? CFG_WS_256x128 : CFG_WS_128x128;
     }
-    // small tiles where large ones would not give every CU one, or would be half padding (P.V with 64 columns, V as [K,N],
-    // 80 x 1024 x 64 x 1024: 46.7 us on the large ones, 19.1 us on the small)
-    return tiles >= 256 && p.N > 64 ? CFG_RAGGED_128 : CFG_RAGGED_64;
+    return pick_ragged(p, tiles, splits_out);
   }
   const bool stream = stream_eligible(p);
   if (p.M <= 64 && p.batch <= 4) {
@@ -3259,15 +3301,15 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
   g_last_config = config;
   p.splits = 1;
   p.kt_split = 0;
-  if (want_splits > 1 && !(k.ws_waves && p.batch == 1)) return fail(TI_E_COMBO, "config %s cannot split K (batch %d)", k.name, p.batch);
-  if (k.ws_waves && p.batch == 1) {
+  if (want_splits > 1 && !(sk_waves(k) && p.batch == 1)) return fail(TI_E_COMBO, "config %s cannot split K (batch %d)", k.name, p.batch);
+  if (sk_waves(k) && p.batch == 1) {
     const int kt = (p.K + k.bk - 1) / k.bk;
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
     int splits = want_splits ? want_splits : auto_splits;
     sk_shape(kt, splits, splits, p.kt_split);
     const size_t item_bytes = (size_t)k.bm * k.bn * sizeof(int);
     if (splits > 1 && static_scratch &&
-        ((size_t)tiles * k.ws_waves > SK_STATIC_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_STATIC_PARTIAL_BYTES)) {
+        ((size_t)tiles * sk_waves(k) > SK_STATIC_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_STATIC_PARTIAL_BYTES)) {
       // a split the caller forced is refused; one the library chose itself gives way to the unsplit launch,
       // which needs no scratch at all (as the allocating path does when its workspace limit is exceeded)
       if (want_splits)
@@ -3281,7 +3323,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
         rc = sk_static_scratch(stream, &p.sk_partial, &p.sk_counter);
         if (rc != TI_OK) return rc;
       }
-    } else if (splits > 1 && ((size_t)tiles * k.ws_waves > SK_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_MAX_PARTIAL_BYTES)) {
+    } else if (splits > 1 && ((size_t)tiles * sk_waves(k) > SK_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_MAX_PARTIAL_BYTES)) {
       if (want_splits) return fail(TI_E_SHAPE, "%d splits of %lld tiles exceed the split-K workspace", splits, (long long)tiles);
       splits = 1;
     }
@@ -3317,7 +3359,8 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
     fn<<<dim3((unsigned)g), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }
-  dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.batch, 1);
+  if ((int64_t)p.tiles_m * p.tiles_n * p.splits > 0x7fffffff) return fail(TI_E_SHAPE, "too many tiles");
+  dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits), (unsigned)p.batch, 1);
   if (dry) {
     dry->grid_x = grid.x; dry->grid_y = grid.y;
     return TI_OK;
@@ -3365,15 +3408,16 @@ static int run_with_residual(GemmParams p, const float* R, int64_t ldr, hipStrea
     return run(p, cfg, stream);
   }
   // the persistent kernels add it in their fp32 epilogue (with split K: in that of a tile's last item, where the
-  // sums are whole); 32-bit offsets into the residual, like the stores
+  // sums are whole); 32-bit offsets into the residual, like the stores.  run() chooses again, the same way: a split passed
+  // to it would count as forced, and a capturing stream without a workspace would be refused instead of run unsplit
   const bool persistent = g_configs[cfg].stream_occ > 0 || g_configs[cfg].ws_waves > 0 || g_configs[cfg].max_k > 0;
   if (persistent && p.batch == 1 && p.out_dtype == TI_F32 && p.epilogue == TI_EPI_SCALE_F &&
       ((int64_t)(p.M + 512) * ldr + p.N) * 4 < ((int64_t)1 << 31)) {
     p.resid = R;
     p.resid_rs = ldr;
-    return run(p, cfg | (splits << 8), stream);
+    return run(p, -1, stream);
   }
-  rc = run(p, cfg | (splits << 8), stream);
+  rc = run(p, -1, stream);
   if (rc != TI_OK) return rc;
   const int vec = (p.N % 4 == 0) && (p.sCm % 4 == 0) && (ldr % 4 == 0) && (((uintptr_t)p.C | (uintptr_t)R) & 15) == 0;
   const int64_t items = (int64_t)p.M * (vec ? p.N / 4 : p.N);
