@@ -83,6 +83,12 @@ double number(PyObject* o) {
   return PyFloat_AsDouble(o);
 }
 
+// A Python bool itself: anything else that counts as true or false is for the Python path to convert.
+bool flag(PyObject* o) {
+  need(PyBool_Check(o));
+  return o == Py_True;
+}
+
 int bias_kind(ScalarType t) {
   switch (t) {
     case ScalarType::Char: return TI_BIAS_I8;
@@ -210,7 +216,7 @@ PyObject* bmm(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Call c(a);
     const Tensor& b = tensor(v[1], c.dev, ScalarType::Char);
     need(a.dim() == 3 && b.dim() == 3 && a.size(0) == b.size(0));
-    const int kn = v[2] == Py_True;  // b is [B, K, N]
+    const bool kn = flag(v[2]);  // b is [B, K, N]
     need(a.size(2) == b.size(kn ? 1 : 2));
     const int64_t B = a.size(0), M = a.size(1), K = a.size(2), N = b.size(kn ? 2 : 1);
     const int dt = (int)integer(v[6]);
@@ -262,7 +268,7 @@ PyObject* layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(g);
     Tensor out = c.empty(x.sizes(), ScalarType::Char);
     const int rc = ti_layernorm_q((const float*)ptr(x), N, g, b, (float)number(v[3]), (int8_t*)mptr(out), N, int32_size(x.numel() / N),
-                                  int32_size(N), v[4] == Py_True, (int)integer(v[5]), nullptr, nullptr, c.stream);
+                                  int32_size(N), flag(v[4]), (int)integer(v[5]), nullptr, nullptr, c.stream);
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -308,9 +314,9 @@ PyObject* layernorm_fp(PyObject*, PyObject* const* v, Py_ssize_t n) {
       skip = ptr(s);
     }
     Tensor out, sout;
-    if (v[6] == Py_True) out = c.empty(x.sizes(), type);
-    if (v[7] == Py_True) sout = c.empty(x.sizes(), type);
-    const int rc = ti_layernorm_fp(ptr(x), N, skip, skip ? N : 0, dt, g, b, (float)number(v[4]), v[5] == Py_True,
+    if (flag(v[6])) out = c.empty(x.sizes(), type);
+    if (flag(v[7])) sout = c.empty(x.sizes(), type);
+    const int rc = ti_layernorm_fp(ptr(x), N, skip, skip ? N : 0, dt, g, b, (float)number(v[4]), flag(v[5]),
                                    out.defined() ? mptr(out) : nullptr, N, sout.defined() ? mptr(sout) : nullptr, N,
                                    int32_size(x.numel() / N), int32_size(N), c.stream);
     need(rc == TI_OK);
