@@ -355,6 +355,7 @@ int ti_kv_append_i8(const int8_t* k_src, int64_t k_src_row_stride, const int8_t*
 /*
  * The same for `seqs` sequences in one launch, source rows q * S + s, cache addresses as in
  * ti_qkv_decode_i8_seqs.  k_dst = NULL: only V^T is written (a prompt without a cache).
+ * Heads of the K cache may lie one after the other or side by side inside a position ([T, heads, D]).
  */
 int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const int8_t* v_src, int64_t v_src_row_stride,
                          int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,

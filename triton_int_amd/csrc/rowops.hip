@@ -767,8 +767,12 @@ int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const in
   if (D & 15) return ti::fail(TI_E_SHAPE, "head dimension %d must be a multiple of 16", D);
   const int64_t H = (int64_t)heads * D;
   if (H > 0x7fffffff) return ti::fail(TI_E_SHAPE, "heads * D too large");
-  if (v_src_row_stride < H || vt_row_stride < S ||
-      (k_dst && (k_src_row_stride < H || k_row_stride < D || k_head_stride < (int64_t)(S - 1) * k_row_stride + D)))
+  // rows of the K cache do not overlap: heads one after the other ([heads, T, D]) or side by side inside a position
+  // ([T, heads, D])
+  const int64_t others = (int64_t)seqs * heads - 1;
+  const bool k_rows_apart = others == 0 || k_head_stride >= (int64_t)(S - 1) * k_row_stride + D ||
+                            (k_head_stride >= D && k_head_stride <= (k_row_stride - D) / others);
+  if (v_src_row_stride < H || vt_row_stride < S || (k_dst && (k_src_row_stride < H || k_row_stride < D || !k_rows_apart)))
     return ti::fail(TI_E_STRIDE, "strides must cover the rows they step over");
   int rc = ti::check_device();
   if (rc != TI_OK) return rc;
