@@ -35,8 +35,12 @@ def _in_layout(values, layout):
     BH, R, C = values.shape
     if layout == "rows_first":  # memory [rows, heads, cols]
         t = torch.zeros((R, BH, C), dtype=torch.int8, device="cuda").transpose(0, 1)
-    else:
-        raise ValueError(layout)
+    elif layout == "cols_first":  # memory [cols, heads, rows]: no unit stride along a row
+        t = torch.zeros((C, BH, R), dtype=torch.int8, device="cuda").permute(1, 2, 0)
+    elif layout == "pitch":  # rows two bytes apart
+        t = torch.zeros((BH, R, C + 2), dtype=torch.int8, device="cuda")[:, :, :C]
+    else:  # contiguous, but from byte `layout` on
+        t = torch.zeros(BH * R * C + layout, dtype=torch.int8, device="cuda")[layout:].view(BH, R, C)
     return t.copy_(values)
 
 
@@ -96,3 +100,19 @@ def test_kv_append_into_a_cache_of_whole_positions(seqs, S, T):
 @pytest.mark.parametrize("S,T", [(1, 53), (20, 53), (20, 80), (200, 400)])
 def test_layer_on_a_k_cache_of_whole_positions(hidden, S, T):
     _check_layer(hidden, S, T, "rows_first", None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden", [256, 1024])
+@pytest.mark.parametrize("k_layout,S,T", [(1, 20, 53), (1, 20, 64), (4, 1, 53), (4, 1, 64), (8, 130, 160), ("pitch", 20, 53), ("cols_first", 1, 53),
+                                          ("cols_first", 20, 64)])
+def test_layer_on_a_k_cache_that_the_attention_kernel_does_not_take(hidden, k_layout, S, T):
+    """Rows of K that do not start at multiples of 16 bytes: the three-launch chain, same bits."""
+    _check_layer(hidden, S, T, k_layout, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vt_layout", [None, 1, "pitch"])
+@pytest.mark.parametrize("S,T", [(1, 53), (1, 64), (20, 53), (130, 144)])
+def test_layer_on_a_vt_cache_at_any_byte(vt_layout, S, T):
+    _check_layer(1024, S, T, None, vt_layout)

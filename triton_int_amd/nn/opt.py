@@ -124,6 +124,13 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         for b in range(B):
             transpose_i8(v_new[b], out=vt_all[b * heads:(b + 1) * heads].view(H, T)[:, T - S:])
 
+    @staticmethod
+    def _kernel_takes(k_all, vt_all):
+        """Whether the attention kernel takes caches that lie like this; the three-launch chain takes any."""
+        ks, vs, T = k_all.stride(), vt_all.stride(), vt_all.shape[2]
+        return (ks[2] == 1 and ks[1] >= k_all.shape[2] and (k_all.data_ptr() | ks[0] | ks[1]) % 16 == 0
+                and (vs[2] == 1 or T == 1) and vs[1] >= T)
+
     @torch.no_grad()
     def forward(self, hidden, kv_cache=None, _trace=None, _mark=None):
         """hidden fp32 [B,S,H].  kv_cache = (K int8 [B*heads, T, D], V^T int8 [B*heads, D, T]) holds the
@@ -153,7 +160,8 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         # short blocks of queries against up to 4096 keys run the attention kernel's one-pass form; a traced
         # forward keeps the three steps of blocks of 17 .. 127 apart so that they can be inspected
         short = T <= 4096 and (S <= 16 or _trace is None)
-        fused = self.fused_attention and (S >= self.fused_attention_min_queries or short) and D == 128 and self.score_scale > 0.0
+        fused = (self.fused_attention and (S >= self.fused_attention_min_queries or short) and D == 128 and self.score_scale > 0.0
+                 and (kv_cache is None or self._kernel_takes(*kv_cache)))
         if kv_cache is None:
             # rows of V^T padded to a multiple of 16 bytes: the attention kernel reads them in 16-byte pieces
             vt_all = torch.empty((B * heads, D, (S + 15) // 16 * 16), dtype=torch.int8, device=hidden.device)[:, :, :S]
