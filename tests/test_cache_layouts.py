@@ -116,3 +116,11 @@ def test_layer_on_a_k_cache_that_the_attention_kernel_does_not_take(hidden, k_la
 @pytest.mark.parametrize("S,T", [(1, 53), (1, 64), (20, 53), (130, 144)])
 def test_layer_on_a_vt_cache_at_any_byte(vt_layout, S, T):
     _check_layer(1024, S, T, None, vt_layout)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k_layout", [1, 2, 4, "pitch", "rows_first"])
+@pytest.mark.parametrize("S,T", [(1, 53), (1, 64), (5, 53)])
+def test_decode_step_on_a_k_cache_that_the_projections_launch_does_not_write(k_layout, S, T):
+    """Rows of K that do not start at multiples of 4 bytes: projections and append as two launches, same bits."""
+    _check_layer(1024, S, T, k_layout, None)

@@ -130,7 +130,8 @@ def linear_qkv_decode_a8_w8_b8_o8(a, w3, bias3, scale_a3, scale_b3, k_cache, vt_
     S = M // seqs
     ks, vs = k_cache.stride(), vt_cache.stride()
     if not (M <= 16 and K >= 1024 and BH * D == seqs * N and D % 16 == 0 and S <= T and vt_cache.shape == (BH, D, T)
-            and ks[2] == 1 and (vs[2] == 1 or T == 1) and (vs[0] == D * vs[1] or BH == 1) and a.stride(1) == 1 and w3.is_contiguous()):
+            and ks[2] == 1 and (vs[2] == 1 or T == 1) and (vs[0] == D * vs[1] or BH == 1) and a.stride(1) == 1 and w3.is_contiguous()
+            and (k_cache.data_ptr() | ks[0] | ks[1]) % 4 == 0):  # the kernel writes K in 4-byte pieces
         return None
     assert a.dtype == w3.dtype == bias3.dtype == k_cache.dtype == vt_cache.dtype == torch.int8
     assert w3.shape == (3 * N, K) and bias3.numel() == 3 * N and seqs * S == M
