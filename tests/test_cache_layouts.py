@@ -124,3 +124,20 @@ def test_layer_on_a_vt_cache_at_any_byte(vt_layout, S, T):
 def test_decode_step_on_a_k_cache_that_the_projections_launch_does_not_write(k_layout, S, T):
     """Rows of K that do not start at multiples of 4 bytes: projections and append as two launches, same bits."""
     _check_layer(1024, S, T, k_layout, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k_layout", [None, "cols_first"])
+@pytest.mark.parametrize("hidden,T", [(256, 53), (1024, 53), (1024, 64)])
+def test_decode_step_on_v_as_it_leaves_the_projection(k_layout, hidden, T):
+    """V kept as [T, heads * 128] and passed as its transposed view: V^T rows without unit stride."""
+    layer, heads = _layer(hidden), hidden // D
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn((1, 1, hidden), device="cuda", generator=g)
+    k0, v = _i8(g, heads, T, D), _i8(g, T, hidden)
+    k, vt = k0.clone(), v.t().contiguous().view(heads, D, T)
+    want = layer(x, kv_cache=(k, vt))
+    k2, vt2 = _in_layout(k0, k_layout), v.t().view(heads, D, T)
+    assert vt2.stride(2) == hidden
+    got = layer(x, kv_cache=(k2, vt2))
+    assert torch.equal(got, want) and torch.equal(k2, k) and torch.equal(vt2, vt)

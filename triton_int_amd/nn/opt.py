@@ -116,7 +116,7 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         B, S, H = v_new.shape
         heads, D, T = self.heads, self.head_dim, vt_all.shape[2]
         vs = vt_all.stride()
-        if D % 16 == 0 and (k_all is None or k_all.stride(2) == 1) and (vs[0] == D * vs[1] or B * heads == 1):
+        if D % 16 == 0 and (k_all is None or k_all.stride(2) == 1) and vs[2] == 1 and (vs[0] == D * vs[1] or B * heads == 1):
             kv_append_i8(k_new.view(B * S, H), v_new.view(B * S, H), k_all, vt_all, seqs=B)
             return
         if k_all is not None:
