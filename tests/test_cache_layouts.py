@@ -141,3 +141,18 @@ def test_decode_step_on_v_as_it_leaves_the_projection(k_layout, hidden, T):
     assert vt2.stride(2) == hidden
     got = layer(x, kv_cache=(k2, vt2))
     assert torch.equal(got, want) and torch.equal(k2, k) and torch.equal(vt2, vt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(1, 16), (1, 5), (2, 2)])
+def test_more_sequences_than_one_launch_takes(S, T):
+    """65600 sequences of one head: the bits of the same sequences in parts."""
+    layer, B = _layer(128), 65600
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn((B, S, 128), device="cuda", generator=g)
+    k0, vt0 = _i8(g, B, T, D), _i8(g, B, D, T)
+    parts = [slice(b, min(b + 30000, B)) for b in range(0, B, 30000)]
+    k, vt, k2, vt2 = k0.clone(), vt0.clone(), k0, vt0
+    want = torch.cat([layer(x[p], kv_cache=(k[p], vt[p])) for p in parts])
+    assert torch.equal(layer(x, kv_cache=(k2, vt2)), want) and torch.equal(k2, k) and torch.equal(vt2, vt)
+    assert torch.equal(layer(x), torch.cat([layer(x[p]) for p in parts]))

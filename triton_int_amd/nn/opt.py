@@ -117,12 +117,22 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         heads, D, T = self.heads, self.head_dim, vt_all.shape[2]
         vs = vt_all.stride()
         if D % 16 == 0 and (k_all is None or k_all.stride(2) == 1) and vs[2] == 1 and (vs[0] == D * vs[1] or B * heads == 1):
-            kv_append_i8(k_new.view(B * S, H), v_new.view(B * S, H), k_all, vt_all, seqs=B)
+            n = self._at_once()
+            if B <= n:
+                kv_append_i8(k_new.view(B * S, H), v_new.view(B * S, H), k_all, vt_all, seqs=B)
+                return
+            for b in range(0, B, n):
+                hs = slice(b * heads, (b + n) * heads)
+                self._append(k_new[b:b + n], v_new[b:b + n], None if k_all is None else k_all[hs], vt_all[hs])
             return
         if k_all is not None:
             k_all[:, T - S:, :] = self._heads(k_new, B, S)
         for b in range(B):
             transpose_i8(v_new[b], out=vt_all[b * heads:(b + 1) * heads].view(H, T)[:, T - S:])
+
+    def _at_once(self):
+        """Sequences of one launch: an attention takes up to 65535 heads, an append up to 32767 sequences."""
+        return max(1, min(32767, 65535 // self.heads))
 
     @staticmethod
     def _kernel_takes(k_all, vt_all):
@@ -179,11 +189,14 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
             if k_all is None:
                 k_all = self._heads(qkv[..., H:2 * H], B, S)
         if fused:
-            # every operand as [B, heads, rows, D] views: all sequences in one launch
+            # every operand as [B, heads, rows, D] views: all sequences in one launch, as far as one launch goes
             by_head = lambda t: t.view(B, S, heads, D).transpose(1, 2)
-            attention_i8(by_head(qkv[..., :H]), by_head(qkv[..., H:2 * H]) if kv_cache is None else k_all.unflatten(0, (B, heads)),
-                         vt_all.unflatten(0, (B, heads)), self.qk_alpha, self.score_scale, self.pv_alpha,
-                         causal_q_len=S if self.causal else 0, out=by_head(ctx))
+            operands = (by_head(qkv[..., :H]), by_head(qkv[..., H:2 * H]) if kv_cache is None else k_all.unflatten(0, (B, heads)),
+                        vt_all.unflatten(0, (B, heads)), by_head(ctx))
+            n = self._at_once()
+            for b in range(0, B, n):
+                q4, k4, vt4, out4 = operands if B <= n else (t[b:b + n] for t in operands)
+                attention_i8(q4, k4, vt4, self.qk_alpha, self.score_scale, self.pv_alpha, causal_q_len=S if self.causal else 0, out=out4)
             mark("attention_i8_fused")
         else:
             scores = bmm_s8t_s8n_s8t(q, k_all, self.qk_alpha)                       # [B*heads, S, T] int8
