@@ -25,3 +25,35 @@ def test_a_flag_that_is_no_bool_counts_as_its_truth_value(rms):
         got, want, other = call(rms), call(bool(rms)), call(not rms)
         assert all(torch.equal(a, b) for a, b in zip(got, want)), name
         assert not torch.equal(want[0], other[0]), f"{name}: the two norms agree, so the test shows nothing"
+
+
+def test_out_of_memory_is_torchs_exception():
+    """An output that does not fit raises torch.OutOfMemoryError, as torch.empty does, from every launcher that allocates."""
+    from triton_int_amd.kernels import bmm, fused, linear
+
+    a, w = (torch.ones(s, dtype=torch.int8, device="cuda") for s in ((1 << 15, 16), (1 << 14, 16)))
+    x, s = torch.ones((1 << 15, 1 << 12), device="cuda"), torch.tensor(1.0, device="cuda")
+    b32, g = torch.zeros(1 << 14, dtype=torch.int32, device="cuda"), torch.ones(1 << 12, device="cuda")
+    calls = {
+        "linear": lambda: linear.linear_a8_w8_b32_o32(a, w, b32),
+        "bmm": lambda: bmm.bmm_s8t_s8n_s32t(a[None], w[None]),
+        "layernorm_q": lambda: fused.layer_norm_fwd_fused_single_pass_q(x, g, None, 1e-5, True),
+        "layernorm": lambda: fused.layer_norm_fwd_fused_single_pass(x, g, None, 1e-5, True),
+        "gelu_q": lambda: fused.gelu_q(x, s),
+        "per_token": lambda: fused.quantize_per_token_absmax(x),
+        "per_tensor": lambda: fused.quantize_per_tensor_absmax(x),
+    }
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (32 << 20)) / total)
+    try:
+        for name, call in calls.items():
+            with pytest.raises(torch.OutOfMemoryError):
+                call()
+                pytest.fail(f"{name}: its output was allocated")
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for name, call in calls.items():
+        call()
+    torch.cuda.synchronize()

@@ -7,8 +7,9 @@
 //
 // Every function returns None, having done nothing, when an argument is anything but the ordinary case (a
 // tensor subclass, another device than the current one, a layout that needs a copy, a python-float scale, a
-// wrong dtype or size, a status from the library).  The Python launcher then takes its own path, which
-// converts or raises: there is one definition of every conversion and every error message.
+// wrong dtype or size, a status from the library, an exception from torch, e.g. out of memory).  The Python
+// launcher then takes its own path, which converts or raises: there is one definition of every conversion and
+// every error, its type included.
 #include <Python.h>
 
 #include <torch/csrc/autograd/python_variable.h>
@@ -153,12 +154,10 @@ PyObject* guarded(Py_ssize_t n, Py_ssize_t want, F f) {
   try {
     return f();
   } catch (const NotOrdinary&) {
-    PyErr_Clear();
-    Py_RETURN_NONE;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {  // nothing is launched yet: the allocations come first
   }
+  PyErr_Clear();
+  Py_RETURN_NONE;
 }
 
 // linear(a, w, bias, alpha, beta, out, epilogue, out_dtype, round_mode, config, groups): kernels/_gemm.py linear and,
