@@ -57,3 +57,43 @@ def test_out_of_memory_is_torchs_exception():
     for name, call in calls.items():
         call()
     torch.cuda.synchronize()
+
+
+def test_launches_from_several_threads():
+    """Eight threads, a stream each, split-K and other kernels: every result is the one of a single thread."""
+    import threading
+
+    from triton_int_amd.kernels import fused, linear
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    i8 = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device="cuda", generator=g)
+    w, b32, gamma = i8(512, 10240), torch.zeros(512, dtype=torch.int32, device="cuda"), torch.ones(10240, device="cuda")
+    xs = [torch.randn((100, 10240), device="cuda", generator=g) for _ in range(8)]
+
+    def once(x):
+        q, scale = fused.quantize_per_token_absmax(x)
+        return linear.linear_a8_w8_b32_o32(q, w, b32), linear.linear_a8_w8_b32_o32(q[:5], w, b32), scale, \
+            fused.layer_norm_fwd_fused_single_pass_q(x, gamma, None, 1e-5, True)
+
+    want = [once(x) for x in xs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for _ in range(20):
+                    got = once(xs[i])
+                    stream.synchronize()
+                    if not all(torch.equal(a, b) for a, b in zip(got, want[i])):
+                        wrong.append(i)
+        except Exception as e:
+            wrong.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

@@ -1,0 +1,25 @@
+"""The extension module's source (csrc/host.cpp): what cannot be seen from a call's result."""
+import os
+import re
+
+SOURCE = os.path.join(os.path.dirname(__file__), "..", "triton_int_amd", "csrc", "host.cpp")
+
+
+def test_every_launch_and_allocation_runs_without_the_interpreters_lock():
+    """A launch may wait for the device (a full queue, a workspace that grows): ctypes releases the lock around a call, and so
+    does every function here.  Python objects are read before."""
+    src = re.sub(r"//.*", "", open(SOURCE).read())
+    bodies = re.split(r"\nPyObject\* (?=\w+\(PyObject\*, PyObject\* const\* v)", src)[1:]
+    assert len(bodies) == len(re.findall(r"TI_METHOD\(\w+\)", src)) - 1  # the macro's own definition
+    for body in bodies:
+        name = body.split("(")[0]
+        parts = body.split("const NoGil unlocked;")
+        assert len(parts) == 2, name
+        depth, end = 1, 0
+        while depth:  # the block that holds the lock's release
+            depth += {"{": 1, "}": -1}.get(parts[1][end], 0)
+            end += 1
+        unlocked, rest = parts[1][:end], parts[0] + parts[1][end:]
+        assert re.search(r"\bti_\w+\(", unlocked), name
+        assert not re.search(r"\bti_\w+\(|c\.empty\(", rest), f"{name}: launches or allocates under the lock"
+        assert not re.search(r"\bPy\w+|THP\w+|\bv\[|\b(integer|number|flag|scale|vector|tensor)\(", unlocked), f"{name}: reads a Python object without the lock"

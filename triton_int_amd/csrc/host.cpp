@@ -10,6 +10,10 @@
 // wrong dtype or size, a status from the library, an exception from torch, e.g. out of memory).  The Python
 // launcher then takes its own path, which converts or raises: there is one definition of every conversion and
 // every error, its type included.
+//
+// The allocations and the C ABI call run without the interpreter's lock (NoGil), as a ctypes call does: a launch can
+// wait (a full hardware queue, a kernel's first launch, a workspace that grows), and other Python threads, host
+// callbacks of the stream among them, go on meanwhile.  So every argument is read before.
 #include <Python.h>
 
 #include <torch/csrc/autograd/python_variable.h>
@@ -23,6 +27,12 @@ namespace {
 
 using at::ScalarType;
 using at::Tensor;
+
+// Releases the interpreter's lock for its lifetime.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
 
 struct NotOrdinary {};  // thrown by the argument readers, turned into None
 
@@ -170,6 +180,7 @@ PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(w.dim() == 2);
     const int64_t groups = integer(v[10]), N = w.size(0), per = groups ? N / groups : N;
     need(!groups || N % groups == 0);
+    const int N32 = int32_size(N), per32 = int32_size(per);
     const Rows r(a, w.size(1));
     int bk = TI_BIAS_NONE;
     const void* bias = nullptr;
@@ -180,28 +191,31 @@ PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
       bias = ptr(b);
     }
     const float *alpha = scale(v[3], c.dev), *beta = scale(v[4], c.dev);
-    const int dt = (int)integer(v[7]);
+    const int epilogue = (int)integer(v[6]), dt = (int)integer(v[7]), round_mode = (int)integer(v[8]), config = (int)integer(v[9]);
     const ScalarType type = out_type(dt);
     const auto sizes = with_last(a, N);
     Tensor out;
-    if (v[5] == Py_None) {
-      out = c.empty(sizes, type);
-    } else {
+    if (v[5] != Py_None) {
       const Tensor& o = tensor(v[5], c.dev, type);
       need(o.numel() == (int64_t)r.M * N && o.is_contiguous());
       out = o.view(sizes);
     }
-    int rc;
     if (groups) {
       for (int i = 3; i < 5; ++i)
         if (v[i] != Py_None) need(THPVariable_Unpack(v[i]).numel() == groups && THPVariable_Unpack(v[i]).is_contiguous());
-      rc = ti_bmm_i8_grouped((const int8_t*)ptr(a), 0, r.pitch, 1, (const int8_t*)ptr(w), per * w.stride(0), w.stride(0), w.stride(1),
-                             mptr(out), per, N, 1, (int)groups, r.M, int32_size(per), r.K, bias, bk, per, alpha, beta, 1,
-                             (int)integer(v[6]), dt, (int)integer(v[8]), (int)integer(v[9]), c.stream);
-    } else {
-      rc = ti_bmm_i8_config((const int8_t*)ptr(a), 0, r.pitch, 1, (const int8_t*)ptr(w), 0, w.stride(0), w.stride(1), mptr(out), 0, N, 1, 1,
-                            r.M, int32_size(N), r.K, bias, bk, alpha, beta, (int)integer(v[6]), dt, (int)integer(v[8]),
-                            (int)integer(v[9]), c.stream);
+    }
+    int rc;
+    {
+      const NoGil unlocked;
+      if (!out.defined()) out = c.empty(sizes, type);
+      if (groups) {
+        rc = ti_bmm_i8_grouped((const int8_t*)ptr(a), 0, r.pitch, 1, (const int8_t*)ptr(w), per * w.stride(0), w.stride(0), w.stride(1),
+                               mptr(out), per, N, 1, (int)groups, r.M, per32, r.K, bias, bk, per, alpha, beta, 1, epilogue, dt, round_mode,
+                               config, c.stream);
+      } else {
+        rc = ti_bmm_i8_config((const int8_t*)ptr(a), 0, r.pitch, 1, (const int8_t*)ptr(w), 0, w.stride(0), w.stride(1), mptr(out), 0, N, 1, 1,
+                              r.M, N32, r.K, bias, bk, alpha, beta, epilogue, dt, round_mode, config, c.stream);
+      }
     }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
@@ -218,18 +232,23 @@ PyObject* bmm(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const bool kn = flag(v[2]);  // b is [B, K, N]
     need(a.size(2) == b.size(kn ? 1 : 2));
     const int64_t B = a.size(0), M = a.size(1), K = a.size(2), N = b.size(kn ? 2 : 1);
-    const int dt = (int)integer(v[6]);
+    const int B32 = int32_size(B), M32 = int32_size(M), N32 = int32_size(N), K32 = int32_size(K);
+    const int epilogue = (int)integer(v[5]), dt = (int)integer(v[6]), round_mode = (int)integer(v[7]), config = (int)integer(v[8]);
+    const float* alpha = scale(v[3], c.dev);
+    const ScalarType type = out_type(dt);
     Tensor out;
-    if (v[4] == Py_None) {
-      out = c.empty({B, M, N}, out_type(dt));
-    } else {
-      out = tensor(v[4], c.dev, out_type(dt));
+    if (v[4] != Py_None) {
+      out = tensor(v[4], c.dev, type);
       need(out.dim() == 3 && out.size(0) == B && out.size(1) == M && out.size(2) == N);
     }
-    const int rc = ti_bmm_i8_config((const int8_t*)ptr(a), a.stride(0), a.stride(1), a.stride(2), (const int8_t*)ptr(b), b.stride(0),
-                                    b.stride(kn ? 2 : 1), b.stride(kn ? 1 : 2), mptr(out), out.stride(0), out.stride(1), out.stride(2),
-                                    int32_size(B), int32_size(M), int32_size(N), int32_size(K), nullptr, TI_BIAS_NONE,
-                                    scale(v[3], c.dev), nullptr, (int)integer(v[5]), dt, (int)integer(v[7]), (int)integer(v[8]), c.stream);
+    int rc;
+    {
+      const NoGil unlocked;
+      if (!out.defined()) out = c.empty({B, M, N}, type);
+      rc = ti_bmm_i8_config((const int8_t*)ptr(a), a.stride(0), a.stride(1), a.stride(2), (const int8_t*)ptr(b), b.stride(0),
+                            b.stride(kn ? 2 : 1), b.stride(kn ? 1 : 2), mptr(out), out.stride(0), out.stride(1), out.stride(2), B32, M32, N32, K32,
+                            nullptr, TI_BIAS_NONE, alpha, nullptr, epilogue, dt, round_mode, config, c.stream);
+    }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -248,9 +267,15 @@ PyObject* linear_residual(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(alpha && beta);
     const float* res = (const float*)vector(v[5], c.dev, ScalarType::Float, (int64_t)r.M * N);
     need(res);
-    Tensor out = c.empty(with_last(a, N), ScalarType::Float);
-    const int rc = ti_linear_i8_residual_f32((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), w.stride(0), bias, alpha, beta, res, N,
-                                             (float*)mptr(out), N, r.M, int32_size(N), r.K, c.stream);
+    const int N32 = int32_size(N);
+    Tensor out;
+    int rc;
+    {
+      const NoGil unlocked;
+      out = c.empty(with_last(a, N), ScalarType::Float);
+      rc = ti_linear_i8_residual_f32((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), w.stride(0), bias, alpha, beta, res, N,
+                                     (float*)mptr(out), N, r.M, N32, r.K, c.stream);
+    }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -265,9 +290,16 @@ PyObject* layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int64_t N = x.size(-1);
     const float *g = (const float*)vector(v[1], c.dev, ScalarType::Float, N), *b = (const float*)vector(v[2], c.dev, ScalarType::Float, N);
     need(g);
-    Tensor out = c.empty(x.sizes(), ScalarType::Char);
-    const int rc = ti_layernorm_q((const float*)ptr(x), N, g, b, (float)number(v[3]), (int8_t*)mptr(out), N, int32_size(x.numel() / N),
-                                  int32_size(N), flag(v[4]), (int)integer(v[5]), nullptr, nullptr, c.stream);
+    const int rows = int32_size(x.numel() / N), cols = int32_size(N), round_mode = (int)integer(v[5]);
+    const float eps = (float)number(v[3]);
+    const bool rms = flag(v[4]);
+    Tensor out;
+    int rc;
+    {
+      const NoGil unlocked;
+      out = c.empty(x.sizes(), ScalarType::Char);
+      rc = ti_layernorm_q((const float*)ptr(x), N, g, b, eps, (int8_t*)mptr(out), N, rows, cols, rms, round_mode, nullptr, nullptr, c.stream);
+    }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -283,11 +315,17 @@ PyObject* dq_add_layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int64_t H = acc.size(-1);
     const float *g = (const float*)vector(v[3], c.dev, ScalarType::Float, H), *b = (const float*)vector(v[4], c.dev, ScalarType::Float, H);
     need(g);
-    const float s = (float)number(v[1]);
-    Tensor rout = c.empty(acc.sizes(), ScalarType::Float), y = c.empty(acc.sizes(), ScalarType::Char);
-    const int rc = ti_dq_add_layernorm_q((const int32_t*)ptr(acc), H, s, nullptr, (const float*)ptr(res), H, g, b, (float)number(v[5]),
-                                         (float*)mptr(rout), H, (int8_t*)mptr(y), H, nullptr, H, int32_size(acc.numel() / H), int32_size(H),
-                                         (int)integer(v[6]), nullptr, nullptr, c.stream);
+    const int rows = int32_size(acc.numel() / H), cols = int32_size(H), round_mode = (int)integer(v[6]);
+    const float s = (float)number(v[1]), eps = (float)number(v[5]);
+    Tensor rout, y;
+    int rc;
+    {
+      const NoGil unlocked;
+      rout = c.empty(acc.sizes(), ScalarType::Float);
+      y = c.empty(acc.sizes(), ScalarType::Char);
+      rc = ti_dq_add_layernorm_q((const int32_t*)ptr(acc), H, s, nullptr, (const float*)ptr(res), H, g, b, eps, (float*)mptr(rout), H,
+                                 (int8_t*)mptr(y), H, nullptr, H, rows, cols, round_mode, nullptr, nullptr, c.stream);
+    }
     need(rc == TI_OK);
     PyObject* pair = PyTuple_New(2);
     PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(rout));
@@ -312,12 +350,18 @@ PyObject* layernorm_fp(PyObject*, PyObject* const* v, Py_ssize_t n) {
       need(s.is_contiguous() && s.numel() == x.numel() && s.size(-1) == N);
       skip = ptr(s);
     }
+    const int rows = int32_size(x.numel() / N), cols = int32_size(N);
+    const float eps = (float)number(v[4]);
+    const bool rms = flag(v[5]), want_out = flag(v[6]), want_skip_out = flag(v[7]);
     Tensor out, sout;
-    if (flag(v[6])) out = c.empty(x.sizes(), type);
-    if (flag(v[7])) sout = c.empty(x.sizes(), type);
-    const int rc = ti_layernorm_fp(ptr(x), N, skip, skip ? N : 0, dt, g, b, (float)number(v[4]), flag(v[5]),
-                                   out.defined() ? mptr(out) : nullptr, N, sout.defined() ? mptr(sout) : nullptr, N,
-                                   int32_size(x.numel() / N), int32_size(N), c.stream);
+    int rc;
+    {
+      const NoGil unlocked;
+      if (want_out) out = c.empty(x.sizes(), type);
+      if (want_skip_out) sout = c.empty(x.sizes(), type);
+      rc = ti_layernorm_fp(ptr(x), N, skip, skip ? N : 0, dt, g, b, eps, rms, want_out ? mptr(out) : nullptr, N,
+                           want_skip_out ? mptr(sout) : nullptr, N, rows, cols, c.stream);
+    }
     need(rc == TI_OK);
     PyObject* pair = PyTuple_New(2);
     const Tensor* both[2] = {&out, &sout};
@@ -337,8 +381,15 @@ PyObject* gelu_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(x.is_contiguous());
     const float* s = scale(v[1], c.dev);
     need(s);
-    Tensor out = c.empty(x.sizes(), ScalarType::Char);
-    need(ti_gelu_q((const float*)ptr(x), s, (int8_t*)mptr(out), x.numel(), (int)integer(v[2]), c.stream) == TI_OK);
+    const int round_mode = (int)integer(v[2]);
+    Tensor out;
+    int rc;
+    {
+      const NoGil unlocked;
+      out = c.empty(x.sizes(), ScalarType::Char);
+      rc = ti_gelu_q((const float*)ptr(x), s, (int8_t*)mptr(out), x.numel(), round_mode, c.stream);
+    }
+    need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
 }
@@ -350,9 +401,15 @@ PyObject* softmax_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Call c(x);
     need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
     const int64_t cols = x.size(-1);
-    Tensor out = c.empty(x.sizes(), ScalarType::Char);
-    const int rc = ti_softmax_q((const int8_t*)ptr(x), cols, (float)number(v[1]), (int8_t*)mptr(out), cols, int32_size(x.numel() / cols),
-                                int32_size(cols), (int)integer(v[2]), c.stream);
+    const int rows = int32_size(x.numel() / cols), cols32 = int32_size(cols), causal = (int)integer(v[2]);
+    const float s = (float)number(v[1]);
+    Tensor out;
+    int rc;
+    {
+      const NoGil unlocked;
+      out = c.empty(x.sizes(), ScalarType::Char);
+      rc = ti_softmax_q((const int8_t*)ptr(x), cols, s, (int8_t*)mptr(out), cols, rows, cols32, causal, c.stream);
+    }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -366,9 +423,15 @@ PyObject* quantize_per_token(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(x.scalar_type() == ScalarType::Float || x.scalar_type() == ScalarType::Half);
     need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
     const int64_t cols = x.size(-1);
-    Tensor q = c.empty(x.sizes(), ScalarType::Char), s = c.empty(with_last(x, 1), x.scalar_type());
-    const int rc = ti_quantize_per_token_absmax(ptr(x), dtype_code(x.scalar_type()), cols, (int8_t*)mptr(q), cols, mptr(s),
-                                                int32_size(x.numel() / cols), int32_size(cols), c.stream);
+    const int rows = int32_size(x.numel() / cols), cols32 = int32_size(cols);
+    Tensor q, s;
+    int rc;
+    {
+      const NoGil unlocked;
+      q = c.empty(x.sizes(), ScalarType::Char);
+      s = c.empty(with_last(x, 1), x.scalar_type());
+      rc = ti_quantize_per_token_absmax(ptr(x), dtype_code(x.scalar_type()), cols, (int8_t*)mptr(q), cols, mptr(s), rows, cols32, c.stream);
+    }
     need(rc == TI_OK);
     PyObject* pair = PyTuple_New(2);
     PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(q));
@@ -385,10 +448,17 @@ PyObject* quantize_per_tensor(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(x.scalar_type() == ScalarType::Float || x.scalar_type() == ScalarType::Half);
     need(x.is_contiguous() && x.numel() > 0);
     const float* ws = scale(v[1], c.dev);
-    Tensor q = c.empty(x.sizes(), ScalarType::Char), s = c.empty({}, x.scalar_type()), al = c.empty({}, ScalarType::Float);
-    Tensor work = c.empty({TI_QUANT_TENSOR_WORKSPACE}, ScalarType::Byte);
-    const int rc = ti_quantize_per_tensor_absmax(ptr(x), dtype_code(x.scalar_type()), x.numel(), (int8_t*)mptr(q), mptr(s), ws,
-                                                 (float*)mptr(al), mptr(work), c.stream);
+    Tensor q, s, al, work;
+    int rc;
+    {
+      const NoGil unlocked;
+      q = c.empty(x.sizes(), ScalarType::Char);
+      s = c.empty({}, x.scalar_type());
+      al = c.empty({}, ScalarType::Float);
+      work = c.empty({TI_QUANT_TENSOR_WORKSPACE}, ScalarType::Byte);
+      rc = ti_quantize_per_tensor_absmax(ptr(x), dtype_code(x.scalar_type()), x.numel(), (int8_t*)mptr(q), mptr(s), ws, (float*)mptr(al),
+                                         mptr(work), c.stream);
+    }
     need(rc == TI_OK);
     PyObject* triple = PyTuple_New(3);
     PyTuple_SET_ITEM(triple, 0, THPVariable_Wrap(q));
@@ -424,18 +494,22 @@ PyObject* attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int64_t S = q.size(-2), D = q.size(-1), T = k.size(-2);
     need(k.dim() == q.dim() && vt.dim() == q.dim() && hk.seqs == hq.seqs && hv.seqs == hq.seqs && hk.heads == hq.heads && hv.heads == hq.heads);
     need(k.size(-1) == D && vt.size(-2) == D && vt.size(-1) == T);
+    const int S32 = int32_size(S), T32 = int32_size(T), D32 = int32_size(D), causal = (int)integer(v[6]);
+    const float qk_alpha = (float)number(v[3]), score_scale = (float)number(v[4]), pv_alpha = (float)number(v[5]);
     Tensor out;
-    if (v[7] == Py_None) {
-      out = c.empty(q.sizes(), ScalarType::Char);
-    } else {
+    if (v[7] != Py_None) {
       out = tensor(v[7], c.dev, ScalarType::Char);
       need(out.sizes() == q.sizes());
     }
-    const Heads ho(out);
-    const int rc = ti_attention_i8_heads((const int8_t*)ptr(q), hq.ss, hq.hs, hq.rs, (const int8_t*)ptr(k), hk.ss, hk.hs, hk.rs,
-                                         (const int8_t*)ptr(vt), hv.ss, hv.hs, hv.rs, (int8_t*)mptr(out), ho.ss, ho.hs, ho.rs, hq.seqs,
-                                         hq.heads, int32_size(S), int32_size(T), int32_size(D), (float)number(v[3]), (float)number(v[4]),
-                                         (float)number(v[5]), (int)integer(v[6]), c.stream);
+    int rc;
+    {
+      const NoGil unlocked;
+      if (!out.defined()) out = c.empty(q.sizes(), ScalarType::Char);
+      const Heads ho(out);
+      rc = ti_attention_i8_heads((const int8_t*)ptr(q), hq.ss, hq.hs, hq.rs, (const int8_t*)ptr(k), hk.ss, hk.hs, hk.rs, (const int8_t*)ptr(vt),
+                                 hv.ss, hv.hs, hv.rs, (int8_t*)mptr(out), ho.ss, ho.hs, ho.rs, hq.seqs, hq.heads, S32, T32, D32, qk_alpha,
+                                 score_scale, pv_alpha, causal, c.stream);
+    }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -476,9 +550,15 @@ PyObject* qkv_decode(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int8_t* bias = (const int8_t*)vector(v[2], c.dev, ScalarType::Char, 3 * N);
     const float *al = (const float*)vector(v[3], c.dev, ScalarType::Float, 3), *be = (const float*)vector(v[4], c.dev, ScalarType::Float, 3);
     need(bias && al && be);
-    Tensor out = c.empty({r.M, 3 * N}, ScalarType::Char);
-    const int rc = ti_qkv_decode_i8_seqs((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), r.K, bias, al, be, (int8_t*)mptr(out), 3 * N,
-                                         (int)seqs, r.M, int32_size(N), r.K, kv.k, kv.k_hs, kv.k_rs, kv.vt, kv.vt_rs, (int)kv.D, c.stream);
+    const int N32 = int32_size(N);
+    Tensor out;
+    int rc;
+    {
+      const NoGil unlocked;
+      out = c.empty({r.M, 3 * N}, ScalarType::Char);
+      rc = ti_qkv_decode_i8_seqs((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), r.K, bias, al, be, (int8_t*)mptr(out), 3 * N, (int)seqs,
+                                 r.M, N32, r.K, kv.k, kv.k_hs, kv.k_rs, kv.vt, kv.vt_rs, (int)kv.D, c.stream);
+    }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
   });
@@ -502,8 +582,13 @@ PyObject* kv_append(PyObject*, PyObject* const* v, Py_ssize_t n) {
       ksrc = (const int8_t*)ptr(kn);
       k_rs = kn.stride(0);
     }
-    const int rc = ti_kv_append_i8_seqs(ksrc, k_rs, (const int8_t*)ptr(vn), vn.stride(0), kv.k, kv.k_hs, kv.k_rs, kv.vt, kv.vt_rs, (int)seqs,
-                                        int32_size(S), (int)(kv.BH / seqs), (int)kv.D, c.stream);
+    const int S32 = int32_size(S);
+    int rc;
+    {
+      const NoGil unlocked;
+      rc = ti_kv_append_i8_seqs(ksrc, k_rs, (const int8_t*)ptr(vn), vn.stride(0), kv.k, kv.k_hs, kv.k_rs, kv.vt, kv.vt_rs, (int)seqs, S32,
+                                (int)(kv.BH / seqs), (int)kv.D, c.stream);
+    }
     need(rc == TI_OK);
     Py_RETURN_TRUE;
   });
