@@ -373,7 +373,7 @@ int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const in
  * The scalars are host floats.  The int8 scores are the BMM's and the probabilities ti_softmax_q's
  * bit for bit (a row's exponentials are summed as integers, so the order in which the keys are
  * visited does not matter): the output equals the three-launch chain's exactly.
- * Launches of few query rows (batch * ceil(S / 16) <= 1024) against T <= 4096 keys run a one-pass kernel,
+ * Launches of few query rows (S <= 16, or batch * ceil(S / 16) <= 1024) against T <= 4096 keys run a one-pass kernel,
  * one to eight workgroups per batch entry and 16 rows.
  * The reference has no fused form (its modules stop at the BMMs, nn/bmm.py:10-74); the
  * three-launch chain remains available and is what this is tested against.
@@ -396,6 +396,12 @@ int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int64_t q_head_
                           int8_t* out, int64_t out_seq_stride, int64_t out_head_stride, int64_t out_row_stride,
                           int seqs, int heads, int S, int T, int D,
                           float qk_alpha, float score_scale, float pv_alpha, int causal_q_len, void* stream);
+
+/*
+ * Query rows of a workgroup that such a launch runs on: 16 (one pass over the keys) or 128 (blocks), for
+ * `heads` (sequence, head) pairs.  Touches no device; lets a test or a benchmark attribute time to the kernel.
+ */
+int ti_attention_i8_rows(int64_t heads, int S, int T, int64_t q_row_stride, int64_t k_row_stride, int64_t vt_row_stride);
 
 /*
  * Dynamic per-token activation quantisation, dynamic_quantize_activation_per_token_absmax

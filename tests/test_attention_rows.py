@@ -1,0 +1,32 @@
+"""Which attention kernel a launch runs on, and that the choice changes no bit."""
+import pytest
+import torch
+
+
+def test_up_to_16_query_rows_run_on_the_one_pass_kernel_at_any_batch():
+    """A 128-row block with 16 live rows walks the keys three times on a quarter of the waves: 27 sequences of 40 heads that
+    decode one token each are more than 1024 groups and still belong on the one-pass kernel."""
+    from triton_int_amd import _lib as L
+
+    rows = lambda heads, S, T: L.lib().ti_attention_i8_rows(heads, S, T, 128, 128, T)
+    for heads in (1, 1024, 1025, 1080, 5120, 65535):
+        for S in (1, 2, 15, 16):
+            assert rows(heads, S, 1) == rows(heads, S, 2048) == rows(heads, S, 4096) == 16, (heads, S)
+            assert rows(heads, S, 4097) == 128  # the scores of a row no longer fit the registers
+    assert rows(64, 256, 1064) == 16 and rows(65, 256, 1064) == 128 and rows(1280, 17, 2048) == 128
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [1, 16, 17])
+@pytest.mark.parametrize("heads,T", [(1024, 33), (1025, 33), (1030, 80), (2600, 17)])
+def test_more_heads_than_four_rounds_of_the_chip(heads, S, T):
+    """All heads in one launch against the same heads in launches of 500, bit for bit."""
+    from triton_int_amd.kernels.fused import attention_i8
+
+    g = torch.Generator(device="cuda").manual_seed(heads + S)
+    i8 = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device="cuda", generator=g)
+    q, k, vt = i8(heads, S, 128), i8(heads, T, 128), i8(heads, 128, T)
+    causal = S if S <= T else 0
+    call = lambda p: attention_i8(q[p], k[p], vt[p], 1e-3, 0.1, 0.05, causal_q_len=causal)
+    got = call(slice(None))
+    assert torch.equal(got, torch.cat([call(slice(i, i + 500)) for i in range(0, heads, 500)])) and got.any()

@@ -555,7 +555,27 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   }
 }
 
+// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them, or as long as they are at most
+// four rounds of the chip (256 workgroups each); 128-row blocks on attention_i8_kernel beyond.  A group walks the keys
+// once on 16 waves; a block walks them three times on 4 waves, 2.1 us per 64 keys however few blocks there are and
+// however few of its rows are live.
+// Measured, causal (us, groups / blocks): 32 heads x 64 rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 /
+// 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81, 64 x 256 x 1064 (1024) 48 / 46,
+// 160 x 96 x 2048 (960) 83 / 81, 40 x 512 x 2048 (1280) 88 / 81, 160 x 128 x 2048 (1280) 103 / 82, 320 x 64 x 2048
+// (1280) 145 / 113, 1280 x 17 x 2048 (2560) 298 / 269, 1280 x 32 x 1024 (2560) 133 / 137.
+// 16 rows and fewer, as many workgroups either way: 1280 x 1 x 2048 156 / 265, 2560 x 16 x 2048 297 / 464, 1056 x 1 x
+// 333 24.8 / 57.8, 20000 x 1 x 304 346 / 707 (20000 x 1 x 64 265 / 242).
+static bool attn_few_rows(int64_t heads, int S, int T, int64_t q_row_stride, int64_t k_row_stride, int64_t vt_row_stride) {
+  const int64_t lim32 = (int64_t)1 << 31;  // descriptor extents and offsets
+  return (S <= 16 || heads * ((S + 15) / 16) <= 1024) && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 &&
+         (int64_t)AT_D * vt_row_stride < lim32 && (int64_t)S * q_row_stride < lim32;
+}
+
 }  // namespace ti
+
+extern "C" int ti_attention_i8_rows(int64_t heads, int S, int T, int64_t q_row_stride, int64_t k_row_stride, int64_t vt_row_stride) {
+  return ti::attn_few_rows(heads, S, T, q_row_stride, k_row_stride, vt_row_stride) ? 16 : ti::AT_ROWS;
+}
 
 extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int64_t q_head_stride, int64_t q_row_stride,
                                      const int8_t* k, int64_t k_seq_stride, int64_t k_head_stride, int64_t k_row_stride,
@@ -582,16 +602,8 @@ extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int6
   const float s2 = score_scale * 1.44269504088896340736f;
   if (!(score_scale > 0.0f) || !(score_scale <= SM_MAX_SCALE))
     return fail(TI_E_COMBO, "score_scale %g outside (0, %g]: the quantised softmax is exact in that range only", (double)score_scale, (double)SM_MAX_SCALE);
-  const int64_t lim32 = (int64_t)1 << 31;
-  // Groups of 16 query rows on attention_decode_i8_kernel as long as they are at most four rounds of the chip
-  // (256 workgroups each), 128-row blocks on attention_i8_kernel beyond.  A group walks the keys once on 16
-  // waves; a block walks them three times on 4 waves, 2.1 us per 64 keys however few blocks there are.
-  // Measured, causal (us, groups / blocks): 32 heads x 64 rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 /
-  // 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81, 64 x 256 x 1064 (1024) 48 / 46,
-  // 160 x 96 x 2048 (960) 83 / 81, 40 x 512 x 2048 (1280) 88 / 81, 160 x 128 x 2048 (1280) 103 / 82.
   const int64_t groups = (int64_t)seqs * heads * ((S + 15) / 16);
-  const bool few_rows = groups <= 1024 && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 && (int64_t)AT_D * vt_row_stride < lim32 &&
-                        (int64_t)S * q_row_stride < lim32;
+  const bool few_rows = attn_few_rows((int64_t)seqs * heads, S, T, q_row_stride, k_row_stride, vt_row_stride);
   int rc = check_device();
   if (rc != TI_OK) return rc;
   const int batch = seqs * heads;
