@@ -176,3 +176,15 @@ def test_split_k_of_the_ragged_kernel_covers_k_once(lib, M, N, K):
             for epi, dt in ((EPI_SCALE_I8, I8), (EPI_SCALE_F, F32)):
                 pr = G.contiguous(1, M, N, K, dt)
                 G.check_launch(pr, G.plan_for(lib, pr, epi, B_NONE, cfg, static))
+
+
+@pytest.mark.parametrize("M,N,K,kn", [(1, 1, (1 << 31) - 50, False), (1, 1, (1 << 31) - 64, True), (1, (1 << 31) - 100, 1, True), (1, (1 << 31) - 100, 1, False),
+                                      ((1 << 31) - 100, 1, 1, False)])
+def test_sizes_at_the_end_of_32_bits_stay_off_the_ragged_kernel(lib, M, N, K, kn):
+    """Its last tile would end past 2^31 - 1: a number of k-tiles, a row or a column that wraps to a negative one."""
+    def name(M, N, K):
+        pr = G.Problem(1, M, N, K, 0, K, 0, 1 if kn else K, 0, N, I32, sBk=N if kn else 1)
+        return G.plan_for(lib, pr, EPI_I32, B_NONE).name
+
+    assert name(M, N, K).startswith("gather")
+    assert name(*(min(v, (1 << 31) - 259) for v in (M, N, K))).startswith("ragged")  # odd: off the aligned kernels

@@ -2746,8 +2746,11 @@ static bool fast_eligible(const GemmParams& p) {
   return true;
 }
 
-// gemm_ragged_kernel: A K-contiguous, B K- or N-contiguous, rows that do not overlap
+// gemm_ragged_kernel: A K-contiguous, B K- or N-contiguous, rows that do not overlap, sizes whose last tile still ends
+// inside 32 bits
 static bool ragged_eligible(const GemmParams& p) {
+  const int most = 0x7fffffff - 256;
+  if (p.M > most || p.N > most || p.K > most) return false;
   if (p.K <= 0 || p.sAk != 1 || (p.M > 1 && p.sAm < p.K)) return false;
   if (out_class(p.out_dtype) == OUT8 && p.sCn != 1) return false;
   if (p.sBk == 1) return p.N == 1 || p.sBn >= p.K;
