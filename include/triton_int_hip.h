@@ -208,7 +208,8 @@ int ti_gemm_last_splits(void);
  * values matter only for their alignment), and writes what would be launched to plan[0..TI_PLAN_INTS):
  *   [0] configuration index  [1] K splits  [2] k-tiles per split  [3] row tiles  [4] column tiles
  *   [5] row tiles per group of the tile order  [6] grid x  [7] grid y  [8] threads per workgroup
- *   [9] waves that split K inside a workgroup (skinny / rows4 kernels)  [10] streaming waves (rows4)
+ *   [9] waves that split K inside a workgroup (skinny / rows4 kernels); weight rows per workgroup / 16, rounded
+ *       up (row-piece kernel)  [10] streaming waves (rows4); bytes of K per stage (row-piece kernel)
  *   [11] bytes of split-K partial sums the launch needs
  * Runs without a GPU.  The autotuner of the reference (kernels/utils.py:6-558) answers the same
  * question -- which tile for which (M, N, K) -- by timing; this reports the static choice.  Used by the

@@ -112,6 +112,53 @@ def plan_for(lib, pr: Problem, epilogue: int, bias_kind: int, config: int = -1, 
     return p
 
 
+def _check_rowpieces_ring(pr: Problem, MT, KC, G, per, workgroups):
+    """The LDS ring of gemm_rowpieces_kernel: stages of packed 1 KB pieces, what producers and consumers touch of it, and
+    that every 16-byte chunk of K is staged once and lies where the consumers read it."""
+    LDS, PW, NST = 160 * 1024, 4, 32
+    assert KC in (256, 512, 1024) and 4 * (G - 1) < per <= 4 * G
+    CH, RPI = KC // 16, 1024 // KC  # chunks of a row in a stage, rows of a piece
+    assert MT % (RPI * PW) == 0 and per * 4 % RPI == 0
+    pieces_a = -(-pr.M // 4) * 4 // RPI if MT == 16 else MT // RPI
+    pieces_w = per * 4 // RPI
+    assert pieces_a * RPI >= pr.M, "activation rows without a piece"
+    stage = (pieces_a + pieces_w) * 1024
+    most = -(-(pieces_a + pieces_w) // PW)
+    depth = min((LDS - (MT + 16 * G) * KC) // stage, 63 // most, NST - 1)
+    assert depth >= 1 and depth * most <= 63, "loads in flight do not fit the counter"
+    # the last stage: what is staged, and what the operand reads take (whole groups of 16 rows)
+    last = depth * stage
+    assert last + stage <= LDS and last + MT * KC <= LDS and last + pieces_a * 1024 + 16 * G * KC <= LDS, "a stage reaches past the LDS"
+    # a producer wave's pieces: within the instantiated counts, every piece of a stage exactly once
+    a_max, w_min, w_max = MT // RPI // PW, (16 * G - 12) // RPI // PW, 16 * G // RPI // PW
+    a_min = a_max // 4 if MT == 16 else a_max
+    got_a, got_w = [], []
+    for pw in range(PW):
+        mine_a = (pieces_a - pw + PW - 1) // PW
+        first_w = pw + mine_a * PW - pieces_a
+        mine_w = (pieces_w - first_w + PW - 1) // PW
+        assert a_min <= mine_a <= a_max and w_min <= mine_w <= w_max, "no producer instantiated for these counts"
+        assert mine_a + mine_w <= most
+        got_a += [pw + i * PW for i in range(mine_a)]
+        got_w += [first_w + i * PW for i in range(mine_w)]
+    assert sorted(got_a) == list(range(pieces_a)) and sorted(got_w) == list(range(pieces_w)), "pieces not staged exactly once"
+    # K: lane l of a piece's load stages, in stage i, chunk (l & 15) ^ (row & 15) of block (l % CH) / 16 + i * KC / 256 counted
+    # from the workgroup's rotation; the consumers take chunk j of a stage from slot j ^ (row & 15)
+    blocks = -(-pr.K // 256)
+    KT = -(-pr.K // KC)
+    lane = np.arange(64, dtype=np.int64)
+    local = (lane % CH // 16)[:, None] + np.arange(KT, dtype=np.int64)[None, :] * (KC // 256)  # [lane, stage]
+    for lin in {0, 1, 7, 8, workgroups - 1}:
+        rot = ((lin >> 3) + (lin & 7) * (blocks * 256 >> 11)) % blocks
+        block = np.where(local < blocks, (local + rot) % blocks, -1)
+        for row in {0, 5, 15}:
+            mine = lane[lane // CH == row % RPI]
+            staged = (block[mine] * 16 + ((mine & 15) ^ (row & 15))[:, None])[block[mine] >= 0]
+            assert np.array_equal(np.sort(staged), np.arange(blocks * 16)), "a chunk of K is not staged exactly once"
+            slot = np.arange(CH) ^ (row & 15)
+            assert np.array_equal(slot // 16, np.arange(CH) // 16) and np.array_equal((slot & 15) ^ (row & 15), np.arange(CH) & 15)
+
+
 # ---- tile order ---------------------------------------------------------------------------------
 
 def tile_from_rank(pl: Plan, lid):
@@ -419,8 +466,9 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
         stats["units"] = NU
         return stats
     if name.endswith("_rowpieces"):
-        # every workgroup of a batch entry: `per` units of 4 weight rows, the whole K in blocks of 256 bytes
-        MT, KC = int(re.search(r"_m(\d+)", name).group(1)), 256
+        # every workgroup of a batch entry: `per` units of 4 weight rows, the whole K in blocks of 256 bytes, KC of them
+        # per stage
+        MT, KC, BLK = int(re.search(r"_m(\d+)", name).group(1)), pl.nwa, 256
         NU = -(-pr.N // 4)
         per = -(-NU // pl.grid_x)
         u0 = np.minimum(NU, np.arange(pl.grid_x, dtype=np.int64) * per)
@@ -428,7 +476,7 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
         assert pr.M <= MT and pl.grid_y == pr.batch and pl.threads == 512
         assert (units > 0).all() and units.sum() == NU and per <= 20, "the workgroups' units do not cover N exactly once"
         chunk = np.arange(16, dtype=np.int64)
-        kmax = ((pr.K - chunk * 16 - 1) // KC) * KC  # the last stage in which a chunk is still inside K (negative: never)
+        kmax = ((pr.K - chunk * 16 - 1) // BLK) * BLK  # the last block in which a chunk is still inside K (negative: never)
         W = 16 * (-(-per // 4))
         n0 = u0 * 4
         w_rows = np.minimum(units * 4, pr.N - n0)
@@ -442,6 +490,7 @@ def check_launch(pr: Problem, pl: Plan, store_sample: int | None = 64, seed: int
             live = (voff[None] + 16 <= extent[:, None, None]) & (kmax >= 0)[None, None, :]
             bad = live & (base[:, None, None] + voff[None] + kmax[None, None, :] + 16 > alloc)
             assert not bad.any(), f"rowpieces {what}: load outside the operand"
+        _check_rowpieces_ring(pr, MT, KC, pl.ksplit, per, pl.grid_x * pl.grid_y)
         stats["units"] = NU
         return stats
     if name.startswith("skinny"):

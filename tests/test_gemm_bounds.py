@@ -188,3 +188,28 @@ def test_sizes_at_the_end_of_32_bits_stay_off_the_ragged_kernel(lib, M, N, K, kn
 
     assert name(M, N, K).startswith("gather")
     assert name(*(min(v, (1 << 31) - 259) for v in (M, N, K))).startswith("ragged")  # odd: off the aligned kernels
+
+
+@pytest.mark.parametrize("K", [16, 272, 1024, 4112, 20480])
+def test_row_piece_rings_of_every_stage_length(lib, K):
+    """Chosen and forced stage lengths (256, 512, 1024 bytes of K) for every height and every share of the weights: planned
+    launches stay inside the LDS ring, and a length that there is no kernel for is refused."""
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    seen = set()
+    for cfg in (i for i, nm in enumerate(names) if nm.endswith("_rowpieces")):
+        MT = int(names[cfg].split("_")[1][1:])
+        for M in sorted({max(1, MT - 15), MT - 9, MT - 3, MT}):
+            for per in range(1, 21):
+                pr = G.contiguous(1, M, per * 1024 - 5, K, I32)
+                for kc in (0, 256, 512, 768, 1024, 1280, 255 * 256):
+                    fits = kc == 0 or kc == 256 or (kc in (512, 1024) and (kc == 512 or MT <= 32) and per <= 12
+                                                    and 3 * (MT + 16 * -(-per // 4)) * kc <= 160 * 1024)
+                    if fits:
+                        pl = G.plan_for(lib, pr, EPI_I32, B_I32, config=cfg | (kc // 256) << 8)
+                        assert kc in (0, pl.nwa), pl
+                        seen.add((MT, pl.ksplit, pl.nwa))
+                        G.check_launch(pr, pl, store_sample=1)
+                    else:
+                        with pytest.raises(AssertionError, match="no stages of"):
+                            G.plan_for(lib, pr, EPI_I32, B_I32, config=cfg | (kc // 256) << 8)
+    assert len(seen) == 20 + 11 + 3, sorted(seen)  # of 256, 512 and 1024 bytes: every kernel there is

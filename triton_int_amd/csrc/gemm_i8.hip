@@ -2685,7 +2685,9 @@ static KernelFn rowpieces_kernel(int g) {
   return fn;
 }
 
+// nullptr: there is no such stage
 static KernelFn rowpieces_kernel(int mt, int g, int kc) {
+  if (kc != RP_KC && kc != 512 && !(kc == 1024 && mt <= 32)) return nullptr;
   switch (mt) {
     case 16: return kc == 1024 ? rowpieces_kernel<16, 1024>(g) : kc == 512 ? rowpieces_kernel<16, 512>(g) : rowpieces_kernel<16, RP_KC>(g);
     case 32: return kc == 1024 ? rowpieces_kernel<32, 1024>(g) : kc == 512 ? rowpieces_kernel<32, 512>(g) : rowpieces_kernel<32, RP_KC>(g);
@@ -3263,17 +3265,18 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
     const int wgs = p.batch >= 256 ? 1 : 256 / p.batch;
     const int rounds = (units + wgs * 4 * RP_GMAX - 1) / (wgs * 4 * RP_GMAX);
     const int per = (units + wgs * rounds - 1) / (wgs * rounds);
-    const int blocks = (units + per - 1) / per;
+    const int blocks = (units + per - 1) / per;  // the units of a block are still `per`: fewer would need more blocks than there are
+    const int g = (per + 3) / 4;
+    // forced by a test: bytes of K per stage, divided by 256
+    const int kc = want_splits ? want_splits * 256 : (k.bm <= 32 && rowpieces_fits(k.bm, g, 1024) ? 1024 : (g <= 3 && rowpieces_fits(k.bm, g, 512) ? 512 : RP_KC));
+    const KernelFn fn = rowpieces_kernel(k.bm, g, kc);
+    if (!fn) return fail(TI_E_COMBO, "config %s: no stages of %d bytes of K for %d weight rows per workgroup", k.name, kc, per * 4);
     g_last_config = config;
     if (dry) {
       dry->config = config; dry->grid_x = (unsigned)blocks; dry->grid_y = (unsigned)p.batch; dry->threads = k.threads;
+      dry->ksplit = g; dry->nwa = kc;
       return TI_OK;
     }
-    const int g = ((units + blocks - 1) / blocks + 3) / 4;
-    // forced by a test: bytes of K per stage, divided by 256
-    const int kc = want_splits ? want_splits * 256 : (k.bm <= 32 && rowpieces_fits(k.bm, g, 1024) ? 1024 : (g <= 3 && rowpieces_fits(k.bm, g, 512) ? 512 : RP_KC));
-    const KernelFn fn = rowpieces_kernel(k.bm, (per + 3) / 4, kc);
-    if (!fn) return fail(TI_E_COMBO, "config %s: stages of %d bytes of K do not fit", k.name, kc);
     fn<<<dim3((unsigned)blocks, (unsigned)p.batch), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }
