@@ -47,12 +47,18 @@ def test_out_of_memory_is_torchs_exception():
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (32 << 20)) / total)
+    taken = []
     try:
+        # what other tests left free inside torch's segments, down to half of the smallest output (128 MB)
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                taken.append(torch.empty(64 << 20, dtype=torch.uint8, device="cuda"))
         for name, call in calls.items():
             with pytest.raises(torch.OutOfMemoryError):
                 call()
                 pytest.fail(f"{name}: its output was allocated")
     finally:
+        taken.clear()
         torch.cuda.set_per_process_memory_fraction(1.0)
     for name, call in calls.items():
         call()
