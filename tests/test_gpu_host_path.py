@@ -234,6 +234,36 @@ def test_every_function_gives_what_the_python_path_gives(monkeypatch):
     assert seen == methods, methods - seen
 
 
+def test_python_float_scales_are_uploaded_before_the_module_is_asked(monkeypatch):
+    """Scales as python floats: the module takes the call instead of declining it, with the bits of device-tensor scales; a
+    scale tensor of the dequantising norm, which the module does not take, is not offered to it."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import bmm, fused, linear
+
+    g, i8, f32, s = _operands()
+    a, w, b8, bf, res = i8(37, 96), i8(48, 96), i8(48), f32(48), f32(37, 48)
+    p, q, x, gm = i8(3, 20, 33), i8(3, 17, 33), f32(9, 160), f32(160)
+    acc = torch.randint(-9999, 9999, (9, 160), dtype=torch.int32, device="cuda", generator=g)
+    calls = [lambda v: linear.linear_a8_w8_b8_o8(a, w, b8, v(1e-3), v(0.5)),
+             lambda v: linear.linear_a8_w8_bfp32_ofp32(a, w, bf, v(1e-3), v(0.5)),
+             lambda v: linear.linear_a8_w8_bfp32_ofp32_residual(a, w, bf, v(1e-3), v(0.5), res),
+             lambda v: bmm.bmm_s8t_s8n_s8t(p, q, v(1e-3)),
+             lambda v: fused.dq_add_layernorm_q(acc, v(0.5), x, gm, None, 1e-5)]
+    for call in calls:
+        records = _Records(L.host)
+        want = _flat(call(s))
+        with monkeypatch.context() as m:
+            m.setattr(L, "host", records)
+            got = _flat(call(float))
+        assert [t for _, t in records.taken] == [True]
+        assert all(torch.equal(u, v) for u, v in zip(got, want))
+    records = _Records(L.host)
+    with monkeypatch.context() as m:
+        m.setattr(L, "host", records)
+        fused.dq_add_layernorm_q(acc, s(0.5), x, gm, None, 1e-5)
+    assert not records.taken
+
+
 def test_what_is_not_the_ordinary_case_is_declined():
     """The module returns None, and nothing has been written, for every argument that the Python path converts or refuses."""
     from triton_int_amd import _lib as L

@@ -118,7 +118,7 @@ def dq_add_layernorm_q(input_int32, input_scale_fp, residual_input_fp, gamma, be
     int8) — or the fp32 LayerNorm output when quantize=False.  Semantics of
     functional/fused.py:6-24; the argument order is that of the intended native op,
     functional/fused.py:27-32."""
-    if quantize and not _return_stats:
+    if quantize and not _return_stats and not torch.is_tensor(input_scale_fp):
         y = L.host.dq_add_layernorm_q(input_int32, input_scale_fp, residual_input_fp, gamma, beta, eps, _round_mode)
         if y is not None:
             return y
