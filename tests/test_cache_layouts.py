@@ -156,15 +156,3 @@ def test_more_sequences_than_one_launch_takes(S, T):
     want = torch.cat([layer(x[p], kv_cache=(k[p], vt[p])) for p in parts])
     assert torch.equal(layer(x, kv_cache=(k2, vt2)), want) and torch.equal(k2, k) and torch.equal(vt2, vt)
     assert torch.equal(layer(x), torch.cat([layer(x[p]) for p in parts]))
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("fused", [True, False])
-@pytest.mark.parametrize("S,T", [(1, 53), (20, 53), (200, 400)])
-def test_a_batch_of_no_sequences(S, T, fused):
-    """An empty batch gives an empty output, with caches and without."""
-    layer = _layer(1024)
-    layer.fused_attention = fused
-    x = torch.empty((0, S, 1024), device="cuda")
-    k, vt = (torch.empty(s, dtype=torch.int8, device="cuda") for s in ((0, T, D), (0, D, T)))
-    assert layer(x).shape == layer(x, kv_cache=(k, vt)).shape == (0, S, 1024)

@@ -155,7 +155,7 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         mark("ln1_layernorm_q")
         w3, b3, a3, s3 = self._qkv_pack()
         qkv = None
-        if kv_cache is not None and 0 < B * S <= 16:
+        if kv_cache is not None and B * S <= 16:
             # decode: projections and KV-cache append in one launch
             qkv = linear_qkv_decode_a8_w8_b8_o8(h8.view(B * S, H), w3, b3, a3, s3, kv_cache[0], kv_cache[1], seqs=B)
         appended = qkv is not None
@@ -178,7 +178,7 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
             k_all = None
         else:
             k_all, vt_all = kv_cache
-        if not appended and B > 0:
+        if not appended:
             # the new K rows and V^T columns go into the last S slots of the cache
             self._append(qkv[..., H:2 * H], v, k_all, vt_all)
         mark("kv_append_v_transpose")
