@@ -310,3 +310,19 @@ def test_what_is_not_the_ordinary_case_is_declined():
     for name in ("linear", "bmm", "softmax_q"):
         with pytest.raises(TypeError):
             getattr(h, name)(a)
+
+
+def test_an_integer_beyond_any_double_is_refused():
+    """As float() refuses it, from every launcher that takes a number, with nothing launched on the value it would leave."""
+    from triton_int_amd.kernels import fused
+
+    g, i8, f32, s = _operands()
+    x, gm, big = f32(9, 160), f32(160), 10 ** 400
+    acc = torch.randint(-9999, 9999, (9, 160), dtype=torch.int32, device="cuda", generator=g)
+    q, k, vt = i8(2, 3, 128), i8(2, 9, 128), i8(2, 128, 9)
+    for call in (lambda: fused.layer_norm_fwd_fused_single_pass_q(x, gm, None, big), lambda: fused.layer_norm_fwd_fused_single_pass(x, gm, None, big),
+                 lambda: fused.dq_add_layernorm_q(acc, big, x, gm, None, 1e-5), lambda: fused.dq_add_layernorm_q(acc, 0.5, x, gm, None, big),
+                 lambda: fused.softmax_q(i8(4, 32), big), lambda: fused.attention_i8(q, k, vt, big, 0.1, 0.05),
+                 lambda: fused.attention_i8(q, k, vt, 1e-3, 0.1, big)):
+        with pytest.raises(OverflowError):
+            call()

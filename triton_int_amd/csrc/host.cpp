@@ -91,7 +91,9 @@ int64_t integer(PyObject* o) {
 
 double number(PyObject* o) {
   need(PyFloat_Check(o) || PyLong_Check(o));
-  return PyFloat_AsDouble(o);
+  const double v = PyFloat_AsDouble(o);
+  need(!(v == -1.0 && PyErr_Occurred()));  // an integer beyond any double
+  return v;
 }
 
 // A Python bool itself: anything else that counts as true or false is for the Python path to convert.
