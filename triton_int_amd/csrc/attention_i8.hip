@@ -401,15 +401,16 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, kq = lane >> 4;  // operand row / 16-byte quarter of a 64-deep k-step
-  // the workgroups of a head are p.batch apart: with a batch that is a multiple of 8 they run on the
-  // same XCD and share its L2 for K
-  const int bh = blockIdx.x % p.batch;
-  const int part = blockIdx.x / p.batch, ngrp = (p.S + 15) >> 4;
-  const int row0 = (part % ngrp) * 16;  // this workgroup's 16 query rows
-  const int dbase = (part / ngrp) * DBW;
+  // Grid: head; 16 query rows and block of output columns; sequence.  The workgroups of a head are p.heads apart: with
+  // a multiple of 8 heads they run on the same XCD and share its L2 for K.  No division on the way to the first loads,
+  // and no branch before all arguments are asked for: at 6 us a launch those are felt (head, sequence, rows and columns divided
+  // out of one grid dimension, and the mask's period: 32 heads x 1 row x 64 keys 6.5 us, so 5.7; 40 x 1 x 512 7.4 / 7.0).
+  constexpr int PARTS = 8 / DBW;
+  const int head = blockIdx.x, seq = blockIdx.z;
+  const int row0 = (int)blockIdx.y / PARTS * 16;  // this workgroup's 16 query rows
+  const int dbase = (int)blockIdx.y % PARTS * DBW;
   const int OOB = 0x7ffffff0;
   const float MAGIC = 12582912.0f;
-  const int seq = bh / p.heads, head = bh - seq * p.heads;
   const int8_t* vb = p.vt + (int64_t)seq * p.sVb + (int64_t)head * p.sVh;
   const __amdgpu_buffer_rsrc_t rQ = __builtin_amdgcn_make_buffer_rsrc((void*)(p.q + (int64_t)seq * p.sQb + (int64_t)head * p.sQh), 0,
                                                                       (int)((p.S - 1) * p.sQm + AT_D), 0x00020000);
@@ -418,23 +419,25 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   // the last chunk of an aligned row may cross T (see attention_i8_kernel)
   const __amdgpu_buffer_rsrc_t rV =
       __builtin_amdgcn_make_buffer_rsrc((void*)vb, 0, (int)((AT_D - 1) * p.sVd + ((p.T + 15) & ~15)), 0x00020000);
+  const int db = dbase + wave % DBW, kh = wave / DBW;
+
+  v4i qf[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+    qf[ks] = __builtin_amdgcn_raw_buffer_load_b128(rQ, row0 + n < p.S ? (row0 + n) * (int)p.sQm + ks * 64 + kq * 16 : OOB, 0, 0);
   // keys that any of the rows sees (under a causal mask the later ones are not even loaded)
   const int rlast = min(row0 + 15, p.S - 1);
-  const int keys = p.causal_q_len > 0 && row0 / p.causal_q_len == rlast / p.causal_q_len ? attn_limit(p, rlast) : p.T;
+  const bool one_period = p.causal_q_len >= p.S;  // of the mask, as in every decoder layer: nothing to divide
+  auto limit_of = [&](int row) { return one_period ? min(p.T, row + (p.T - p.causal_q_len) + 1) : attn_limit(p, row); };
+  const int keys = one_period || (p.causal_q_len > 0 && row0 / p.causal_q_len == rlast / p.causal_q_len) ? limit_of(rlast) : p.T;
   auto load_v = [&](int d, int col) -> v4i {
     if constexpr (VANY) return load16_tail(vb + (int64_t)d * p.sVd, col, p.T);
     else return __builtin_amdgcn_raw_buffer_load_b128(rV, col < keys ? d * (int)p.sVd + col : OOB, 0, 0);
   };
   const int NCH = (keys + 15) >> 4;  // 16-key chunks; rows of K past T read as zeros and are masked
   const int NG = (keys + 63) >> 6;   // 64-key groups
-  const int db = dbase + wave % DBW, kh = wave / DBW;
-
+  const int limit = limit_of(min(row0 + n, rlast));
   // ---- scores: f = the int8 score as a float, -inf where masked or beyond T
-  v4i qf[2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks)
-    qf[ks] = __builtin_amdgcn_raw_buffer_load_b128(rQ, row0 + n < p.S ? (row0 + n) * (int)p.sQm + ks * 64 + kq * 16 : OOB, 0, 0);
-  const int limit = attn_limit(p, row0 + n);
   const float NEG = -__builtin_inff();
   float f[CPW][4];
   constexpr int NB = CPW < 8 ? CPW : (CPW > 8 ? 4 : 8);  // chunks whose K operands are in flight together
@@ -624,7 +627,7 @@ extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int6
     // 24 us for 8, which no longer fit one round)
     int dbw = 8;
     while (dbw > 1 && groups * (16 / dbw) <= 256) dbw /= 2;
-    const dim3 grid((unsigned)(groups * (8 / dbw))), block(AD_WAVES * 64);
+    const dim3 grid((unsigned)heads, (unsigned)((S + 15) / 16 * (8 / dbw)), (unsigned)seqs), block(AD_WAVES * 64);
 #define TI_AD_LAUNCH(C, V) \
     (dbw == 8 ? attention_decode_i8_kernel<C, 8, V><<<grid, block, 0, st>>>(p) : dbw == 4 ? attention_decode_i8_kernel<C, 4, V><<<grid, block, 0, st>>>(p) \
      : dbw == 2 ? attention_decode_i8_kernel<C, 2, V><<<grid, block, 0, st>>>(p) : attention_decode_i8_kernel<C, 1, V><<<grid, block, 0, st>>>(p))
