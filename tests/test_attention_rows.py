@@ -16,6 +16,18 @@ def test_up_to_16_query_rows_run_on_the_one_pass_kernel_at_any_batch():
     assert rows(64, 256, 1064) == 16 and rows(65, 256, 1064) == 128 and rows(1280, 17, 2048) == 128
 
 
+def test_more_query_rows_run_on_the_kernel_that_measures_faster():
+    """Several rounds of 16-row groups against few keys, or against caches that every round reads again, cost more than one
+    round of 128-row blocks."""
+    from triton_int_amd import _lib as L
+
+    rows = lambda heads, S, T: L.lib().ti_attention_i8_rows(heads, S, T, 128, 128, T)
+    for heads, S, T in ((160, 64, 64), (80, 128, 128), (512, 32, 128), (512, 17, 1024), (256, 64, 2048), (160, 48, 64), (340, 48, 2048), (40, 384, 384)):
+        assert rows(heads, S, T) == 128, (heads, S, T)
+    for heads, S, T in ((32, 64, 1064), (64, 128, 333), (8, 17, 64), (32, 512, 2048), (40, 128, 512), (128, 17, 2048), (40, 333, 2048), (1, 129, 4096)):
+        assert rows(heads, S, T) == 16, (heads, S, T)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("S", [1, 16, 17])
 @pytest.mark.parametrize("heads,T", [(1024, 33), (1025, 33), (1030, 80), (2600, 17)])

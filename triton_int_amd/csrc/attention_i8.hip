@@ -558,19 +558,30 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   }
 }
 
-// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them, or as long as they are at most
-// four rounds of the chip (256 workgroups each); 128-row blocks on attention_i8_kernel beyond.  A group walks the keys
-// once on 16 waves; a block walks them three times on 4 waves, 2.1 us per 64 keys however few blocks there are and
-// however few of its rows are live.
-// Measured, causal (us, groups / blocks): 32 heads x 64 rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 /
-// 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81, 64 x 256 x 1064 (1024) 48 / 46,
-// 160 x 96 x 2048 (960) 83 / 81, 40 x 512 x 2048 (1280) 88 / 81, 160 x 128 x 2048 (1280) 103 / 82, 320 x 64 x 2048
-// (1280) 145 / 113, 1280 x 17 x 2048 (2560) 298 / 269, 1280 x 32 x 1024 (2560) 133 / 137.
+// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them.  Up to four rounds of the chip
+// (256 workgroups each) on whichever kernel takes less: a round of groups walks the keys once, 0.4 us per 64 of them and
+// 3.5 us besides, or as long as 4 TB/s take for the caches of the heads in it (up to 256: each is then read again in the
+// next round); the blocks of 128 rows on attention_i8_kernel, all in one round, 2.4 us per 64 keys and 3.5 us besides
+// however few their rows.  128-row blocks beyond four rounds.
+// Measured (us, groups / blocks), 340 launches of 17 .. 512 rows against 16 .. 4096 keys, with and without a mask: the
+// estimate's choice is 0.4 % above the better one on average, and nowhere more than 3 % above the blocks.  Causal: 32 heads x 64
+// rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 / 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81;
+// but 160 x 64 x 64 13.3 / 7.7, 80 x 192 x 256 19.3 / 15.0, 512 x 32 x 128 19.1 / 11.9, 256 x 64 x 2048 120 / 83, 512 x 17 x 1024
+// 59 / 48.  Beyond: 40 x 512 x 2048 (1280) 88 / 81, 320 x 64 x 2048 (1280) 145 / 113, 1280 x 17 x 2048 (2560) 298 / 269, 1280
+// x 32 x 1024 (2560) 133 / 137.
 // 16 rows and fewer, as many workgroups either way: 1280 x 1 x 2048 156 / 265, 2560 x 16 x 2048 297 / 464, 1056 x 1 x
 // 333 24.8 / 57.8, 20000 x 1 x 304 346 / 707 (20000 x 1 x 64 265 / 242).
+static bool attn_groups_lead(int64_t heads, int S, int T) {
+  const int64_t groups = heads * ((S + 15) / 16);
+  if (S <= 16) return true;
+  if (groups > 1024) return false;
+  const double walk = 3.5 + 0.4 * T / 64, fetch = (double)(heads < 256 ? heads : 256) * T * 2 * AT_D / 4.0e6;
+  return (double)((groups + 255) / 256) * (walk > fetch ? walk : fetch) <= 3.5 + 2.4 * T / 64;
+}
+
 static bool attn_few_rows(int64_t heads, int S, int T, int64_t q_row_stride, int64_t k_row_stride, int64_t vt_row_stride) {
   const int64_t lim32 = (int64_t)1 << 31;  // descriptor extents and offsets
-  return (S <= 16 || heads * ((S + 15) / 16) <= 1024) && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 &&
+  return attn_groups_lead(heads, S, T) && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 &&
          (int64_t)AT_D * vt_row_stride < lim32 && (int64_t)S * q_row_stride < lim32;
 }
 
