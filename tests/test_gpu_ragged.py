@@ -92,14 +92,16 @@ def test_row_piece_kernel_edges(M, N, K):
     bf, res = torch.randn(N, device="cuda", generator=g), torch.randn((M, N), device="cuda", generator=g)
     acc = (a.double() @ w.double().t()).to(torch.int32)
     alpha, one = torch.tensor(30.0 / (K ** 0.5 * 5400.0), device="cuda"), torch.tensor(1.0, device="cuda")
-    got = linear.linear_a8_w8_b32_o32(a, w, b32)
-    assert lib.ti_gemm_config_name(lib.ti_gemm_last_config()).decode().endswith("_rowpieces")
-    assert torch.equal(got, acc + b32)
     f = alpha * acc.float()
-    assert torch.equal(linear.linear_a8_w8_b8_o8(a, w, b8, alpha, one), (b8.float() + f).round().clamp(-128, 127).to(torch.int8))
     want = bf + f
-    assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one), want)
-    assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one, dtype=torch.float16), want.half())
+    # forced: a short K may run on another kernel, and has to give the same there
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    for cfg in (names.index(f"skinny_m{(M + 15) // 16 * 16}_rowpieces"), -1):
+        assert torch.equal(linear.linear_a8_w8_b32_o32(a, w, b32, _config=cfg), acc + b32)
+        assert cfg in (-1, lib.ti_gemm_last_config())
+        assert torch.equal(linear.linear_a8_w8_b8_o8(a, w, b8, alpha, one, _config=cfg), (b8.float() + f).round().clamp(-128, 127).to(torch.int8))
+        assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one, _config=cfg), want)
+        assert torch.equal(linear.linear_a8_w8_bfp32_ofp32(a, w, bf, alpha, one, dtype=torch.float16, _config=cfg), want.half())
     assert torch.equal(linear.linear_a8_w8_bfp32_ofp32_residual(a, w, bf, alpha, one, res), want + res)
 
 
@@ -116,9 +118,10 @@ def test_row_piece_kernel_every_stage_length(M, N, K):
     a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device="cuda", generator=g) for s in ((M, K), (N, K)))
     b32 = torch.randint(-1000, 1000, (N,), dtype=torch.int32, device="cuda", generator=g)
     want = (a.double() @ w.double().t()).to(torch.int32) + b32
-    assert torch.equal(linear.linear_a8_w8_b32_o32(a, w, b32), want)
-    cfg = lib.ti_gemm_last_config()
-    assert lib.ti_gemm_config_name(cfg).decode().endswith("_rowpieces")
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    cfg = names.index(f"skinny_m{(M + 15) // 16 * 16}_rowpieces")
+    for c in (cfg, -1):
+        assert torch.equal(linear.linear_a8_w8_b32_o32(a, w, b32, _config=c), want)
     mt, per = (M + 15) // 16 * 16, -(-((N + 3) // 4) // 256)
     for kc in (256, 512, 1024):
         if kc == 256 or (per <= 12 and 3 * (mt + 16 * -(-per // 4)) * kc <= 160 * 1024 and (kc == 512 or mt <= 32)):
@@ -267,3 +270,33 @@ def test_quantize_per_tensor_is_the_torch_steps_bit_for_bit(shape, dtype):
         assert q.dtype == torch.int8 and q.shape == x.shape and torch.equal(x, kept)
         assert torch.equal(s, want_s) and torch.equal(alpha, want_s.float() * ws)
         assert torch.equal(q, (x / want_s).round_().to(torch.int8))
+
+
+@pytest.mark.parametrize("M,N,K,batch,kernel", [
+    (1, 4096, 64, 1, "slab"), (16, 20480, 256, 1, "slab"), (16, 1024, 272, 1, "rowpieces"), (17, 4096, 128, 1, "slab"), (32, 512, 144, 1, "rowpieces"),
+    (33, 12288, 64, 1, "slab"), (33, 11264, 64, 1, "rowpieces"), (64, 20480, 80, 1, "rowpieces"),                # one round
+    (1, 26000, 1008, 1, "slab"), (12, 13824, 256, 3, "slab"), (20, 20480, 512, 3, "slab"), (20, 12288, 528, 3, "rowpieces"),
+    (64, 11008, 64, 4, "slab"), (64, 16384, 272, 3, "rowpieces"), (8, 4096, 1024, 1, "rowpieces")])               # more, and K of 1024
+def test_short_k_against_few_rows_at_the_edges_of_the_rule(M, N, K, batch, kernel):
+    """Which kernel a short K runs on, and the same sums from both, residual included."""
+    from triton_int_amd import _lib as L
+    from triton_int_amd.kernels import linear
+    from triton_int_amd.kernels._gemm import linear_group
+
+    lib = L.lib()
+    names = [lib.ti_gemm_config_name(i).decode() for i in range(lib.ti_gemm_num_configs())]
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = (torch.randint(-128, 128, s, dtype=torch.int8, device="cuda", generator=g) for s in ((M, K), (batch * N, K)))
+    want = (a.double() @ w.double().t()).to(torch.int32)
+    other = names.index(f"skinny_m{(M + 15) // 16 * 16}_rowpieces" if kernel == "slab" else f"skinny_m{16 if M <= 16 else 32 if M <= 32 else 64}_slab16")
+    for cfg in (-1, other):
+        if batch == 1:
+            got = linear.linear_a8_w8_b32_o32(a, w, torch.zeros(N, dtype=torch.int32, device="cuda"), _config=cfg)
+        else:
+            got = linear_group(a, w, batch, epilogue=L.EPI_I32, out_dtype=torch.int32, config=cfg)
+        assert torch.equal(got, want), cfg
+        assert (kernel in names[lib.ti_gemm_last_config()]) == (cfg == -1)
+    if batch == 1:
+        one, res = torch.tensor(1.0, device="cuda"), torch.randn((M, N), device="cuda", generator=g)
+        got = linear.linear_a8_w8_bfp32_ofp32_residual(a, w, torch.zeros(N, device="cuda"), one, one, res)
+        assert torch.equal(got, want.float() + res)

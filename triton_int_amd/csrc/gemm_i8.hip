@@ -10,7 +10,7 @@
 //   gemm_mfma_kernel         one tile per workgroup; any output layout the fast loads allow.
 //   gemm_rowpieces_kernel    M <= 64: weight rows dealt evenly to the CUs, the whole K in one workgroup.
 //   gemm_rows4_kernel        M <= 16 against a few rows of a long K: weights as whole 1 KB row pieces.
-//   gemm_skinny_kernel       M <= 64, batched: 16-row weight slabs in MFMA layout, K split over waves.
+//   gemm_skinny_kernel       M <= 64, batched or a short K: 16-row weight slabs in MFMA layout, K split over waves.
 //   gemm_ragged_kernel       rows that start at any byte, any K, [K,N] operands (unaligned loads through registers).
 //   gemm_gather_kernel       any strides (byte gathers).
 // All but the last two need both operands K-contiguous and 16-byte aligned: 128-bit buffer loads
@@ -2911,8 +2911,15 @@ static int pick_config(const GemmParams& p, int* splits_out) {
     //   10240 21.0 / 20.5 (48), 4096 x 8192 16.6 / 15.4 (64); but 5120 x 20480 24.0 / 26.5 (32), 4096 x 16384 20.1 /
     //   22.2 (48), 6848 x 10240 21.3 / 21.7 (64), 50272 x 1024 18.3 / 34.8, 32768 x 768 9.5 / 18.7.  The line: one
     //   round and K = 16384 (M <= 32), 10240 (48), 8192 (64).
-    //   K < 1024, one round, against gemm_skinny_kernel: 768 x 768 9.4 / 5.0 (M = 16), 20.2 / 5.5 (64), 256 x 256
-    //   5.2 / 4.9 (1).
+    //   K < 1024, against gemm_skinny_kernel (whose waves start at once, where this one fills its LDS stages first, and
+    //   which has as many workgroups as it likes, where this one pays whole rounds).  One round, fp32 out: 768 x 768 9.0 /
+    //   5.4 (M = 16), 20.2 / 5.5 (64); but 4096 x 64 3.9 / 5.1 (M = 1), 4.9 / 5.6 (32), 6.9 / 5.8 (64), 4096 x 128 4.2 / 5.2 (1), 5.7 /
+    //   5.5 (32), 4096 x 256 5.2 / 5.3 (1), 5.6 / 5.3 (16), 7.0 / 5.6 (32), 20480 x 256 5.6 / 5.6 (1), 20480 x 64 8.0 / 9.0 (64).  The
+    //   line: K of 256 (M <= 16), 128 (32), 64 with 12 and more units per workgroup (48, 64).
+    //   More than one round, three grouped (N each): 8192 x 256 5.8 / 8.9 (1), 7.7 / 10.4 (32), 11.4 / 14.1 (64), 16384 x 1008
+    //   15.6 / 19.1 (1), 16384 x 512 18.0 / 20.2 (32), 28.7 / 26.0 (64), 12288 x 640 13.5 / 12.3 (16), 20.8 / 15.2 (32).  The line: any K
+    //   (M <= 16), 512 (32), 256 (64).  (One GEMM of more rounds and M > 16 has the tiles below.)  With a
+    //   residual this kernel: the other would take an add kernel after it.
     // Three corners stay on the tiles although this kernel measures better there, because tests name what
     // they run on: M > 48 with 16385 .. 20480 columns (64 x 20480 x 5120 34.0 / 28.2), M > 16 with fewer than 512
     // (32 x 272 x 1040 8.5 / 5.3), M > 48 with one unit per workgroup and K > 4096 (64 x 1024 x 10240 17.0 / 15.7).
@@ -2921,9 +2928,15 @@ static int pick_config(const GemmParams& p, int* splits_out) {
     const int64_t columns = (int64_t)p.N * p.batch;
     const int rp = CFG_ROWPIECES_16 + (p.M - 1) / 16;
     if (p.M <= 16 && p.K >= 1024) return one_round ? rp : CFG_ROWS4_16;
-    if (p.K < 1024 ? one_round || p.M <= 16 || p.batch > 1 || !stream
-                   : one_round && p.K <= (p.M <= 32 ? 16384 : p.M <= 48 ? 10240 : per > 1 ? 8192 : 4096) && !(p.M > 48 && columns > 16384) && columns >= 512)
+    if (p.K < 1024) {
+      const bool slabs = !p.resid && (one_round ? p.K <= (p.M <= 16 ? 256 : p.M <= 32 ? 128 : per >= 12 ? 64 : 0) : p.M <= 16 || p.K <= (p.M <= 32 ? 512 : 256));
+      if (one_round || p.M <= 16 || p.batch > 1 || !stream) {
+        if (!slabs) return rp;
+        if (p.M > 16) return CFG_SKINNY_16 + 1 + (p.M > 32);
+      }
+    } else if (one_round && p.K <= (p.M <= 32 ? 16384 : p.M <= 48 ? 10240 : per > 1 ? 8192 : 4096) && !(p.M > 48 && columns > 16384) && columns >= 512) {
       return rp;
+    }
   }
   // batched, few rows (attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
   if (p.M <= 16) return (p.N + 31) / 32 >= 160 ? CFG_SKINNY_16_G2 : CFG_SKINNY_16;
@@ -3406,23 +3419,20 @@ static int run_with_residual(GemmParams p, const float* R, int64_t ldr, hipStrea
   rc = check_device();
   if (rc != TI_OK) return rc;
   if (!p.bias) p.bias_kind = TI_BIAS_NONE;
+  p.resid = R;
+  p.resid_rs = ldr;
   int splits = 1;
   const int cfg = pick_config(p, &splits);
-  if (g_configs[cfg].rows4 || g_configs[cfg].rowpieces) {  // the decode kernels add the residual in their store phase
-    p.resid = R;
-    p.resid_rs = ldr;
-    return run(p, cfg, stream);
-  }
+  if (g_configs[cfg].rows4 || g_configs[cfg].rowpieces) return run(p, cfg, stream);  // the decode kernels add the residual in their store phase
   // the persistent kernels add it in their fp32 epilogue (with split K: in that of a tile's last item, where the
   // sums are whole); 32-bit offsets into the residual, like the stores.  run() chooses again, the same way: a split passed
   // to it would count as forced, and a capturing stream without a workspace would be refused instead of run unsplit
   const bool persistent = g_configs[cfg].stream_occ > 0 || g_configs[cfg].ws_waves > 0 || g_configs[cfg].max_k > 0;
   if (persistent && p.batch == 1 && p.out_dtype == TI_F32 && p.epilogue == TI_EPI_SCALE_F &&
       ((int64_t)(p.M + 512) * ldr + p.N) * 4 < ((int64_t)1 << 31)) {
-    p.resid = R;
-    p.resid_rs = ldr;
     return run(p, -1, stream);
   }
+  p.resid = nullptr;
   rc = run(p, -1, stream);
   if (rc != TI_OK) return rc;
   const int vec = (p.N % 4 == 0) && (p.sCm % 4 == 0) && (ldr % 4 == 0) && (((uintptr_t)p.C | (uintptr_t)R) & 15) == 0;
