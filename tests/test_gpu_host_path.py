@@ -177,7 +177,11 @@ def _ordinary_calls():
                 add("layernorm_fp", lambda rms=rms, beta=beta, c=c: fused.skip_layer_norm_fwd_fused_single_pass2(c(x), c(x * 2), c(gm), c(beta), 1e-6, rms))
     acc = torch.randint(-9999, 9999, (2, 9, 160), dtype=torch.int32, device="cuda", generator=g)
     add("dq_add_layernorm_q", lambda: fused.dq_add_layernorm_q(acc, 1e-4, x, gm, bt, 1e-5))
+    acc_wide = torch.randint(-9999, 9999, (2, 9, 192), dtype=torch.int32, device="cuda", generator=g)
+    w160, w160x160 = i8(48, 160), i8(160, 160)
     add("gelu_q", lambda: fused.gelu_q(x, s(30.0)))
+    add("gelu_q", lambda: fused.gelu_q(x, 30.0))
+    add("linear", lambda: linear.linear_a8_w8_b8_o8(a, w, b8, al, 1))
     scores = i8(3, 20, 33)
     add("softmax_q", lambda: fused.softmax_q(scores, 0.1))
     add("softmax_q", lambda: fused.softmax_q(scores, 0.1, 20))
@@ -185,6 +189,19 @@ def _ordinary_calls():
         add("quantize_per_token", lambda t=t: fused.quantize_per_token_absmax(t.contiguous()))
         add("quantize_per_tensor", lambda t=t: fused.quantize_per_tensor_absmax(t.contiguous(), s(0.25)))
     add("quantize_per_tensor", lambda: fused.quantize_per_tensor_absmax(x))
+    # rows that are slices of wider ones, with any leading dimensions that make one row after the other
+    for cut in (lambda t: t[..., 3:163], lambda t: t[0, :, 16:176], lambda t: t[:, 4:5, :160], lambda t: t[1:, :1, 8:168], lambda t: t[:1, :0, :160]):
+        y, z = cut(f32(2, 9, 200)), cut(f32(2, 9, 184))
+        add("layernorm_q", lambda y=y: fused.layer_norm_fwd_fused_single_pass_q(y, gm, bt, 1e-5))
+        for dt in (torch.float32, torch.float16):
+            wide = [cut(t.to(dt)) for t in (f32(2, 9, 200), f32(2, 9, 176))]
+            add("layernorm_fp", lambda t=wide, dt=dt: fused.skip_layer_norm_fwd_fused_single_pass2(t[0], t[1], gm.to(dt), bt.to(dt), 1e-6))
+        add("dq_add_layernorm_q", lambda z=z, b=cut(acc_wide): fused.dq_add_layernorm_q(b, 1e-4, z, gm, bt, 1e-5))
+        add("softmax_q", lambda b=cut(i8(2, 9, 209)): fused.softmax_q(b, 0.1))
+        add("quantize_per_token", lambda y=y: fused.quantize_per_token_absmax(y))
+        cut8 = lambda n, c=cut: c(i8(2, 9, n))
+        add("linear", lambda b=cut8(208): linear.linear_a8_w8_b32_o32(b, w160, b32))
+        add("linear_residual", lambda b=cut8(208), r=cut(f32(2, 9, 240)): linear.linear_a8_w8_bfp32_ofp32_residual(b, w160x160, gm, al, be, r))
     for lead in ((4,), (2, 3)):
         Q, K, V = i8(*lead, 5, 128), i8(*lead, 21, 128), i8(*lead, 128, 21)
         add("attention", lambda Q=Q, K=K, V=V: fused.attention_i8(Q, K, V, 1e-3, 0.1, 0.05, 5))

@@ -138,16 +138,32 @@ int int32_size(int64_t v) {
   return (int)v;
 }
 
+// Distance of the rows [..., n] with unit stride along the last dimension and one distance between all of them (a
+// slice of wider rows); n for a single row.  Anything else needs a copy.
+int64_t row_pitch(const Tensor& t) {
+  const int64_t d = t.dim();
+  need(d >= 1);
+  int64_t pitch = t.size(d - 1), next = -1;
+  if (t.is_contiguous()) return pitch;
+  need(t.stride(d - 1) == 1);
+  for (int64_t i = d - 2; i >= 0; --i) {
+    if (t.size(i) == 1) continue;
+    if (next < 0) pitch = t.stride(i);
+    need(next < 0 || t.stride(i) == next);
+    next = t.stride(i) * t.size(i);
+  }
+  return pitch;
+}
+
 // activations [..., K] as M rows of one pitch
 struct Rows {
   int M, K;
   int64_t pitch;
   Rows(const Tensor& a, int64_t k) {
     need(a.dim() >= 2 && a.size(-1) == k && k > 0);
-    need(a.dim() == 2 ? a.stride(1) == 1 : a.is_contiguous());
     K = int32_size(k);
     M = int32_size(a.numel() / k);
-    pitch = a.dim() == 2 ? a.stride(0) : k;
+    pitch = row_pitch(a);
   }
 };
 
@@ -267,15 +283,16 @@ PyObject* linear_residual(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Rows r(a, w.size(1));
     const float *bias = (const float*)vector(v[2], c.dev, ScalarType::Float, N), *alpha = scale(v[3], c.dev), *beta = scale(v[4], c.dev);
     need(alpha && beta);
-    const float* res = (const float*)vector(v[5], c.dev, ScalarType::Float, (int64_t)r.M * N);
-    need(res);
+    const Tensor& res = tensor(v[5], c.dev, ScalarType::Float);
+    need(res.numel() == (int64_t)r.M * N && (res.is_contiguous() || res.size(-1) == N));
+    const int64_t res_pitch = res.is_contiguous() ? N : row_pitch(res);
     const int N32 = int32_size(N);
     Tensor out;
     int rc;
     {
       const NoGil unlocked;
       out = c.empty(with_last(a, N), ScalarType::Float);
-      rc = ti_linear_i8_residual_f32((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), w.stride(0), bias, alpha, beta, res, N,
+      rc = ti_linear_i8_residual_f32((const int8_t*)ptr(a), r.pitch, (const int8_t*)ptr(w), w.stride(0), bias, alpha, beta, (const float*)ptr(res), res_pitch,
                                      (float*)mptr(out), N, r.M, N32, r.K, c.stream);
     }
     need(rc == TI_OK);
@@ -288,8 +305,8 @@ PyObject* layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* {
     const Tensor& x = tensor(v[0], -1, ScalarType::Float);
     const Call c(x);
-    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
-    const int64_t N = x.size(-1);
+    need(x.dim() >= 1 && x.size(-1) > 0);
+    const int64_t N = x.size(-1), pitch = row_pitch(x);
     const float *g = (const float*)vector(v[1], c.dev, ScalarType::Float, N), *b = (const float*)vector(v[2], c.dev, ScalarType::Float, N);
     need(g);
     const int rows = int32_size(x.numel() / N), cols = int32_size(N), round_mode = (int)integer(v[5]);
@@ -300,7 +317,7 @@ PyObject* layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     {
       const NoGil unlocked;
       out = c.empty(x.sizes(), ScalarType::Char);
-      rc = ti_layernorm_q((const float*)ptr(x), N, g, b, eps, (int8_t*)mptr(out), N, rows, cols, rms, round_mode, nullptr, nullptr, c.stream);
+      rc = ti_layernorm_q((const float*)ptr(x), pitch, g, b, eps, (int8_t*)mptr(out), N, rows, cols, rms, round_mode, nullptr, nullptr, c.stream);
     }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
@@ -313,8 +330,8 @@ PyObject* dq_add_layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Tensor& acc = tensor(v[0], -1, ScalarType::Int);
     const Call c(acc);
     const Tensor& res = tensor(v[2], c.dev, ScalarType::Float);
-    need(acc.dim() >= 1 && acc.is_contiguous() && res.is_contiguous() && acc.sizes() == res.sizes() && acc.size(-1) > 0);
-    const int64_t H = acc.size(-1);
+    need(acc.dim() >= 1 && acc.sizes() == res.sizes() && acc.size(-1) > 0);
+    const int64_t H = acc.size(-1), pitch = row_pitch(acc), res_pitch = row_pitch(res);
     const float *g = (const float*)vector(v[3], c.dev, ScalarType::Float, H), *b = (const float*)vector(v[4], c.dev, ScalarType::Float, H);
     need(g);
     const int rows = int32_size(acc.numel() / H), cols = int32_size(H), round_mode = (int)integer(v[6]);
@@ -325,7 +342,7 @@ PyObject* dq_add_layernorm_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
       const NoGil unlocked;
       rout = c.empty(acc.sizes(), ScalarType::Float);
       y = c.empty(acc.sizes(), ScalarType::Char);
-      rc = ti_dq_add_layernorm_q((const int32_t*)ptr(acc), H, s, nullptr, (const float*)ptr(res), H, g, b, eps, (float*)mptr(rout), H,
+      rc = ti_dq_add_layernorm_q((const int32_t*)ptr(acc), pitch, s, nullptr, (const float*)ptr(res), res_pitch, g, b, eps, (float*)mptr(rout), H,
                                  (int8_t*)mptr(y), H, nullptr, H, rows, cols, round_mode, nullptr, nullptr, c.stream);
     }
     need(rc == TI_OK);
@@ -343,13 +360,15 @@ PyObject* layernorm_fp(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Call c(x);
     const ScalarType type = x.scalar_type();
     const int dt = dtype_code(type);
-    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
-    const int64_t N = x.size(-1);
+    need(x.dim() >= 1 && x.size(-1) > 0);
+    const int64_t N = x.size(-1), pitch = row_pitch(x);
+    int64_t skip_pitch = 0;
     const void *g = vector(v[2], c.dev, type, N), *b = vector(v[3], c.dev, type, N), *skip = nullptr;
     need(g);
     if (v[1] != Py_None) {
       const Tensor& s = tensor(v[1], c.dev, type);
-      need(s.is_contiguous() && s.numel() == x.numel() && s.size(-1) == N);
+      need(s.numel() == x.numel() && s.size(-1) == N);
+      skip_pitch = row_pitch(s);
       skip = ptr(s);
     }
     const int rows = int32_size(x.numel() / N), cols = int32_size(N);
@@ -361,7 +380,7 @@ PyObject* layernorm_fp(PyObject*, PyObject* const* v, Py_ssize_t n) {
       const NoGil unlocked;
       if (want_out) out = c.empty(x.sizes(), type);
       if (want_skip_out) sout = c.empty(x.sizes(), type);
-      rc = ti_layernorm_fp(ptr(x), N, skip, skip ? N : 0, dt, g, b, eps, rms, want_out ? mptr(out) : nullptr, N,
+      rc = ti_layernorm_fp(ptr(x), pitch, skip, skip_pitch, dt, g, b, eps, rms, want_out ? mptr(out) : nullptr, N,
                            want_skip_out ? mptr(sout) : nullptr, N, rows, cols, c.stream);
     }
     need(rc == TI_OK);
@@ -401,8 +420,8 @@ PyObject* softmax_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 3, [&]() -> PyObject* {
     const Tensor& x = tensor(v[0], -1, ScalarType::Char);
     const Call c(x);
-    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
-    const int64_t cols = x.size(-1);
+    need(x.dim() >= 1 && x.size(-1) > 0);
+    const int64_t cols = x.size(-1), pitch = row_pitch(x);
     const int rows = int32_size(x.numel() / cols), cols32 = int32_size(cols), causal = (int)integer(v[2]);
     const float s = (float)number(v[1]);
     Tensor out;
@@ -410,7 +429,7 @@ PyObject* softmax_q(PyObject*, PyObject* const* v, Py_ssize_t n) {
     {
       const NoGil unlocked;
       out = c.empty(x.sizes(), ScalarType::Char);
-      rc = ti_softmax_q((const int8_t*)ptr(x), cols, s, (int8_t*)mptr(out), cols, rows, cols32, causal, c.stream);
+      rc = ti_softmax_q((const int8_t*)ptr(x), pitch, s, (int8_t*)mptr(out), cols, rows, cols32, causal, c.stream);
     }
     need(rc == TI_OK);
     return THPVariable_Wrap(out);
@@ -423,8 +442,8 @@ PyObject* quantize_per_token(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const Tensor& x = tensor(v[0]);
     const Call c(x);
     need(x.scalar_type() == ScalarType::Float || x.scalar_type() == ScalarType::Half);
-    need(x.dim() >= 1 && x.is_contiguous() && x.size(-1) > 0);
-    const int64_t cols = x.size(-1);
+    need(x.dim() >= 1 && x.size(-1) > 0);
+    const int64_t cols = x.size(-1), pitch = row_pitch(x);
     const int rows = int32_size(x.numel() / cols), cols32 = int32_size(cols);
     Tensor q, s;
     int rc;
@@ -432,7 +451,7 @@ PyObject* quantize_per_token(PyObject*, PyObject* const* v, Py_ssize_t n) {
       const NoGil unlocked;
       q = c.empty(x.sizes(), ScalarType::Char);
       s = c.empty(with_last(x, 1), x.scalar_type());
-      rc = ti_quantize_per_token_absmax(ptr(x), dtype_code(x.scalar_type()), cols, (int8_t*)mptr(q), cols, mptr(s), rows, cols32, c.stream);
+      rc = ti_quantize_per_token_absmax(ptr(x), dtype_code(x.scalar_type()), pitch, (int8_t*)mptr(q), cols, mptr(s), rows, cols32, c.stream);
     }
     need(rc == TI_OK);
     PyObject* pair = PyTuple_New(2);

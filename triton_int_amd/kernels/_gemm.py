@@ -65,9 +65,9 @@ def linear(a, w, *, epilogue, out_dtype, bias=None, alpha=None, beta=None, out=N
     """Common body of the linear_* launchers (reference: kernels/linear.py:257-288 and siblings).  The ordinary
     call is one function of the extension module; what it declines is converted or refused here."""
     # the extension module takes scales as device tensors only, and a call that it declines has cost 1.7 us
-    if alpha.__class__ is float and a.is_cuda:
+    if alpha.__class__ in (float, int) and a.is_cuda:
         alpha = L.scale_tensor(alpha, a.device)
-    if beta.__class__ is float and a.is_cuda:
+    if beta.__class__ in (float, int) and a.is_cuda:
         beta = L.scale_tensor(beta, a.device)
     y = L.host.linear(a, w, bias, alpha, beta, out, epilogue, L.TORCH_TO_DT[out_dtype], round_mode, config, 0)
     if y is not None:
@@ -92,7 +92,7 @@ def linear(a, w, *, epilogue, out_dtype, bias=None, alpha=None, beta=None, out=N
 
 def bmm(a, b, *, b_is_kn, epilogue, out_dtype, alpha=None, out=None, round_mode=L.ROUND_RNE_CLAMP, config=-1):
     """Common body of the bmm_* launchers (reference: kernels/bmm.py:577-612 and siblings); as in `linear`."""
-    if alpha.__class__ is float and a.is_cuda:  # as in `linear`
+    if alpha.__class__ in (float, int) and a.is_cuda:  # as in `linear`
         alpha = L.scale_tensor(alpha, a.device)
     y = L.host.bmm(a, b, b_is_kn, alpha, out, epilogue, L.TORCH_TO_DT[out_dtype], round_mode, config)
     if y is not None:

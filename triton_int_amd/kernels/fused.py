@@ -167,6 +167,8 @@ def dq_add_layernorm_q(input_int32, input_scale_fp, residual_input_fp, gamma, be
 
 def gelu_q(x, scale, *, _round_mode=L.ROUND_RNE_CLAMP):
     """q8(gelu_tanh(x) * scale) element-wise, x fp32 -> int8 (math of kernels/fused.py:76-79)."""
+    if scale.__class__ in (float, int) and x.is_cuda:  # the module takes scales as device tensors only
+        scale = L.scale_tensor(scale, x.device)
     y = L.host.gelu_q(x, scale, _round_mode)
     if y is not None:
         return y

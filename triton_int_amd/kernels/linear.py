@@ -75,7 +75,7 @@ def linear_a8_w8_bfp32_ofp32_residual(a, b, bias, scale_a, scale_b, residual, ou
     `out` must not overlap `residual`."""
     if out is None:
         if a.is_cuda:  # the module takes scales as device tensors only
-            scale_a, scale_b = (L.scale_tensor(s, a.device) if s.__class__ is float else s for s in (scale_a, scale_b))
+            scale_a, scale_b = (L.scale_tensor(s, a.device) if s.__class__ in (float, int) else s for s in (scale_a, scale_b))
         y = L.host.linear_residual(a, b, bias, scale_a, scale_b, residual)
         if y is not None:
             return y
