@@ -306,9 +306,10 @@ int ti_transpose_i8(const int8_t* src, int64_t src_row_stride, int8_t* dst, int6
  * (`fc2(x) + residual` in a decoder layer):
  *     C[m][n] = (alpha * f(acc[m][n]) + beta * bias[n]) + residual[m][n]        fp32, rounded per step
  * A [M,K], W [N,K] int8 with unit column stride, bias fp32 [N] or NULL, residual and C fp32 with unit
- * column stride (row strides in elements).  With M <= 16 the weight-streaming decode kernel adds the
- * residual as it stores, and the persistent kernels that serve large outputs add it in their epilogue (one
- * launch instead of two); otherwise the GEMM is followed by an add kernel.
+ * column stride (row strides in elements).  The kernels for 64 rows and fewer add the residual as they store, and
+ * the persistent kernels that serve larger outputs add it in their epilogue, with K split in that of a tile's
+ * last item (one launch instead of two); the kernels with one tile per workgroup and the gather kernel are followed
+ * by an add kernel.
  * Same bits as the linear followed by an fp32 add.  C must not overlap the residual.
  */
 int ti_linear_i8_residual_f32(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const float* bias,
@@ -374,8 +375,8 @@ int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const in
  * The scalars are host floats.  The int8 scores are the BMM's and the probabilities ti_softmax_q's
  * bit for bit (a row's exponentials are summed as integers, so the order in which the keys are
  * visited does not matter): the output equals the three-launch chain's exactly.
- * Launches of few query rows (S <= 16, or batch * ceil(S / 16) <= 1024) against T <= 4096 keys run a one-pass kernel,
- * one to eight workgroups per batch entry and 16 rows.
+ * Launches of few query rows against T <= 4096 keys (S <= 16; more rows where up to 1024 groups of 16 take less time
+ * than blocks of 128) run a one-pass kernel, one to eight workgroups per batch entry and 16 rows.
  * The reference has no fused form (its modules stop at the BMMs, nn/bmm.py:10-74); the
  * three-launch chain remains available and is what this is tested against.
  */

@@ -9,7 +9,7 @@
 //   gemm_mfma_stream_kernel  persistent, loads issued by the MFMA waves (256x256 tiles, short K).
 //   gemm_mfma_kernel         one tile per workgroup; any output layout the fast loads allow.
 //   gemm_rowpieces_kernel    M <= 64: weight rows dealt evenly to the CUs, the whole K in one workgroup.
-//   gemm_rows4_kernel        M <= 16 against a few rows of a long K: weights as whole 1 KB row pieces.
+//   gemm_rows4_kernel        M <= 16, more than one round of weight rows: weights as whole 1 KB row pieces.
 //   gemm_skinny_kernel       M <= 64, batched or a short K: 16-row weight slabs in MFMA layout, K split over waves.
 //   gemm_ragged_kernel       rows that start at any byte, any K, [K,N] operands (unaligned loads through registers).
 //   gemm_gather_kernel       any strides (byte gathers).
@@ -3255,9 +3255,10 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       if (want_splits) return fail(TI_E_COMBO, "config %s: %d units per workgroup do not fit one pass with K split over %d waves", k.name, per, p.ksplit);
       p.ksplit = 1;
     }
-    // 6 or fewer units per workgroup: 6 streaming waves with 4 ring stages each instead of 8 with 3
-    // (weights rotated through > 600 MB: 5120 x 20480 28.6 -> 25.3 us, 4096 x 16384 24.0 -> 20.0 us,
-    // 4096 x 4096 10.0 -> 8.7 us; 4 waves with 6 stages: equal or slower than 6 with 4)
+    // 8 streaming waves: the choice of configuration comes here with more than 20 units per workgroup only.  The
+    // kernels of 6 and 4 waves serve launches that force this configuration for 6 units or fewer (6 waves with 4 ring
+    // stages each against 8 with 3, weights rotated through > 600 MB: 5120 x 20480 28.6 -> 25.3 us, 4096 x 16384 24.0 -> 20.0;
+    // 4 with 6 equal or slower), which gemm_rowpieces_kernel serves otherwise
     int nwa = want_nwa ? want_nwa : (p.ksplit == 1 && per <= 6 ? 6 : 8);
     if (nwa < 8 && per > nwa) return fail(TI_E_COMBO, "config %s: %d units per workgroup need more than %d waves", k.name, per, nwa);
     g_last_config = config;

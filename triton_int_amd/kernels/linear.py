@@ -69,9 +69,9 @@ def linear_a8_w8_bfp32_ofp32(a, b, bias, scale_a, scale_b, out=None, dtype=None,
 
 def linear_a8_w8_bfp32_ofp32_residual(a, b, bias, scale_a, scale_b, residual, out=None):
     """`linear_a8_w8_bfp32_ofp32(a, b, bias, scale_a, scale_b) + residual` in fp32 as one library call
-    (reference: kernels/linear.py:819-853 followed by the caller's add): with 16 or fewer rows the
-    decode kernel adds the residual while it stores, the persistent kernels that serve large outputs add it in
-    their epilogue, otherwise an add kernel follows the GEMM.
+    (reference: kernels/linear.py:819-853 followed by the caller's add): the kernels for 64 rows and fewer add the
+    residual while they store, the persistent kernels that serve larger outputs in their epilogue (split K
+    included); an add kernel follows the others.
     `out` must not overlap `residual`."""
     if out is None:
         if a.is_cuda:  # the module takes scales as device tensors only

@@ -18,7 +18,7 @@ end-to-end tests: every heavy step is one of the package's HIP kernels, torch on
       resid, h8 = DQ_Add_LayerNorm_Q(hidden, acc)           (ti_dq_add_layernorm_q)
       f8     = W8A8BFP32OFP32_GeLu_Q(h8) -> int8            (GEMM + GELU-quant epilogue)   fc1
       out    = W8A8BFP32OFP32Linear(f8) + resid -> fp32                                  fc2
-               (one library call, ti_linear_i8_residual_f32: in decode the GEMM kernel adds the residual)
+               (one library call, ti_linear_i8_residual_f32: the GEMM kernel adds the residual)
 """
 from __future__ import annotations
 
@@ -167,7 +167,7 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         v = qkv[..., 2 * H:]                                                       # [B,S,H] int8, row pitch 3H
         mark("qkv_3x_linear_o8")
         T = S if kv_cache is None else kv_cache[0].shape[1]
-        # short blocks of queries against up to 4096 keys run the attention kernel's one-pass form; a traced
+        # short blocks of queries against up to 4096 keys run the attention kernel too; a traced
         # forward keeps the three steps of blocks of 17 .. 127 apart so that they can be inspected
         short = T <= 4096 and (S <= 16 or _trace is None)
         fused = (self.fused_attention and (S >= self.fused_attention_min_queries or short) and D == 128 and self.score_scale > 0.0
