@@ -117,10 +117,10 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         heads, D, T = self.heads, self.head_dim, vt_all.shape[2]
         vs = vt_all.stride()
         if D % 16 == 0 and (k_all is None or k_all.stride(2) == 1) and vs[2] == 1 and (vs[0] == D * vs[1] or B * heads == 1):
-            n = self._at_once()
-            if B <= n:
+            if B * heads <= 32767 or B <= self._at_once():
                 kv_append_i8(k_new.view(B * S, H), v_new.view(B * S, H), k_all, vt_all, seqs=B)
                 return
+            n = self._at_once()
             for b in range(0, B, n):
                 hs = slice(b * heads, (b + n) * heads)
                 self._append(k_new[b:b + n], v_new[b:b + n], None if k_all is None else k_all[hs], vt_all[hs])
@@ -135,11 +135,11 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         return max(1, min(32767, 65535 // self.heads))
 
     @staticmethod
-    def _kernel_takes(k_all, vt_all):
+    def _kernel_takes(k_all, vt_all, T, D):
         """Whether the attention kernel takes caches that lie like this; the three-launch chain takes any."""
-        ks, vs, T = k_all.stride(), vt_all.stride(), vt_all.shape[2]
-        return (ks[2] == 1 and ks[1] >= k_all.shape[2] and (k_all.data_ptr() | ks[0] | ks[1]) % 16 == 0
-                and (vs[2] == 1 or T == 1) and vs[1] >= T)
+        kh, kr, kc = k_all.stride()
+        vr, vc = vt_all.stride()[1:]
+        return kc == 1 and kr >= D and (k_all.data_ptr() | kh | kr) % 16 == 0 and (vc == 1 or T == 1) and vr >= T
 
     @torch.no_grad()
     def forward(self, hidden, kv_cache=None, _trace=None, _mark=None):
@@ -171,7 +171,7 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         # forward keeps the three steps of blocks of 17 .. 127 apart so that they can be inspected
         short = T <= 4096 and (S <= 16 or _trace is None)
         fused = (self.fused_attention and (S >= self.fused_attention_min_queries or short) and D == 128 and self.score_scale > 0.0
-                 and (kv_cache is None or self._kernel_takes(*kv_cache)))
+                 and (kv_cache is None or self._kernel_takes(*kv_cache, T, D)))
         if kv_cache is None:
             # rows of V^T padded to a multiple of 16 bytes: the attention kernel reads them in 16-byte pieces
             vt_all = torch.empty((B * heads, D, (S + 15) // 16 * 16), dtype=torch.int8, device=hidden.device)[:, :, :S]
@@ -191,12 +191,14 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         if fused:
             # every operand as [B, heads, rows, D] views: all sequences in one launch, as far as one launch goes
             by_head = lambda t: t.view(B, S, heads, D).transpose(1, 2)
-            operands = (by_head(qkv[..., :H]), by_head(qkv[..., H:2 * H]) if kv_cache is None else k_all.unflatten(0, (B, heads)),
-                        vt_all.unflatten(0, (B, heads)), by_head(ctx))
-            n = self._at_once()
-            for b in range(0, B, n):
-                q4, k4, vt4, out4 = operands if B <= n else (t[b:b + n] for t in operands)
-                attention_i8(q4, k4, vt4, self.qk_alpha, self.score_scale, self.pv_alpha, causal_q_len=S if self.causal else 0, out=out4)
+            q4, k4 = by_head(qkv[..., :H]), by_head(qkv[..., H:2 * H]) if kv_cache is None else k_all.unflatten(0, (B, heads))
+            vt4, out4, causal = vt_all.unflatten(0, (B, heads)), by_head(ctx), S if self.causal else 0
+            n = B if B * heads <= 65535 else self._at_once()
+            if n == B:
+                attention_i8(q4, k4, vt4, self.qk_alpha, self.score_scale, self.pv_alpha, causal_q_len=causal, out=out4)
+            else:
+                for b in (slice(b, b + n) for b in range(0, B, n)):
+                    attention_i8(q4[b], k4[b], vt4[b], self.qk_alpha, self.score_scale, self.pv_alpha, causal_q_len=causal, out=out4[b])
             mark("attention_i8_fused")
         else:
             scores = bmm_s8t_s8n_s8t(q, k_all, self.qk_alpha)                       # [B*heads, S, T] int8
