@@ -563,8 +563,8 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
 // 3.5 us besides, or as long as 4 TB/s take for the caches of the heads in it (up to 256: each is then read again in the
 // next round); the blocks of 128 rows on attention_i8_kernel, all in one round, 2.4 us per 64 keys and 3.5 us besides
 // however few their rows.  128-row blocks beyond four rounds.
-// Measured (us, groups / blocks), 340 launches of 17 .. 512 rows against 16 .. 4096 keys, with and without a mask: the
-// estimate's choice is 0.4 % above the better one on average, and nowhere more than 3 % above the blocks.  Causal: 32 heads x 64
+// Measured (us, groups / blocks), 815 sizes of 17 .. 512 rows against 16 .. 4096 keys, with and without a mask: the
+// estimate's choice is 0.5 % above the better one on average, and nowhere more than 3 % above the blocks.  Causal: 32 heads x 64
 // rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 / 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81;
 // but 160 x 64 x 64 13.3 / 7.7, 80 x 192 x 256 19.3 / 15.0, 512 x 32 x 128 19.1 / 11.9, 256 x 64 x 2048 120 / 83, 512 x 17 x 1024
 // 59 / 48.  Beyond: 40 x 512 x 2048 (1280) 88 / 81, 320 x 64 x 2048 (1280) 145 / 113, 1280 x 17 x 2048 (2560) 298 / 269, 1280
