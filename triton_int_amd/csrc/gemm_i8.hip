@@ -2127,19 +2127,17 @@ constexpr int R4_NW = 8, R4_RG = 4, R4_KC = 1024, R4_PITCH = R4_KC + 16, R4_WPIT
               R4_UMAX = 4;
 
 // Four neighbouring outputs n0 .. n0+3 of row `row` from their int32 sums: converted and stored as one piece
-// where the output's layout allows.
+// where the output's layout allows.  col: the columns' terms (bits; EPI_I32: the int32 bias); resid: the four residuals, or null.
 template <int OUTCLS>
 __device__ __forceinline__ void store4(const EpiCtx& e, char* Cz, int64_t sCm, int64_t sCn, int N, int out_dtype, int row, int n0,
-                                       v4i a, const float* resid, int64_t resid_rs, int bz, const GemmParams* kp) {
+                                       v4i a, const unsigned (&col)[4], const float* resid, int bz, const GemmParams* kp) {
   constexpr int ESZ = OUTCLS == OUT8 ? 1 : (OUTCLS == OUT32 ? 4 : 2);
   unsigned b[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int n = min(n0 + i, N - 1);
-    const int bias_i32 = (e.epilogue == TI_EPI_I32 && e.bias_kind == TI_BIAS_I32) ? ((const int*)e.bias)[n] : 0;
-    b[i] = convert_one<OUTCLS>(e, a[i], column_term(e, n), bias_i32, out_dtype);
+    b[i] = convert_one<OUTCLS>(e, a[i], __uint_as_float(col[i]), (int)col[i], out_dtype);
     if constexpr (OUTCLS == OUT32) {
-      if (resid) b[i] = __float_as_uint(__uint_as_float(b[i]) + resid[(int64_t)row * resid_rs + n]);  // fp32 epilogues only (host)
+      if (resid) b[i] = __float_as_uint(__uint_as_float(b[i]) + resid[i]);  // fp32 epilogues only (host)
     }
   }
   char* dst = Cz + ((int64_t)row * sCm + (int64_t)n0 * sCn) * ESZ;
@@ -2193,7 +2191,15 @@ __device__ __attribute__((noinline)) void rows4_store_tile(const EpiCtx e, char*
   if (!(row < M && unit < u_end && grp < max_units)) return;
   const unsigned addr = tile0 + (row >> 1) * RING + (row & 1) * 2048 + grp * 16;
   const v4i a = *(const __attribute__((address_space(3))) v4i*)(uintptr_t)addr;
-  store4<OUTCLS>(e, Cz, sCm, sCn, N, out_dtype, row, unit * R4_RG, a, resid, resid_rs, bz, kp);
+  unsigned col[4];
+  float res[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int n = min(unit * R4_RG + i, N - 1);
+    col[i] = e.epilogue == TI_EPI_I32 ? (e.bias_kind == TI_BIAS_I32 ? ((const unsigned*)e.bias)[n] : 0u) : __float_as_uint(column_term(e, n));
+    res[i] = OUTCLS == OUT32 && resid ? resid[(int64_t)row * resid_rs + n] : 0.0f;
+  }
+  store4<OUTCLS>(e, Cz, sCm, sCn, N, out_dtype, row, unit * R4_RG, a, col, resid ? res : nullptr, bz, kp);
 }
 
 template <int OUTCLS, int NWA, int NST>
@@ -2402,17 +2408,89 @@ __host__ __device__ __forceinline__ void with_count(int n, F f) {
   f(std::integral_constant<int, MAX>{});
 }
 
-template <int OUTCLS>
-__device__ __attribute__((noinline)) void rowpieces_store(const EpiCtx e, char* Cz, int64_t sCm, int64_t sCn, int M, int N, int out_dtype,
-                                                         unsigned red, int wave_bytes, int gu, int tid, int n_first, int units,
-                                                         const float* resid, int64_t resid_rs, int bz, const GemmParams* kp) {
-  for (int idx = tid; idx < M * units; idx += (RP_PW + RP_CW) * 64) {
-    const int m = idx / units, u = idx - m * units;
-    const unsigned addr = red + (((m >> 4) * gu + u) * 17 + (m & 15)) * 16;
-    v4i a = {0, 0, 0, 0};
+// What the store phase of gemm_rowpieces_kernel reads besides the sums, fetched by the consumer waves before their first stage:
+// consumer thread t stores items t, t + 256, ... of the workgroup's (row, unit) pairs.  The first stage lands about 3 us
+// after a workgroup's start, so these reads cost nothing there; after the last stage the chain scales (cold scalar loads) ->
+// bias -> residual took 2.2 us (now 0.7): 1 x 5120 x 5120 9.0 -> 7.5 us, 1 x 20480 x 5120 20.1 -> 18.6, 16 x 4096 x 16384 15.4 ->
+// 13.8, 64 x 4096 x 4096 10.2 -> 8.9, 64 x 16384 x 4096 17.0 -> 16.5.
+template <int J>
+struct RowpiecesPre {
+  int at[J];            // row << 8 | unit
+  unsigned col[J][4];   // beta * bias as fp32 bits (EPI_I32: the int32 bias)
+  float resid[J][4];
+};
+
+template <int J>
+__device__ __forceinline__ void rowpieces_prefetch(RowpiecesPre<J>& r, const GemmParams& p, const EpiCtx& e, int tid, int n_first, int units) {
+  const int total = p.M * units;
+  int n[J][4];
 #pragma unroll
-    for (int w = 0; w < RP_CW; ++w) a += *(const __attribute__((address_space(3))) v4i*)(uintptr_t)(addr + w * wave_bytes);
-    store4<OUTCLS>(e, Cz, sCm, sCn, N, out_dtype, m, n_first + 4 * u, a, resid, resid_rs, bz, kp);
+  for (int j = 0; j < J; ++j) {
+    const int idx = min(tid + j * RP_CW * 64, total - 1), m = idx / units, u = idx - m * units;
+    r.at[j] = m << 8 | u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) n[j][i] = min(n_first + 4 * u + i, p.N - 1);
+  }
+  // the branch on the bias type is outside the loops, so that all loads are issued before the first is waited for
+  const auto fetch = [&](auto element) {
+    using T = decltype(element);
+    const T* bias = (const T*)e.bias;
+    T b[J][4];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[j][i] = bias[n[j][i]];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float f;
+        if constexpr (std::is_same<T, uint16_t>::value) f = __uint_as_float((unsigned)b[j][i] << 16);  // bf16
+        else f = (float)b[j][i];
+        r.col[j][i] = __float_as_uint(e.epilogue == TI_EPI_GELU_I8 ? f : f * e.beta);
+        if constexpr (std::is_same<T, int32_t>::value) {
+          if (e.epilogue == TI_EPI_I32) r.col[j][i] = (unsigned)b[j][i];
+        }
+      }
+  };
+  float res[J][4];
+  if (p.resid) {
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) res[j][i] = p.resid[(int64_t)(r.at[j] >> 8) * p.resid_rs + n[j][i]];
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.col[j][i] = 0;
+  switch (e.bias_kind) {
+    case TI_BIAS_I8: fetch(int8_t{}); break;
+    case TI_BIAS_I32: fetch(int32_t{}); break;
+    case TI_BIAS_F32: fetch(float{}); break;
+    case TI_BIAS_F16: fetch(_Float16{}); break;
+    case TI_BIAS_BF16: fetch(uint16_t{}); break;
+    default: break;
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.resid[j][i] = p.resid ? res[j][i] : 0.0f;
+}
+
+template <int OUTCLS, int J>
+__device__ __forceinline__ void rowpieces_store(const GemmParams& p, const EpiCtx& e, const RowpiecesPre<J>& r, char* Cz, unsigned red,
+                                                int wave_bytes, int gu, int tid, int n_first, int units, int bz, const GemmParams* kp) {
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    if (tid + j * RP_CW * 64 < p.M * units) {
+      const int m = r.at[j] >> 8, u = r.at[j] & 255;
+      const unsigned addr = red + (((m >> 4) * gu + u) * 17 + (m & 15)) * 16;
+      v4i a = {0, 0, 0, 0};
+#pragma unroll
+      for (int w = 0; w < RP_CW; ++w) a += *(const __attribute__((address_space(3))) v4i*)(uintptr_t)(addr + w * wave_bytes);
+      store4<OUTCLS>(e, Cz, p.sCm, p.sCn, p.N, p.out_dtype, m, n_first + 4 * u, a, r.col[j], p.resid ? r.resid[j] : nullptr, bz, kp);
+    }
   }
 }
 
@@ -2508,8 +2586,14 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     with_count<MT == 16 ? A_MAX / 4 : A_MAX, A_MAX>(mine_a, [&](auto a_tag) {
       with_count<W_MIN, W_MAX>((pieces_w - first_w + RP_PW - 1) / RP_PW, [&](auto w_tag) { produce(a_tag, w_tag); });
     });
+    asm volatile("s_barrier" ::: "memory");  // the consumers' exchange of sums
   } else {
     const int r16 = lane & 15, c4 = lane >> 4;
+    // scales, bias and residual now, under the wait for the first stage, and not after the last one
+    constexpr int J = (MT * 4 * G + RP_CW * 64 - 1) / (RP_CW * 64);
+    const EpiCtx e = make_epi(p, bz);
+    RowpiecesPre<J> pre;
+    rowpieces_prefetch<J>(pre, p, e, tid, n0, units);
     v4i acc[G][MB];
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -2563,15 +2647,14 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     for (int m = 0; m < MB; ++m)
 #pragma unroll
       for (int g = 0; g < G; ++g) *(v4i*)(red + ((m * 4 * G + g * 4 + c4) * 17 + r16) * 16) = acc[g][m];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const GemmParams* kp = (const GemmParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    const int esz = p.out_dtype == TI_I8 ? 1 : ((p.out_dtype == TI_F16 || p.out_dtype == TI_BF16) ? 2 : 4);
+    char* Cz = (char*)p.C + (int64_t)bz * p.sCb * esz;
+    if (esz == 1) rowpieces_store<OUT8, J>(p, e, pre, Cz, lds_base, WAVE_RED, 4 * G, tid, n0, units, bz, kp);
+    else if (esz == 2) rowpieces_store<OUT16, J>(p, e, pre, Cz, lds_base, WAVE_RED, 4 * G, tid, n0, units, bz, kp);
+    else rowpieces_store<OUT32, J>(p, e, pre, Cz, lds_base, WAVE_RED, 4 * G, tid, n0, units, bz, kp);
   }
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  const EpiCtx e = make_epi(p, bz);
-  const GemmParams* kp = (const GemmParams*)__builtin_amdgcn_kernarg_segment_ptr();
-  const int esz = p.out_dtype == TI_I8 ? 1 : ((p.out_dtype == TI_F16 || p.out_dtype == TI_BF16) ? 2 : 4);
-  char* Cz = (char*)p.C + (int64_t)bz * p.sCb * esz;
-  if (esz == 1) rowpieces_store<OUT8>(e, Cz, p.sCm, p.sCn, p.M, p.N, p.out_dtype, lds_base, WAVE_RED, 4 * G, tid, n0, units, nullptr, 0, bz, kp);
-  else if (esz == 2) rowpieces_store<OUT16>(e, Cz, p.sCm, p.sCn, p.M, p.N, p.out_dtype, lds_base, WAVE_RED, 4 * G, tid, n0, units, nullptr, 0, bz, kp);
-  else rowpieces_store<OUT32>(e, Cz, p.sCm, p.sCn, p.M, p.N, p.out_dtype, lds_base, WAVE_RED, 4 * G, tid, n0, units, p.resid, p.resid_rs, bz, kp);
 }
 
 // ---- host side ---------------------------------------------------------------------------------
