@@ -1,0 +1,44 @@
+"""The choice of tile and K splits for 65 and more rows: what it plans stays inside its operands, and launches agree with float64."""
+import pytest
+import torch
+
+from tests import gemm_bounds_model as G
+from triton_int_amd import _lib as L
+
+# one row past 64, edges of the 64-, 128- and 256-row tiles, K just beyond 1024 and no multiple of a k-tile, few and many columns
+SIZES = [(1, 65, 4096, 1040), (1, 100, 4096, 4096), (1, 129, 304, 16384), (1, 200, 1024, 4096), (1, 257, 512, 20480), (1, 384, 4096, 4080),
+         (1, 1000, 1024, 4096), (3, 100, 1024, 2048), (4, 65, 272, 1536), (1, 513, 6848, 1520)]
+
+
+@pytest.mark.parametrize("B,M,N,K", SIZES)
+def test_planned_launches(B, M, N, K):
+    lib = L.lib()
+    for epi, dt, bias in ((L.EPI_SCALE_I8, 0, 1), (L.EPI_SCALE_F, 2, 3), (L.EPI_SCALE_F, 3, 3)):
+        pr = G.contiguous(B, M, N, K, dt)
+        pl = G.plan_for(lib, pr, epi, bias)
+        assert pl.name.startswith("ws_") and (B == 1 or pl.splits == 1)
+        G.check_launch(pr, pl, store_sample=12)
+        G.check_launch(pr, G.plan_for(lib, pr, epi, bias, static_scratch=1), store_sample=4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,K", SIZES)
+def test_outputs(B, M, N, K):
+    from triton_int_amd.kernels.linear import linear_a8_w8_b32_o32, linear_a8_w8_b8_o8, linear_a8_w8_bfp32_ofp32, linear_group_a8_w8_b8_o8
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    a = torch.randint(-127, 128, (M, K), dtype=torch.int8, device=dev, generator=g)
+    w = torch.randint(-127, 128, (B * N, K), dtype=torch.int8, device=dev, generator=g)
+    acc = a.double() @ w.double().t()  # exact: below 2^53
+    b8 = torch.randint(-127, 128, (B * N,), dtype=torch.int8, device=dev, generator=g)
+    al, be = torch.tensor(2.0e-4, device=dev), torch.tensor(0.5, device=dev)
+    want = (b8.float() * be + acc.float() * al).round().clamp(-128, 127).to(torch.int8)
+    if B > 1:
+        got = linear_group_a8_w8_b8_o8(a, w, b8, al.repeat(B), be.repeat(B), B)
+        assert torch.equal(got, want)
+        return
+    assert torch.equal(linear_a8_w8_b8_o8(a, w, b8, al, be), want)
+    assert torch.equal(linear_a8_w8_b32_o32(a, w, None).double(), acc)
+    bias = torch.randn(N, device=dev, generator=g)
+    for dt in (torch.float32, torch.float16):
+        assert torch.equal(linear_a8_w8_bfp32_ofp32(a, w, bias, al, be, dtype=dt), (bias * be + acc.float() * al).to(dt))

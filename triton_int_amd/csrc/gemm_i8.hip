@@ -2871,6 +2871,8 @@ static bool kn_eligible(const GemmParams& p) {
   return stream_stores(p);
 }
 
+constexpr size_t SK_MAX_PARTIAL_BYTES = (size_t)96 << 20;  // split-K workspace: < 2 GiB, the kernel addresses it with 32-bit offsets
+
 // k-tiles per split and the number of non-empty splits for `want` splits of a K of `kt` k-tiles
 static void sk_shape(int kt, int want, int& splits, int& kt_split) {
   want = want < 1 ? 1 : (want > kt ? (kt > 0 ? kt : 1) : want);
@@ -2929,6 +2931,54 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
   }
   if (cost_out) *cost_out = cost;
   return used;
+}
+
+// Time in us of a GEMM with K > 1024 on a wave-specialised configuration in `want` K splits: a round of items costs its
+// k-tiles (`tile` each, and `busy` more the more of the chip works on outputs that exist: that part is power and
+// shared memory), `item` and `out` once (pipeline fill, epilogue, stores), the weights their bytes at 5 TB/s times
+// `mem`, a split the exchange of its sums.  Least squares over 8044 launches: M = 65 .. 3000, 24
+// shapes of N and K from 256 to 20480, one GEMM and three grouped, int8 and fp32 outputs, every tile in 1, 2, 3, 4, 6 and 8
+// splits, weights from HBM.  Over those 648 sizes its choice is 1.3 % above the fastest on average; the estimate it replaces,
+// which knew neither the 64-row tile beyond 128 rows nor splits shorter than 2560 bytes of K, was 10.4 % above.  us, that one /
+// this: 100 x 4096 x 4096 16.2 / 11.5, 200 x 4096 x 4096 21.9 / 13.8, 384 x 4096 x 4096 21.2 / 16.7, 300 x 1024 x 4096 15.0 / 10.0, 128 x
+// 20480 x 5120 48 / 34, 160 x 5120 x 5120 25.2 / 16.1, 1000 x 5120 x 20480 122 / 102, three grouped 100 x 4096 x 4096 20.7 / 17.3.
+// Where it loses (3 % and more at 23 of them): 384 x 2048 x 2048 9.1 / 10.2, 140 x 4096 x 11008 22.0 / 24.4.
+// K <= 1024 is left to config_cost: the rounds there are mostly epilogue.
+struct WsCost {
+  int cfg;
+  double start, tile, busy, out8, out4, split, per_split, item, mem, sums;
+};
+
+static double ws_time(const GemmParams& p, const Config& k, const WsCost& c, int want, int& splits) {
+  const int64_t tiles = (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bn - 1) / k.bn);
+  int kts;
+  sk_shape((p.K + k.bk - 1) / k.bk, want, splits, kts);
+  const int64_t items = tiles * p.batch * splits, rounds = (items + 255) / 256;
+  const double filled = (double)items / 256.0, real = (double)p.M * p.N / ((double)tiles * k.bm * k.bn);
+  return c.start + kts * (rounds * c.tile + filled * real * c.busy) + rounds * (out_class(p.out_dtype) == OUT8 ? c.out8 : c.out4) +
+         (splits > 1 ? c.split + splits * (c.per_split + filled * c.sums) : 0.0) + filled * c.item + (double)p.N * p.K * p.batch / 5e6 * c.mem;
+}
+
+static int pick_ws(const GemmParams& p, int* splits_out) {
+  static const WsCost costs[] = {
+      {CFG_WS_64x128, 1.495, 0.227, 0.122, 2.583, 2.809, 1.722, 0.216, 0.000, 0.587, 0.342},
+      {CFG_WS_128x128, 0.000, 0.292, 0.180, 3.614, 4.137, 2.237, 0.240, 0.000, 0.642, 0.764},
+      {CFG_WS_256x128, 0.000, 0.438, 0.252, 4.620, 5.677, 2.824, 0.393, 0.000, 0.581, 1.467},
+      {CFG_WS_256x160, 0.000, 0.526, 0.292, 9.049, 6.328, 3.050, 0.730, 0.825, 0.520, 1.645},
+  };
+  int best = CFG_WS_128x128;
+  double best_time = -1.0;
+  for (const WsCost& c : costs) {
+    const Config& k = g_configs[c.cfg];
+    const int64_t tiles = (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bn - 1) / k.bn);
+    for (int want : {1, 2, 3, 4, 6, 8}) {
+      if (want > 1 && (p.batch != 1 || tiles * want > 520 || p.K < 384 * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
+      int splits;
+      const double t = ws_time(p, k, c, want, splits);
+      if (best_time < 0 || t < best_time) best_time = t, best = c.cfg, *splits_out = splits;
+    }
+  }
+  return best;
 }
 
 // Tile and K splits of gemm_ragged_kernel.  A k-tile costs a workgroup 0.5-0.8 us of load latency whatever else the chip
@@ -3023,14 +3073,14 @@ static int pick_config(const GemmParams& p, int* splits_out) {
   }
   // batched, few rows (attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
   if (p.M <= 16) return (p.N + 31) / 32 >= 160 ? CFG_SKINNY_16_G2 : CFG_SKINNY_16;
-  if (p.M <= 128 && stream && p.batch == 1 && (p.K >= 1024 || p.M <= 64)) {
+  if (stream && p.M > 64 && p.K > 1024 && p.batch <= 4) return pick_ws(p, splits_out);
+  if (p.M <= 64 && stream && p.batch == 1) {
     // a few rows against a long K: the GEMM is a read of the weight matrix, and what decides its speed is how
     // many weight bytes a CU keeps in flight.  K is split over enough workgroups to have every CU pulling its
     // own slab, and the tile has no more activation rows than needed, so that the LDS holds more stages of
     // weights: 32 x 128 tiles with 7 stages up to 32 rows, 64 x 128 with 6 stages beyond (a 128 x 128 tile has
     // room for 4).  Measured in steady state, weights rotated through 350 MB, N = 6848, K = 10240, against
-    // the 128 x 128 tile: M = 17 .. 32 34 -> 22-23 us, M = 64 35 -> 28.5 us, M = 128 38 -> 33 us; N = K = 5120:
-    // 18.5-19 -> 15-16 us, M = 128 20.4 -> 16.6 us.
+    // the 128 x 128 tile: M = 17 .. 32 34 -> 22-23 us, M = 64 35 -> 28.5 us; N = K = 5120: 18.5-19 -> 15-16 us.
     const int cfg = p.M <= 32 ? CFG_WS_32x128 : CFG_WS_64x128;
     *splits_out = pick_splits(p, g_configs[cfg], 1.0, nullptr);
     return cfg;
@@ -3140,7 +3190,6 @@ static thread_local int g_last_splits = 1;
 // so they can share it; launches on different streams may overlap and get their own.  It grows on
 // demand.
 constexpr size_t SK_COUNTER_INTS = 1 << 16;             // tiles x consumer waves of one launch
-constexpr size_t SK_MAX_PARTIAL_BYTES = (size_t)96 << 20;  // < 2 GiB: the kernel addresses it with 32-bit offsets
 struct SkWorkspace { int dev; hipStream_t stream; char* base; size_t partial_bytes; std::vector<char*> outgrown; };
 static std::mutex g_sk_mutex;
 static std::vector<SkWorkspace> g_sk_ws;
