@@ -110,14 +110,15 @@ class _MissingHost:
         self._error = error
 
     def __getattr__(self, name):
-        raise RuntimeError(f"triton_int_amd._host cannot be loaded ({self._error}): build it with "
+        raise RuntimeError(f"triton_int_amd._host or _layer_host cannot be loaded ({self._error}): build it with "
                            "`python -m triton_int_amd.build` (g++, hipcc, gfx950)")
 
 
 try:
     from . import _host as host  # the launchers' host path; its functions return None for what is not the ordinary case
+    from . import _layer_host as layer_host  # the same for a whole decoder layer
 except ImportError as e:
-    host = _MissingHost(e)
+    host = layer_host = _MissingHost(e)
 
 
 def lib() -> ctypes.CDLL:

@@ -1,5 +1,6 @@
 """Builds libtriton_int_hip.so (gfx950 only) from triton_int_amd/csrc/*.hip with hipcc, and the extension
-module _host.so (the launchers' host path, csrc/host.cpp, against torch's headers) with g++.
+modules _host.so and _layer_host.so (the host path of launchers and decoder layer, csrc/host*.cpp, against torch's headers)
+with g++.
 
     python -m triton_int_amd.build
 
@@ -21,8 +22,7 @@ OBJ_DIR = os.path.join(HERE, "_obj")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libtriton_int_hip.so")
 
-HOST_SRC = os.path.join(CSRC, "host.cpp")
-HOST_PATH = os.path.join(HERE, "_host.so")
+HOST_MODULES = {"host.cpp": os.path.join(HERE, "_host.so"), "host_layer.cpp": os.path.join(HERE, "_layer_host.so")}
 
 SOURCES = ["lib.hip", "gemm_i8.hip", "rowops.hip", "attention_i8.hip", "quant.hip", "layernorm_fp.hip"]
 
@@ -46,7 +46,7 @@ def _compile(src: str) -> str:
     return obj
 
 
-def _build_host() -> None:
+def _build_host(src: str) -> None:
     import torch
 
     root = os.path.dirname(torch.__file__)
@@ -57,11 +57,11 @@ def _build_host() -> None:
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-isystem{d}" for d in (os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                                       os.path.join(rocm, "include"), sysconfig.get_paths()["include"])),
-           HOST_SRC, "-o", HOST_PATH, f"-L{os.path.join(root, 'lib')}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu",
+           os.path.join(CSRC, src), "-o", HOST_MODULES[src], f"-L{os.path.join(root, 'lib')}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu",
            "-lc10_hip", "-lc10", f"-L{LIB_DIR}", "-l:libtriton_int_hip.so", "-Wl,-rpath,$ORIGIN/lib"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{r.stderr}")
+        raise RuntimeError(f"{cmd[0]} failed on {src}:\n{r.stderr}")
     if r.stderr.strip():
         sys.stderr.write(r.stderr + "\n")
 
@@ -76,7 +76,8 @@ def build(verbose: bool = True) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
-    _build_host()
+    with concurrent.futures.ThreadPoolExecutor(max_workers=len(HOST_MODULES)) as ex:
+        list(ex.map(_build_host, HOST_MODULES))
     if verbose:
         print(f"built {LIB_PATH} ({os.path.getsize(LIB_PATH) // 1024} KiB)")
     return LIB_PATH

@@ -23,7 +23,9 @@ end-to-end tests: every heavy step is one of the package's HIP kernels, torch on
 from __future__ import annotations
 
 import torch
+from torch.nn.modules import module as _torch_module
 
+from .. import _lib as L
 from ..kernels.bmm import bmm_s8t_s8n_s8t
 from ..kernels.fused import attention_i8, kv_append_i8, softmax_q, transpose_i8
 from ..kernels.linear import linear_group_a8_w8_b8_o8, linear_qkv_decode_a8_w8_b8_o8
@@ -141,14 +143,25 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         vr, vc = vt_all.stride()[1:]
         return kc == 1 and kr >= D and (k_all.data_ptr() | kh | kr) % 16 == 0 and (vc == 1 or T == 1) and vr >= T
 
-    @torch.no_grad()
     def forward(self, hidden, kv_cache=None, _trace=None, _mark=None):
         """hidden fp32 [B,S,H].  kv_cache = (K int8 [B*heads, T, D], V^T int8 [B*heads, D, T]) holds the
         T-S earlier positions in its first T-S slots; the S new positions are written into the last S
         slots before attention (decode / chunked prefill).  Returns fp32 [B,S,H].  A dict passed as
         `_trace` receives every intermediate tensor (for stage-by-stage parity tests); a callable
         passed as `_mark` is called with a stage name after that stage's launches (for timing the
-        stages in sequence with stream events)."""
+        stages in sequence with stream events).
+
+        The ordinary call is one function of the extension module, which makes the launches below from the modules' buffers
+        (csrc/host_layer.cpp); what it declines (hooks on a module, other module types, caches that need a copy)
+        runs step by step."""
+        if _trace is None and _mark is None and self.head_dim == 128 and self.fused_attention:
+            out = L.layer_host.decoder_layer(self, hidden, kv_cache, _TYPES, _GLOBAL_HOOKS)
+            if out is not None:
+                return out
+        return self._forward_steps(hidden, kv_cache, _trace, _mark)
+
+    @torch.no_grad()
+    def _forward_steps(self, hidden, kv_cache, _trace, _mark):
         mark = _mark if _mark is not None else (lambda name: None)
         B, S, H = hidden.shape
         h8 = self.ln1(hidden)
@@ -231,3 +244,10 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
             _trace.update(h8=h8, q=q, k_all=k_all, vt_all=vt_all, scores=scores, probs=probs, ctx=ctx, acc=acc,
                           resid=resid, h8b=h8b, f8=f8, fc2=y, out=out)
         return out
+
+
+# What the extension module's function stands for: exactly these types, nothing hooked into any module
+_TYPES = (W8A8OPTDecoderLayer, LayerNormQ, W8A8B8O8Linear, W8A8B8O8Linear, W8A8B8O8Linear, W8A8B32O32LinearWithoutScaling, DQ_Add_LayerNorm_Q,
+          W8A8BFP32OFP32_GeLu_Q, W8A8BFP32OFP32Linear)
+_GLOBAL_HOOKS = tuple(getattr(_torch_module, name) for name in ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
+                                                                "_global_backward_pre_hooks"))
