@@ -343,6 +343,30 @@ int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t
                           int64_t vt_row_stride, int D, void* stream);
 
 /*
+ * The same with the LayerNormQ in front in the same launch: x fp32 [M, K], unit column stride, row stride in elements, gamma
+ * and beta (may be NULL) as ti_layernorm_q takes them.  The bits are those of ti_layernorm_q followed by the call above.  At
+ * most 4 rows, 1024 <= K <= 5120, 16-byte aligned rows; TI_E_COMBO, with nothing done, for everything else (the
+ * caller makes the two calls).
+ */
+int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const float* gamma, const float* beta, float eps,
+                                    const int8_t* W, int64_t ldw, const int8_t* bias, const float* alpha3, const float* beta3,
+                                    int8_t* C, int64_t ldc, int seqs, int M, int N, int K, int8_t* k_dst,
+                                    int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride, int D,
+                                    void* stream);
+
+/*
+ * ti_dq_add_layernorm_q (kernels/fused.py:235-382 behind nn/fused.py:59-78) and the GELU-quant linear on its int8 rows
+ * (kernels/fused.py:197-231) as one launch: resid_out = resid + in_scale * acc, C = q8(gelu(scale_a * (LN(resid_out) . W) + bias) *
+ * scale_b).  Limits and TI_E_COMBO as above.
+ */
+int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_stride, float in_scale, const float* resid,
+                                       int64_t resid_row_stride, const float* gamma, const float* beta, float eps,
+                                       float* resid_out, int64_t resid_out_row_stride, const int8_t* W, int64_t ldw,
+                                       const float* bias, const float* scale_a, const float* scale_b, int8_t* C, int64_t ldc,
+                                       int M, int N, int K, void* stream);
+
+
+/*
  * Appends S new positions to an int8 KV cache in one launch: K [S, heads*D] (row stride
  * k_src_row_stride) is copied to k_dst[h][s][d] = k_dst + h * k_head_stride + s * D + d (k_dst points at
  * the first new slot of head 0 in a [heads, T, D] cache, k_head_stride = T * D), and V [S, heads*D]

@@ -35,6 +35,20 @@ __device__ unsigned long long g_timeline[1024 * 8];
 #define TI_TL(slot) do { } while (0)
 #endif
 
+// The LayerNorm that makes a GEMM's activations (gemm_rowpieces_kernel): rows x, or acc * in_scale + resid (written to
+// resid_out), normalised and quantised as in rownorm_vec_kernel.
+enum NormKind { NORM_NONE = 0, NORM_LN, NORM_DQ_ADD_LN };
+struct NormArgs {
+  int kind = NORM_NONE;
+  const float* x;  // NORM_DQ_ADD_LN: the residual
+  const int32_t* acc;
+  float* resid_out;
+  int64_t x_rs, acc_rs, rout_rs;
+  const float* gamma;
+  const float* beta;
+  float in_scale, eps;
+};
+
 struct GemmParams {
   const int8_t* A;
   const int8_t* B;
@@ -68,6 +82,7 @@ struct GemmParams {
   int splits, kt_split;
   int* sk_partial;   // [tile][split][consumer wave][accumulator dword][lane]
   int* sk_counter;   // [tile][consumer wave], zero between launches
+  NormArgs norm;
 };
 
 enum OutClass { OUT8 = 0, OUT32 = 1, OUT16 = 2 };
@@ -2494,7 +2509,110 @@ __device__ __forceinline__ void rowpieces_store(const GemmParams& p, const EpiCt
   }
 }
 
-template <int MT, int G, int KC>
+// The activations of up to RPN_ROWS rows from their LayerNorm (p.norm), by the consumer waves of every workgroup, while the
+// producers fill the stages with weights: int8 rows of `pitch` bytes at x8.  The statistics are those of rownorm_vec_kernel (256
+// threads, the same order of every sum), so the bits are too.  `red`: 2 x RPN_ROWS x RP_CW floats.
+// Joins two barriers; the caller's next one publishes x8.
+constexpr int RPN_ROWS = 4, RPN_K = 5120;  // more of either do not fit the registers
+template <int KIND, int VPT>
+__device__ __forceinline__ void rowpieces_norm(const GemmParams& p, char* x8, int pitch, float* red, int tid, bool store_resid) {
+  static_assert(RP_CW * 64 == 256, "the threads of rownorm_vec_kernel");
+  const NormArgs& a = p.norm;
+  const unsigned bytes = (unsigned)p.K * 4u;
+  const auto rsrc = [](const void* row, unsigned n) { return __builtin_amdgcn_make_buffer_rsrc((void*)row, 0, (int)n, 0x00020000); };
+  const auto load = [](__amdgpu_buffer_rsrc_t r, int vec) { return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, vec * 16, 0, 0)); };
+  v4f x[RPN_ROWS][VPT], w[VPT], b[VPT];
+  v4i acc[KIND == NORM_DQ_ADD_LN ? RPN_ROWS : 1][VPT];
+#pragma unroll
+  for (int r = 0; r < RPN_ROWS; ++r) {
+    // a row past the last has an empty descriptor: zeros, no memory touched
+    const __amdgpu_buffer_rsrc_t rx = rsrc(a.x + (int64_t)(r < p.M ? r : 0) * a.x_rs, r < p.M ? bytes : 0u);
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) x[r][j] = load(rx, tid + j * 256);
+    if constexpr (KIND == NORM_DQ_ADD_LN) {
+      const __amdgpu_buffer_rsrc_t ra = rsrc(a.acc + (int64_t)(r < p.M ? r : 0) * a.acc_rs, r < p.M ? bytes : 0u);
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) acc[r][j] = __builtin_bit_cast(v4i, load(ra, tid + j * 256));
+    }
+  }
+  const bool has_b = a.beta != nullptr;
+  const __amdgpu_buffer_rsrc_t rg = rsrc(a.gamma, bytes), rb = rsrc(a.beta, has_b ? bytes : 0u);
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) w[j] = load(rg, tid + j * 256), b[j] = load(rb, tid + j * 256);
+  const float inv_n = 1.0f / (float)p.K;
+  const int nvec = p.K >> 2, wave = tid >> 6;
+  float mean[RPN_ROWS], rstd[RPN_ROWS];
+  const auto put = [&](float v, int set, int r) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if ((tid & 63) == 0) red[(set * RPN_ROWS + r) * RP_CW + wave] = v;
+  };
+  const auto total = [&](int set, int r) {
+    const float* q = red + (set * RPN_ROWS + r) * RP_CW;
+    float t = q[0];
+#pragma unroll
+    for (int i = 1; i < RP_CW; ++i) t += q[i];
+    return t;
+  };
+#pragma unroll
+  for (int r = 0; r < RPN_ROWS; ++r) {
+    if (r >= p.M) break;
+    if constexpr (KIND == NORM_DQ_ADD_LN) {
+      const __amdgpu_buffer_rsrc_t ro = rsrc(a.resid_out + (int64_t)r * a.rout_rs, store_resid ? bytes : 0u);
+#pragma unroll
+      for (int j = 0; j < VPT; ++j) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float prod = a.in_scale * (float)acc[r][j][t];
+          x[r][j][t] = x[r][j][t] + prod;
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, x[r][j]), ro, (tid + j * 256) * 16, 0, 0);
+      }
+    }
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) s += (x[r][j][0] + x[r][j][1]) + (x[r][j][2] + x[r][j][3]);
+    put(s, 0, r);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int r = 0; r < RPN_ROWS; ++r) {
+    if (r >= p.M) break;
+    mean[r] = total(0, r) * inv_n;
+    float m2 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      if (tid + j * 256 < nvec) {
+        const float d0 = x[r][j][0] - mean[r], d1 = x[r][j][1] - mean[r], d2 = x[r][j][2] - mean[r], d3 = x[r][j][3] - mean[r];
+        m2 += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+      }
+    }
+    put(m2, 1, r);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int r = 0; r < RPN_ROWS; ++r) {
+    if (r >= p.M) break;
+    const float var = total(1, r) * inv_n;
+    rstd[r] = 1.0f / sqrtf(var + a.eps);
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+      const int v = tid + j * 256;
+      if (v < nvec) {
+        int q[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          float o = ((x[r][j][t] - mean[r]) * rstd[r]) * w[j][t];
+          if (has_b) o = o + b[j][t];
+          q[t] = q8(o, TI_ROUND_RNE_CLAMP);
+        }
+        *(unsigned*)(x8 + r * pitch + v * 4) = pack4(q[0], q[1], q[2], q[3]);
+      }
+    }
+  }
+}
+
+template <int MT, int G, int KC, int NORM = NORM_NONE, int VPT = 1>
 __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(GemmParams p) {
   constexpr int MB = MT / 16, CH = KC / 16, RPI = 1024 / KC;        // RPI: rows per load instruction
   constexpr int KPW = KC / 64 / RP_CW;                              // 64-deep k-steps of a consumer wave per stage
@@ -2518,11 +2636,20 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
   // A stage holds the 1 KB pieces that have rows, one after the other: the activations' (whole groups of four rows; with
   // more than 16 rows, all MT of them), then the weights'.  What the operand reads take beyond a stage's pieces belongs to sums that
   // are never stored.
-  const int pieces_a = MT == 16 ? (p.M + 3) / 4 * 4 / RPI : MT / RPI, pieces_w = per * 4 / RPI;
+  // With a norm the activations lie in LDS as a whole, behind the rings, and the stages hold weights only.
+  const int pieces_a = NORM ? 0 : MT == 16 ? (p.M + 3) / 4 * 4 / RPI : MT / RPI, pieces_w = per * 4 / RPI;
+  const int k_blocks = (p.K + 255) & ~255;
+  // rows 64 bytes apart in the banks: the four 16-byte pieces that 16 lanes read of each of four rows do not collide
+  const int x8_pitch = k_blocks + 64, x8_bytes = NORM ? RPN_ROWS * x8_pitch + 2 * RPN_ROWS * RP_CW * 4 : 0;
   const int stage_bytes = (pieces_a + pieces_w) * 1024;
   const int most = (pieces_a + pieces_w + RP_PW - 1) / RP_PW;  // loads of a producer wave per stage
-  const int depth = __builtin_amdgcn_readfirstlane(min(min((LDS_BYTES - (MT + 16 * G) * KC) / stage_bytes, 63 / most), RP_NST - 1));
+  const int depth = __builtin_amdgcn_readfirstlane(min(min((LDS_BYTES - x8_bytes - ((NORM ? 0 : MT) + 16 * G) * KC) / stage_bytes, 63 / most), RP_NST - 1));
   const int ring_bytes = (depth + 1) * stage_bytes;
+  // K is walked from another 256-byte block by every workgroup (integer sums: any order gives the same bits):
+  // neighbours on an XCD one block apart, the XCDs an eighth of K.  In step, they would all ask the same L2 channel
+  // and the same part of HBM for rows that lie a power of two apart.
+  const unsigned lin = blockIdx.y * gridDim.x + blockIdx.x;
+  const int rot = __builtin_amdgcn_readfirstlane((int)(((lin >> 3) + (lin & 7) * (unsigned)(k_blocks >> 11)) % (unsigned)(k_blocks >> 8)) * 256);
 
   if (wave >= RP_CW) {
     // this wave's pieces of a stage: every fourth activation piece, then every fourth weight piece from where those
@@ -2535,12 +2662,6 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     const v4i rW = make_rsrc(p.B + (int64_t)bz * p.sBb + (int64_t)n0 * ldb, (min(units * 4, p.N - n0) - 1) * ldb + p.K);
     const int mine_a = (pieces_a - pw + RP_PW - 1) / RP_PW;
     const int first_w = pw + mine_a * RP_PW - pieces_a;
-    // K is walked from another 256-byte block by every workgroup (integer sums: any order gives the same bits):
-    // neighbours on an XCD one block apart, the XCDs an eighth of K.  In step, they would all ask the same L2 channel
-    // and the same part of HBM for rows that lie a power of two apart.
-    const int k_blocks = (p.K + 255) & ~255;
-    const unsigned lin = blockIdx.y * gridDim.x + blockIdx.x;
-    const int rot = __builtin_amdgcn_readfirstlane((int)(((lin >> 3) + (lin & 7) * (unsigned)(k_blocks >> 11)) % (unsigned)(k_blocks >> 8)) * 256);
     auto produce = [&](auto a_tag, auto w_tag) {
       constexpr int LA = decltype(a_tag)::value, L = LA + decltype(w_tag)::value;
       constexpr int MAXD = 63 / (L > 0 ? L : 1) < RP_NST - 1 ? 63 / (L > 0 ? L : 1) : RP_NST - 1;
@@ -2570,6 +2691,7 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
       };
       int issued = 0;
       for (; issued < depth && issued < KT; ++issued) issue();
+      if constexpr (NORM != NORM_NONE) asm volatile("s_barrier\n\ts_barrier" ::: "memory");  // rowpieces_norm's
       wait_stages<L, 0, MAXD>(issued - 1);  // stage 0 landed
       asm volatile("s_barrier" ::: "memory");
       for (int g = 0; g < KT; ++g) {
@@ -2583,7 +2705,7 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     };
     // 4 * (G - 1) < per <= 4 * G (host)
     constexpr int A_MAX = MT / RPI / RP_PW, W_MIN = (16 * G - 12) / RPI / RP_PW, W_MAX = 16 * G / RPI / RP_PW;
-    with_count<MT == 16 ? A_MAX / 4 : A_MAX, A_MAX>(mine_a, [&](auto a_tag) {
+    with_count<NORM ? 0 : MT == 16 ? A_MAX / 4 : A_MAX, NORM ? 0 : A_MAX>(mine_a, [&](auto a_tag) {
       with_count<W_MIN, W_MAX>((pieces_w - first_w + RP_PW - 1) / RP_PW, [&](auto w_tag) { produce(a_tag, w_tag); });
     });
     asm volatile("s_barrier" ::: "memory");  // the consumers' exchange of sums
@@ -2592,6 +2714,11 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
     // scales, bias and residual now, under the wait for the first stage, and not after the last one
     constexpr int J = (MT * 4 * G + RP_CW * 64 - 1) / (RP_CW * 64);
     const EpiCtx e = make_epi(p, bz);
+    char* const x8 = lds + (LDS_BYTES - x8_bytes);
+    if constexpr (NORM != NORM_NONE) {
+      rowpieces_norm<NORM, VPT>(p, x8, x8_pitch, (float*)(x8 + RPN_ROWS * x8_pitch), tid, lin == 0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // x8 is written before the barrier that opens stage 0
+    }
     RowpiecesPre<J> pre;
     rowpieces_prefetch<J>(pre, p, e, tid, n0, units);
     v4i acc[G][MB];
@@ -2600,17 +2727,25 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
 #pragma unroll
       for (int m = 0; m < MB; ++m) acc[g][m] = (v4i){0, 0, 0, 0};
     v4i xf[2][KPW][MB], wf[2][KPW][G];
+    int pos = 0;  // of the stage in this workgroup's walk over K
     auto read = [&](auto set_tag, int stage) {
       constexpr int set = decltype(set_tag)::value;
       const char* sp = lds + stage;
 #pragma unroll
       for (int k = 0; k < KPW; ++k) {
         const int off = r16 * KC + ((((wave * KPW + k) * 4 + c4) ^ r16) * 16);
+        if constexpr (NORM != NORM_NONE) {
+          // blocks past the last meet weights that are zero; rows past the last are never stored
+          const int at = pos + (wave * KPW + k) * 64, kk = at >= k_blocks ? 0 : (at + rot >= k_blocks ? at + rot - k_blocks : at + rot);
+          xf[set][k][0] = *(const v4i*)(x8 + min(r16, p.M - 1) * x8_pitch + kk + c4 * 16);
+        } else {
 #pragma unroll
         for (int m = 0; m < MB; ++m) xf[set][k][m] = *(const v4i*)(sp + m * 16 * KC + off);
+        }
 #pragma unroll
         for (int g = 0; g < G; ++g) wf[set][k][g] = *(const v4i*)(sp + pieces_a * 1024 + g * 16 * KC + off);
       }
+      if constexpr (NORM != NORM_NONE) pos += KC;
     };
     auto compute = [&](auto set_tag) {
       constexpr int set = decltype(set_tag)::value;
@@ -2777,6 +2912,25 @@ static KernelFn rowpieces_kernel(int mt, int g, int kc) {
     case 48: return kc == 512 ? rowpieces_kernel<48, 512>(g) : rowpieces_kernel<48, RP_KC>(g);
     default: return kc == 512 ? rowpieces_kernel<64, 512>(g) : rowpieces_kernel<64, RP_KC>(g);
   }
+}
+
+// gemm_rowpieces_kernel with a norm in front: up to 16 * g weight rows per workgroup, K up to RPN_K.  Stages as long as the
+// LDS beside the activations allows.
+static KernelFn rowpieces_norm_kernel(int kind, int g, int K) {
+  KernelFn fn = nullptr;
+  const auto pick = [&](auto kind_tag, auto vpt_tag) {
+    with_count<1, RP_GMAX>(g, [&](auto g_tag) {
+      constexpr int G = decltype(g_tag)::value, KC = G <= 2 ? 1024 : G == 3 ? 512 : RP_KC;
+      fn = gemm_rowpieces_kernel<16, G, KC, decltype(kind_tag)::value, decltype(vpt_tag)::value>;
+    });
+  };
+  const auto by_k = [&](auto kind_tag) {
+    if (K <= 4096) pick(kind_tag, std::integral_constant<int, 4>{});
+    else pick(kind_tag, std::integral_constant<int, 5>{});
+  };
+  if (kind == NORM_LN) by_k(std::integral_constant<int, NORM_LN>{});
+  else by_k(std::integral_constant<int, NORM_DQ_ADD_LN>{});
+  return fn;
 }
 
 static const Config g_configs[] = {
@@ -3415,7 +3569,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
     const int g = (per + 3) / 4;
     // forced by a test: bytes of K per stage, divided by 256
     const int kc = want_splits ? want_splits * 256 : (k.bm <= 32 && rowpieces_fits(k.bm, g, 1024) ? 1024 : (g <= 3 && rowpieces_fits(k.bm, g, 512) ? 512 : RP_KC));
-    const KernelFn fn = rowpieces_kernel(k.bm, g, kc);
+    const KernelFn fn = p.norm.kind ? rowpieces_norm_kernel(p.norm.kind, g, p.K) : rowpieces_kernel(k.bm, g, kc);
     if (!fn) return fail(TI_E_COMBO, "config %s: no stages of %d bytes of K for %d weight rows per workgroup", k.name, kc, per * 4);
     g_last_config = config;
     if (dry) {
@@ -3623,16 +3777,26 @@ int ti_bmm_i8_grouped(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, co
   return ti::run(p, config, (hipStream_t)stream);
 }
 
-int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
-                          const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
-                          int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
-                          int D, void* stream) {
+// Whether gemm_rowpieces_kernel can make these activations from their LayerNorm: few rows, whole 16-byte pieces of every row
+static bool rows_take_norm(const ti::GemmParams& p) {
+  const ti::NormArgs& a = p.norm;
+  const bool dq = a.kind == ti::NORM_DQ_ADD_LN;
+  const uintptr_t at = (uintptr_t)a.x | (uintptr_t)a.gamma | (uintptr_t)a.beta | (dq ? (uintptr_t)a.acc | (uintptr_t)a.resid_out : 0);
+  const int64_t pitch = a.x_rs | (dq ? a.acc_rs | a.rout_rs : 0);
+  return p.M <= ti::RPN_ROWS && p.K >= 1024 && p.K <= ti::RPN_K && ti::fast_eligible(p) && (at & 15) == 0 && (p.M == 1 || (pitch & 3) == 0);
+}
+
+static int qkv_decode(const ti::NormArgs& norm, const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+                      const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
+                      int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
+                      int D, void* stream) {
   using namespace ti;
   if (seqs < 1 || M % seqs) return fail(TI_E_SHAPE, "%d rows are not %d sequences of one length", M, seqs);
   if (M > 16 || K < 1024 || D <= 0 || (D & 15) || N % D) return fail(TI_E_COMBO, "needs M <= 16, K >= 1024, D %% 16 == 0, N %% D == 0");
   if (!k_dst || !vt_dst) return fail(TI_E_NULL, "k_dst and vt_dst are required");
   if (((uintptr_t)k_dst & 3) || (k_head_stride & 3) || (k_row_stride & 3)) return fail(TI_E_STRIDE, "k_dst and its strides must be multiples of 4 bytes");
   GemmParams p;
+  p.norm = norm;
   p.A = A; p.B = W; p.C = C;
   p.sAb = 0; p.sAm = lda; p.sAk = 1;
   p.sBb = (int64_t)N * ldw; p.sBn = ldw; p.sBk = 1;
@@ -3655,8 +3819,61 @@ int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t
   int splits = 1;
   const int cfg = pick_config(p, &splits);
   if (!g_configs[cfg].rows4 && !g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "operands not eligible for the decode kernel (16-byte aligned, K-contiguous)");
+  if (norm.kind && !(rows_take_norm(p) && g_configs[cfg].rowpieces)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
   return run(p, cfg, (hipStream_t)stream);
 }
+
+int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+                          const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
+                          int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
+                          int D, void* stream) {
+  return qkv_decode(ti::NormArgs{}, A, lda, W, ldw, bias, alpha3, beta3, C, ldc, seqs, M, N, K, k_dst, k_head_stride, k_row_stride, vt_dst, vt_row_stride, D, stream);
+}
+
+int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const float* gamma, const float* beta, float eps, const int8_t* W, int64_t ldw,
+                                    const int8_t* bias, const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
+                                    int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride, int D, void* stream) {
+  if (M > 0 && (!x || !gamma)) return ti::fail(TI_E_NULL, "x and gamma are required");
+  ti::NormArgs n{};
+  n.kind = ti::NORM_LN;
+  n.x = x; n.x_rs = x_row_stride; n.gamma = gamma; n.beta = beta; n.eps = eps;
+  return qkv_decode(n, (const int8_t*)x, K, W, ldw, bias, alpha3, beta3, C, ldc, seqs, M, N, K, k_dst, k_head_stride, k_row_stride, vt_dst, vt_row_stride, D, stream);
+}
+
+int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_stride, float in_scale, const float* resid, int64_t resid_row_stride, const float* gamma,
+                                       const float* beta, float eps, float* resid_out, int64_t resid_out_row_stride, const int8_t* W, int64_t ldw,
+                                       const float* bias, const float* scale_a, const float* scale_b, int8_t* C, int64_t ldc, int M, int N, int K, void* stream) {
+  using namespace ti;
+  if (M > 0 && (!acc || !resid || !gamma || !resid_out)) return fail(TI_E_NULL, "acc, resid, gamma and resid_out are required");
+  GemmParams p;
+  p.norm.kind = NORM_DQ_ADD_LN;
+  p.norm.x = resid; p.norm.x_rs = resid_row_stride;
+  p.norm.acc = acc; p.norm.acc_rs = acc_row_stride; p.norm.in_scale = in_scale;
+  p.norm.resid_out = resid_out; p.norm.rout_rs = resid_out_row_stride;
+  p.norm.gamma = gamma; p.norm.beta = beta; p.norm.eps = eps;
+  p.A = (const int8_t*)resid; p.B = W; p.C = C;
+  p.sAb = 0; p.sAm = K; p.sAk = 1;
+  p.sBb = 0; p.sBn = ldw; p.sBk = 1;
+  p.sCb = 0; p.sCm = ldc; p.sCn = 1;
+  p.batch = 1; p.M = M; p.N = N; p.K = K;
+  p.bias = bias; p.bias_kind = bias ? TI_BIAS_F32 : TI_BIAS_NONE;
+  p.alpha = scale_a; p.beta = scale_b;
+  p.epilogue = TI_EPI_GELU_I8; p.out_dtype = TI_I8; p.round_mode = TI_ROUND_RNE_CLAMP;
+  p.tiles_m = p.tiles_n = 0; p.group_m = 1; p.ksplit = 1;
+  p.bias_bs = 0; p.scale_bs = 0;
+  p.resid = nullptr; p.resid_rs = 0;
+  p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
+  p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
+  int rc = validate(p);
+  if (rc != TI_OK) return rc;
+  if (M == 0 || N == 0) return TI_OK;
+  int splits = 1;
+  if (!rows_take_norm(p)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
+  const int cfg = pick_config(p, &splits);
+  if (!g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for this size");
+  return run(p, cfg, (hipStream_t)stream);
+}
+
 
 int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
                      const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int M, int N, int K,

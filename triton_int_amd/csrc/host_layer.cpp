@@ -165,6 +165,8 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(S >= min_queries || T <= 4096);
     const int T32 = int32_size(T);
 
+    const bool few = M <= 4 && H >= 1024 && ((x_rs & 3) == 0 || M == 1) && (((uintptr_t)ptr(x) | (uintptr_t)ln1.g | (uintptr_t)ln1.b | (uintptr_t)ln2.g |
+                                                                              (uintptr_t)ln2.b) & 15) == 0;  // the norms go into the launches after them
     int rc = TI_OK;
     Tensor out;
     {
@@ -181,9 +183,15 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
       float* resid = (float*)(base + at[4]);
       const float* xp = (const float*)ptr(x);
       const auto run = [&]() {
-        if ((rc = ti_layernorm_q(xp, x_rs, ln1.g, ln1.b, ln1.eps, h8, H, M32, H32, 0, TI_ROUND_RNE_CLAMP, nullptr, nullptr, c.stream))) return;
         bool appended = false;
-        if (cached && M <= 16 && H >= 1024 && ((((int64_t)k_dst | dst_hs | dst_rs) & 3) == 0)) {
+        if (few && cached) {
+          rc = ti_layernorm_qkv_decode_i8_seqs(xp, x_rs, ln1.g, ln1.b, ln1.eps, (const int8_t*)ptr(w3), H, b3, a3, s3, qkv, 3 * H, B32, M32, H32, H32, k_dst, dst_hs,
+                                               dst_rs, vt_dst, vt_rs, (int)D, c.stream);
+          if (rc && rc != TI_E_COMBO) return;
+          appended = rc == TI_OK;
+        }
+        if (!appended && (rc = ti_layernorm_q(xp, x_rs, ln1.g, ln1.b, ln1.eps, h8, H, M32, H32, 0, TI_ROUND_RNE_CLAMP, nullptr, nullptr, c.stream))) return;
+        if (!appended && cached && M <= 16 && H >= 1024 && ((((int64_t)k_dst | dst_hs | dst_rs) & 3) == 0)) {
           rc = ti_qkv_decode_i8_seqs(h8, H, (const int8_t*)ptr(w3), H, b3, a3, s3, qkv, 3 * H, B32, M32, H32, H32, k_dst, dst_hs, dst_rs, vt_dst, vt_rs, (int)D, c.stream);
           if (rc && rc != TI_E_COMBO) return;
           appended = rc == TI_OK;
@@ -199,10 +207,16 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
                                         vt_rs, ctx, S * H, D, H, B32, (int)heads, S32, T32, (int)D, qk_alpha, score_scale, pv_alpha, causal, c.stream))) return;
         if ((rc = ti_bmm_i8_config(ctx, 0, H, 1, out_proj.w, 0, out_proj.ldw, 1, acc, 0, H, 1, 1, M32, H32, H32, out_proj.bias, TI_BIAS_I32, nullptr, nullptr,
                                    TI_EPI_I32, TI_I32, TI_ROUND_RNE_CLAMP, -1, c.stream))) return;
-        if ((rc = ti_dq_add_layernorm_q(acc, H, in_scale, nullptr, xp, x_rs, ln2.g, ln2.b, ln2.eps, resid, H, h8b, H, nullptr, H, M32, H32, TI_ROUND_RNE_CLAMP,
-                                        nullptr, nullptr, c.stream))) return;
-        if ((rc = ti_bmm_i8_config(h8b, 0, H, 1, fc1.w, 0, fc1.ldw, 1, f8, 0, fc1.N, 1, 1, M32, F32, H32, fc1.bias, TI_BIAS_F32, fc1.a, fc1.b, TI_EPI_GELU_I8, TI_I8,
-                                   TI_ROUND_RNE_CLAMP, -1, c.stream))) return;
+        rc = few ? ti_dq_add_layernorm_linear_gelu_i8(acc, H, in_scale, xp, x_rs, ln2.g, ln2.b, ln2.eps, resid, H, fc1.w, fc1.ldw, (const float*)fc1.bias, fc1.a, fc1.b,
+                                                      f8, fc1.N, M32, F32, H32, c.stream)
+                 : TI_E_COMBO;
+        if (rc && rc != TI_E_COMBO) return;
+        if (rc) {
+          if ((rc = ti_dq_add_layernorm_q(acc, H, in_scale, nullptr, xp, x_rs, ln2.g, ln2.b, ln2.eps, resid, H, h8b, H, nullptr, H, M32, H32, TI_ROUND_RNE_CLAMP,
+                                          nullptr, nullptr, c.stream))) return;
+          if ((rc = ti_bmm_i8_config(h8b, 0, H, 1, fc1.w, 0, fc1.ldw, 1, f8, 0, fc1.N, 1, 1, M32, F32, H32, fc1.bias, TI_BIAS_F32, fc1.a, fc1.b, TI_EPI_GELU_I8, TI_I8,
+                                     TI_ROUND_RNE_CLAMP, -1, c.stream))) return;
+        }
         rc = ti_linear_i8_residual_f32(f8, fc1.N, fc2.w, fc2.ldw, (const float*)fc2.bias, fc2.a, fc2.b, resid, H, (float*)mptr(out), H, M32, H32, F32, c.stream);
       };
       run();
