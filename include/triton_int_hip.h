@@ -357,14 +357,13 @@ int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const 
 /*
  * ti_dq_add_layernorm_q (kernels/fused.py:235-382 behind nn/fused.py:59-78) and the GELU-quant linear on its int8 rows
  * (kernels/fused.py:197-231) as one launch: resid_out = resid + in_scale * acc, C = q8(gelu(scale_a * (LN(resid_out) . W) + bias) *
- * scale_b).  Limits and TI_E_COMBO as above.
+ * scale_b).  Limits and TI_E_COMBO as above; also where resid_out shares memory with resid or acc.
  */
 int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_stride, float in_scale, const float* resid,
                                        int64_t resid_row_stride, const float* gamma, const float* beta, float eps,
                                        float* resid_out, int64_t resid_out_row_stride, const int8_t* W, int64_t ldw,
                                        const float* bias, const float* scale_a, const float* scale_b, int8_t* C, int64_t ldc,
                                        int M, int N, int K, void* stream);
-
 
 /*
  * Appends S new positions to an int8 KV cache in one launch: K [S, heads*D] (row stride

@@ -68,4 +68,7 @@ def test_declined():
     for m, k, xp in ((5, 4096, x.data_ptr()), (1, 5136, x.data_ptr()), (1, 1008, x.data_ptr()), (1, 4096, x.data_ptr() + 4), (1, 4090, x.data_ptr())):
         assert lib.ti_dq_add_layernorm_linear_gelu_i8(acc.data_ptr(), K, 1.0, xp, K, gamma.data_ptr(), 0, 1e-5, r.data_ptr(), K, w.data_ptr(), K, 0, s.data_ptr(),
                                                       s.data_ptr(), out.data_ptr(), N, m, N, k, st) == COMBO
-    assert (out == 3).all() and (r == 7.0).all()
+    for a, xp, ro in ((acc, x, x), (acc, x, acc), (acc, x, x[1:]), (acc[1:], x, acc)):  # in place: other workgroups still read what one writes
+        assert lib.ti_dq_add_layernorm_linear_gelu_i8(a.data_ptr(), K, 1.0, xp.data_ptr(), K, gamma.data_ptr(), 0, 1e-5, ro.data_ptr(), K, w.data_ptr(), K, 0,
+                                                      s.data_ptr(), s.data_ptr(), out.data_ptr(), N, 2, N, 4096, st) == COMBO
+    assert (out == 3).all() and (r == 7.0).all() and (x == 0).all() and (acc == 0).all()

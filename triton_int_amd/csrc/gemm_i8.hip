@@ -3845,6 +3845,12 @@ int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_strid
                                        const float* bias, const float* scale_a, const float* scale_b, int8_t* C, int64_t ldc, int M, int N, int K, void* stream) {
   using namespace ti;
   if (M > 0 && (!acc || !resid || !gamma || !resid_out)) return fail(TI_E_NULL, "acc, resid, gamma and resid_out are required");
+  // every workgroup reads all of acc and resid while the first one writes resid_out
+  const auto meets = [&](const void* q, int64_t rs) {
+    const uintptr_t a = (uintptr_t)resid_out, b = (uintptr_t)q;
+    return M > 0 && a < b + 4 * ((M - 1) * rs + K) && b < a + 4 * ((M - 1) * resid_out_row_stride + K);
+  };
+  if (meets(acc, acc_row_stride) || meets(resid, resid_row_stride)) return fail(TI_E_COMBO, "resid_out lies in acc or resid");
   GemmParams p;
   p.norm.kind = NORM_DQ_ADD_LN;
   p.norm.x = resid; p.norm.x_rs = resid_row_stride;
@@ -3873,7 +3879,6 @@ int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_strid
   if (!g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for this size");
   return run(p, cfg, (hipStream_t)stream);
 }
-
 
 int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
                      const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int M, int N, int K,
