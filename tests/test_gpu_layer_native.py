@@ -1,5 +1,7 @@
 """The extension module's decoder layer against the step-by-step path: the same bits over the forms both take, and everything
 that only Python can honour is left to it."""
+import threading
+
 import pytest
 import torch
 
@@ -122,3 +124,30 @@ def test_on_another_stream_and_captured(layer):
         graph.replay()
         assert torch.equal(static, want)
         torch.cuda.synchronize()
+
+
+def test_buffers_replaced_by_another_thread(layer):
+    x = torch.randn(2, 3, HIDDEN, device=DEV)
+    want = layer(x)
+    first, stop = layer.fc2.weight, threading.Event()
+
+    def replace():
+        stream = torch.cuda.Stream()
+        while not stop.is_set():
+            with torch.cuda.stream(stream):
+                fresh = first.clone()
+                stream.synchronize()
+            layer.fc2.weight = fresh
+
+    stream0 = torch.cuda.current_stream()
+    worker = threading.Thread(target=replace)
+    worker.start()
+    try:
+        for _ in range(50):
+            got = layer(x)
+            stream0.synchronize()
+            assert torch.equal(got, want)
+    finally:
+        stop.set()
+        worker.join()
+        layer.fc2.weight = first

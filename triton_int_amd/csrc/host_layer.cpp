@@ -58,23 +58,39 @@ PyObject* step(PyObject* modules, int i, PyObject* type) {
   return d;
 }
 
+// The tensors that a call reads, held until it returns: another thread may replace a module's buffer while this one launches
+// without the interpreter's lock.
+struct Held {
+  c10::SmallVector<Tensor, 32> all;
+  const Tensor& tensor(PyObject* o, int dev, ScalarType type) {
+    const Tensor& t = ::tensor(o, dev, type);
+    all.push_back(t);
+    return t;
+  }
+  const void* vector(PyObject* o, int dev, ScalarType type, int64_t n) {
+    const void* at = ::vector(o, dev, type, n);
+    if (at) all.push_back(THPVariable_Unpack(o));
+    return at;
+  }
+};
+
 // the buffers of an int8 linear [N, K]
 struct Linear {
   const int8_t* w;
   const void* bias;
   const float *a = nullptr, *b = nullptr;
   int64_t N, ldw;
-  Linear(PyObject* dict, int dev, int64_t K, ScalarType bias_type, bool scales) {
+  Linear(Held& held, PyObject* dict, int dev, int64_t K, ScalarType bias_type, bool scales) {
     PyObject* buffers = item(dict, names().buffers);
     need(PyDict_Check(buffers));
-    const Tensor& wt = tensor(item(buffers, names().weight), dev, ScalarType::Char);
+    const Tensor& wt = held.tensor(item(buffers, names().weight), dev, ScalarType::Char);
     need(wt.dim() == 2 && wt.size(1) == K && wt.stride(1) == 1);
     N = wt.size(0), ldw = wt.stride(0), w = (const int8_t*)ptr(wt);
-    bias = vector(item(buffers, names().bias), dev, bias_type, N);
+    bias = held.vector(item(buffers, names().bias), dev, bias_type, N);
     need(bias);
     if (!scales) return;
     for (int i = 0; i < 2; ++i) {
-      const Tensor& t = tensor(item(buffers, i ? names().b : names().a), dev, ScalarType::Float);
+      const Tensor& t = held.tensor(item(buffers, i ? names().b : names().a), dev, ScalarType::Float);
       need(t.numel() == 1);
       (i ? b : a) = (const float*)ptr(t);
     }
@@ -84,11 +100,11 @@ struct Linear {
 struct Norm {
   const float *g, *b;
   float eps;
-  Norm(PyObject* dict, int dev, int64_t H) {
+  Norm(Held& held, PyObject* dict, int dev, int64_t H) {
     PyObject* buffers = item(dict, names().buffers);
     need(PyDict_Check(buffers));
-    g = (const float*)vector(item(buffers, names().weight), dev, ScalarType::Float, H);
-    b = (const float*)vector(item(buffers, names().bias), dev, ScalarType::Float, H);
+    g = (const float*)held.vector(item(buffers, names().weight), dev, ScalarType::Float, H);
+    b = (const float*)held.vector(item(buffers, names().bias), dev, ScalarType::Float, H);
     need(g != nullptr);
     eps = (float)number(item(dict, names().eps));
   }
@@ -110,7 +126,8 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
     PyObject* d[8];
     for (int i = 0; i < 8; ++i) d[i] = step(modules, i, PyTuple_GET_ITEM(v[3], i + 1));
 
-    const Tensor& x = tensor(v[1], -1, ScalarType::Float);
+    Held held;
+    const Tensor& x = held.tensor(v[1], -1, ScalarType::Float);
     const Call c(x);
     need(x.dim() == 3 && x.numel() > 0);
     const int64_t B = x.size(0), S = x.size(1), H = x.size(2), M = B * S, x_rs = row_pitch(x);
@@ -119,22 +136,22 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int M32 = int32_size(M), S32 = int32_size(S), B32 = (int)B, H32 = int32_size(H);
     int32_size(3 * H);
 
-    const Norm ln1(d[0], c.dev, H), ln2(d[5], c.dev, H);
+    const Norm ln1(held, d[0], c.dev, H), ln2(held, d[5], c.dev, H);
     // the projections' buffers have to be slices of the pack, whose rows are contiguous
     PyObject* pack = item(self, nm.qkv);
     need(PyTuple_Check(pack) && PyTuple_GET_SIZE(pack) == 4);
-    const Tensor& w3 = tensor(PyTuple_GET_ITEM(pack, 0), c.dev, ScalarType::Char);
+    const Tensor& w3 = held.tensor(PyTuple_GET_ITEM(pack, 0), c.dev, ScalarType::Char);
     need(w3.dim() == 2 && w3.size(0) == 3 * H && w3.size(1) == H && w3.is_contiguous());
-    const int8_t* b3 = (const int8_t*)vector(PyTuple_GET_ITEM(pack, 1), c.dev, ScalarType::Char, 3 * H);
-    const float *a3 = (const float*)vector(PyTuple_GET_ITEM(pack, 2), c.dev, ScalarType::Float, 3),
-                *s3 = (const float*)vector(PyTuple_GET_ITEM(pack, 3), c.dev, ScalarType::Float, 3);
+    const int8_t* b3 = (const int8_t*)held.vector(PyTuple_GET_ITEM(pack, 1), c.dev, ScalarType::Char, 3 * H);
+    const float *a3 = (const float*)held.vector(PyTuple_GET_ITEM(pack, 2), c.dev, ScalarType::Float, 3),
+                *s3 = (const float*)held.vector(PyTuple_GET_ITEM(pack, 3), c.dev, ScalarType::Float, 3);
     need(b3 && a3 && s3);
     for (int i = 0; i < 3; ++i) {
-      const Linear p(d[1 + i], c.dev, H, ScalarType::Char, true);
+      const Linear p(held, d[1 + i], c.dev, H, ScalarType::Char, true);
       need(p.N == H && p.ldw == H && p.w == (const int8_t*)ptr(w3) + i * H * H && p.bias == b3 + i * H && p.a == a3 + i && p.b == s3 + i);
     }
-    const Linear out_proj(d[4], c.dev, H, ScalarType::Int, false), fc1(d[6], c.dev, H, ScalarType::Float, true),
-        fc2(d[7], c.dev, fc1.N, ScalarType::Float, true);
+    const Linear out_proj(held, d[4], c.dev, H, ScalarType::Int, false), fc1(held, d[6], c.dev, H, ScalarType::Float, true),
+        fc2(held, d[7], c.dev, fc1.N, ScalarType::Float, true);
     need(out_proj.N == H && fc2.N == H);
     const int F32 = int32_size(fc1.N);
 
