@@ -1,6 +1,9 @@
 """The extension module's source (csrc/host.cpp): what cannot be seen from a call's result."""
 import os
 import re
+import struct
+
+import pytest
 
 SOURCE = os.path.join(os.path.dirname(__file__), "..", "triton_int_amd", "csrc", "host.cpp")
 
@@ -23,3 +26,16 @@ def test_every_launch_and_allocation_runs_without_the_interpreters_lock():
         assert re.search(r"\bti_\w+\(", unlocked), name
         assert not re.search(r"\bti_\w+\(|c\.empty\(", rest), f"{name}: launches or allocates under the lock"
         assert not re.search(r"\bPy\w+|THP\w+|\bv\[|\b(integer|number|flag|scale|vector|tensor)\(", unlocked), f"{name}: reads a Python object without the lock"
+
+
+@pytest.mark.parametrize("name", ["_host.so", "_layer_host.so"])
+def test_no_thread_local_storage(name):
+    """A module with thread-local storage of its own, loaded after torch and HIP, puts every thread-local access of those on the
+    slow path (glibc before 2.39)."""
+    path = os.path.join(os.path.dirname(SOURCE), "..", name)
+    with open(path, "rb") as f:
+        elf = f.read()
+    table, = struct.unpack_from("<Q", elf, 32)
+    size, count = struct.unpack_from("<HH", elf, 54)
+    types = [struct.unpack_from("<I", elf, table + i * size)[0] for i in range(count)]
+    assert 1 in types and 7 not in types  # PT_LOAD, PT_TLS
