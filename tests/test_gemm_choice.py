@@ -42,3 +42,26 @@ def test_outputs(B, M, N, K):
     bias = torch.randn(N, device=dev, generator=g)
     for dt in (torch.float32, torch.float16):
         assert torch.equal(linear_a8_w8_bfp32_ofp32(a, w, bias, al, be, dtype=dt), (bias * be + acc.float() * al).to(dt))
+
+
+# few 64 x 64 tiles against the lines of small_tiles_lead: K 16 short of a line and on it, 128-byte rows and others, 256 tiles and one more
+# row of them, one GEMM and grouped, weights of 4 MB and beyond
+SMALL = [(1, 129, 1440, 1232, True), (1, 1024, 1024, 1152, True), (1, 1025, 1024, 1152, False), (1, 383, 624, 2416, True), (1, 383, 624, 2432, False),
+         (1, 200, 512, 1408, True), (1, 200, 512, 1536, False), (3, 143, 352, 1040, True), (2, 111, 1168, 6320, True), (2, 111, 1168, 6272, False),
+         (1, 256, 3584, 1152, True), (1, 256, 3712, 1152, False)]
+
+
+@pytest.mark.parametrize("B,M,N,K,small", SMALL)
+def test_few_small_tiles(B, M, N, K, small):
+    lib = L.lib()
+    for epi, dt, bias in ((L.EPI_SCALE_I8, 0, 1), (L.EPI_SCALE_F, 2, 3), (L.EPI_SCALE_F, 4, 3)):
+        pr = G.contiguous(B, M, N, K, dt)
+        pl = G.plan_for(lib, pr, epi, bias)
+        assert pl.name.startswith("mfma_64x64" if small else "ws_")
+        G.check_launch(pr, pl, store_sample=12)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,K,small", SMALL)
+def test_outputs_of_few_small_tiles(B, M, N, K, small):
+    test_outputs(B, M, N, K)

@@ -3113,7 +3113,24 @@ static double ws_time(const GemmParams& p, const Config& k, const WsCost& c, int
          (splits > 1 ? c.split + splits * (c.per_split + filled * c.sums) : 0.0) + filled * c.item + (double)p.N * p.K * p.batch / 5e6 * c.mem;
 }
 
+// Up to one 64 x 64 tile per CU, a short K and few weights: gemm_mfma_kernel, whose workgroups start at once, where the
+// wave-specialised ones fill 4 .. 6 stages first.  us, that one / the best of these: 580 x 400 x 1136 6.5 / 8.1, 129 x 1440 x 1232 6.8 / 8.2, 902 x
+// 592 x 1232 7.3 / 8.7, 522 x 1024 x 1024 6.5 / 7.0, 383 x 624 x 2064 9.5 / 11.1.  The lines: 256 tiles (3072 x 1024 at 225 rows, 192 tiles, 6.6 /
+// 7.1, at 532 rows, 432 tiles, 7.7 / 7.2); K below 1536 where its rows are whole 128-byte lines (384 x 2048 x 2048 9.5 / 8.8, 507 x 1984 x
+// 2176 9.8 / 9.0) and 2432 for one GEMM whose rows are not, which cost the longer stages more (1959 x 496 x 2064 10.4 / 11.2); 4 MB of
+// weights, since half as many columns per tile ask for the activations twice as often (212 x 4096 x 1024 6.3 / 6.8, but 65 x 8192 x 1024 8.5 /
+// 7.8).  Grouped GEMMs cannot split K: with ragged rows and few tiles this one leads at any K (4 x 122 x 544 x 17584 83 / 94, 2 x 125 x 880
+// x 8016 39.8 / 45.5, 4 x 334 x 416 x 2080 10.1 / 10.9 at 168 tiles).  Not with a residual, which it would need a second launch to add.
+static bool small_tiles_lead(const GemmParams& p) {
+  if (p.resid) return false;
+  const int64_t tiles = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * p.batch;
+  const bool lines = p.K % 128 == 0;
+  if (p.batch > 1 && !lines && tiles <= 200) return true;
+  return tiles <= 256 && p.K < (lines || p.batch > 1 ? 1536 : 2432) && (int64_t)p.N * p.K * p.batch <= 4 << 20;
+}
+
 static int pick_ws(const GemmParams& p, int* splits_out) {
+  if (small_tiles_lead(p)) return CFG_TILE_64x64;
   static const WsCost costs[] = {
       {CFG_WS_64x128, 1.495, 0.227, 0.122, 2.583, 2.809, 1.722, 0.216, 0.000, 0.587, 0.342},
       {CFG_WS_128x128, 0.000, 0.292, 0.180, 3.614, 4.137, 2.237, 0.240, 0.000, 0.642, 0.764},
