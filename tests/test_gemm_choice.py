@@ -65,3 +65,20 @@ def test_few_small_tiles(B, M, N, K, small):
 @pytest.mark.parametrize("B,M,N,K,small", SMALL)
 def test_outputs_of_few_small_tiles(B, M, N, K, small):
     test_outputs(B, M, N, K)
+
+
+# K = 1024: few small tiles, and the wave-specialised tiles where there are many or their weights are large
+@pytest.mark.parametrize("M,N", [(65, 256), (65, 4096), (100, 3072), (128, 4096), (65, 4112), (65, 8192), (128, 8192), (100, 16384), (128, 16384)])
+def test_k_1024(M, N):
+    lib = L.lib()
+    for epi, dt, bias in ((L.EPI_SCALE_I8, 0, 1), (L.EPI_SCALE_F, 2, 3), (L.EPI_SCALE_F, 3, 3)):
+        pr = G.contiguous(1, M, N, 1024, dt)
+        pl = G.plan_for(lib, pr, epi, bias)
+        assert pl.name.startswith("mfma_64x64" if N <= 4096 else "ws_")
+        G.check_launch(pr, pl, store_sample=12)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(65, 256), (128, 4096), (65, 4112), (100, 8192)])
+def test_outputs_at_k_1024(M, N):
+    test_outputs(1, M, N, 1024)

@@ -3087,7 +3087,7 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
   return used;
 }
 
-// Time in us of a GEMM with K > 1024 on a wave-specialised configuration in `want` K splits: a round of items costs its
+// Time in us of a GEMM with K >= 1024 on a wave-specialised configuration in `want` K splits: a round of items costs its
 // k-tiles (`tile` each, and `busy` more the more of the chip works on outputs that exist: that part is power and
 // shared memory), `item` and `out` once (pipeline fill, epilogue, stores), the weights their bytes at 5 TB/s times
 // `mem`, a split the exchange of its sums.  Least squares over 8044 launches: M = 65 .. 3000, 24
@@ -3097,7 +3097,12 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
 // this: 100 x 4096 x 4096 16.2 / 11.5, 200 x 4096 x 4096 21.9 / 13.8, 384 x 4096 x 4096 21.2 / 16.7, 300 x 1024 x 4096 15.0 / 10.0, 128 x
 // 20480 x 5120 48 / 34, 160 x 5120 x 5120 25.2 / 16.1, 1000 x 5120 x 20480 122 / 102, three grouped 100 x 4096 x 4096 20.7 / 17.3.
 // Where it loses (3 % and more at 23 of them): 384 x 2048 x 2048 9.1 / 10.2, 140 x 4096 x 11008 22.0 / 24.4.
-// K <= 1024 is left to config_cost: the rounds there are mostly epilogue.
+// Checked on 1451 other sizes, with the 64 x 64 tile of gemm_mfma_kernel (below) and the 256 x 256 tile beside it: M up to 16384, N from
+// 256 and K from 1024 up to 20480, one GEMM and 2 .. 4 grouped, every output type, K a multiple of 128 and not.  Choice / fastest 1.008 on
+// average; choice / the estimate's choice 0.91 (M > 3000 0.97, 16-bit outputs 0.92, 2 and 4 grouped 0.90, K = 1024 0.97), more than 1.04 at
+// 30 of them: 136 x 8112 x 5536 24.0 / 28.9, 343 x 7248 x 2048 three times 26.4 / 30.2, 3 x 571 x 4096 x 4096 int8 38.9 / 43.9, 264 x 20480 x 5120
+// int8 48.9 / 53.3, 128 x 16384 x 1024 8.7 / 9.5.  The 256 x 256 tile, no candidate, leads by more than 3 % at 20 of 327 (547 x 6752 x 9824
+// three times 143 / 170).  K < 1024, where rounds are mostly epilogue, and sizes beyond these are left to config_cost.
 struct WsCost {
   int cfg;
   double start, tile, busy, out8, out4, split, per_split, item, mem, sums;
@@ -3112,6 +3117,8 @@ static double ws_time(const GemmParams& p, const Config& k, const WsCost& c, int
   return c.start + kts * (rounds * c.tile + filled * real * c.busy) + rounds * (out_class(p.out_dtype) == OUT8 ? c.out8 : c.out4) +
          (splits > 1 ? c.split + splits * (c.per_split + filled * c.sums) : 0.0) + filled * c.item + (double)p.N * p.K * p.batch / 5e6 * c.mem;
 }
+
+static bool ws_range(const GemmParams& p) { return p.M > 64 && p.K >= 1024 && p.batch <= 4; }
 
 // Up to one 64 x 64 tile per CU, a short K and few weights: gemm_mfma_kernel, whose workgroups start at once, where the
 // wave-specialised ones fill 4 .. 6 stages first.  us, that one / the best of these: 580 x 400 x 1136 6.5 / 8.1, 129 x 1440 x 1232 6.8 / 8.2, 902 x
@@ -3244,7 +3251,7 @@ static int pick_config(const GemmParams& p, int* splits_out) {
   }
   // batched, few rows (attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
   if (p.M <= 16) return (p.N + 31) / 32 >= 160 ? CFG_SKINNY_16_G2 : CFG_SKINNY_16;
-  if (stream && p.M > 64 && p.K > 1024 && p.batch <= 4) return pick_ws(p, splits_out);
+  if (stream && ws_range(p)) return pick_ws(p, splits_out);
   if (p.M <= 64 && stream && p.batch == 1) {
     // a few rows against a long K: the GEMM is a read of the weight matrix, and what decides its speed is how
     // many weight bytes a CU keeps in flight.  K is split over enough workgroups to have every CU pulling its
