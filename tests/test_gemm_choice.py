@@ -82,3 +82,14 @@ def test_k_1024(M, N):
 @pytest.mark.parametrize("M,N", [(65, 256), (128, 4096), (65, 4112), (100, 8192)])
 def test_outputs_at_k_1024(M, N):
     test_outputs(1, M, N, 1024)
+
+
+def test_sizes_beyond_the_measured_ones():
+    """The times behind the choice hold up to 20480 columns and K = 28672; beyond, the estimate in units of work decides."""
+    lib = L.lib()
+    for M, N, K, name, splits in ((300, 20480, 4096, "ws_256x160", 1), (300, 50272, 4096, "ws_128x128", 1), (384, 50272, 1024, "ws_128x128", 1),
+                                  (500, 4096, 28672, "ws_256x128", 4), (500, 4096, 28688, "ws_128x128", 2)):
+        pr = G.contiguous(1, M, N, K, 2)
+        pl = G.plan_for(lib, pr, L.EPI_SCALE_F, 3)
+        assert pl.name.startswith(name) and pl.splits == splits, (M, N, K, pl)
+        G.check_launch(pr, pl, store_sample=2)

@@ -3102,7 +3102,10 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
 // average; choice / the estimate's choice 0.91 (M > 3000 0.97, 16-bit outputs 0.92, 2 and 4 grouped 0.90, K = 1024 0.97), more than 1.04 at
 // 30 of them: 136 x 8112 x 5536 24.0 / 28.9, 343 x 7248 x 2048 three times 26.4 / 30.2, 3 x 571 x 4096 x 4096 int8 38.9 / 43.9, 264 x 20480 x 5120
 // int8 48.9 / 53.3, 128 x 16384 x 1024 8.7 / 9.5.  The 256 x 256 tile, no candidate, leads by more than 3 % at 20 of 327 (547 x 6752 x 9824
-// three times 143 / 170).  K < 1024, where rounds are mostly epilogue, and sizes beyond these are left to config_cost.
+// three times 143 / 170).  Left to config_cost: K < 1024, where rounds are mostly epilogue; more
+// than 20480 columns (config_cost's choice / this one's: 300 x 50272 x 1024 39.8 / 47.7, 300 x 50272 x 4096 97 / 107, 384 x 50272 x 2048 59.2 / 64.7;
+// up to 128 rows the same); K beyond 28672 (4096 x 28672 1.08 above the fastest / 1.02, 5120 x 24576 1.03 / 1.02, 11264 x 32768 1.01 / 1.01).
+// M has no end: 17000 .. 32768 rows 1.025 / 1.004.
 struct WsCost {
   int cfg;
   double start, tile, busy, out8, out4, split, per_split, item, mem, sums;
@@ -3118,7 +3121,7 @@ static double ws_time(const GemmParams& p, const Config& k, const WsCost& c, int
          (splits > 1 ? c.split + splits * (c.per_split + filled * c.sums) : 0.0) + filled * c.item + (double)p.N * p.K * p.batch / 5e6 * c.mem;
 }
 
-static bool ws_range(const GemmParams& p) { return p.M > 64 && p.K >= 1024 && p.batch <= 4; }
+static bool ws_range(const GemmParams& p) { return p.M > 64 && p.N <= 20480 && p.K >= 1024 && p.K <= 28672 && p.batch <= 4; }
 
 // Up to one 64 x 64 tile per CU, a short K and few weights: gemm_mfma_kernel, whose workgroups start at once, where the
 // wave-specialised ones fill 4 .. 6 stages first.  us, that one / the best of these: 580 x 400 x 1136 6.5 / 8.1, 129 x 1440 x 1232 6.8 / 8.2, 902 x
