@@ -1,0 +1,58 @@
+"""What a launch does whose K split finds no memory: it chooses among the unsplit launches, instead of running the split's tile with
+whole K (three quarters of the chip idle).  On the CPU, against the library as it is built: native/split_memory.cpp stands in for HIP."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from tests import gemm_bounds_model as G
+from triton_int_amd import _lib as L
+from triton_int_amd import build as B
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+# the split choice needs more than 32 MiB of partial sums at the first four, 32 MiB at the last
+SIZES = [(666, 4096, 16384), (768, 4096, 16384), (300, 10240, 20480), (128, 20480, 20480), (384, 4096, 16384)]
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("native") / "split_memory")
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(B.HIPCC)))
+    rocm = rocm if os.path.isdir(os.path.join(rocm, "include", "hip")) else "/opt/rocm"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", f"-isystem{rocm}/include", os.path.join(HERE, "native", "split_memory.cpp"), "-o", out,
+                    "-rdynamic", f"-L{B.LIB_DIR}", "-l:libtriton_int_hip.so", f"-Wl,-rpath,{B.LIB_DIR}", f"-L{rocm}/lib", f"-Wl,-rpath,{rocm}/lib", "-lamdhip64"],
+                   check=True)
+
+    def run(mode, room, *sizes):
+        r = subprocess.run([out, mode, str(room), *(",".join(map(str, s)) for s in sizes)], capture_output=True, text=True, check=True, timeout=60)
+        rows = [line.split() for line in r.stdout.splitlines()]
+        return [(int(rc), name, int(splits), int(n), int(held)) for rc, name, splits, n, held in rows]
+    return run
+
+
+def workgroups(name, M, N):
+    bm, bn = map(int, re.match(r"ws_(\d+)x(\d+)x", name).groups())
+    return -(-M // bm) * -(-N // bn)
+
+
+def test_static_scratch_plans_an_unsplit_choice():
+    lib = L.lib()
+    for M, N, K in SIZES[:4]:
+        pr = G.contiguous(1, M, N, K, 2)
+        split = G.plan_for(lib, pr, L.EPI_SCALE_F, 3)
+        assert split.splits > 1 and split.partial_bytes > 32 << 20
+        pl = G.plan_for(lib, pr, L.EPI_SCALE_F, 3, static_scratch=1)
+        assert pl.splits == 1 and pl.name.startswith("ws_128x128") and pl.tiles_m * pl.tiles_n >= 160 > split.tiles_m * split.tiles_n
+        G.check_launch(pr, pl, store_sample=2)
+
+
+def test_capture_without_a_workspace(program):
+    for (rc, name, splits, launches, held), (M, N, K) in zip(program("capturing", 1 << 40, *SIZES), SIZES):
+        assert (rc, splits, launches, held) == (0, 1, 1, 0)
+        assert workgroups(name, M, N) >= 160, name
+
+
+def test_workspace_is_given(program):
+    for rc, name, splits, launches, held in program("none", 1 << 40, *SIZES):
+        assert rc == 0 and splits > 1 and launches in (1, 2) and held > 0  # the clearing kernel of a new workspace

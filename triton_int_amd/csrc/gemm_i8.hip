@@ -3139,7 +3139,7 @@ static bool small_tiles_lead(const GemmParams& p) {
   return tiles <= 256 && p.K < (lines || p.batch > 1 ? 1536 : 2432) && (int64_t)p.N * p.K * p.batch <= 4 << 20;
 }
 
-static int pick_ws(const GemmParams& p, int* splits_out) {
+static int pick_ws(const GemmParams& p, int* splits_out, bool may_split) {
   if (small_tiles_lead(p)) return CFG_TILE_64x64;
   static const WsCost costs[] = {
       {CFG_WS_64x128, 1.495, 0.227, 0.122, 2.583, 2.809, 1.722, 0.216, 0.000, 0.587, 0.342},
@@ -3153,7 +3153,7 @@ static int pick_ws(const GemmParams& p, int* splits_out) {
     const Config& k = g_configs[c.cfg];
     const int64_t tiles = (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bn - 1) / k.bn);
     for (int want : {1, 2, 3, 4, 6, 8}) {
-      if (want > 1 && (p.batch != 1 || tiles * want > 520 || p.K < 384 * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
+      if (want > 1 && (!may_split || p.batch != 1 || tiles * want > 520 || p.K < 384 * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
       int splits;
       const double t = ws_time(p, k, c, want, splits);
       if (best_time < 0 || t < best_time) best_time = t, best = c.cfg, *splits_out = splits;
@@ -3194,7 +3194,10 @@ static int pick_ragged(const GemmParams& p, int64_t tiles128, int* splits_out) {
 // Tile choice: the configuration (and K split) with the lowest estimated run time.  The class
 // efficiencies were measured with weights streamed from HBM.  Outputs the persistent kernels can
 // store (row-major, aligned) go to them; the rest to the one-tile kernels.
-static int pick_config(const GemmParams& p, int* splits_out) {
+// may_split: whether the launch can get memory for split-K partial sums.  pick_ws weighs tile and splits together: a launch
+// that then ran its tile with whole K would leave the chip idle (768 x 4096 x 16384: 256 x 160 in 3 splits 58 us, whole K
+// on the 78 tiles 92; the 128 x 128 tile 67, by the estimate).  Elsewhere the caller drops the split and keeps the tile.
+static int pick_config(const GemmParams& p, int* splits_out, bool may_split = true) {
   *splits_out = 1;
   if (!fast_eligible(p)) {
     if (!ragged_eligible(p)) return CFG_GATHER;
@@ -3254,7 +3257,7 @@ static int pick_config(const GemmParams& p, int* splits_out) {
   }
   // batched, few rows (attention BMMs): MFMA-layout loads, two slabs per wave while enough waves remain
   if (p.M <= 16) return (p.N + 31) / 32 >= 160 ? CFG_SKINNY_16_G2 : CFG_SKINNY_16;
-  if (stream && ws_range(p)) return pick_ws(p, splits_out);
+  if (stream && ws_range(p)) return pick_ws(p, splits_out, may_split);
   if (p.M <= 64 && stream && p.batch == 1) {
     // a few rows against a long K: the GEMM is a read of the weight matrix, and what decides its speed is how
     // many weight bytes a CU keeps in flight.  K is split over enough workgroups to have every CU pulling its
@@ -3505,7 +3508,8 @@ struct LaunchPlan {
 // launch whose partial sums do not fit it is refused (nothing is allocated or freed on this path).
 // dry: every decision is taken as for a launch (same code), but no device is touched, nothing is
 // allocated or launched, and *dry receives the launch's configuration and grid.
-static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch = false, LaunchPlan* dry = nullptr) {
+// may_split: a configuration that is chosen here may split K; false where a first choice found no memory for the split.
+static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch = false, LaunchPlan* dry = nullptr, bool may_split = true) {
   g_last_splits = 1;
   int want_splits = config < 0 ? 0 : (config >> 8) & 0xff;
   if (config >= 0) config = (config & 0xff) == 0xff ? -1 : (config & 0xff);
@@ -3521,10 +3525,12 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
   // on the gather kernel
   const bool trunc8 = p.round_mode == TI_ROUND_TRUNC && out_class(p.out_dtype) == OUT8;
   int auto_splits = 1;
-  if (config < 0) {
+  const bool chosen = config < 0;
+  if (chosen) {
     // int8 truncation (a test-time switch) is implemented by the gather kernel and the M <= 64 kernels
     if (trunc8 && (p.M > 16 || !fast_eligible(p))) config = (p.M <= 64 && fast_eligible(p)) ? CFG_SKINNY_16 + 1 + (p.M > 32) : CFG_GATHER;
-    else config = pick_config(p, &auto_splits);
+    else config = pick_config(p, &auto_splits, may_split);
+    if (!may_split) auto_splits = 1;
   }
   else if (config < g_num_configs && !want_splits && g_configs[config].ws_waves) auto_splits = pick_splits(p, g_configs[config], 1.0, nullptr);
   if (config >= g_num_configs) return fail(TI_E_COMBO, "config %d out of range", config);
@@ -3643,12 +3649,13 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
     const size_t item_bytes = (size_t)k.bm * k.bn * sizeof(int);
     if (splits > 1 && static_scratch &&
         ((size_t)tiles * sk_waves(k) > SK_STATIC_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_STATIC_PARTIAL_BYTES)) {
-      // a split the caller forced is refused; one the library chose itself gives way to the unsplit launch,
+      // a split the caller forced is refused; one the library chose itself gives way to an unsplit launch,
       // which needs no scratch at all (as the allocating path does when its workspace limit is exceeded)
       if (want_splits)
         return fail(TI_E_SHAPE, "%d K splits of %lld tiles need %zu bytes of partial sums: more than the %zu bytes of static scratch "
                     "(use ti_bmm_i8, which allocates its workspace)", splits, (long long)tiles, (size_t)tiles * splits * item_bytes,
                     SK_STATIC_PARTIAL_BYTES);
+      if (chosen) return run(p, -1, stream, static_scratch, dry, false);
       sk_shape(kt, 1, splits, p.kt_split);
     }
     if (splits > 1 && static_scratch) {
@@ -3658,14 +3665,18 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       }
     } else if (splits > 1 && ((size_t)tiles * sk_waves(k) > SK_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_MAX_PARTIAL_BYTES)) {
       if (want_splits) return fail(TI_E_SHAPE, "%d splits of %lld tiles exceed the split-K workspace", splits, (long long)tiles);
+      if (chosen) return run(p, -1, stream, static_scratch, dry, false);
       splits = 1;
     }
     if (splits > 1 && !static_scratch && !dry) {
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
       (void)hipStreamIsCapturing(stream, &cap);
       rc = sk_workspace(stream, (size_t)tiles * splits * item_bytes, cap == hipStreamCaptureStatusNone, &p.sk_partial, &p.sk_counter);
-      if (rc == TI_E_COMBO && !want_splits) splits = 1;  // capturing and nothing allocated yet: run unsplit
-      else if (rc == TI_E_COMBO) return fail(TI_E_COMBO, "no split-K workspace on this stream and none can be allocated during graph capture");
+      // capturing without a large enough workspace: an automatic split gives way
+      if (!want_splits && rc == TI_E_COMBO) {
+        if (chosen) return run(p, -1, stream, false, nullptr, false);
+        splits = 1;
+      } else if (rc == TI_E_COMBO) return fail(TI_E_COMBO, "no split-K workspace on this stream and none can be allocated during graph capture");
       else if (rc != TI_OK) return rc;
     }
     p.splits = splits;
