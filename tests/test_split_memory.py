@@ -56,3 +56,16 @@ def test_capture_without_a_workspace(program):
 def test_workspace_is_given(program):
     for rc, name, splits, launches, held in program("none", 1 << 40, *SIZES):
         assert rc == 0 and splits > 1 and launches in (1, 2) and held > 0  # the clearing kernel of a new workspace
+
+
+def test_no_memory_for_a_workspace(program):
+    """The launches run all the same, and a smaller workspace that is there is kept and used."""
+    for (rc, name, splits, launches, held), (M, N, K) in zip(program("none", 0, *SIZES), SIZES):
+        assert (rc, splits, launches, held) == (0, 1, 1, 0)
+        assert workgroups(name, M, N) >= 160, name
+    small = (100, 1024, 4096)
+    room = program("none", 1 << 40, small)[0][4]
+    first, second, third = program("none", room, small, SIZES[0], small)
+    assert first[0] == 0 and first[2] > 1 and first[4] == room
+    assert second[0] == 0 and second[2] == 1 and second[4] == room
+    assert third == (0, first[1], first[2], 1, room)

@@ -3672,8 +3672,9 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
       (void)hipStreamIsCapturing(stream, &cap);
       rc = sk_workspace(stream, (size_t)tiles * splits * item_bytes, cap == hipStreamCaptureStatusNone, &p.sk_partial, &p.sk_counter);
-      // capturing without a large enough workspace: an automatic split gives way
-      if (!want_splits && rc == TI_E_COMBO) {
+      // capturing without a large enough workspace, or no memory for one: an automatic split gives way
+      if (!want_splits && (rc == TI_E_COMBO || rc == (int)hipErrorOutOfMemory)) {
+        if (rc != TI_E_COMBO) (void)hipGetLastError();  // launch_status below asks for the launch's own
         if (chosen) return run(p, -1, stream, false, nullptr, false);
         splits = 1;
       } else if (rc == TI_E_COMBO) return fail(TI_E_COMBO, "no split-K workspace on this stream and none can be allocated during graph capture");
