@@ -7,7 +7,7 @@ import torch
 
 from tests.util import DEV
 from triton_int_amd import _lib as L
-from triton_int_amd.nn import opt
+from triton_int_amd.nn import fused, linear, opt
 from triton_int_amd.nn.linear import W8A8B8O8Linear, W8A8BFP32OFP32Linear
 
 pytestmark = pytest.mark.gpu
@@ -105,6 +105,26 @@ def test_what_only_python_can_honour(layer):
     for kv in ((k[:, :, :64], vt), (k[1:], vt[1:]), (k, vt.half()), [k, vt], (k, None)):
         assert native(layer, x, kv) is None
     assert native(layer, torch.randn(1, 9, HIDDEN, device=DEV), (k, vt)) is None  # more new positions than the cache holds
+
+
+@pytest.mark.parametrize("where,name", [
+    (fused.LayerNormQ, "forward"), (fused.DQ_Add_LayerNorm_Q, "forward"), (linear.W8A8B32O32LinearWithoutScaling, "_launch"), (linear._Int8Linear, "forward"),
+    (fused.W8A8BFP32OFP32_GeLu_Q, "_launch"), (W8A8BFP32OFP32Linear, "forward_add"), (torch.nn.Module, "__call__"), (torch.nn.Module, "_call_impl"),
+    (opt.W8A8OPTDecoderLayer, "_append"), (opt.W8A8OPTDecoderLayer, "_qkv_pack"), (opt.W8A8OPTDecoderLayer, "_forward_steps"),
+    (opt, "attention_i8"), (opt, "linear_group_a8_w8_b8_o8"), (fused, "dq_add_layernorm_q_cpp"), (linear, "linear_a8_w8_b32_o32")])
+def test_replaced_for_every_instance(layer, monkeypatch, where, name):
+    """A method replaced on a class, or a launcher in the module that calls it, runs inside the layer."""
+    x = torch.randn(1, 17, HIDDEN, device=DEV)
+    want, seen, original = layer(x), [], getattr(where, name)
+
+    def replacement(*args, **kwargs):
+        seen.append(name)
+        return original(*args, **kwargs)
+    with monkeypatch.context() as m:
+        m.setattr(where, name, replacement)
+        assert native(layer, x, None) is None
+        assert torch.equal(layer(x), want) and seen
+    assert torch.equal(native(layer, x, None), want)
 
 
 def test_on_another_stream_and_captured(layer):

@@ -3,9 +3,10 @@
 // The seven to eight launches of W8A8OPTDecoderLayer.forward cost 60 us of Python (module calls, attribute
 // look-ups, views, one allocation per step) where their kernels on a 1024-wide layer take 30.  This is the same
 // sequence of C ABI calls on the modules' buffers as they are now: nothing is kept from one call for the next.
-// Intermediates share one allocation.  Anything that Python would notice (hooks, another module type, a replaced
-// method) or that the plain sequence does not cover is declined, as is a status from the library: the steps
-// before it have written nothing that the Python path, which then runs them all, does not write again.
+// Intermediates share one allocation.  Anything that Python would notice (hooks, another module type, a method replaced on
+// an instance or on a class, a launcher replaced in the module that calls it) or that the plain sequence does not cover is
+// declined, as is a status from the library: the steps before it have written nothing that the Python path, which then
+// runs them all, does not write again.
 #include "host_common.h"
 
 namespace {
@@ -16,9 +17,9 @@ struct Names {
            *eps = key("eps"), *input_scale = key("input_scale"), *qkv = key("_qkv"), *hidden = key("hidden"), *heads = key("heads"),
            *causal = key("causal"), *qk_alpha = key("qk_alpha"), *score_scale = key("score_scale"), *pv_alpha = key("pv_alpha"),
            *fused_attention = key("fused_attention"), *min_queries = key("fused_attention_min_queries"), *fused_residual = key("fused_residual");
-  PyObject* replaced[4] = {key("forward"), key("_launch"), key("forward_add"), key("__call__")};
+  PyObject* replaced[5] = {key("forward"), key("_launch"), key("forward_add"), key("_call_impl"), key("_compiled_call_impl")};
   PyObject* hooks[4] = {key("_forward_hooks"), key("_forward_pre_hooks"), key("_backward_hooks"), key("_backward_pre_hooks")};
-  PyObject* layer_methods[6] = {key("forward"), key("_forward_steps"), key("_qkv_pack"), key("_heads"), key("_append"), key("_kernel_takes")};
+  PyObject* layer_methods[7] = {key("forward"), key("_forward_steps"), key("_qkv_pack"), key("_heads"), key("_append"), key("_at_once"), key("_kernel_takes")};
   PyObject* steps[8] = {key("ln1"), key("q_proj"), key("k_proj"), key("v_proj"), key("out_proj"), key("ln2"), key("fc1"), key("fc2")};
 };
 const Names& names() {
@@ -50,7 +51,7 @@ PyObject* step(PyObject* modules, int i, PyObject* type) {
   PyObject* m = item(modules, names().steps[i]);
   need((PyObject*)Py_TYPE(m) == type);
   PyObject* d = dict_of(m);
-  need(none_of(d, names().replaced, 4));
+  need(none_of(d, names().replaced, 5));
   for (PyObject* h : names().hooks) {
     PyObject* hooks = item(d, h);
     need(PyDict_Check(hooks) && PyDict_Size(hooks) == 0);
@@ -110,16 +111,31 @@ struct Norm {
   }
 };
 
+// What the Python steps look up in classes and modules while they run, as (class or module dictionary, name, what was found
+// there when the package was loaded): nobody has replaced any of it.  The 41 look-ups cost 0.3 us of
+// the call's 21.
+void unchanged(PyObject* found) {
+  need(PyTuple_Check(found));
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(found); ++i) {
+    PyObject* e = PyTuple_GET_ITEM(found, i);
+    need(PyTuple_Check(e) && PyTuple_GET_SIZE(e) == 3);
+    PyObject *where = PyTuple_GET_ITEM(e, 0), *name = PyTuple_GET_ITEM(e, 1);
+    need(PyDict_Check(where) || PyType_Check(where));
+    need((PyDict_Check(where) ? PyDict_GetItem(where, name) : _PyType_Lookup((PyTypeObject*)where, name)) == PyTuple_GET_ITEM(e, 2));
+  }
+}
+
 // decoder_layer(layer, hidden, kv_cache, types, global_hooks): W8A8OPTDecoderLayer.forward without trace and marks.  types: of the layer
-// and of its eight steps; global_hooks: torch's dictionaries of hooks on every module.
+// and of its eight steps, then what unchanged() takes; global_hooks: torch's dictionaries of hooks on every module.
 PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 5, [&]() -> PyObject* {
     const Names& nm = names();
-    need(PyTuple_Check(v[3]) && PyTuple_GET_SIZE(v[3]) == 9 && PyTuple_Check(v[4]));
+    need(PyTuple_Check(v[3]) && PyTuple_GET_SIZE(v[3]) == 10 && PyTuple_Check(v[4]));
     need((PyObject*)Py_TYPE(v[0]) == PyTuple_GET_ITEM(v[3], 0));
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(v[4]); ++i) need(PyDict_Check(PyTuple_GET_ITEM(v[4], i)) && PyDict_Size(PyTuple_GET_ITEM(v[4], i)) == 0);
     PyObject* self = dict_of(v[0]);
-    need(none_of(self, nm.layer_methods, 6));
+    need(none_of(self, nm.layer_methods, 7));
+    unchanged(PyTuple_GET_ITEM(v[3], 9));
     need(flag(item(self, nm.fused_attention)) && flag(item(self, nm.fused_residual)));
     PyObject* modules = item(self, nm.modules);
     need(PyDict_Check(modules));

@@ -22,6 +22,8 @@ end-to-end tests: every heavy step is one of the package's HIP kernels, torch on
 """
 from __future__ import annotations
 
+import sys
+
 import torch
 from torch.nn.modules import module as _torch_module
 
@@ -29,6 +31,7 @@ from .. import _lib as L
 from ..kernels.bmm import bmm_s8t_s8n_s8t
 from ..kernels.fused import attention_i8, kv_append_i8, softmax_q, transpose_i8
 from ..kernels.linear import linear_group_a8_w8_b8_o8, linear_qkv_decode_a8_w8_b8_o8
+from . import fused as _fused, linear as _linear
 from .fused import DQ_Add_LayerNorm_Q, LayerNormQ, W8A8BFP32OFP32_GeLu_Q
 from .linear import W8A8B8O8Linear, W8A8B32O32LinearWithoutScaling, W8A8BFP32OFP32Linear
 
@@ -246,8 +249,22 @@ class W8A8OPTDecoderLayer(torch.nn.Module):
         return out
 
 
-# What the extension module's function stands for: exactly these types, nothing hooked into any module
+# What the extension module's function stands for: exactly these types, nothing hooked into any module, and the methods and launchers that
+# the steps above look up as they are here
+def _found(where, *names):
+    tables = [vars(c) for c in where.__mro__] if isinstance(where, type) else [vars(where)]
+    return tuple((where if isinstance(where, type) else vars(where), n, next(t[n] for t in tables if n in t)) for n in names)
+
+
+_CALL = ("__call__", "_call_impl", "_compiled_call_impl", "__getattr__", "forward")
+_UNCHANGED = (*_found(W8A8OPTDecoderLayer, "__getattr__", "_forward_steps", "_qkv_pack", "_heads", "_append", "_at_once", "_kernel_takes"),
+              *_found(LayerNormQ, *_CALL), *_found(DQ_Add_LayerNorm_Q, *_CALL), *_found(W8A8B8O8Linear, "__getattr__"),
+              *_found(W8A8B32O32LinearWithoutScaling, *_CALL, "_launch"), *_found(W8A8BFP32OFP32_GeLu_Q, *_CALL, "_launch"),
+              *_found(W8A8BFP32OFP32Linear, "__getattr__", "forward_add"),
+              *_found(sys.modules[__name__], "linear_qkv_decode_a8_w8_b8_o8", "linear_group_a8_w8_b8_o8", "kv_append_i8", "attention_i8"),
+              *_found(_fused, "layer_norm_fwd_fused_single_pass_q", "dq_add_layernorm_q_cpp", "linear_a8_w8_bfp32_ofp32_GeLu_Q"),
+              *_found(_linear, "linear_a8_w8_b32_o32", "linear_a8_w8_bfp32_ofp32_residual"))
 _TYPES = (W8A8OPTDecoderLayer, LayerNormQ, W8A8B8O8Linear, W8A8B8O8Linear, W8A8B8O8Linear, W8A8B32O32LinearWithoutScaling, DQ_Add_LayerNorm_Q,
-          W8A8BFP32OFP32_GeLu_Q, W8A8BFP32OFP32Linear)
+          W8A8BFP32OFP32_GeLu_Q, W8A8BFP32OFP32Linear, _UNCHANGED)
 _GLOBAL_HOOKS = tuple(getattr(_torch_module, name) for name in ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
                                                                 "_global_backward_pre_hooks"))
