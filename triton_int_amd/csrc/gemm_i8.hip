@@ -3195,8 +3195,8 @@ static int pick_ragged(const GemmParams& p, int64_t tiles128, int* splits_out) {
 // efficiencies were measured with weights streamed from HBM.  Outputs the persistent kernels can
 // store (row-major, aligned) go to them; the rest to the one-tile kernels.
 // may_split: whether the launch can get memory for split-K partial sums.  pick_ws weighs tile and splits together: a launch
-// that then ran its tile with whole K would leave the chip idle (768 x 4096 x 16384: 256 x 160 in 3 splits 58 us, whole K
-// on the 78 tiles 92; the 128 x 128 tile 67, by the estimate).  Elsewhere the caller drops the split and keeps the tile.
+// that then ran its tile with whole K would leave the chip idle (us, 256 x 160 in 3 splits / whole K on its 78 tiles / whole K on 128 x
+// 128: 768 x 4096 x 16384 62.0 / 102 / 69.6, 666 x 4096 x 16384 57.0 / 96.8 / 59.0).  Elsewhere the caller drops the split and keeps the tile.
 static int pick_config(const GemmParams& p, int* splits_out, bool may_split = true) {
   *splits_out = 1;
   if (!fast_eligible(p)) {
