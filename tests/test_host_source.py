@@ -39,3 +39,23 @@ def test_no_thread_local_storage(name):
     size, count = struct.unpack_from("<HH", elf, 54)
     types = [struct.unpack_from("<I", elf, table + i * size)[0] for i in range(count)]
     assert 1 in types and 7 not in types  # PT_LOAD, PT_TLS
+
+
+def test_the_layer_reads_held_tensors_without_the_interpreters_lock():
+    """Another thread may replace what a Python tensor object holds while the layer launches: every tensor that is read without the
+    lock is the copy that the call holds."""
+    src = re.sub(r"//.*", "", open(os.path.join(os.path.dirname(SOURCE), "host_layer.cpp")).read())
+    assert re.search(r"const Tensor& tensor\([^)]*\) \{[^}]*all\.push_back\(::tensor\(o, dev, type\)\);\s*return all\.back\(\);", src)
+    before, after = src.split("const NoGil unlocked;")
+    unlocked = after[:after.index("need(rc == TI_OK)")]
+    assert not re.search(r"\bPy\w+|THP\w+|\bv\[", unlocked)
+    used = set(re.findall(r"\bm?ptr\((\w+)\)", unlocked)) | set(re.findall(r"(\w+)\.sizes\(\)", unlocked))
+    own = set(re.findall(r"Tensor (\w+)(?: = c\.empty|;)", src))
+    assert src.count("held.tensor(PyTuple_GET_ITEM(v[2], ") == 2  # the caches
+    for name in used - own:
+        assert f"const Tensor& {name} = held.tensor(" in before, name
+    # references into the vector stay valid: it never grows past its inline storage
+    room = int(re.search(r"SmallVector<Tensor, (\d+)> all;", src).group(1))
+    linears, norms = 6, 2
+    caches = 2
+    assert 1 + 4 + linears * 4 + norms * 2 + caches <= room and f"need(all.size() < {room})" in src

@@ -59,18 +59,19 @@ PyObject* step(PyObject* modules, int i, PyObject* type) {
   return d;
 }
 
-// The tensors that a call reads, held until it returns: another thread may replace a module's buffer while this one launches
-// without the interpreter's lock.
+// The tensors that a call reads, held until it returns: another thread may replace a module's buffer, or what a tensor object
+// holds, while this one launches without the interpreter's lock.  The references stay valid: nothing moves within the
+// inline storage.
 struct Held {
-  c10::SmallVector<Tensor, 32> all;
+  c10::SmallVector<Tensor, 40> all;
   const Tensor& tensor(PyObject* o, int dev, ScalarType type) {
-    const Tensor& t = ::tensor(o, dev, type);
-    all.push_back(t);
-    return t;
+    need(all.size() < 40);
+    all.push_back(::tensor(o, dev, type));
+    return all.back();
   }
   const void* vector(PyObject* o, int dev, ScalarType type, int64_t n) {
     const void* at = ::vector(o, dev, type, n);
-    if (at) all.push_back(THPVariable_Unpack(o));
+    if (at) tensor(o, dev, type);
     return at;
   }
 };
@@ -192,7 +193,8 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
       k_dst = kv.k, vt_dst = kv.vt, dst_hs = kv.k_hs, dst_rs = kv.k_rs, vt_rs = kv.vt_rs;
       k = kv.k - (T - S) * kv.k_rs, vt = kv.vt - (T - S);
       k_hs = kv.k_hs, k_rs = kv.k_rs, k_ss = heads * k_hs;
-      vt_hs = THPVariable_Unpack(PyTuple_GET_ITEM(v[2], 1)).stride(0);
+      held.tensor(PyTuple_GET_ITEM(v[2], 0), c.dev, ScalarType::Char);
+      vt_hs = held.tensor(PyTuple_GET_ITEM(v[2], 1), c.dev, ScalarType::Char).stride(0);
       need(k_rs >= D && (((int64_t)k | k_hs | k_rs) & 15) == 0 && vt_rs >= T);
     }
     need(S >= min_queries || T <= 4096);
