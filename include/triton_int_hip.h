@@ -345,8 +345,8 @@ int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t
 /*
  * The same with the LayerNormQ in front in the same launch: x fp32 [M, K], unit column stride, row stride in elements, gamma
  * and beta (may be NULL) as ti_layernorm_q takes them.  The bits are those of ti_layernorm_q followed by the call above.  At
- * most 4 rows, 1024 <= K <= 5120, 16-byte aligned rows; TI_E_COMBO, with nothing done, for everything else (the
- * caller makes the two calls).
+ * most 4 rows, 1024 <= K <= 5120, 16-byte aligned rows, outputs that share no memory with x, gamma, beta or each other;
+ * TI_E_COMBO, with nothing done, for everything else (the caller makes the two calls).
  */
 int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const float* gamma, const float* beta, float eps,
                                     const int8_t* W, int64_t ldw, const int8_t* bias, const float* alpha3, const float* beta3,
@@ -357,7 +357,7 @@ int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const 
 /*
  * ti_dq_add_layernorm_q (kernels/fused.py:235-382 behind nn/fused.py:59-78) and the GELU-quant linear on its int8 rows
  * (kernels/fused.py:197-231) as one launch: resid_out = resid + in_scale * acc, C = q8(gelu(scale_a * (LN(resid_out) . W) + bias) *
- * scale_b).  Limits and TI_E_COMBO as above; also where resid_out shares memory with resid or acc.
+ * scale_b).  Limits and TI_E_COMBO as above; no output may share memory with an input or the other output.
  */
 int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_stride, float in_scale, const float* resid,
                                        int64_t resid_row_stride, const float* gamma, const float* beta, float eps,

@@ -1,0 +1,25 @@
+"""The entry points with a LayerNorm in front of a GEMM decline what only two launches compute as their header says, on the CPU."""
+import subprocess
+
+import pytest
+
+from tests.native import build_native
+
+OK, COMBO = 0, -3
+
+
+@pytest.fixture(scope="module")
+def said(tmp_path_factory):
+    program = build_native("norm_in_front.cpp", tmp_path_factory.mktemp("native"))
+    out = subprocess.run([program], capture_output=True, text=True, check=True, timeout=60).stdout
+    return {name: (int(rc), int(launches)) for name, rc, launches in (line.split() for line in out.splitlines())}
+
+
+def test_outputs_that_share_memory(said):
+    apart = {"fc1", "fc1_no_bias", "fc1_out_after_acc", "fc1_out_before_x", "qkv", "qkv_out_after_x", "qkv_k_ends_before_x"}
+    shared = [n for n in said if ("_in_" in n or "_is_" in n)]
+    assert len(shared) >= 14
+    for name in apart:
+        assert said[name] == (OK, 1), name
+    for name in shared:
+        assert said[name] == (COMBO, 0), name

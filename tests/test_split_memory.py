@@ -1,28 +1,21 @@
 """What a launch does whose K split finds no memory: it chooses among the unsplit launches, instead of running the split's tile with
-whole K (three quarters of the chip idle).  On the CPU, against the library as it is built: native/split_memory.cpp stands in for HIP."""
-import os
+whole K (three quarters of the chip idle).  On the CPU, against the library as it is built: native/fake_hip.h stands in for HIP."""
 import re
 import subprocess
 
 import pytest
 
 from tests import gemm_bounds_model as G
+from tests.native import build_native
 from triton_int_amd import _lib as L
-from triton_int_amd import build as B
 
-HERE = os.path.dirname(os.path.abspath(__file__))
 # the split choice needs more than 32 MiB of partial sums at the first four, 32 MiB at the last
 SIZES = [(666, 4096, 16384), (768, 4096, 16384), (300, 10240, 20480), (128, 20480, 20480), (384, 4096, 16384)]
 
 
 @pytest.fixture(scope="module")
 def program(tmp_path_factory):
-    out = str(tmp_path_factory.mktemp("native") / "split_memory")
-    rocm = os.path.dirname(os.path.dirname(os.path.realpath(B.HIPCC)))
-    rocm = rocm if os.path.isdir(os.path.join(rocm, "include", "hip")) else "/opt/rocm"
-    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", f"-isystem{rocm}/include", os.path.join(HERE, "native", "split_memory.cpp"), "-o", out,
-                    "-rdynamic", f"-L{B.LIB_DIR}", "-l:libtriton_int_hip.so", f"-Wl,-rpath,{B.LIB_DIR}", f"-L{rocm}/lib", f"-Wl,-rpath,{rocm}/lib", "-lamdhip64"],
-                   check=True)
+    out = build_native("split_memory.cpp", tmp_path_factory.mktemp("native"))
 
     def run(mode, room, *sizes):
         r = subprocess.run([out, mode, str(room), *(",".join(map(str, s)) for s in sizes)], capture_output=True, text=True, check=True, timeout=60)

@@ -3825,6 +3825,30 @@ static bool rows_take_norm(const ti::GemmParams& p) {
   return p.M <= ti::RPN_ROWS && p.K >= 1024 && p.K <= ti::RPN_K && ti::fast_eligible(p) && (at & 15) == 0 && (p.M == 1 || (pitch & 3) == 0);
 }
 
+// Addresses from the first to past the last byte of n1 x n2 pieces of `bytes`, s1 and s2 bytes apart
+struct Span {
+  uintptr_t lo = 0, hi = 0;
+  Span(const void* at, int64_t bytes, int64_t n1 = 1, int64_t s1 = 0, int64_t n2 = 1, int64_t s2 = 0) {
+    if (!at || bytes <= 0 || n1 <= 0 || n2 <= 0) return;
+    const int64_t e1 = (n1 - 1) * s1, e2 = (n2 - 1) * s2;
+    lo = (uintptr_t)at + (e1 < 0 ? e1 : 0) + (e2 < 0 ? e2 : 0);
+    hi = (uintptr_t)at + (e1 > 0 ? e1 : 0) + (e2 > 0 ? e2 : 0) + bytes;
+  }
+  bool meets(const Span& o) const { return lo < o.hi && o.lo < hi; }
+};
+
+// With a norm in front every workgroup reads what the norm reads, while others already store: outputs that share memory with it, or
+// with each other, are well defined in two launches only.
+static bool shares(std::initializer_list<Span> written, std::initializer_list<Span> read) {
+  for (const Span* w = written.begin(); w != written.end(); ++w) {
+    for (const Span& r : read)
+      if (w->meets(r)) return true;
+    for (const Span* v = written.begin(); v != w; ++v)
+      if (w->meets(*v)) return true;
+  }
+  return false;
+}
+
 static int qkv_decode(const ti::NormArgs& norm, const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
                       const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
                       int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
@@ -3858,6 +3882,12 @@ static int qkv_decode(const ti::NormArgs& norm, const int8_t* A, int64_t lda, co
   int splits = 1;
   const int cfg = pick_config(p, &splits);
   if (!g_configs[cfg].rows4 && !g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "operands not eligible for the decode kernel (16-byte aligned, K-contiguous)");
+  if (norm.kind) {
+    const int64_t heads = (int64_t)seqs * (N / D), row = 4 * (int64_t)K;
+    if (shares({{C, 3 * (int64_t)N, M, ldc}, {k_dst, D, heads, k_head_stride, p.kv_S, k_row_stride}, {vt_dst, p.kv_S, heads * D, vt_row_stride}},
+               {{norm.x, row, M, 4 * norm.x_rs}, {norm.gamma, row}, {norm.beta, row}}))
+      return fail(TI_E_COMBO, "an output lies in what the LayerNorm reads");
+  }
   if (norm.kind && !(rows_take_norm(p) && g_configs[cfg].rowpieces)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
   return run(p, cfg, (hipStream_t)stream);
 }
@@ -3884,12 +3914,10 @@ int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_strid
                                        const float* bias, const float* scale_a, const float* scale_b, int8_t* C, int64_t ldc, int M, int N, int K, void* stream) {
   using namespace ti;
   if (M > 0 && (!acc || !resid || !gamma || !resid_out)) return fail(TI_E_NULL, "acc, resid, gamma and resid_out are required");
-  // every workgroup reads all of acc and resid while the first one writes resid_out
-  const auto meets = [&](const void* q, int64_t rs) {
-    const uintptr_t a = (uintptr_t)resid_out, b = (uintptr_t)q;
-    return M > 0 && a < b + 4 * ((M - 1) * rs + K) && b < a + 4 * ((M - 1) * resid_out_row_stride + K);
-  };
-  if (meets(acc, acc_row_stride) || meets(resid, resid_row_stride)) return fail(TI_E_COMBO, "resid_out lies in acc or resid");
+  const int64_t row = 4 * (int64_t)K;
+  if (shares({{resid_out, row, M, 4 * resid_out_row_stride}, {C, N, M, ldc}},
+             {{acc, row, M, 4 * acc_row_stride}, {resid, row, M, 4 * resid_row_stride}, {gamma, row}, {beta, row}, {W, K, N, ldw}, {bias, 4 * (int64_t)N}, {scale_a, 4}, {scale_b, 4}}))
+    return fail(TI_E_COMBO, "an output lies in what the launch reads");
   GemmParams p;
   p.norm.kind = NORM_DQ_ADD_LN;
   p.norm.x = resid; p.norm.x_rs = resid_row_stride;
