@@ -61,5 +61,14 @@ int main() {
   with<Qkv>("qkv_k_ends_in_x", [](Qkv& t) { t.k = t.x - (2 * 8 - 1) * 64 * 128 - 112; });
   with<Qkv>("qkv_k_ends_before_x", [](Qkv& t) { t.k = t.x - (2 * 8 - 1) * 64 * 128 - 128; });
   with<Qkv>("qkv_v_in_beta", [](Qkv& t) { t.v = t.beta + 16; });
+  for (int m = 1; m <= 2; ++m) {
+    const char* const names[2][5] = {{"fc1_one_row", "fc1_one_row_odd_x", "fc1_one_row_odd_acc", "fc1_one_row_odd_resid_out", "qkv_one_row_odd_x"},
+                                     {"fc1_two_rows", "fc1_two_rows_odd_x", "fc1_two_rows_odd_acc", "fc1_two_rows_odd_resid_out", "qkv_two_rows_odd_x"}};
+    with<Fc1>(names[m - 1][0], [=](Fc1& t) { t.M = m, t.x_rs += 4, t.acc_rs += 8, t.ro_rs += 12; });
+    with<Fc1>(names[m - 1][1], [=](Fc1& t) { t.M = m, t.x_rs += 2; });
+    with<Fc1>(names[m - 1][2], [=](Fc1& t) { t.M = m, t.acc_rs += 1; });
+    with<Fc1>(names[m - 1][3], [=](Fc1& t) { t.M = m, t.ro_rs += 3; });
+    with<Qkv>(names[m - 1][4], [=](Qkv& t) { t.M = t.seqs = m, t.x_rs += 2; });
+  }
   return 0;
 }

@@ -23,3 +23,10 @@ def test_outputs_that_share_memory(said):
         assert said[name] == (OK, 1), name
     for name in shared:
         assert said[name] == (COMBO, 0), name
+
+
+def test_pitches_of_whole_pieces(said):
+    """The separate norm sums rows at other pitches in another order, a single row among them."""
+    for name, got in said.items():
+        if "_row" in name:
+            assert got == ((COMBO, 0) if "_odd_" in name else (OK, 1)), name

@@ -3816,13 +3816,14 @@ int ti_bmm_i8_grouped(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, co
   return ti::run(p, config, (hipStream_t)stream);
 }
 
-// Whether gemm_rowpieces_kernel can make these activations from their LayerNorm: few rows, whole 16-byte pieces of every row
+// Whether gemm_rowpieces_kernel can make these activations from their LayerNorm: few rows, whole 16-byte pieces of every row, and
+// the pitches that rownorm_vec_kernel takes, a single row's too: rownorm_any_kernel sums in another order
 static bool rows_take_norm(const ti::GemmParams& p) {
   const ti::NormArgs& a = p.norm;
   const bool dq = a.kind == ti::NORM_DQ_ADD_LN;
   const uintptr_t at = (uintptr_t)a.x | (uintptr_t)a.gamma | (uintptr_t)a.beta | (dq ? (uintptr_t)a.acc | (uintptr_t)a.resid_out : 0);
   const int64_t pitch = a.x_rs | (dq ? a.acc_rs | a.rout_rs : 0);
-  return p.M <= ti::RPN_ROWS && p.K >= 1024 && p.K <= ti::RPN_K && ti::fast_eligible(p) && (at & 15) == 0 && (p.M == 1 || (pitch & 3) == 0);
+  return p.M <= ti::RPN_ROWS && p.K >= 1024 && p.K <= ti::RPN_K && ti::fast_eligible(p) && (at & 15) == 0 && (pitch & 3) == 0;
 }
 
 // Addresses from the first to past the last byte of n1 x n2 pieces of `bytes`, s1 and s2 bytes apart

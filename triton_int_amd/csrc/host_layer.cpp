@@ -200,7 +200,7 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need(S >= min_queries || T <= 4096);
     const int T32 = int32_size(T);
 
-    const bool few = M <= 4 && H >= 1024 && ((x_rs & 3) == 0 || M == 1) && (((uintptr_t)ptr(x) | (uintptr_t)ln1.g | (uintptr_t)ln1.b | (uintptr_t)ln2.g |
+    const bool few = M <= 4 && H >= 1024 && (x_rs & 3) == 0 && (((uintptr_t)ptr(x) | (uintptr_t)ln1.g | (uintptr_t)ln1.b | (uintptr_t)ln2.g |
                                                                               (uintptr_t)ln2.b) & 15) == 0;  // the norms go into the launches after them
     int rc = TI_OK;
     Tensor out;
