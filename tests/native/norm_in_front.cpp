@@ -70,5 +70,8 @@ int main() {
     with<Fc1>(names[m - 1][3], [=](Fc1& t) { t.M = m, t.ro_rs += 3; });
     with<Qkv>(names[m - 1][4], [=](Qkv& t) { t.M = t.seqs = m, t.x_rs += 2; });
   }
+  with<Fc1>("fc1_no_columns", [](Fc1& t) { t.N = 0; });
+  with<Fc1>("fc1_empty", [](Fc1& t) { t.M = 0; });
+  with<Fc1>("fc1_empty_no_columns", [](Fc1& t) { t.M = t.N = 0; });
   return 0;
 }

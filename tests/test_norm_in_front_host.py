@@ -30,3 +30,9 @@ def test_pitches_of_whole_pieces(said):
     for name, got in said.items():
         if "_row" in name:
             assert got == ((COMBO, 0) if "_odd_" in name else (OK, 1)), name
+
+
+def test_no_columns(said):
+    """The residual is an output whatever the number of columns: without any, the separate launches write it."""
+    assert said["fc1_no_columns"] == (COMBO, 0)
+    assert said["fc1_empty"] == said["fc1_empty_no_columns"] == (OK, 0)

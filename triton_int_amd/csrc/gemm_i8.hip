@@ -3940,7 +3940,8 @@ int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_strid
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   int rc = validate(p);
   if (rc != TI_OK) return rc;
-  if (M == 0 || N == 0) return TI_OK;
+  if (M == 0) return TI_OK;
+  if (N == 0) return fail(TI_E_COMBO, "no columns: resid_out is left to the separate launches");
   int splits = 1;
   if (!rows_take_norm(p)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
   const int cfg = pick_config(p, &splits);
