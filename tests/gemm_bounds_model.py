@@ -112,26 +112,31 @@ def plan_for(lib, pr: Problem, epilogue: int, bias_kind: int, config: int = -1, 
     return p
 
 
-def _check_rowpieces_ring(pr: Problem, MT, KC, G, per, workgroups):
+def _check_rowpieces_ring(pr: Problem, MT, KC, G, per, workgroups, norm=False):
     """The LDS ring of gemm_rowpieces_kernel: stages of packed 1 KB pieces, what producers and consumers touch of it, and
-    that every 16-byte chunk of K is staged once and lies where the consumers read it."""
+    that every 16-byte chunk of K is staged once and lies where the consumers read it.  norm: the activations, made from their
+    LayerNorm, lie behind the ring as a whole, and the stages hold weights only."""
     LDS, PW, NST = 160 * 1024, 4, 32
+    if norm:
+        LDS -= _check_norm_rows(pr, KC, workgroups)
     assert KC in (256, 512, 1024) and 4 * (G - 1) < per <= 4 * G
     CH, RPI = KC // 16, 1024 // KC  # chunks of a row in a stage, rows of a piece
     assert MT % (RPI * PW) == 0 and per * 4 % RPI == 0
-    pieces_a = -(-pr.M // 4) * 4 // RPI if MT == 16 else MT // RPI
+    pieces_a = 0 if norm else -(-pr.M // 4) * 4 // RPI if MT == 16 else MT // RPI
     pieces_w = per * 4 // RPI
-    assert pieces_a * RPI >= pr.M, "activation rows without a piece"
+    assert norm or pieces_a * RPI >= pr.M, "activation rows without a piece"
     stage = (pieces_a + pieces_w) * 1024
     most = -(-(pieces_a + pieces_w) // PW)
-    depth = min((LDS - (MT + 16 * G) * KC) // stage, 63 // most, NST - 1)
+    depth = min((LDS - ((0 if norm else MT) + 16 * G) * KC) // stage, 63 // most, NST - 1)
     assert depth >= 1 and depth * most <= 63, "loads in flight do not fit the counter"
     # the last stage: what is staged, and what the operand reads take (whole groups of 16 rows)
     last = depth * stage
-    assert last + stage <= LDS and last + MT * KC <= LDS and last + pieces_a * 1024 + 16 * G * KC <= LDS, "a stage reaches past the LDS"
+    assert last + stage <= LDS and (norm or last + MT * KC <= LDS) and last + pieces_a * 1024 + 16 * G * KC <= LDS, "a stage reaches past the LDS"
     # a producer wave's pieces: within the instantiated counts, every piece of a stage exactly once
     a_max, w_min, w_max = MT // RPI // PW, (16 * G - 12) // RPI // PW, 16 * G // RPI // PW
     a_min = a_max // 4 if MT == 16 else a_max
+    if norm:
+        a_min = a_max = 0
     got_a, got_w = [], []
     for pw in range(PW):
         mine_a = (pieces_a - pw + PW - 1) // PW
@@ -157,6 +162,46 @@ def _check_rowpieces_ring(pr: Problem, MT, KC, G, per, workgroups):
             assert np.array_equal(np.sort(staged), np.arange(blocks * 16)), "a chunk of K is not staged exactly once"
             slot = np.arange(CH) ^ (row & 15)
             assert np.array_equal(slot // 16, np.arange(CH) // 16) and np.array_equal((slot & 15) ^ (row & 15), np.arange(CH) & 15)
+
+
+def _check_norm_rows(pr: Problem, KC, workgroups):
+    """The int8 rows that a norm in front leaves behind the ring, and the fp32 sums of its waves after them: what is loaded, written and
+    read, and that a consumer's operand is the K that its weights are.  Returns the bytes of LDS they take."""
+    ROWS, THREADS, WAVES = 4, 256, 4
+    assert 1 <= pr.M <= ROWS and 1024 <= pr.K <= 5120 and pr.K % 16 == 0
+    blocks = -(-pr.K // 256)
+    pitch, vectors = blocks * 256 + 64, 4 if pr.K <= 4096 else 5
+    # a thread's vectors of four: every one of a row's, those past its end dropped by the descriptor's extent of 4 * K bytes
+    vec = np.arange(THREADS * vectors, dtype=np.int64)
+    assert vec.size * 4 >= pr.K and pr.K % 4 == 0
+    inside = vec * 16 + 16 <= pr.K * 4
+    assert np.array_equal(inside, vec < pr.K // 4), "a vector is half inside its row"
+    assert (vec[vec < pr.K // 4] * 4 + 4 <= pr.K).all() and pr.K <= pitch, "an int8 piece is written past its row"
+    size = ROWS * pitch + 2 * ROWS * WAVES * 4
+    assert (ROWS * pitch) % 4 == 0 and ((2 * ROWS - 1) * WAVES + WAVES) * 4 <= 2 * ROWS * WAVES * 4 and (160 * 1024 - size) % 16 == 0
+    # the consumers' reads: 64 bytes of K a step, KC / 64 of them a stage; slot j of a stage is chunk j of the workgroup's walk
+    for lin in {0, 1, 7, 8, workgroups - 1}:
+        rot = ((lin >> 3) + (lin & 7) * (blocks * 256 >> 11)) % blocks
+        at = np.arange(-(-pr.K // KC) * KC, step=64, dtype=np.int64)
+        kk = np.where(at >= blocks * 256, 0, np.where(at + rot * 256 >= blocks * 256, at + rot * 256 - blocks * 256, at + rot * 256))
+        byte = kk[:, None] + np.arange(4)[None, :] * 16
+        assert byte.min() >= 0 and byte.max() + 16 <= pitch, "an operand read leaves its row"
+        slot = at[:, None] // 16 + np.arange(4)[None, :]  # of the walk
+        live = slot // 16 < blocks
+        assert np.array_equal(byte[live], (((slot // 16 + rot) % blocks) * 256 + slot % 16 * 16)[live]), "activations and weights of different K"
+    return size
+
+
+def check_norm_in_front(batch, M, N, K):
+    """A launch of gemm_rowpieces_kernel with a norm in front: the host's split of N and choice of stage length, then the LDS.  Returns the
+    weight rows' share (in groups of 16) and the stage length."""
+    units, wgs = -(-N // 4), 256 // batch
+    rounds = -(-units // (wgs * 20))
+    per = -(-units // (wgs * rounds))
+    blocks, G = -(-units // per), -(-per // 4)
+    KC = 1024 if G <= 2 else 512 if G == 3 else 256
+    _check_rowpieces_ring(contiguous(batch, M, N, K, 0), 16, KC, G, per, blocks * batch, norm=True)
+    return G, KC
 
 
 # ---- tile order ---------------------------------------------------------------------------------

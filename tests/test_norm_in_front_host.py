@@ -3,6 +3,7 @@ import subprocess
 
 import pytest
 
+from tests import gemm_bounds_model as G
 from tests.native import build_native
 
 OK, COMBO = 0, -3
@@ -36,3 +37,16 @@ def test_no_columns(said):
     """The residual is an output whatever the number of columns: without any, the separate launches write it."""
     assert said["fc1_no_columns"] == (COMBO, 0)
     assert said["fc1_empty"] == said["fc1_empty_no_columns"] == (OK, 0)
+
+
+@pytest.mark.parametrize("K", [1024, 1040, 1264, 1280, 2000, 4080, 4096, 4112, 5104, 5120])
+def test_lds_of_every_share_of_the_weights(K):
+    """Every kernel with a norm in front, at every number of rows and of units per workgroup, one GEMM and three grouped."""
+    seen = set()
+    for batch in (1, 3):
+        wgs = 256 // batch
+        for per in range(1, 21):
+            for N in (per * wgs * 4, per * wgs * 4 - 5):
+                for M in range(1, 5):
+                    seen.add(G.check_norm_in_front(batch, M, N, K))
+    assert seen == {(1, 1024), (2, 1024), (3, 512), (4, 256), (5, 256)}
