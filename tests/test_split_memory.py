@@ -62,3 +62,34 @@ def test_no_memory_for_a_workspace(program):
     assert first[0] == 0 and first[2] > 1 and first[4] == room
     assert second[0] == 0 and second[2] == 1 and second[4] == room
     assert third == (0, first[1], first[2], 1, room)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(100, 1024, 4096), (300, 1024, 8192), (666, 512, 16384)])
+def test_captured_without_a_workspace(M, N, K):
+    """On a stream that never split K: the unsplit choice's outputs, with and without a residual, at every replay."""
+    import torch
+
+    from triton_int_amd.kernels.linear import linear_a8_w8_b32_o32, linear_a8_w8_bfp32_ofp32_residual
+    lib, dev = L.lib(), torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, w = (torch.randint(-127, 128, s, dtype=torch.int8, device=dev, generator=g) for s in ((M, K), (N, K)))
+    bias, resid = torch.randn(N, device=dev, generator=g), torch.randn(M, N, device=dev, generator=g)
+    al, be = torch.tensor(2.0e-4, device=dev), torch.tensor(0.5, device=dev)
+    want, want_r = linear_a8_w8_b32_o32(a, w, None), linear_a8_w8_bfp32_ofp32_residual(a, w, bias, al, be, resid)
+    assert lib.ti_gemm_last_splits() > 1
+    assert torch.equal(want.double(), a.double() @ w.double().t())
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    L.release_workspaces(all_streams=True)
+    with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+        got = linear_a8_w8_b32_o32(a, w, None)
+        assert lib.ti_gemm_last_splits() == 1
+        got_r = linear_a8_w8_bfp32_ofp32_residual(a, w, bias, al, be, resid)
+        assert lib.ti_gemm_last_splits() == 1
+    for _ in range(3):
+        got.zero_(), got_r.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        assert torch.equal(got, want) and torch.equal(got_r, want_r)
+        torch.cuda.synchronize()

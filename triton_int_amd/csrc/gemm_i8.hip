@@ -2513,7 +2513,9 @@ __device__ __forceinline__ void rowpieces_store(const GemmParams& p, const EpiCt
 // producers fill the stages with weights: int8 rows of `pitch` bytes at x8.  The statistics are those of rownorm_vec_kernel (256
 // threads, the same order of every sum), so the bits are too.  `red`: 2 x RPN_ROWS x RP_CW floats.
 // Joins two barriers; the caller's next one publishes x8.
-constexpr int RPN_ROWS = 4, RPN_K = 5120;  // more of either do not fit the registers
+// One limit for rows and one for K, although the registers hold rows x K: four rows of 5120 are what fits (20 vectors of x a thread, and as
+// many of acc).  Fewer rows of a longer K would fit as well; no kernel is built for them.
+constexpr int RPN_ROWS = 4, RPN_K = 5120;
 template <int KIND, int VPT>
 __device__ __forceinline__ void rowpieces_norm(const GemmParams& p, char* x8, int pitch, float* red, int tid, bool store_resid) {
   static_assert(RP_CW * 64 == 256, "the threads of rownorm_vec_kernel");
