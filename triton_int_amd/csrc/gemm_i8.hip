@@ -39,7 +39,7 @@ __device__ unsigned long long g_timeline[1024 * 8];
 // resid_out), normalised and quantised as in rownorm_vec_kernel.
 enum NormKind { NORM_NONE = 0, NORM_LN, NORM_DQ_ADD_LN };
 struct NormArgs {
-  int kind = NORM_NONE;
+  int kind;
   const float* x;  // NORM_DQ_ADD_LN: the residual
   const int32_t* acc;
   float* resid_out;
@@ -82,8 +82,15 @@ struct GemmParams {
   int splits, kt_split;
   int* sk_partial;   // [tile][split][consumer wave][accumulator dword][lane]
   int* sk_counter;   // [tile][consumer wave], zero between launches
+};
+
+// The arguments of the kernels with a norm in front.  The others do not carry them: 80 more bytes of arguments cost a short launch 0.2 us
+// (354 x 320 x 561 on gemm_ragged_kernel 7.13 / 7.36).
+struct GemmNormParams : GemmParams {
   NormArgs norm;
 };
+template <int NORM>
+using RowpiecesParams = typename std::conditional<NORM == NORM_NONE, GemmParams, GemmNormParams>::type;
 
 enum OutClass { OUT8 = 0, OUT32 = 1, OUT16 = 2 };
 
@@ -2509,7 +2516,7 @@ __device__ __forceinline__ void rowpieces_store(const GemmParams& p, const EpiCt
   }
 }
 
-// The activations of up to RPN_ROWS rows from their LayerNorm (p.norm), by the consumer waves of every workgroup, while the
+// The activations of up to RPN_ROWS rows from their LayerNorm, by the consumer waves of every workgroup, while the
 // producers fill the stages with weights: int8 rows of `pitch` bytes at x8.  The statistics are those of rownorm_vec_kernel (256
 // threads, the same order of every sum), so the bits are too.  `red`: 2 x RPN_ROWS x RP_CW floats.
 // Joins two barriers; the caller's next one publishes x8.
@@ -2517,7 +2524,7 @@ __device__ __forceinline__ void rowpieces_store(const GemmParams& p, const EpiCt
 // many of acc).  Fewer rows of a longer K would fit as well; no kernel is built for them.
 constexpr int RPN_ROWS = 4, RPN_K = 5120;
 template <int KIND, int VPT>
-__device__ __forceinline__ void rowpieces_norm(const GemmParams& p, char* x8, int pitch, float* red, int tid, bool store_resid) {
+__device__ __forceinline__ void rowpieces_norm(const GemmNormParams& p, char* x8, int pitch, float* red, int tid, bool store_resid) {
   static_assert(RP_CW * 64 == 256, "the threads of rownorm_vec_kernel");
   const NormArgs& a = p.norm;
   const unsigned bytes = (unsigned)p.K * 4u;
@@ -2615,7 +2622,7 @@ __device__ __forceinline__ void rowpieces_norm(const GemmParams& p, char* x8, in
 }
 
 template <int MT, int G, int KC, int NORM = NORM_NONE, int VPT = 1>
-__global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(GemmParams p) {
+__global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(RowpiecesParams<NORM> p) {
   constexpr int MB = MT / 16, CH = KC / 16, RPI = 1024 / KC;        // RPI: rows per load instruction
   constexpr int KPW = KC / 64 / RP_CW;                              // 64-deep k-steps of a consumer wave per stage
   constexpr int WAVE_RED = MB * 4 * G * 17 * 16;                    // a wave's sums, 16-byte pieces padded against bank conflicts
@@ -2797,6 +2804,7 @@ __global__ __launch_bounds__((RP_PW + RP_CW) * 64) void gemm_rowpieces_kernel(Ge
 // ---- host side ---------------------------------------------------------------------------------
 
 typedef void (*KernelFn)(GemmParams);
+typedef void (*NormKernelFn)(GemmNormParams);
 
 struct Config {
   const char* name;
@@ -2918,8 +2926,8 @@ static KernelFn rowpieces_kernel(int mt, int g, int kc) {
 
 // gemm_rowpieces_kernel with a norm in front: up to 16 * g weight rows per workgroup, K up to RPN_K.  Stages as long as the
 // LDS beside the activations allows.
-static KernelFn rowpieces_norm_kernel(int kind, int g, int K) {
-  KernelFn fn = nullptr;
+static NormKernelFn rowpieces_norm_kernel(int kind, int g, int K) {
+  NormKernelFn fn = nullptr;
   const auto pick = [&](auto kind_tag, auto vpt_tag) {
     with_count<1, RP_GMAX>(g, [&](auto g_tag) {
       constexpr int G = decltype(g_tag)::value, KC = G <= 2 ? 1024 : G == 3 ? 512 : RP_KC;
@@ -3511,7 +3519,9 @@ struct LaunchPlan {
 // dry: every decision is taken as for a launch (same code), but no device is touched, nothing is
 // allocated or launched, and *dry receives the launch's configuration and grid.
 // may_split: a configuration that is chosen here may split K; false where a first choice found no memory for the split.
-static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch = false, LaunchPlan* dry = nullptr, bool may_split = true) {
+// norm: makes the activations (gemm_rowpieces_kernel only; the caller has asked rows_take_norm).
+static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch = false, LaunchPlan* dry = nullptr, bool may_split = true,
+               const NormArgs* norm = nullptr) {
   g_last_splits = 1;
   int want_splits = config < 0 ? 0 : (config >> 8) & 0xff;
   if (config >= 0) config = (config & 0xff) == 0xff ? -1 : (config & 0xff);
@@ -3604,15 +3614,24 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
     const int g = (per + 3) / 4;
     // forced by a test: bytes of K per stage, divided by 256
     const int kc = want_splits ? want_splits * 256 : (k.bm <= 32 && rowpieces_fits(k.bm, g, 1024) ? 1024 : (g <= 3 && rowpieces_fits(k.bm, g, 512) ? 512 : RP_KC));
-    const KernelFn fn = p.norm.kind ? rowpieces_norm_kernel(p.norm.kind, g, p.K) : rowpieces_kernel(k.bm, g, kc);
-    if (!fn) return fail(TI_E_COMBO, "config %s: no stages of %d bytes of K for %d weight rows per workgroup", k.name, kc, per * 4);
+    const KernelFn fn = norm ? nullptr : rowpieces_kernel(k.bm, g, kc);
+    const NormKernelFn norm_fn = norm ? rowpieces_norm_kernel(norm->kind, g, p.K) : nullptr;
+    if (!fn && !norm_fn) return fail(TI_E_COMBO, "config %s: no stages of %d bytes of K for %d weight rows per workgroup", k.name, kc, per * 4);
     g_last_config = config;
     if (dry) {
       dry->config = config; dry->grid_x = (unsigned)blocks; dry->grid_y = (unsigned)p.batch; dry->threads = k.threads;
       dry->ksplit = g; dry->nwa = kc;
       return TI_OK;
     }
-    fn<<<dim3((unsigned)blocks, (unsigned)p.batch), dim3(k.threads), 0, stream>>>(p);
+    const dim3 grid((unsigned)blocks, (unsigned)p.batch);
+    if (norm) {
+      GemmNormParams q;
+      static_cast<GemmParams&>(q) = p;
+      q.norm = *norm;
+      norm_fn<<<grid, dim3(k.threads), 0, stream>>>(q);
+    } else {
+      fn<<<grid, dim3(k.threads), 0, stream>>>(p);
+    }
     return launch_status(k.name);
   }
   if (k.skinny) {
@@ -3820,8 +3839,7 @@ int ti_bmm_i8_grouped(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, co
 
 // Whether gemm_rowpieces_kernel can make these activations from their LayerNorm: few rows, whole 16-byte pieces of every row, and
 // the pitches that rownorm_vec_kernel takes, a single row's too: rownorm_any_kernel sums in another order
-static bool rows_take_norm(const ti::GemmParams& p) {
-  const ti::NormArgs& a = p.norm;
+static bool rows_take_norm(const ti::GemmParams& p, const ti::NormArgs& a) {
   const bool dq = a.kind == ti::NORM_DQ_ADD_LN;
   const uintptr_t at = (uintptr_t)a.x | (uintptr_t)a.gamma | (uintptr_t)a.beta | (dq ? (uintptr_t)a.acc | (uintptr_t)a.resid_out : 0);
   const int64_t pitch = a.x_rs | (dq ? a.acc_rs | a.rout_rs : 0);
@@ -3852,7 +3870,7 @@ static bool shares(std::initializer_list<Span> written, std::initializer_list<Sp
   return false;
 }
 
-static int qkv_decode(const ti::NormArgs& norm, const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+static int qkv_decode(const ti::NormArgs* norm, const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
                       const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
                       int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
                       int D, void* stream) {
@@ -3862,7 +3880,6 @@ static int qkv_decode(const ti::NormArgs& norm, const int8_t* A, int64_t lda, co
   if (!k_dst || !vt_dst) return fail(TI_E_NULL, "k_dst and vt_dst are required");
   if (((uintptr_t)k_dst & 3) || (k_head_stride & 3) || (k_row_stride & 3)) return fail(TI_E_STRIDE, "k_dst and its strides must be multiples of 4 bytes");
   GemmParams p;
-  p.norm = norm;
   p.A = A; p.B = W; p.C = C;
   p.sAb = 0; p.sAm = lda; p.sAk = 1;
   p.sBb = (int64_t)N * ldw; p.sBn = ldw; p.sBk = 1;
@@ -3885,21 +3902,21 @@ static int qkv_decode(const ti::NormArgs& norm, const int8_t* A, int64_t lda, co
   int splits = 1;
   const int cfg = pick_config(p, &splits);
   if (!g_configs[cfg].rows4 && !g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "operands not eligible for the decode kernel (16-byte aligned, K-contiguous)");
-  if (norm.kind) {
+  if (norm) {
     const int64_t heads = (int64_t)seqs * (N / D), row = 4 * (int64_t)K;
     if (shares({{C, 3 * (int64_t)N, M, ldc}, {k_dst, D, heads, k_head_stride, p.kv_S, k_row_stride}, {vt_dst, p.kv_S, heads * D, vt_row_stride}},
-               {{norm.x, row, M, 4 * norm.x_rs}, {norm.gamma, row}, {norm.beta, row}}))
+               {{norm->x, row, M, 4 * norm->x_rs}, {norm->gamma, row}, {norm->beta, row}}))
       return fail(TI_E_COMBO, "an output lies in what the LayerNorm reads");
+    if (!rows_take_norm(p, *norm) || !g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
   }
-  if (norm.kind && !(rows_take_norm(p) && g_configs[cfg].rowpieces)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
-  return run(p, cfg, (hipStream_t)stream);
+  return run(p, cfg, (hipStream_t)stream, false, nullptr, true, norm);
 }
 
 int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
                           const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
                           int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst, int64_t vt_row_stride,
                           int D, void* stream) {
-  return qkv_decode(ti::NormArgs{}, A, lda, W, ldw, bias, alpha3, beta3, C, ldc, seqs, M, N, K, k_dst, k_head_stride, k_row_stride, vt_dst, vt_row_stride, D, stream);
+  return qkv_decode(nullptr, A, lda, W, ldw, bias, alpha3, beta3, C, ldc, seqs, M, N, K, k_dst, k_head_stride, k_row_stride, vt_dst, vt_row_stride, D, stream);
 }
 
 int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const float* gamma, const float* beta, float eps, const int8_t* W, int64_t ldw,
@@ -3909,7 +3926,7 @@ int ti_layernorm_qkv_decode_i8_seqs(const float* x, int64_t x_row_stride, const 
   ti::NormArgs n{};
   n.kind = ti::NORM_LN;
   n.x = x; n.x_rs = x_row_stride; n.gamma = gamma; n.beta = beta; n.eps = eps;
-  return qkv_decode(n, (const int8_t*)x, K, W, ldw, bias, alpha3, beta3, C, ldc, seqs, M, N, K, k_dst, k_head_stride, k_row_stride, vt_dst, vt_row_stride, D, stream);
+  return qkv_decode(&n, (const int8_t*)x, K, W, ldw, bias, alpha3, beta3, C, ldc, seqs, M, N, K, k_dst, k_head_stride, k_row_stride, vt_dst, vt_row_stride, D, stream);
 }
 
 int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_stride, float in_scale, const float* resid, int64_t resid_row_stride, const float* gamma,
@@ -3922,11 +3939,12 @@ int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_strid
              {{acc, row, M, 4 * acc_row_stride}, {resid, row, M, 4 * resid_row_stride}, {gamma, row}, {beta, row}, {W, K, N, ldw}, {bias, 4 * (int64_t)N}, {scale_a, 4}, {scale_b, 4}}))
     return fail(TI_E_COMBO, "an output lies in what the launch reads");
   GemmParams p;
-  p.norm.kind = NORM_DQ_ADD_LN;
-  p.norm.x = resid; p.norm.x_rs = resid_row_stride;
-  p.norm.acc = acc; p.norm.acc_rs = acc_row_stride; p.norm.in_scale = in_scale;
-  p.norm.resid_out = resid_out; p.norm.rout_rs = resid_out_row_stride;
-  p.norm.gamma = gamma; p.norm.beta = beta; p.norm.eps = eps;
+  NormArgs norm{};
+  norm.kind = NORM_DQ_ADD_LN;
+  norm.x = resid; norm.x_rs = resid_row_stride;
+  norm.acc = acc; norm.acc_rs = acc_row_stride; norm.in_scale = in_scale;
+  norm.resid_out = resid_out; norm.rout_rs = resid_out_row_stride;
+  norm.gamma = gamma; norm.beta = beta; norm.eps = eps;
   p.A = (const int8_t*)resid; p.B = W; p.C = C;
   p.sAb = 0; p.sAm = K; p.sAk = 1;
   p.sBb = 0; p.sBn = ldw; p.sBk = 1;
@@ -3945,10 +3963,10 @@ int ti_dq_add_layernorm_linear_gelu_i8(const int32_t* acc, int64_t acc_row_strid
   if (M == 0) return TI_OK;
   if (N == 0) return fail(TI_E_COMBO, "no columns: resid_out is left to the separate launches");
   int splits = 1;
-  if (!rows_take_norm(p)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
+  if (!rows_take_norm(p, norm)) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for these operands");
   const int cfg = pick_config(p, &splits);
   if (!g_configs[cfg].rowpieces) return fail(TI_E_COMBO, "no kernel with a LayerNorm in front for this size");
-  return run(p, cfg, (hipStream_t)stream);
+  return run(p, cfg, (hipStream_t)stream, false, nullptr, true, &norm);
 }
 
 int ti_qkv_decode_i8(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
