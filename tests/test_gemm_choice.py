@@ -93,3 +93,15 @@ def test_sizes_beyond_the_measured_ones():
         pl = G.plan_for(lib, pr, L.EPI_SCALE_F, 3)
         assert pl.name.startswith(name) and pl.splits == splits, (M, N, K, pl)
         G.check_launch(pr, pl, store_sample=2)
+
+
+@pytest.mark.parametrize("M,N,K", [(1036, 4096, 16384), (1234, 4096, 16384), (799, 4096, 16384), (395, 4096, 16384), (427, 4096, 16384), (666, 4096, 16384), (100, 5120, 20480)])
+def test_splits_fill_one_round(M, N, K):
+    """No more items than CUs; 395 and 427 rows are the ones that 256 x 128 tiles in four splits lost to 128 x 128 tiles in two."""
+    lib = L.lib()
+    pr = G.contiguous(1, M, N, K, 2)
+    pl = G.plan_for(lib, pr, L.EPI_SCALE_F, 3)
+    assert pl.splits == 1 or pl.tiles_m * pl.tiles_n * pl.splits <= 256, pl
+    assert M not in (395, 427) or (pl.name.startswith("ws_128x128") and pl.splits == 2), pl
+    assert M < 1000 or (pl.name.startswith("ws_256x128") and pl.splits == 1), pl
+    G.check_launch(pr, pl, store_sample=4)

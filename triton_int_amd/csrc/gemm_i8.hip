@@ -3107,15 +3107,18 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
 // this: 100 x 4096 x 4096 16.2 / 11.5, 200 x 4096 x 4096 21.9 / 13.8, 384 x 4096 x 4096 21.2 / 16.7, 300 x 1024 x 4096 15.0 / 10.0, 128 x
 // 20480 x 5120 48 / 34, 160 x 5120 x 5120 25.2 / 16.1, 1000 x 5120 x 20480 122 / 102, three grouped 100 x 4096 x 4096 20.7 / 17.3.
 // Where it loses (3 % and more at 23 of them): 384 x 2048 x 2048 9.1 / 10.2, 140 x 4096 x 11008 22.0 / 24.4.
-// Checked on 1451 other sizes, with the 64 x 64 tile of gemm_mfma_kernel (below) and the 256 x 256 tile beside it: M up to 16384, N from
-// 256 and K from 1024 up to 20480, one GEMM and 2 .. 4 grouped, every output type, K a multiple of 128 and not.  Choice / fastest 1.008 on
-// average; choice / the estimate's choice 0.91 (M > 3000 0.97, 16-bit outputs 0.92, 2 and 4 grouped 0.90, K = 1024 0.97), more than 1.04 at
-// 30 of them: 136 x 8112 x 5536 24.0 / 28.9, 343 x 7248 x 2048 three times 26.4 / 30.2, 3 x 571 x 4096 x 4096 int8 38.9 / 43.9, 264 x 20480 x 5120
-// int8 48.9 / 53.3, 128 x 16384 x 1024 8.7 / 9.5.  The 256 x 256 tile, no candidate, leads by more than 3 % at 20 of 327 (547 x 6752 x 9824
-// three times 143 / 170).  Left to config_cost: K < 1024, where rounds are mostly epilogue; more
-// than 20480 columns (config_cost's choice / this one's: 300 x 50272 x 1024 39.8 / 47.7, 300 x 50272 x 4096 97 / 107, 384 x 50272 x 2048 59.2 / 64.7;
-// up to 128 rows the same); K beyond 28672 (4096 x 28672 1.08 above the fastest / 1.02, 5120 x 24576 1.03 / 1.02, 11264 x 32768 1.01 / 1.01).
-// M has no end: 17000 .. 32768 rows 1.025 / 1.004.
+// Checked on 1931 other sizes, with the 64 x 64 tile of gemm_mfma_kernel (below) and the 256 x 256 tile beside it: M up to 16384, N from
+// 256 and K from 1024 up to 20480, one GEMM and 2 .. 4 grouped, every output type, K a multiple of 128 and not, and all GEMMs of three decoder
+// layers.  Choice / fastest 1.009 on average; choice / the estimate's choice 0.92 (M > 3000 0.97, 16-bit outputs 0.92, 2 and 4 grouped 0.90, K =
+// 1024 0.97), more than 1.04 at 29 of them: 136 x 8112 x 5536 24.0 / 28.9, 343 x 7248 x 2048 three times 26.4 / 30.2, 3 x 571 x 4096 x 4096 int8
+// 38.9 / 43.9, 264 x 20480 x 5120 int8 48.9 / 53.3, 104 x 5120 x 20480 34.5 / 38.6, 799 x 4096 x 16384 65.4 / 71.9.  The 256 x 256 tile, no
+// candidate, leads by more than 3 % at 20 of 327 (547 x 6752 x 9824 three times 143 / 170).
+// Splits are limited to one round of items, and 2 us were added to the fitted 2.824 of a 256 x 128 split: two rounds of splits lost wherever they were chosen
+// (whole K / 3 splits on 256 x 128: 1036 x 4096 x 16384 96 / 104, 1234 x 4096 x 16384 102 / 118), as did 256 x 128 in 4 splits against 128 x 128
+// in 2 (395 x 4096 x 16384 42.7 / 46.0).
+// Left to config_cost: K < 1024, where rounds are mostly epilogue; more than 20480 columns (config_cost's choice / this one's: 300 x 50272 x
+// 1024 39.8 / 47.7, 300 x 50272 x 4096 97 / 107, 384 x 50272 x 2048 59.2 / 64.7; up to 128 rows the same); K beyond 28672 (N = 4096, K = 28672 1.08
+// of the fastest / 1.02, 5120 x 24576 1.03 / 1.02, 11264 x 32768 1.01 / 1.01).  M has no end: 17000 .. 32768 rows 1.025 / 1.004.
 struct WsCost {
   int cfg;
   double start, tile, busy, out8, out4, split, per_split, item, mem, sums;
@@ -3154,7 +3157,7 @@ static int pick_ws(const GemmParams& p, int* splits_out, bool may_split) {
   static const WsCost costs[] = {
       {CFG_WS_64x128, 1.495, 0.227, 0.122, 2.583, 2.809, 1.722, 0.216, 0.000, 0.587, 0.342},
       {CFG_WS_128x128, 0.000, 0.292, 0.180, 3.614, 4.137, 2.237, 0.240, 0.000, 0.642, 0.764},
-      {CFG_WS_256x128, 0.000, 0.438, 0.252, 4.620, 5.677, 2.824, 0.393, 0.000, 0.581, 1.467},
+      {CFG_WS_256x128, 0.000, 0.438, 0.252, 4.620, 5.677, 4.824, 0.393, 0.000, 0.581, 1.467},
       {CFG_WS_256x160, 0.000, 0.526, 0.292, 9.049, 6.328, 3.050, 0.730, 0.825, 0.520, 1.645},
   };
   int best = CFG_WS_128x128;
@@ -3163,7 +3166,7 @@ static int pick_ws(const GemmParams& p, int* splits_out, bool may_split) {
     const Config& k = g_configs[c.cfg];
     const int64_t tiles = (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bn - 1) / k.bn);
     for (int want : {1, 2, 3, 4, 6, 8}) {
-      if (want > 1 && (!may_split || p.batch != 1 || tiles * want > 520 || p.K < 384 * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
+      if (want > 1 && (!may_split || p.batch != 1 || tiles * want > 256 || p.K < 384 * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
       int splits;
       const double t = ws_time(p, k, c, want, splits);
       if (best_time < 0 || t < best_time) best_time = t, best = c.cfg, *splits_out = splits;
