@@ -399,7 +399,8 @@ int ti_kv_append_i8_seqs(const int8_t* k_src, int64_t k_src_row_stride, const in
  * bit for bit (a row's exponentials are summed as integers, so the order in which the keys are
  * visited does not matter): the output equals the three-launch chain's exactly.
  * Launches of few query rows against T <= 4096 keys (S <= 16; more rows where up to 1024 groups of 16 take less time
- * than blocks of 128) run a one-pass kernel, one to eight workgroups per batch entry and 16 rows.
+ * than blocks of 128) run a one-pass kernel, one to eight workgroups per batch entry and 16 rows; a single row (S = 1)
+ * runs one of its own, on the dot-product instructions.
  * The reference has no fused form (its modules stop at the BMMs, nn/bmm.py:10-74); the
  * three-launch chain remains available and is what this is tested against.
  */

@@ -42,3 +42,30 @@ def test_more_heads_than_four_rounds_of_the_chip(heads, S, T):
     call = lambda p: attention_i8(q[p], k[p], vt[p], 1e-3, 0.1, 0.05, causal_q_len=causal)
     got = call(slice(None))
     assert torch.equal(got, torch.cat([call(slice(i, i + 500)) for i in range(0, heads, 500)])) and got.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("seqs,heads", [(1, 3), (1, 33), (13, 5), (43, 3)])  # 8, 4, 2 and 1 workgroups per head
+def test_one_query_row_equals_the_three_kernels(seqs, heads, aligned):
+    """All lengths at which a wave, a group of loads or a piece of V^T ends, against scores -> softmax -> P.V, bit for bit."""
+    from triton_int_amd.kernels import bmm
+    from triton_int_amd.kernels.fused import attention_i8, softmax_q
+
+    H = seqs * heads
+    g = torch.Generator(device="cuda").manual_seed(H)
+    i8 = lambda *s: torch.randint(-127, 128, s, dtype=torch.int8, device="cuda", generator=g)
+    for T in (1, 15, 16, 17, 63, 64, 65, 511, 1008, 1023, 1024, 1025, 2033, 2048, 2049, 4095, 4096):
+        room = (T + 31) // 16 * 16 + (0 if aligned else 3)
+        q, k, vt = i8(H, 1, 128), i8(H, T, 128), i8(H, 128, room)[:, :, :T]
+        for qk_alpha, scale, pv_alpha in ((1e-3, 0.05, 0.05), (-2e-3, 0.5, 0.02), (6e-4, 0.5, 0.05)):
+            p = softmax_q(bmm.bmm_s8t_s8n_s8t(q, k, qk_alpha), scale)
+            want = bmm.bmm_s8t_s8n_s8t(p, vt.contiguous(), pv_alpha)
+            for causal in (0, 1):
+                got = attention_i8(q, k, vt, qk_alpha, scale, pv_alpha, causal_q_len=causal)
+                assert torch.equal(got, want), (T, qk_alpha, causal)
+        assert want.any()  # few saturated scores: probabilities above 1/254 however long the row
+        # one score for every key: a wave's sum of 256 largest exponentials
+        got = attention_i8(torch.zeros_like(q), k, vt, 1e-3, 0.05, 0.5)
+        p = softmax_q(torch.zeros((H, 1, T), dtype=torch.int8, device="cuda"), 0.05)
+        assert torch.equal(got, bmm.bmm_s8t_s8n_s8t(p, vt.contiguous(), 0.5)), T

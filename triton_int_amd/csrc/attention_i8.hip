@@ -20,7 +20,7 @@
 // half-wave swaps put a row's keys in order) and feeds them to the P.V MFMAs, so P never goes
 // through memory.
 //
-// (Launches of few query rows take attention_decode_i8_kernel further down instead.)
+// (Launches of few query rows take attention_decode_i8_kernel, and of one row attention_row_i8_kernel, further down instead.)
 //
 // Workgroup = 4 waves = 128 query rows of one head; a wave owns 32 rows.  K and V^T are staged
 // through LDS in tiles of 64 keys, double-buffered, one barrier per tile.  Causal masking skips
@@ -558,7 +558,201 @@ __global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(Attn
   }
 }
 
-// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them.  Up to four rounds of the chip
+// ---- one query row (a decode step): one workgroup per head, or several that share its V^T ----------------
+//
+// With one row the matrix units have nothing to do that the dot-product instructions do not do as well, and what their
+// operand layout costs is the order of the reads: 16 rows x 64 bytes per instruction, of K as of V^T, and sixteen queries' worth
+// of softmax for one.  Here a wave reads 1 KB of consecutive bytes per instruction: 8 rows of K (a lane one 16-byte piece, v_dot4, three
+// additions across 8 lanes) and 64 x 16 keys of one row of V^T.  Scores end up one per lane, so the softmax of 1024 keys is one or two
+// values a lane; int8 probabilities go through LDS once, and every lane keeps its 16 of each 1024 keys for all its rows of V^T.
+// The loads of K and then V^T are one sequence with AR_WINDOW of them in flight, so V^T is on its way before the
+// first reduction.  Sums are integers: the bits are those of the other kernels.
+// Bound: HBM where the heads fill the chip, else what a CU takes in.  attention_decode_i8_kernel / this one, caches from HBM: 512
+// heads x 1007 keys 30.7 / 24.9 us (5.3 TB/s), 640 x 2048 87 / 57.7 (5.8 TB/s), 40 x 1531 12.9 / 7.6, 32 x 64 5.6 / 4.2, rows of V^T at any
+// byte 512 x 1007 36.9 / 23.6.  V^T (and K where one workgroup reads it) is loaded non-temporally: read once; 640 x 2048 60.6 -> 57.4.
+// 24 loads in flight instead of 16: 1 - 3 % slower.
+constexpr int AR_WINDOW = 16;
+typedef v4i v4i_any __attribute__((aligned(1)));  // at any byte
+
+// f(integral_constant i) for A <= i < B
+template <int A, int B, class F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (A < B) {
+    f(std::integral_constant<int, A>{});
+    static_for<A + 1, B>(f);
+  }
+}
+
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v) { return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false); }
+
+// lanes 0..31 of the result: a's sum over both halves of the wave; lanes 32..63: b's
+__device__ __forceinline__ int merge32(int a, int b) {
+  const auto s = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+  return (int)s[0] + (int)s[1];
+}
+// the same with neighbouring rows of 16 lanes
+__device__ __forceinline__ int merge16(int a, int b) {
+  const auto s = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+  return (int)s[0] + (int)s[1];
+}
+__device__ __forceinline__ int sum16(int v) {
+  v += dpp<0x128>(v);
+  v += dpp<0x124>(v);
+  v += dpp<0x122>(v);
+  return v + dpp<0x121>(v);
+}
+__device__ __forceinline__ float wave_max(float f) {
+  const auto other = [&](int v) { f = fmaxf(f, __int_as_float(v)); };
+  other(dpp<0x128>(__float_as_int(f)));
+  other(dpp<0x124>(__float_as_int(f)));
+  other(dpp<0x122>(__float_as_int(f)));
+  other(dpp<0x121>(__float_as_int(f)));
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(f), __float_as_uint(f), false, false);
+  f = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(f), __float_as_uint(f), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// NW waves; RW rows of V^T per wave (a workgroup has NW * RW of the 128); GR: T <= 64 * NW * GR.
+// VANY: rows of V^T start at any byte (T >= 16): the lane with the row's end reads the row's last 16 bytes, against
+// probabilities that lie the same way.
+template <int NW, int RW, int GR, bool VANY>
+__global__ __launch_bounds__(NW * 64, 4) void attention_row_i8_kernel(AttnParams p) {
+  constexpr int KS = 8 * GR, SL = NW * GR * 64 / 1024, NV = RW * SL, W = AR_WINDOW, NT = 2;
+  static_assert(SL * 1024 == NW * GR * 64 && NW * 64 * GR <= AD_MAXT && GR <= 4, "every probability has a slot; a wave's sum fits 32 bits");
+  __shared__ __attribute__((aligned(16))) char p_lds[SL * 1024];
+  __shared__ __attribute__((aligned(16))) char p_tail[16];
+  __shared__ __attribute__((aligned(16))) float red_max[NW];
+  __shared__ __attribute__((aligned(16))) unsigned red_sum[NW];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int head = blockIdx.x, seq = blockIdx.z;
+  const int d0 = ((int)blockIdx.y * NW + wave) * RW;
+  const float MAGIC = 12582912.0f, NEG = -__builtin_inff();
+  const int8_t* qb = p.q + (int64_t)seq * p.sQb + (int64_t)head * p.sQh;
+  const int8_t* vb = p.vt + (int64_t)seq * p.sVb + (int64_t)head * p.sVh;
+  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)(p.k + (int64_t)seq * p.sKb + (int64_t)head * p.sKh), 0,
+                                                                      (int)((p.T - 1) * p.sKn + AT_D), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rV =
+      __builtin_amdgcn_make_buffer_rsrc((void*)vb, 0, (int)((AT_D - 1) * p.sVd + ((p.T + 15) & ~15)), 0x00020000);
+  const v4i qf = *(const v4i*)(qb + (lane & 7) * 16);
+  // keys from T on lie past K's descriptor and read as zeros
+  const int koff = (wave * 8 + (lane >> 3)) * (int)p.sKn + (lane & 7) * 16, kstep = NW * 8 * (int)p.sKn;
+  int voff[SL];
+#pragma unroll
+  for (int s = 0; s < SL; ++s) {
+    const int col = s * 1024 + lane * 16;
+    voff[s] = VANY ? min(col, p.T - 16) : (col < p.T ? col : 0x7ffffff0);
+  }
+  v4i slot[W];
+  const auto issue = [&](auto at) {
+    constexpr int i = decltype(at)::value;
+    if constexpr (i < KS) {
+      slot[i % W] = __builtin_amdgcn_raw_buffer_load_b128(rK, koff + i * kstep, 0, NW * RW == AT_D ? NT : 0);
+    } else if constexpr (i < KS + NV) {
+      constexpr int s = (i - KS) / RW, r = (i - KS) % RW;
+      if constexpr (VANY) slot[i % W] = __builtin_nontemporal_load((const v4i_any*)(vb + (int64_t)(d0 + r) * p.sVd + voff[s]));
+      else slot[i % W] = __builtin_amdgcn_raw_buffer_load_b128(rV, voff[s], (d0 + r) * (int)p.sVd, NT);
+    }
+  };
+  static_for<0, W>(issue);
+  if (VANY && tid < 16) p_tail[tid] = 0;
+
+  // ---- scores: lane l keeps those of loads i with i % 8 == l % 8, key (i * NW + wave) * 8 + l / 8
+  float f[GR];
+  const int key0 = ((lane & 7) * NW + wave) * 8 + (lane >> 3);
+  static_for<0, GR>([&](auto gt) {
+    constexpr int g = decltype(gt)::value;
+    int acc = 0;
+    static_for<0, 8>([&](auto it) {
+      constexpr int i = g * 8 + decltype(it)::value;
+      int a = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a = __builtin_amdgcn_sdot4(slot[i % W][t], qf[t], a, false);
+      issue(std::integral_constant<int, i + W>{});
+      a += dpp<0xB1>(a);   // neighbour
+      a += dpp<0x4E>(a);   // pairs
+      a += dpp<0x141>(a);  // halves of 8 lanes
+      acc = (lane & 7) == decltype(it)::value ? a : acc;
+    });
+    float v = (float)acc * p.qk_alpha;
+    v = __builtin_amdgcn_fmed3f(v, -128.0f, 127.0f);
+    f[g] = key0 + g * 64 * NW < p.T ? __builtin_rintf(v) : NEG;
+  });
+
+  float mx = f[0];
+#pragma unroll
+  for (int g = 1; g < GR; ++g) mx = fmaxf(mx, f[g]);
+  mx = wave_max(mx);
+  if (lane == 0) red_max[wave] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) mx = fmaxf(mx, red_max[w]);
+  const float c0 = -(mx * p.s2);
+  unsigned bits = 0;
+#pragma unroll
+  for (int g = 0; g < GR; ++g) {
+    f[g] = __builtin_amdgcn_exp2f(__builtin_fmaf(f[g], p.s2, c0));
+    bits += sm_unit_bits(f[g]);
+  }
+  bits -= (unsigned)GR * SM_ONE_BITS;
+  bits = (unsigned)sum16((int)bits);
+  bits = (unsigned)merge16((int)bits, (int)bits);
+  bits = (unsigned)merge32((int)bits, (int)bits);
+  if (lane == 0) red_sum[wave] = bits;
+  __syncthreads();
+  unsigned long long sum = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) sum += red_sum[w];
+  const float rcp = sm_scale_from_sum(sum);
+#pragma unroll
+  for (int g = 0; g < GR; ++g) {
+    const int key = key0 + g * 64 * NW;
+    const char b = (char)__float_as_uint(__builtin_fmaf(f[g], rcp, MAGIC));
+    p_lds[key] = b;  // 0 from T on
+    if (VANY && key >= (p.T & ~15) && key < p.T) p_tail[key - (p.T - 16)] = b;
+  }
+  __syncthreads();
+
+  // ---- P.V
+  int o[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) o[r] = 0;
+  v4i pf[SL];
+#pragma unroll
+  for (int s = 0; s < SL; ++s) {
+    const int col = s * 1024 + lane * 16;
+    pf[s] = *(const v4i*)(VANY && col < p.T && col + 16 > p.T ? p_tail : p_lds + col);
+  }
+  static_for<0, NV>([&](auto it) {
+    constexpr int i = KS + decltype(it)::value, s = decltype(it)::value / RW, r = decltype(it)::value % RW;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[r] = __builtin_amdgcn_sdot4(slot[i % W][t], pf[s][t], o[r], false);
+    issue(std::integral_constant<int, i + W>{});
+  });
+  // sums over the wave: two rows meet in the halves of a register, then four in its quarters
+  constexpr int H = (RW + 1) / 2, Q = (H + 1) / 2;
+  int q4[Q];
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    const auto half = [&](int i) { return merge32(o[2 * i], o[RW > 1 ? 2 * i + 1 : 0]); };
+    const int lo = half(2 * j);
+    q4[j] = sum16(merge16(lo, H > 1 ? half(H > 1 ? 2 * j + 1 : 0) : lo));
+  }
+  // lane (half h, quarter q, i): row 4 i + 2 q + h
+  const int i = lane & 15, h = lane >> 5, q = lane >> 4 & 1;
+  int v = q4[0];
+#pragma unroll
+  for (int j = 1; j < Q; ++j) v = i == j ? q4[j] : v;
+  const int r = 4 * i + (H > 1 ? 2 * q : 0) + (RW > 1 ? h : 0);
+  float x = (float)v * p.pv_alpha;
+  x = __builtin_amdgcn_fmed3f(x, -128.0f, 127.0f);
+  if (i < Q && (H > 1 || q == 0) && (RW > 1 || h == 0))
+    p.out[(int64_t)seq * p.sOb + (int64_t)head * p.sOh + d0 + r] = (int8_t)__float_as_uint(x + MAGIC);
+}
+
+// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them (a single row goes on to attention_row_i8_kernel).  Up to four rounds of the chip
 // (256 workgroups each) on whichever kernel takes less: a round of groups walks the keys once, 0.4 us per 64 of them and
 // 3.5 us besides, or as long as 4 TB/s take for the caches of the heads in it (up to 256: each is then read again in the
 // next round); the blocks of 128 rows on attention_i8_kernel, all in one round, 2.4 us per 64 keys and 3.5 us besides
@@ -583,6 +777,39 @@ static bool attn_few_rows(int64_t heads, int S, int T, int64_t q_row_stride, int
   const int64_t lim32 = (int64_t)1 << 31;  // descriptor extents and offsets
   return attn_groups_lead(heads, S, T) && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 &&
          (int64_t)AT_D * vt_row_stride < lim32 && (int64_t)S * q_row_stride < lim32;
+}
+
+// One query row: what attention_row_i8_kernel takes of the calls for few rows.  An unaligned row of V^T needs 16 bytes; the
+// offsets of all its score slots (up to AD_MAXT keys, those past T included) fit 32 bits.
+static bool attn_one_row(int S, int T, bool vany, int64_t k_row_stride) {
+  return S == 1 && (T >= 16 || !vany) && AD_MAXT * k_row_stride < (int64_t)1 << 31;
+}
+
+// A head is spread over as many workgroups (each reads K again, from L2) as fit one round of the 256 CUs; beyond one round K read
+// once is worth more than an even last round.  us for 1 / 2 / 4 / 8 workgroups per head, caches from HBM: 8 heads x 1500 keys 7.9 / 7.7 /
+// 6.4 / 6.0, 32 x 1000 5.7 / 6.4 / 5.3 / 4.9, 40 x 2047 10.0 / 10.0 / 7.4 / 10.3, 64 x 1500 10.1 / 9.7 / 8.3 / 11.0, 65 x 1500 10.0 / 10.0 / 15.1 / 21.0,
+// 128 x 2047 14.2 / 13.7 / 16.8 / 21.9, 129 x 2047 13.9 / 22.0 / 31.0 / 49.0, 512 x 1000 25.0 / 35.0 / 52.7 / 89.3.  Up to 2048 keys
+// 8 waves, which leave room for two workgroups on a CU; beyond, 16 (a wave's scores stay four registers): 3000 keys 1 / 2 / 4 per head, 40
+// heads 16.5 / 15.0 / 12.5, 100 19.9 / 20.2 / 28.4.
+static int launch_attention_row(const AttnParams& p, int seqs, bool vany, hipStream_t st) {
+  const auto launch = [&](auto nw, auto rw, auto gr) {
+    constexpr int NW = decltype(nw)::value, RW = decltype(rw)::value, GR = decltype(gr)::value;
+    const dim3 grid((unsigned)p.heads, AT_D / (NW * RW), (unsigned)seqs), block(NW * 64);
+    if (vany) attention_row_i8_kernel<NW, RW, GR, true><<<grid, block, 0, st>>>(p);
+    else attention_row_i8_kernel<NW, RW, GR, false><<<grid, block, 0, st>>>(p);
+  };
+  const auto spread = [&](auto nw, auto gr) {
+    constexpr int NW = decltype(nw)::value, RW = AT_D / NW;
+    if (NW == 8 && p.batch <= 32) launch(nw, std::integral_constant<int, 2>{}, gr);
+    else if (p.batch <= 64) launch(nw, std::integral_constant<int, RW / 4>{}, gr);
+    else if (p.batch <= 128) launch(nw, std::integral_constant<int, RW / 2>{}, gr);
+    else launch(nw, std::integral_constant<int, RW>{}, gr);
+  };
+  using W8 = std::integral_constant<int, 8>;
+  if (p.T <= 1024) spread(W8{}, std::integral_constant<int, 2>{});
+  else if (p.T <= 2048) spread(W8{}, std::integral_constant<int, 4>{});
+  else spread(std::integral_constant<int, 16>{}, std::integral_constant<int, 4>{});
+  return launch_status("attention_row_i8_kernel");
 }
 
 }  // namespace ti
@@ -632,9 +859,10 @@ extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int6
   p.nblk = (S + AT_ROWS - 1) / AT_ROWS;
   p.batch = batch; p.heads = heads;
   const hipStream_t st = (hipStream_t)stream;
+  if (few_rows && attn_one_row(S, T, vany, k_row_stride)) return launch_attention_row(p, seqs, vany, st);
   if (few_rows) {
     // spread a head over as many workgroups as keep the launch within one round of the 256 CUs
-    // (measured, 40 heads x 16 rows x 2048 keys: 18.9 / 15.3 / 13.6 us for 1 / 2 / 4 workgroups per head,
+    // (40 heads x 16 rows x 2048 keys: 18.9 / 15.3 / 13.6 us for 1 / 2 / 4 workgroups per head,
     // 24 us for 8, which no longer fit one round)
     int dbw = 8;
     while (dbw > 1 && groups * (16 / dbw) <= 256) dbw /= 2;
