@@ -57,6 +57,7 @@ struct GemmParams {
   int batch, M, N, K;
   const void* bias;
   int bias_kind;
+  int keep;  // persistent kernels: the outputs are stored for the next launch to find in the Infinity Cache, else streamed past it
   const float* alpha;
   const float* beta;
   int epilogue, out_dtype, round_mode;
@@ -653,27 +654,25 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (WAVES_M * WAVES_N * OCC + 3
 // number of store instructions per tile does not depend on the tile (2-byte outputs: one of two
 // constants, by out16_pairs()).  `strip` is the wave's private
 // LDS area (int8 outputs only): 32*WTN bytes for the row strip plus WTN floats of column terms.
-#ifndef TI_STREAM_STORE_AUX
-#define TI_STREAM_STORE_AUX 2  // nt: the outputs are streamed, keep the operand panels in L2
-#endif
 // bytes of the per-wave LDS strip of the int8 epilogue: 32 rows of the wave's WTN output bytes when
 // WTN / 16 is a power of two (the swizzle below needs that), none otherwise (direct stores)
 constexpr int epi_strip_bytes(int wtn) { return ((wtn / 16) & (wtn / 16 - 1)) == 0 ? 32 * wtn : 0; }
 
-// 4-byte outputs: every store instruction writes two whole 128-byte lines, which go out non-temporal
-// (measured on the P.V shape with fp32 output: 192 -> 162 us)
-#ifndef TI_STREAM_STORE32_AUX
-#define TI_STREAM_STORE32_AUX 2
-#endif
+// Cache policy of the stores.  Non-temporal leaves the operand panels in L2 and the Infinity Cache (P.V with fp32 output,
+// 168 MB of probabilities: 192 -> 162 us; every store instruction of a 4-byte output writes two whole 128-byte lines), but the
+// launch that reads the outputs then fetches them from HBM.  Device scope (sc1) writes them through L2 into the
+// Infinity Cache, where that launch finds them: keep_outputs() says which.
+constexpr int STORE_STREAM = 2, STORE_KEEP = 16;
+
 // 2-byte outputs: pairs of neighbouring elements of a row can go out as one aligned dword
 __device__ __forceinline__ bool out16_pairs(const GemmParams& p) {
   return !(p.N & 1) && !(p.sCm & 1) && !(p.sCb & 1) && !((uintptr_t)p.C & 3);
 }
 // LDS_COLS false: `strip` has no room for the column terms; int8 launches with a bias or GELU are not
 // compiled in (the host refuses them for such a kernel).
-template <int TM, int TN, int OUTCLS, bool LDS_COLS = true>
-__device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
-                                                int mw, int nw, char* strip, int lane) {
+template <int TM, int TN, int OUTCLS, bool LDS_COLS, int AUX>
+__device__ __forceinline__ void store_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
+                                               int mw, int nw, char* strip, int lane) {
   constexpr int WTN = TN * 32;
   constexpr int ESZ = OUTCLS == OUT8 ? 1 : (OUTCLS == OUT32 ? 4 : 2);
   const int OOB = (int)0x80000000;
@@ -762,7 +761,7 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
             const int row = q * RP + r_row;
             const v4u v = *(const v4u*)(strip + row * WTN + ((r_seg ^ ((row / WRAP) & (SEG - 1))) * 16));
             const int R = i * 32 + q * RP;  // row mw + R + r_row
-            __builtin_amdgcn_raw_buffer_store_b128(v, rC, (R < s_rows_left ? s_base : OOB) + R * ldc, 0, TI_STREAM_STORE_AUX);
+            __builtin_amdgcn_raw_buffer_store_b128(v, rC, (R < s_rows_left ? s_base : OOB) + R * ldc, 0, AUX);
           }
         }
       }
@@ -840,7 +839,7 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
                   const unsigned got = (unsigned)__builtin_amdgcn_mov_dpp((int)give, 0xB1, 0xf, 0xf, true);  // lane ^ 1
                   const unsigned dword = odd ? (got | (hi_row << 16)) : (lo_row | (got << 16));
                   const int R = i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);  // row mw + R + odd
-                  __builtin_amdgcn_raw_buffer_store_b32(dword, rC, in[h] ? base2[jp] : OOB, R * pitch, TI_STREAM_STORE32_AUX);
+                  __builtin_amdgcn_raw_buffer_store_b32(dword, rC, in[h] ? base2[jp] : OOB, R * pitch, AUX);
                 }
               }
             }
@@ -867,7 +866,7 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
                 const unsigned got = (unsigned)__builtin_amdgcn_mov_dpp((int)give, 0xB1, 0xf, 0xf, true);
                 const unsigned dword = odd ? (got | (row[1] << 16)) : (row[0] | (got << 16));
                 const int R = i * 32 + 8 * (r >> 2) + (r & 3);  // row mw + R + 4 * lhi + odd
-                __builtin_amdgcn_raw_buffer_store_b32(dword, rC, R < rows_left - odd ? base : OOB, R * pitch, TI_STREAM_STORE32_AUX);
+                __builtin_amdgcn_raw_buffer_store_b32(dword, rC, R < rows_left - odd ? base : OOB, R * pitch, AUX);
               }
             }
           }
@@ -919,7 +918,7 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
                 const float vb = colr[j] + v;
                 v = has_bias ? vb : v;
                 v = v + res[g & 1][t][j];
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rC, in ? base_c[j] : OOB, R * pitch, TI_STREAM_STORE32_AUX);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rC, in ? base_c[j] : OOB, R * pitch, AUX);
               }
             }
           }
@@ -949,13 +948,13 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
             const int off = in ? base[j] : OOB;
             const int a = acc[i][j][r];
             if constexpr (KIND == 0) {
-              __builtin_amdgcn_raw_buffer_store_b32((unsigned)a + (unsigned)bias_i32[j], rC, off, soff, TI_STREAM_STORE32_AUX);
+              __builtin_amdgcn_raw_buffer_store_b32((unsigned)a + (unsigned)bias_i32[j], rC, off, soff, AUX);
             } else {
               float v = (float)a * e.alpha;
               const float vb = col[j] + v;
               v = has_bias ? vb : v;
-              if constexpr (KIND == 1) __builtin_amdgcn_raw_buffer_store_b32((unsigned)q32(v, e.round_mode), rC, off, soff, TI_STREAM_STORE32_AUX);
-              else if constexpr (KIND == 2) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rC, off, soff, TI_STREAM_STORE32_AUX);
+              if constexpr (KIND == 1) __builtin_amdgcn_raw_buffer_store_b32((unsigned)q32(v, e.round_mode), rC, off, soff, AUX);
+              else if constexpr (KIND == 2) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rC, off, soff, AUX);
               else if constexpr (KIND == 3) __builtin_amdgcn_raw_buffer_store_b16(f32_to_f16_bits(v), rC, off, soff, 0);
               else __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16_bits(v), rC, off, soff, 0);
             }
@@ -972,6 +971,15 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
       else body(std::integral_constant<int, 4>{});
     }
   }
+}
+
+template <int TM, int TN, int OUTCLS, bool LDS_COLS = true>
+__device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
+                                                int mw, int nw, char* strip, int lane) {
+  // int8 without a strip stores with the default policy
+  constexpr bool CHOICE = OUTCLS != OUT8 || epi_strip_bytes(TN * 32) != 0;
+  if (!CHOICE || p.keep) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_KEEP>(p, e, acc, bz, mw, nw, strip, lane);
+  else store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_STREAM>(p, e, acc, bz, mw, nw, strip, lane);
 }
 
 // ---- persistent ("stream") variant of the fast family --------------------------------------------
@@ -3347,6 +3355,16 @@ static int pick_group_m(const GemmParams& p, const Config& k) {
   return best;
 }
 
+// Whether the outputs of a launch on a persistent kernel stay in the 256 MB Infinity Cache for the launch that reads them:
+// where that, with what this launch reads, takes less than half of it.  us of a launch and the one after it, stored
+// non-temporally / for the cache: Q.K^T 40 x 1024^2 and its softmax 40.0 / 38.8, 80 x 1024^2 63.1 / 58.2, but 160 x 1024^2 (168 MB of
+// scores) 120 / 123; P.V with fp32 output 40 x 1024 x 128 17.3 / 14.1, but 80 x 1024 (136 MB) 30.3 / 31.4 and 160 x 1024 49.8 / 55.0.
+static bool keep_outputs(const GemmParams& p) {
+  const int esz = p.out_dtype == TI_I8 ? 1 : ((p.out_dtype == TI_F16 || p.out_dtype == TI_BF16) ? 2 : 4);
+  const double a = (double)p.M * p.K * (p.sAb ? p.batch : 1), b = (double)p.N * p.K * p.batch, c = (double)p.M * p.N * p.batch * esz;
+  return a + b + c <= 128e6;
+}
+
 static int validate(const GemmParams& p) {
   if (p.batch < 0 || p.M < 0 || p.N < 0 || p.K < 0) return fail(TI_E_SHAPE, "negative size");
   if (p.batch == 0 || p.M == 0 || p.N == 0) return TI_OK;
@@ -3725,6 +3743,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       return TI_OK;
     }
     const KernelFn fn = kn ? ws_kn_kernel(k.bm, out_class(p.out_dtype)) : k.fn[out_class(p.out_dtype)];
+    p.keep = keep_outputs(p);
     fn<<<dim3((unsigned)g), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }

@@ -10,6 +10,8 @@
 // vectors (thread t owns vectors t, t+256, ...: every load/store instruction of a wave is one
 // contiguous 1 KB / 256 B run), so x is read from HBM exactly once; mean and the centred sum of
 // squares are exact two-pass statistics reduced with wave shuffles and one LDS hop.
+#include <type_traits>
+
 #include "ti_common.h"
 
 namespace ti {
@@ -77,14 +79,24 @@ __device__ __forceinline__ float norm_one(float x, float mean, float rstd, float
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* row_ptr, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)row_ptr, 0, (int)bytes, 0x00020000);
 }
+// Cache policy of a launch's rows.  KEEP: plain loads, and stores of device scope (sc1), which go through L2 into the Infinity
+// Cache (256 MB), where the next launch finds them, as this one finds what was left there for it.  Otherwise non-temporal
+// both ways: rows that pass the caches by cost less there.
+template <bool KEEP>
+constexpr int LOAD_AUX = KEEP ? 0 : 2;
+template <bool KEEP>
+constexpr int STORE_AUX = KEEP ? 16 : 2;
+
+template <bool KEEP>
 __device__ __forceinline__ v4f row_load_f4(__amdgpu_buffer_rsrc_t r, int vec) {
-  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, vec * 16, 0, 2));  // 2: non-temporal
+  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, vec * 16, 0, LOAD_AUX<KEEP>));
 }
+template <bool KEEP>
 __device__ __forceinline__ void row_store_f4(__amdgpu_buffer_rsrc_t r, int vec, v4f v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, v), r, vec * 16, 0, 2);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, v), r, vec * 16, 0, STORE_AUX<KEEP>);
 }
 
-template <int VPT, bool DQ>
+template <int VPT, bool DQ, bool KEEP>
 __global__ __launch_bounds__(RN_THREADS) void rownorm_vec_kernel(RowNormParams p) {
   __shared__ float red[2 * RN_WAVES];
   int red_k = 0;
@@ -109,7 +121,7 @@ __global__ __launch_bounds__(RN_THREADS) void rownorm_vec_kernel(RowNormParams p
     const bool in = row < p.rows;
     const __amdgpu_buffer_rsrc_t rx = row_rsrc(p.x + (int64_t)(in ? row : 0) * p.x_rs, in ? row_bytes : 0u);
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) dst[j] = row_load_f4(rx, tid + j * RN_THREADS);
+    for (int j = 0; j < VPT; ++j) dst[j] = row_load_f4<KEEP>(rx, tid + j * RN_THREADS);
   };
 
   v4f x[VPT], xn[VPT];
@@ -131,8 +143,8 @@ __global__ __launch_bounds__(RN_THREADS) void rownorm_vec_kernel(RowNormParams p
       v4f r[VPT];
 #pragma unroll
       for (int j = 0; j < VPT; ++j) {
-        a[j] = __builtin_amdgcn_raw_buffer_load_b128(ra, (tid + j * RN_THREADS) * 16, 0, 2);
-        r[j] = row_load_f4(rr, tid + j * RN_THREADS);
+        a[j] = __builtin_amdgcn_raw_buffer_load_b128(ra, (tid + j * RN_THREADS) * 16, 0, LOAD_AUX<KEEP>);
+        r[j] = row_load_f4<KEEP>(rr, tid + j * RN_THREADS);
       }
 #pragma unroll
       for (int j = 0; j < VPT; ++j) {
@@ -144,7 +156,7 @@ __global__ __launch_bounds__(RN_THREADS) void rownorm_vec_kernel(RowNormParams p
           o[t] = r[j][t] + prod;
         }
         x[j] = o;  // vectors past the row's end: 0 + scale * 0
-        row_store_f4(ro, tid + j * RN_THREADS, o);
+        row_store_f4<KEEP>(ro, tid + j * RN_THREADS, o);
       }
     } else {
 #pragma unroll
@@ -183,10 +195,10 @@ __global__ __launch_bounds__(RN_THREADS) void rownorm_vec_kernel(RowNormParams p
       v4f o;
 #pragma unroll
       for (int t = 0; t < 4; ++t) o[t] = norm_one(x[j][t], mean, rstd, w[j][t], b[j][t], has_b);
-      row_store_f4(rl, v, o);  // an empty descriptor when there is no fp32 output
+      row_store_f4<KEEP>(rl, v, o);  // an empty descriptor when there is no fp32 output
       const int q0 = q8(o[0], p.round_mode), q1 = q8(o[1], p.round_mode), q2 = q8(o[2], p.round_mode),
                 q3 = q8(o[3], p.round_mode);
-      __builtin_amdgcn_raw_buffer_store_b32((int)pack4(q0, q1, q2, q3), ry, v * 4, 0, 2);
+      __builtin_amdgcn_raw_buffer_store_b32((int)pack4(q0, q1, q2, q3), ry, v * 4, 0, STORE_AUX<KEEP>);
       if (p.y && !y_vec && v < nvec) {  // int8 rows that are not 4-byte aligned
         int8_t* dst = p.y + (int64_t)row * p.y_rs + v * 4;
         dst[0] = (int8_t)q0; dst[1] = (int8_t)q1; dst[2] = (int8_t)q2; dst[3] = (int8_t)q3;
@@ -275,13 +287,21 @@ static int launch_rownorm(const RowNormParams& p, hipStream_t stream) {
   const unsigned per_cu = DQ ? (vpt <= 2 ? 3u : 2u) : ln_per_cu;
   const unsigned slots = 256u * per_cu;
   if (grid.x > slots) grid.x = slots;
-  if (vpt <= 1) rownorm_vec_kernel<1, DQ><<<grid, block, 0, stream>>>(p);
-  else if (vpt <= 2) rownorm_vec_kernel<2, DQ><<<grid, block, 0, stream>>>(p);
-  else if (vpt <= 3) rownorm_vec_kernel<3, DQ><<<grid, block, 0, stream>>>(p);
-  else if (vpt <= 4) rownorm_vec_kernel<4, DQ><<<grid, block, 0, stream>>>(p);
-  else if (vpt <= 5) rownorm_vec_kernel<5, DQ><<<grid, block, 0, stream>>>(p);
-  else if (vpt <= 6) rownorm_vec_kernel<6, DQ><<<grid, block, 0, stream>>>(p);
-  else rownorm_vec_kernel<8, DQ><<<grid, block, 0, stream>>>(p);
+  const auto launch = [&](auto keep) {
+    constexpr bool KEEP = decltype(keep)::value;
+    if (vpt <= 1) rownorm_vec_kernel<1, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+    else if (vpt <= 2) rownorm_vec_kernel<2, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+    else if (vpt <= 3) rownorm_vec_kernel<3, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+    else if (vpt <= 4) rownorm_vec_kernel<4, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+    else if (vpt <= 5) rownorm_vec_kernel<5, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+    else if (vpt <= 6) rownorm_vec_kernel<6, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+    else rownorm_vec_kernel<8, DQ, KEEP><<<grid, block, 0, stream>>>(p);
+  };
+  // Rows for the Infinity Cache up to 20 M elements (dq + add: 273 MB read and written, plain: 105 MB).  us, non-temporal / for the cache,
+  // 5120 columns, the residual read by the launch before: dq + add 500 rows 9.2 / 7.0, 1000 15.6 / 12.6, 2000 26.1 / 22.3, 4000 46.8 / 44.2, 6000
+  // 68.5 / 68.5, 8192 91.5 / 92.4; plain 1000 8.9 / 9.1, 4000 22.0 / 21.4, 6000 28.8 / 31.6, 8192 36.8 / 46.3.
+  if ((int64_t)p.rows * p.cols <= (int64_t)20 << 20) launch(std::true_type{});
+  else launch(std::false_type{});
   return launch_status("rownorm_vec_kernel");
 }
 
@@ -315,7 +335,7 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned v) {
 // first use: buffer loads whose offset is pushed out of range for chunks beyond the causal limit
 // (they return 0 without touching memory), then masking in registers.  Stores are range-checked
 // buffer stores, so neither phase branches around a memory instruction.
-template <int VPT>
+template <int VPT, bool KEEP>
 __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_kernel(const int8_t* __restrict__ x, int64_t x_rs,
                                                                   float scale, int8_t* __restrict__ y, int64_t y_rs,
                                                                   int rows, int cols, int causal_q_len) {
@@ -334,7 +354,7 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_kernel(const int8_t* 
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int c0 = (j * 64 + lane) * 16;
-    w[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, c0 < limit ? c0 : OOB, 0, 2);
+    w[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, c0 < limit ? c0 : OOB, 0, LOAD_AUX<KEEP>);
   }
   float f[VPT][16];
   float mx = NEG;
@@ -388,14 +408,14 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_kernel(const int8_t* 
         o[g] = (int)(__builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) | __builtin_amdgcn_perm(b3, b2, 0x04000c0cu));
       }
     }
-    __builtin_amdgcn_raw_buffer_store_b128(o, ry, c0, 0, 2);  // dropped beyond the row's end
+    __builtin_amdgcn_raw_buffer_store_b128(o, ry, c0, 0, STORE_AUX<KEEP>);  // dropped beyond the row's end
   }
 }
 // Any alignment, length and scale >= 0: 16 unaligned bytes per lane.  160 x 1001 rows of 1001 columns 311 (byte loads
 // and stores) -> 84 us, 40 x 2047 rows of 2047 341 -> 61 us (aligned rows of 2048: 54 us).
 typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(1)));
 
-template <int VPT>
+template <int VPT, bool KEEP>
 __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8_t* __restrict__ x, int64_t x_rs,
                                                                   float scale, int8_t* __restrict__ y, int64_t y_rs,
                                                                   int rows, int cols, int causal_q_len) {
@@ -481,7 +501,8 @@ __global__ __launch_bounds__(SM_WAVES * 64) void softmax_q_any_kernel(const int8
     }
     const int left = cols - c0;
     if (left >= 16) {
-      __builtin_nontemporal_store(o, (v4u_any*)(yr + c0));
+      if constexpr (KEEP) *(v4u_any*)(yr + c0) = o;
+      else __builtin_nontemporal_store(o, (v4u_any*)(yr + c0));
     } else {  // the lane with the row's end: 8, 4, 2 and 1 bytes
       int8_t* d = yr + c0;
       if (left & 8) {
@@ -702,16 +723,23 @@ int ti_softmax_q(const int8_t* x, int64_t x_row_stride, float scale, int8_t* y, 
   dim3 grid((unsigned)((rows + ti::SM_WAVES - 1) / ti::SM_WAVES)), block(ti::SM_WAVES * 64);
   const int vpt = (cols + 1023) / 1024;
   const bool aligned = ((((uintptr_t)x) | ((uintptr_t)y) | (uintptr_t)x_row_stride | (uintptr_t)y_row_stride | (uintptr_t)cols) & 15) == 0;
-#define TI_SOFTMAX_LAUNCH(KERNEL)                                                                          \
-  do {                                                                                                     \
-    if (vpt <= 1) KERNEL<1><<<grid, block, 0, s>>>(x, x_row_stride, scale, y, y_row_stride, rows, cols, causal_q_len);      \
-    else if (vpt <= 2) KERNEL<2><<<grid, block, 0, s>>>(x, x_row_stride, scale, y, y_row_stride, rows, cols, causal_q_len); \
-    else if (vpt <= 4) KERNEL<4><<<grid, block, 0, s>>>(x, x_row_stride, scale, y, y_row_stride, rows, cols, causal_q_len); \
-    else KERNEL<8><<<grid, block, 0, s>>>(x, x_row_stride, scale, y, y_row_stride, rows, cols, causal_q_len);               \
-  } while (0)
-  if (aligned && scale > 0.0f) TI_SOFTMAX_LAUNCH(ti::softmax_q_kernel);
-  else TI_SOFTMAX_LAUNCH(ti::softmax_q_any_kernel);
-#undef TI_SOFTMAX_LAUNCH
+  // for the Infinity Cache (see LOAD_AUX) up to 168 MB of scores, us, non-temporal / for the cache: 40 x 1024^2 22.0 / 20.3, 80 x 1024^2
+  // 36.3 / 31.4, 40 x 2048^2 55.9 / 51.6, but 80 x 2048^2 110 / 125, 160 x 2048^2 215 / 248
+  const bool keep = (int64_t)rows * cols <= (int64_t)160 << 20, vec = aligned && scale > 0.0f;
+  const auto launch = [&](auto vpt_tag, auto keep_tag) {
+    constexpr int VPT = decltype(vpt_tag)::value;
+    constexpr bool KEEP = decltype(keep_tag)::value;
+    const auto kernel = vec ? ti::softmax_q_kernel<VPT, KEEP> : ti::softmax_q_any_kernel<VPT, KEEP>;
+    kernel<<<grid, block, 0, s>>>(x, x_row_stride, scale, y, y_row_stride, rows, cols, causal_q_len);
+  };
+  const auto by_length = [&](auto keep_tag) {
+    if (vpt <= 1) launch(std::integral_constant<int, 1>{}, keep_tag);
+    else if (vpt <= 2) launch(std::integral_constant<int, 2>{}, keep_tag);
+    else if (vpt <= 4) launch(std::integral_constant<int, 4>{}, keep_tag);
+    else launch(std::integral_constant<int, 8>{}, keep_tag);
+  };
+  if (keep) by_length(std::true_type{});
+  else by_length(std::false_type{});
   return ti::launch_status("softmax_q_kernel");
 }
 
