@@ -343,7 +343,17 @@ int ti_qkv_decode_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t
                           int64_t vt_row_stride, int D, void* stream);
 
 /*
- * The same with the LayerNormQ in front in the same launch: x fp32 [M, K], unit column stride, row stride in elements, gamma
+ * The same for up to 64 rows, and with k_dst = NULL for a prompt without a cache (only V^T is written; k is read from C).
+ * TI_E_COMBO, with nothing done, for more rows, for caches that share memory with an operand and where no kernel takes it (the
+ * caller then makes the two calls).
+ */
+int ti_qkv_append_i8_seqs(const int8_t* A, int64_t lda, const int8_t* W, int64_t ldw, const int8_t* bias,
+                          const float* alpha3, const float* beta3, int8_t* C, int64_t ldc, int seqs, int M, int N, int K,
+                          int8_t* k_dst, int64_t k_head_stride, int64_t k_row_stride, int8_t* vt_dst,
+                          int64_t vt_row_stride, int D, void* stream);
+
+/*
+ * ti_qkv_decode_i8_seqs with the LayerNormQ in front in the same launch: x fp32 [M, K], unit column stride, row stride in elements, gamma
  * and beta (may be NULL) as ti_layernorm_q takes them.  The bits are those of ti_layernorm_q followed by the call above.  At
  * most 4 rows, 1024 <= K <= 5120, 16-byte aligned rows, outputs that share no memory with x, gamma, beta or each other;
  * TI_E_COMBO, with nothing done, for everything else (the caller makes the two calls).

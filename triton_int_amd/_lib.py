@@ -27,7 +27,7 @@ TORCH_TO_BIAS = {torch.int8: BIAS_I8, torch.int32: BIAS_I32, torch.float32: BIAS
 
 EXPORTS = ("ti_version", "ti_last_error", "ti_mfma_i8_probe", "ti_bmm_i8", "ti_bmm_i8_config", "ti_bmm_i8_grouped", "ti_bmm_i8_static_scratch", "ti_gemm_num_configs",
            "ti_gemm_config_name", "ti_gemm_last_config", "ti_gemm_last_splits", "ti_gemm_plan", "ti_release_workspaces", "ti_layernorm_q", "ti_dq_add_layernorm_q", "ti_gelu_q", "ti_softmax_q", "ti_transpose_i8", "ti_attention_i8", "ti_attention_i8_heads", "ti_attention_i8_rows", "ti_quantize_per_token_absmax", "ti_quantize_per_tensor_absmax", "ti_kv_append_i8", "ti_kv_append_i8_seqs", "ti_layernorm_qkv_decode_i8_seqs", "ti_dq_add_layernorm_linear_gelu_i8",
-           "ti_layernorm_fp", "ti_linear_i8_residual_f32", "ti_qkv_decode_i8", "ti_qkv_decode_i8_seqs")
+           "ti_layernorm_fp", "ti_linear_i8_residual_f32", "ti_qkv_decode_i8", "ti_qkv_decode_i8_seqs", "ti_qkv_append_i8_seqs")
 
 _lib = None
 
@@ -97,6 +97,8 @@ def _declare(lib):
     lib.ti_qkv_decode_i8_seqs.restype = _int
     lib.ti_qkv_decode_i8_seqs.argtypes = [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _int, _int, _int, _int,
                                           _vp, _i64, _i64, _vp, _i64, _int, _vp]
+    lib.ti_qkv_append_i8_seqs.restype = _int
+    lib.ti_qkv_append_i8_seqs.argtypes = lib.ti_qkv_decode_i8_seqs.argtypes
     lib.ti_layernorm_qkv_decode_i8_seqs.restype = _int
     lib.ti_layernorm_qkv_decode_i8_seqs.argtypes = [_vp, _i64, _vp, _vp, _f32, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _int, _int, _int, _int,
                                                     _vp, _i64, _i64, _vp, _i64, _int, _vp]

@@ -226,15 +226,15 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
           appended = rc == TI_OK;
         }
         if (!appended && (rc = ti_layernorm_q(xp, x_rs, ln1.g, ln1.b, ln1.eps, h8, H, M32, H32, 0, TI_ROUND_RNE_CLAMP, nullptr, nullptr, c.stream))) return;
-        if (!appended && cached && M <= 16 && H >= 1024 && ((((int64_t)k_dst | dst_hs | dst_rs) & 3) == 0)) {
-          rc = ti_qkv_decode_i8_seqs(h8, H, (const int8_t*)ptr(w3), H, b3, a3, s3, qkv, 3 * H, B32, M32, H32, H32, k_dst, dst_hs, dst_rs, vt_dst, vt_rs, (int)D, c.stream);
+        int8_t* const vd = cached ? vt_dst : (int8_t*)base + at[7];
+        if (!appended && M <= 64 && H >= 1024 && ((((int64_t)k_dst | dst_hs | dst_rs) & 3) == 0)) {
+          rc = ti_qkv_append_i8_seqs(h8, H, (const int8_t*)ptr(w3), H, b3, a3, s3, qkv, 3 * H, B32, M32, H32, H32, k_dst, dst_hs, dst_rs, vd, vt_rs, (int)D, c.stream);
           if (rc && rc != TI_E_COMBO) return;
           appended = rc == TI_OK;
         }
         if (!appended) {
           if ((rc = ti_bmm_i8_grouped(h8, 0, H, 1, (const int8_t*)ptr(w3), H * H, H, 1, qkv, H, 3 * H, 1, 3, M32, H32, H32, b3, TI_BIAS_I8, H, a3, s3, 1,
                                       TI_EPI_SCALE_I8, TI_I8, TI_ROUND_RNE_CLAMP, -1, c.stream))) return;
-          int8_t* vd = cached ? vt_dst : (int8_t*)base + at[7];
           if ((rc = ti_kv_append_i8_seqs(cached ? qkv + H : nullptr, cached ? 3 * H : 0, qkv + 2 * H, 3 * H, k_dst, dst_hs, dst_rs, vd, vt_rs, B32, S32,
                                          (int)heads, (int)D, c.stream))) return;
         }
