@@ -382,18 +382,20 @@ __global__ __launch_bounds__(256, 2) void attention_i8_kernel(AttnParams p) {
 constexpr int AD_WAVES = 16;
 constexpr int AD_MAXT = 4096;
 
-// CPW: 16-key chunks per wave (T <= 256 * CPW).  DBW: 16-column blocks of the output a workgroup
+// CPW: 16-key chunks per wave (T <= 256 * CPW), in steps of 256 keys up to 1536: chunks past the last key cost their loads' latency, scores and
+// exponentials like any other.  us, 4 chunks at least and then 8 and 16 / these: 32 heads x 64 rows x 64 keys 6.2 / 4.5, x 128 x 128 7.1 / 5.3, x 64 x
+// 1064 12.7 / 11.1, 64 x 140 x 437 27.7 / 19.9, 40 x 7 x 1200 11.5 / 10.1, 8 x 27 x 27 5.5 / 4.1.  DBW: 16-column blocks of the output a workgroup
 // produces (8: the whole head; fewer: the head is spread over 8 / DBW workgroups, each of which
 // repeats the scores and the softmax and reads only its rows of V^T — a single CU fills its caches at
 // about 30 GB/s, so a head's 512 KB of K and V^T through one CU alone would take 17 us).
 // VANY: V^T rows without alignment, as in attention_i8_kernel.
 template <int CPW, int DBW, bool VANY>
-__global__ __launch_bounds__(AD_WAVES * 64) void attention_decode_i8_kernel(AttnParams p) {
+__global__ __launch_bounds__(AD_WAVES * 64, CPW <= 2 ? 8 : 4) void attention_decode_i8_kernel(AttnParams p) {
   constexpr int TMAX = 256 * CPW;
   constexpr int PP = TMAX + 16;             // LDS pitch of a query's probabilities
   constexpr int KPARTS = AD_WAVES / DBW;    // waves that share an output block and split the keys
   constexpr int GPW = (TMAX / 64 + KPARTS - 1) / KPARTS;  // 64-key groups per wave in P.V
-  constexpr int HOIST = CPW >= 16 ? (GPW < 4 ? GPW : 4) : GPW;  // V^T operands fetched before the softmax reductions
+  constexpr int HOIST = CPW >= 12 ? (GPW < 4 ? GPW : 4) : GPW;  // V^T operands fetched before the softmax reductions
   __shared__ __attribute__((aligned(16))) char p_lds[16 * PP];
   __shared__ float red_max[AD_WAVES][16];
   __shared__ unsigned red_sum[AD_WAVES][16];
@@ -752,25 +754,24 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_row_i8_kernel(AttnParams
     p.out[(int64_t)seq * p.sOb + (int64_t)head * p.sOh + d0 + r] = (int8_t)__float_as_uint(x + MAGIC);
 }
 
-// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them (a single row goes on to attention_row_i8_kernel).  Up to four rounds of the chip
-// (256 workgroups each) on whichever kernel takes less: a round of groups walks the keys once, 0.4 us per 64 of them and
-// 3.5 us besides, or as long as 4 TB/s take for the caches of the heads in it (up to 256: each is then read again in the
-// next round); the blocks of 128 rows on attention_i8_kernel, all in one round, 2.4 us per 64 keys and 3.5 us besides
-// however few their rows.  128-row blocks beyond four rounds.
-// Measured (us, groups / blocks), 815 sizes of 17 .. 512 rows against 16 .. 4096 keys, with and without a mask: the
-// estimate's choice is 0.5 % above the better one on average, and nowhere more than 3 % above the blocks.  Causal: 32 heads x 64
-// rows x 1064 keys 11.9 / 43.3, 64 x 128 x 333 11.7 / 20.2, 40 x 333 x 2048 (840 groups) 72 / 80, 32 x 512 x 2048 (1024) 71 / 81;
-// but 160 x 64 x 64 13.3 / 7.7, 80 x 192 x 256 19.3 / 15.0, 512 x 32 x 128 19.1 / 11.9, 256 x 64 x 2048 120 / 83, 512 x 17 x 1024
-// 59 / 48.  Beyond: 40 x 512 x 2048 (1280) 88 / 81, 320 x 64 x 2048 (1280) 145 / 113, 1280 x 17 x 2048 (2560) 298 / 269, 1280
-// x 32 x 1024 (2560) 133 / 137.
+// Groups of 16 query rows on attention_decode_i8_kernel where a head has one of them (a single row goes on to attention_row_i8_kernel).  Up to four
+// rounds of the chip (256 workgroups each) on whichever kernel takes less: a round of groups walks the keys once, 0.2 us per 64 of them and
+// 2.5 us besides, or as long as 4 TB/s take for the caches of the heads in it (up to 256: each is then read again in the
+// next round); two workgroups on a CU fill a last round that is partly empty.  The blocks of 128 rows on attention_i8_kernel, all in one round,
+// 1.8 us per 64 keys and 3 us besides however few their rows.  128-row blocks beyond four rounds.
+// Measured over 170 sizes of 17 .. 600 rows against 17 .. 1950 keys, masked: the estimate's choice is 1.6 % above the better one on
+// average (the one before it, fitted when a workgroup had four chunks of keys a wave at least, 5.3 %).  us, groups / blocks: 40 heads x 205
+// rows x 205 keys 9.1 / 15.2, 80 x 107 x 196 10.6 / 16.2, 32 x 371 x 371 13.7 / 20.3, 8 x 19 x 1103 10.1 / 46.9, 96 x 57 x 755 22.5 / 37.9; but 80 x 377 x 377
+// 28.6 / 20.6, 160 x 232 x 434 58.8 / 32.0.  Where it loses: 80 x 139 x 139 9.4 / 12.2, 32 x 516 x 516 (1056 groups) 20.4 / 25.9.
 // 16 rows and fewer, as many workgroups either way: 1280 x 1 x 2048 156 / 265, 2560 x 16 x 2048 297 / 464, 1056 x 1 x
 // 333 24.8 / 57.8, 20000 x 1 x 304 346 / 707 (20000 x 1 x 64 265 / 242).
 static bool attn_groups_lead(int64_t heads, int S, int T) {
   const int64_t groups = heads * ((S + 15) / 16);
   if (S <= 16) return true;
   if (groups > 1024) return false;
-  const double walk = 3.5 + 0.4 * T / 64, fetch = (double)(heads < 256 ? heads : 256) * T * 2 * AT_D / 4.0e6;
-  return (double)((groups + 255) / 256) * (walk > fetch ? walk : fetch) <= 3.5 + 2.4 * T / 64;
+  const double walk = 2.5 + 0.2 * T / 64, fetch = (double)(heads < 256 ? heads : 256) * T * 2 * AT_D / 4.0e6;
+  const double rounds = groups > 256 ? (double)groups / 256 : 1.0;
+  return rounds * (walk > fetch ? walk : fetch) <= 3.0 + 1.8 * T / 64;
 }
 
 static bool attn_few_rows(int64_t heads, int S, int T, int64_t q_row_stride, int64_t k_row_stride, int64_t vt_row_stride) {
@@ -870,8 +871,14 @@ extern "C" int ti_attention_i8_heads(const int8_t* q, int64_t q_seq_stride, int6
 #define TI_AD_LAUNCH(C, V) \
     (dbw == 8 ? attention_decode_i8_kernel<C, 8, V><<<grid, block, 0, st>>>(p) : dbw == 4 ? attention_decode_i8_kernel<C, 4, V><<<grid, block, 0, st>>>(p) \
      : dbw == 2 ? attention_decode_i8_kernel<C, 2, V><<<grid, block, 0, st>>>(p) : attention_decode_i8_kernel<C, 1, V><<<grid, block, 0, st>>>(p))
-    if (T <= 1024) vany ? TI_AD_LAUNCH(4, true) : TI_AD_LAUNCH(4, false);
+    if (T <= 256) vany ? TI_AD_LAUNCH(1, true) : TI_AD_LAUNCH(1, false);
+    else if (T <= 512) vany ? TI_AD_LAUNCH(2, true) : TI_AD_LAUNCH(2, false);
+    else if (T <= 768) vany ? TI_AD_LAUNCH(3, true) : TI_AD_LAUNCH(3, false);
+    else if (T <= 1024) vany ? TI_AD_LAUNCH(4, true) : TI_AD_LAUNCH(4, false);
+    else if (T <= 1280) vany ? TI_AD_LAUNCH(5, true) : TI_AD_LAUNCH(5, false);
+    else if (T <= 1536) vany ? TI_AD_LAUNCH(6, true) : TI_AD_LAUNCH(6, false);
     else if (T <= 2048) vany ? TI_AD_LAUNCH(8, true) : TI_AD_LAUNCH(8, false);
+    else if (T <= 3072) vany ? TI_AD_LAUNCH(12, true) : TI_AD_LAUNCH(12, false);
     else vany ? TI_AD_LAUNCH(16, true) : TI_AD_LAUNCH(16, false);
 #undef TI_AD_LAUNCH
     return launch_status("attention_decode_i8_kernel");
