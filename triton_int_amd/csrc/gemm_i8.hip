@@ -1559,6 +1559,9 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
     int b_extent = 0, b_n0 = 0;
     // one column of tiles: every byte of A is read exactly once, so it need not stay in the caches
     const bool a_once = p.tiles_n == 1;
+    // Tiles of 64 columns: weights read once (one row tile) of 96 MB and more pass the caches by, 128 x 5120 x 20480 37.3 / 36.2 us, 128 x 16384 x 16384
+    // 65.7 / 61.7; smaller ones may still lie in the Infinity Cache, 64 x 6848 x 10240 16.5 / 19.5
+    const bool b_once = p.tiles_m == 1 && (int64_t)p.N * p.K * p.batch >= 96000000;
     auto aim = [&](int i) {
       kt_left = KT;
       k_issue = 0;
@@ -1606,10 +1609,15 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
         b_kn += (int64_t)BK * ldb;
         b_extent = max(b_extent - BK * ldb, 0);
       } else {
+        if (BN == 64 && b_once) {
 #pragma unroll
-        for (int d = 0; d < B_IT; ++d)
-          dma16_to_lds(rB, (k_issue < lb.klim[d]) ? lb.voff[d] : OOB, k_issue,
-                       wave_slot + st_issue * STAGE + A_BYTES + d * NTP * 16);
+          for (int d = 0; d < B_IT; ++d)
+            dma16_to_lds_stream(rB, (k_issue < lb.klim[d]) ? lb.voff[d] : OOB, k_issue, wave_slot + st_issue * STAGE + A_BYTES + d * NTP * 16);
+        } else {
+#pragma unroll
+          for (int d = 0; d < B_IT; ++d)
+            dma16_to_lds(rB, (k_issue < lb.klim[d]) ? lb.voff[d] : OOB, k_issue, wave_slot + st_issue * STAGE + A_BYTES + d * NTP * 16);
+        }
       }
       k_issue += BK;
       st_issue = (st_issue + 1 == NSTAGE) ? 0 : st_issue + 1;
@@ -2908,6 +2916,8 @@ enum ConfigId {
   CFG_ROWPIECES_64,
   CFG_RAGGED_128,      // rows at any byte, any K, [K,N] operands
   CFG_RAGGED_64,
+  CFG_WS_64x64,        // one row tile: every weight row belongs to one workgroup, read in 256-byte pieces
+  CFG_WS_128x64,
 };
 
 constexpr int RP_KC = 256;
@@ -2981,6 +2991,8 @@ static const Config g_configs[] = {
     TI_ROWPIECES(64),
     {"ragged_128x128x64", TI_RAGGED(128, 128, false), 128, 128, 64, 256, false, false, 0, false, 0, 0, false, true},
     {"ragged_64x64x64", TI_RAGGED(64, 64, false), 64, 64, 64, 256, false, false, 0, false, 0, 0, false, true},
+    TI_WS(64, 64, 256, 2, 2, 0, 4, 4),
+    TI_WS(128, 64, 256, 2, 2, 0, 3, 4),
 };
 static const int g_num_configs = (int)(sizeof(g_configs) / sizeof(g_configs[0]));
 
@@ -3128,6 +3140,11 @@ static int pick_splits(const GemmParams& p, const Config& k, double eff, double*
 // Splits are limited to one round of items, and 2 us were added to the fitted 2.824 of a 256 x 128 split: two rounds of splits lost wherever they were chosen
 // (whole K / 3 splits on 256 x 128: 1036 x 4096 x 16384 96 / 104, 1234 x 4096 x 16384 102 / 118), as did 256 x 128 in 4 splits against 128 x 128
 // in 2 (395 x 4096 x 16384 42.7 / 46.0).
+// 128 x 64 tiles, up to 128 rows: every workgroup streams weight rows of its own, in 256-byte pieces, where two row tiles of 64 x 128 ask for each of them
+// twice.  Fitted to 204 launches of 65 .. 128 rows, less 0.9 us: with the choice between both in mind.  Splits of 1280 and more (128 x 4096 x 4096, three /
+// four splits 12.1 / 13.7).  us, the best of the others / this, weights from HBM: 75 x 4384 x 2464 13.1 / 10.9, 85 x 6160 x 4960 20.5 /
+// 17.0, 128 x 5120 x 20480 41.7 / 37.1, 104 x 576 x 20016 17.4 / 15.1, three grouped 90 x 4096 x 4096 21.3 / 20.0; 128 x 4096 x 4096 12.1 / 12.1; but 90 x 20480 x
+// 5120 (320 tiles) 38.6 / 40.5, 128 x 4096 x 1024 7.5 / 7.7.
 // Left to config_cost: K < 1024, where rounds are mostly epilogue; more than 20480 columns (config_cost's choice / this one's: 300 x 50272 x
 // 1024 39.8 / 47.7, 300 x 50272 x 4096 97 / 107, 384 x 50272 x 2048 59.2 / 64.7; up to 128 rows the same); K beyond 28672 (N = 4096, K = 28672 1.08
 // of the fastest / 1.02, 5120 x 24576 1.03 / 1.02, 11264 x 32768 1.01 / 1.01).  M has no end: 17000 .. 32768 rows 1.025 / 1.004.
@@ -3171,14 +3188,17 @@ static int pick_ws(const GemmParams& p, int* splits_out, bool may_split) {
       {CFG_WS_128x128, 0.000, 0.292, 0.180, 3.614, 4.137, 2.237, 0.240, 0.000, 0.642, 0.764},
       {CFG_WS_256x128, 0.000, 0.438, 0.252, 4.620, 5.677, 4.824, 0.393, 0.000, 0.581, 1.467},
       {CFG_WS_256x160, 0.000, 0.526, 0.292, 9.049, 6.328, 3.050, 0.730, 0.825, 0.520, 1.645},
+      {CFG_WS_128x64, 0.100, 0.455, 0.255, 3.699, 3.998, 1.421, 0.304, 0.000, 0.544, 0.179},
   };
   int best = CFG_WS_128x128;
   double best_time = -1.0;
   for (const WsCost& c : costs) {
+    const bool narrow = c.cfg == CFG_WS_128x64;
+    if (narrow && p.M > 128) continue;
     const Config& k = g_configs[c.cfg];
     const int64_t tiles = (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bn - 1) / k.bn);
     for (int want : {1, 2, 3, 4, 6, 8}) {
-      if (want > 1 && (!may_split || p.batch != 1 || tiles * want > 256 || p.K < 384 * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
+      if (want > 1 && (!may_split || p.batch != 1 || tiles * want > 256 || p.K < (narrow ? 1280 : 384) * want || (size_t)tiles * want * k.bm * k.bn * sizeof(int) > SK_MAX_PARTIAL_BYTES)) break;
       int splits;
       const double t = ws_time(p, k, c, want, splits);
       if (best_time < 0 || t < best_time) best_time = t, best = c.cfg, *splits_out = splits;
@@ -3290,6 +3310,17 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
     // weights: 32 x 128 tiles with 7 stages up to 32 rows, 64 x 128 with 6 stages beyond (a 128 x 128 tile has
     // room for 4).  Measured in steady state, weights rotated through 350 MB, N = 6848, K = 10240, against
     // the 128 x 128 tile: M = 17 .. 32 34 -> 22-23 us, M = 64 35 -> 28.5 us; N = K = 5120: 18.5-19 -> 15-16 us.
+    // Up to 256 tiles of 64 columns and K from 1536 on, 64 x 64: twice the CUs for the same splits, weight rows in
+    // 256-byte pieces.  us, 32 x 128 or 64 x 128 / this, weights in the Infinity Cache; from HBM: 64 x 6848 x 10240 18.1 / 16.5; 23.6 / 22.3, 64 x 4096 x 16384 18.5 /
+    // 17.0; 21.9 / 21.9, 40 x 5120 x 20480 29.1 / 25.5, 57 x 13008 x 18160 72.3 / 65.3, 46 x 416 x 10000 16.5 / 10.0; 18.0 / 10.2, 24 x 352 x 17584 14.3 / 10.9;
+    // more tiles than CUs: 64 x 20480 x 5120 35.6 / 35.6, 32 x 17792 x 14096 55.0 / 83; whole K on 129 .. 191 CUs: 18 x 8656 x 20144 50 / 56, 45 x
+    // 10560 x 20048 59 / 66; K below: 32 x 272 x 1152 6.6 / 6.6.
+    const int64_t tiles = (p.N + 63) / 64;
+    if ((tiles <= 128 || (tiles >= 192 && tiles <= 256)) && p.K >= 1536) {
+      const int64_t fill = 256 / tiles, by_k = p.K / 1024, want = fill < by_k ? fill : by_k;
+      *splits_out = !may_split || want < 1 ? 1 : want > 8 ? 8 : (int)want;
+      return CFG_WS_64x64;
+    }
     const int cfg = p.M <= 32 ? CFG_WS_32x128 : CFG_WS_64x128;
     *splits_out = pick_splits(p, g_configs[cfg], 1.0, nullptr);
     return cfg;
