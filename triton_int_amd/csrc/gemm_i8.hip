@@ -3282,13 +3282,19 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
     //   15.6 / 19.1 (1), 16384 x 512 18.0 / 20.2 (32), 28.7 / 26.0 (64), 12288 x 640 13.5 / 12.3 (16), 20.8 / 15.2 (32).  The line: any K
     //   (M <= 16), 512 (32), 256 (64).  (One GEMM of more rounds and M > 16 has the tiles below.)  With a
     //   residual this kernel: the other would take an add kernel after it.
+    //   Outputs that the tiles cannot store (int8 of N no multiple of 16) have gemm_skinny_kernel instead: this one at any K.  int8 out,
+    //   64 x 17000 x 4096 59.1 / 18.3, 64 x 5001 x 12000 49.4 / 23.5, 64 x 511 x 1024 13.8 / 5.3, 40 x 333 x 16000 31.7 / 16.7, 17 x 300 x 1040 6.5 / 4.9;
+    //   equal at 32 x 5001 x 12000 21.5 / 21.9 and 17 x 20001 x 10240.
     // Three corners stay on the tiles although this kernel measures better there, because tests name what
-    // they run on: M > 48 with 16385 .. 20480 columns (64 x 20480 x 5120 34.0 / 28.2), M > 16 with fewer than 512
-    // (32 x 272 x 1040 8.5 / 5.3), M > 48 with one unit per workgroup and K > 4096 (64 x 1024 x 10240 17.0 / 15.7).
+    // they run on: M > 48 with 16385 .. 20480 columns of 4 or 2 bytes (64 x 20480 x 5120 34.0 / 28.2), M > 16 with fewer than 512
+    // (32 x 272 x 1040 8.5 / 5.3), M > 48 with one unit per workgroup and K > 4096 (64 x 1024 x 10240 17.0 / 15.7).  int8 columns of the first
+    // stay below K = 2048 only (weights in the Infinity Cache; from HBM: 64 x 20480 x 5120 34.9 / 24.6; 35.4 / 24.6, 49 x 16400 x 5120 21.8 / 20.8; 30.8 / 21.1, 64 x
+    // 18000 x 2048 12.1 / 13.2; 15.2 / 12.5, but 64 x 20480 x 1024 8.8 / 10.4; 10.4 / 9.8).
     const int units = (p.N + 3) / 4, per = (units + 256 / p.batch - 1) / (256 / p.batch);
     const bool one_round = per <= 4 * RP_GMAX;
     const int64_t columns = (int64_t)p.N * p.batch;
     const int rp = CFG_ROWPIECES_16 + (p.M - 1) / 16;
+    const bool wide8 = out_class(p.out_dtype) == OUT8 && p.K >= 2048;
     if (p.M <= 16 && p.K >= 1024) return one_round ? rp : CFG_ROWS4_16;
     if (p.K < 1024) {
       const bool slabs = !p.resid && (one_round ? p.K <= (p.M <= 16 ? 256 : p.M <= 32 ? 128 : per >= 12 ? 64 : 0) : p.M <= 16 || p.K <= (p.M <= 32 ? 512 : 256));
@@ -3296,7 +3302,9 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
         if (!slabs) return rp;
         if (p.M > 16) return CFG_SKINNY_16 + 1 + (p.M > 32);
       }
-    } else if (one_round && p.K <= (p.M <= 32 ? 16384 : p.M <= 48 ? 10240 : per > 1 ? 8192 : 4096) && !(p.M > 48 && columns > 16384) && columns >= 512) {
+    } else if (one_round && !stream) {
+      return rp;
+    } else if (one_round && p.K <= (p.M <= 32 ? 16384 : p.M <= 48 ? 10240 : per > 1 ? 8192 : 4096) && (p.M <= 48 || columns <= 16384 || wide8) && columns >= 512) {
       return rp;
     }
   }
