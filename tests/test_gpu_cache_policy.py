@@ -33,12 +33,12 @@ def test_row_norms(rows, cols):
         assert torch.equal(resid[a:b], r) and torch.equal(z[a:b], q)
 
 
-@pytest.mark.parametrize("rows,cols,causal", [(82000, 2048, 0), (82000, 2048, 2000), (82000, 2047, 0), (81920, 2048, 0)])  # 160 Mi scores is the line
+@pytest.mark.parametrize("rows,cols,causal", [(82000, 2048, 0), (82000, 2048, 2000), (82000, 2047, 0), (49152, 2048, 0)])  # beyond 96 Mi scores
 def test_softmax(rows, cols, causal):
     g = torch.Generator(device=DEV).manual_seed(2)
     s = _int8(g, rows, cols)
     p = softmax_q(s, 0.05, causal_q_len=causal)
-    for a, b in ((0, 2000), (40000, 42000), (rows - 2000 if causal == 0 else 80000, rows if causal == 0 else 82000)):
+    for a, b in ((0, 2000), (40000, 42000) if causal else (30000, 32000), (rows - 2000 if causal == 0 else 80000, rows if causal == 0 else 82000)):
         assert torch.equal(p[a:b], softmax_q(s[a:b], 0.05, causal_q_len=causal))
 
 

@@ -57,7 +57,7 @@ struct GemmParams {
   int batch, M, N, K;
   const void* bias;
   int bias_kind;
-  int keep;  // persistent kernels: the outputs are stored for the next launch to find in the Infinity Cache, else streamed past it
+  int keep;  // gemm_mfma_shortk_kernel: int8 outputs are stored for the next launch to find in the Infinity Cache, else streamed past it
   const float* alpha;
   const float* beta;
   int epilogue, out_dtype, round_mode;
@@ -661,7 +661,7 @@ constexpr int epi_strip_bytes(int wtn) { return ((wtn / 16) & (wtn / 16 - 1)) ==
 // Cache policy of the stores.  Non-temporal leaves the operand panels in L2 and the Infinity Cache (P.V with fp32 output,
 // 168 MB of probabilities: 192 -> 162 us; every store instruction of a 4-byte output writes two whole 128-byte lines), but the
 // launch that reads the outputs then fetches them from HBM.  Device scope (sc1) writes them through L2 into the
-// Infinity Cache, where that launch finds them: keep_outputs() says which.
+// Infinity Cache, where that launch finds them: stream_epilogue says which.
 constexpr int STORE_STREAM = 2, STORE_KEEP = 16;
 
 // 2-byte outputs: pairs of neighbouring elements of a row can go out as one aligned dword
@@ -976,9 +976,12 @@ __device__ __forceinline__ void store_epilogue(const GemmParams& p, const EpiCtx
 template <int TM, int TN, int OUTCLS, bool LDS_COLS = true>
 __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
                                                 int mw, int nw, char* strip, int lane) {
-  // int8 without a strip stores with the default policy
-  constexpr bool CHOICE = OUTCLS != OUT8 || epi_strip_bytes(TN * 32) != 0;
-  if (!CHOICE || p.keep) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_KEEP>(p, e, acc, bz, mw, nw, strip, lane);
+  // One copy of the code each, except in the kernel for a short K (the one without column terms): a second one cost the launches of a linear set 1 %.
+  // int8 outputs are read by the next launch and a quarter of the bytes: for the cache.  4- and 2-byte ones stream: kept, the output of fc2 gained
+  // its launch nothing, and P.V over 168 MB of probabilities lost 10 %.
+  if constexpr (OUTCLS == OUT8 && LDS_COLS) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_KEEP>(p, e, acc, bz, mw, nw, strip, lane);
+  else if constexpr (OUTCLS != OUT8) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_STREAM>(p, e, acc, bz, mw, nw, strip, lane);
+  else if (p.keep) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_KEEP>(p, e, acc, bz, mw, nw, strip, lane);
   else store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_STREAM>(p, e, acc, bz, mw, nw, strip, lane);
 }
 
@@ -3341,6 +3344,14 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
     const int64_t tm = (p.M + 255) / 256, tn = (p.N + 255) / 256;
     if (tm * tn * p.batch >= 512 && (double)p.M * p.N >= 0.6 * (double)(tm * 256) * (double)(tn * 256)) return CFG_SHORTK_256x256;
   }
+  // Attention scores that the persistent kernels cannot store (an odd number of keys): the epilogue is most of the launch.  128 x 128 tiles, and 64 x 64
+  // of gemm_ragged_kernel where they are a fifth less padding or the larger are few.  us, the 256-row tiles that the estimate took / 128 x 128 / 64 x 64: 149 heads x
+  // 1000 x 1000 95.0 / 90.3 / 123, 40 x 1366 57.5 / 52.0 / 67, 107 x 234 9.8 / 8.8 / 10.8, 30 x 510, K = 64 11.1 / 9.8 / 10.2, 100 x 150 7.5 / 6.2 / 5.9, 90 x 190 9.7 / 7.9 /
+  // 7.2, 141 x 137 8.7 / 10.2 / 8.1, 150 x 90 7.4 / 5.9 / 5.4; 160 x 130 7.5 / 11.1 / 8.4 loses.
+  if (!stream && out_class(p.out_dtype) == OUT8 && p.batch > 4 && p.K <= 128) {
+    const int64_t t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64), t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
+    return (ragged_eligible(p) && (t64 * 5 < t128 * 16 || t128 * p.batch <= 192)) ? CFG_RAGGED_64 : CFG_TILE_128x128;
+  }
   // short K: the epilogue dominates and the larger tile halves the operand traffic per output
   const double big = p.K <= 512 ? 1.20 : 0.92;
   // 256 x 160 tiles: as good as 256 x 128 per unit of work with 2- and 4-byte outputs; with int8 outputs
@@ -3398,14 +3409,13 @@ static int pick_group_m(const GemmParams& p, const Config& k) {
   return best;
 }
 
-// Whether the outputs of a launch on a persistent kernel stay in the 256 MB Infinity Cache for the launch that reads them:
-// where that, with what this launch reads, takes less than half of it.  us of a launch and the one after it, stored
-// non-temporally / for the cache: Q.K^T 40 x 1024^2 and its softmax 40.0 / 38.8, 80 x 1024^2 63.1 / 58.2, but 160 x 1024^2 (168 MB of
-// scores) 120 / 123; P.V with fp32 output 40 x 1024 x 128 17.3 / 14.1, but 80 x 1024 (136 MB) 30.3 / 31.4 and 160 x 1024 49.8 / 55.0.
+// Whether int8 scores from gemm_mfma_shortk_kernel stay in the 256 MB Infinity Cache for the launch that reads them: where they, with what this
+// launch reads, take 96 MB of it at most.  us of a launch and its softmax, streamed / kept: 40 x 1024^2 40.0 / 38.8, but 160 x 1024^2 (168 MB
+// of scores) 120 / 123, 40 x 2048^2 with P.V 141 / 155.
 static bool keep_outputs(const GemmParams& p) {
   const int esz = p.out_dtype == TI_I8 ? 1 : ((p.out_dtype == TI_F16 || p.out_dtype == TI_BF16) ? 2 : 4);
   const double a = (double)p.M * p.K * (p.sAb ? p.batch : 1), b = (double)p.N * p.K * p.batch, c = (double)p.M * p.N * p.batch * esz;
-  return a + b + c <= 128e6;
+  return a + b + c <= 96e6;
 }
 
 static int validate(const GemmParams& p) {

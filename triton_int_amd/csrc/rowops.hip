@@ -723,9 +723,9 @@ int ti_softmax_q(const int8_t* x, int64_t x_row_stride, float scale, int8_t* y, 
   dim3 grid((unsigned)((rows + ti::SM_WAVES - 1) / ti::SM_WAVES)), block(ti::SM_WAVES * 64);
   const int vpt = (cols + 1023) / 1024;
   const bool aligned = ((((uintptr_t)x) | ((uintptr_t)y) | (uintptr_t)x_row_stride | (uintptr_t)y_row_stride | (uintptr_t)cols) & 15) == 0;
-  // for the Infinity Cache (see LOAD_AUX) up to 168 MB of scores, us, non-temporal / for the cache: 40 x 1024^2 22.0 / 20.3, 80 x 1024^2
-  // 36.3 / 31.4, 40 x 2048^2 55.9 / 51.6, but 80 x 2048^2 110 / 125, 160 x 2048^2 215 / 248
-  const bool keep = (int64_t)rows * cols <= (int64_t)160 << 20, vec = aligned && scale > 0.0f;
+  // for the Infinity Cache (see LOAD_AUX) up to 100 MB of scores, us, non-temporal / for the cache: 40 x 1024^2 22.0 / 20.3, 80 x 1024^2
+  // 36.3 / 31.4, but 80 x 2048^2 110 / 125, 160 x 2048^2 215 / 248
+  const bool keep = (int64_t)rows * cols <= (int64_t)96 << 20, vec = aligned && scale > 0.0f;
   const auto launch = [&](auto vpt_tag, auto keep_tag) {
     constexpr int VPT = decltype(vpt_tag)::value;
     constexpr bool KEEP = decltype(keep_tag)::value;
