@@ -132,7 +132,11 @@ int ti_bmm_i8(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk,
  * the number of streaming waves (4, 6, 8); 0 = choose.  Returns TI_E_COMBO if the configuration
  * cannot run the given shape or stride pattern (e.g. "shortk_..." takes 16 <= K <= 128 and, for
  * int8 outputs, neither bias nor GELU) or cannot split K that way.
+ * Bit 16 (TI_CONFIG_NEXT_READS) of a non-negative config says that the caller's next launch reads the
+ * outputs: int8 ones are then stored for it to find in the Infinity Cache up to 256 MB.  The bits of the
+ * outputs do not depend on it.  0xff | TI_CONFIG_NEXT_READS chooses like -1.
  */
+#define TI_CONFIG_NEXT_READS 0x10000
 int ti_bmm_i8_config(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk,
                      const int8_t* B, int64_t sBb, int64_t sBn, int64_t sBk,
                      void* C, int64_t sCb, int64_t sCm, int64_t sCn,
@@ -201,6 +205,9 @@ const char* ti_gemm_config_name(int config);
 int ti_gemm_last_config(void);
 /* Number of K splits that launch used (1 = K not split). */
 int ti_gemm_last_splits(void);
+/* 1 if the persistent kernels store the int8 outputs of such a launch (shared_a: sAb = 0) for the next launch to find in the
+ * Infinity Cache, 0 if they stream them past it.  Runs without a GPU. */
+int ti_gemm_keeps_outputs(int batch, int shared_a, int M, int N, int K, int config);
 /*
  * Dry run of ti_bmm_i8_config (static_scratch != 0: of ti_bmm_i8_static_scratch): takes every decision
  * the launch would take, through the same host code (validation, choice of configuration, K split, tile

@@ -26,7 +26,7 @@ TORCH_TO_BIAS = {torch.int8: BIAS_I8, torch.int32: BIAS_I32, torch.float32: BIAS
                  torch.bfloat16: BIAS_BF16}
 
 EXPORTS = ("ti_version", "ti_last_error", "ti_mfma_i8_probe", "ti_bmm_i8", "ti_bmm_i8_config", "ti_bmm_i8_grouped", "ti_bmm_i8_static_scratch", "ti_gemm_num_configs",
-           "ti_gemm_config_name", "ti_gemm_last_config", "ti_gemm_last_splits", "ti_gemm_plan", "ti_release_workspaces", "ti_layernorm_q", "ti_dq_add_layernorm_q", "ti_gelu_q", "ti_softmax_q", "ti_transpose_i8", "ti_attention_i8", "ti_attention_i8_heads", "ti_attention_i8_rows", "ti_quantize_per_token_absmax", "ti_quantize_per_tensor_absmax", "ti_kv_append_i8", "ti_kv_append_i8_seqs", "ti_layernorm_qkv_decode_i8_seqs", "ti_dq_add_layernorm_linear_gelu_i8",
+           "ti_gemm_config_name", "ti_gemm_last_config", "ti_gemm_last_splits", "ti_gemm_keeps_outputs", "ti_gemm_plan", "ti_release_workspaces", "ti_layernorm_q", "ti_dq_add_layernorm_q", "ti_gelu_q", "ti_softmax_q", "ti_transpose_i8", "ti_attention_i8", "ti_attention_i8_heads", "ti_attention_i8_rows", "ti_quantize_per_token_absmax", "ti_quantize_per_tensor_absmax", "ti_kv_append_i8", "ti_kv_append_i8_seqs", "ti_layernorm_qkv_decode_i8_seqs", "ti_dq_add_layernorm_linear_gelu_i8",
            "ti_layernorm_fp", "ti_linear_i8_residual_f32", "ti_qkv_decode_i8", "ti_qkv_decode_i8_seqs", "ti_qkv_append_i8_seqs")
 
 _lib = None
@@ -63,6 +63,8 @@ def _declare(lib):
     lib.ti_gemm_last_config.argtypes = []
     lib.ti_gemm_last_splits.restype = _int
     lib.ti_gemm_last_splits.argtypes = []
+    lib.ti_gemm_keeps_outputs.restype = _int
+    lib.ti_gemm_keeps_outputs.argtypes = [_int] * 6
     lib.ti_gemm_config_name.restype = ctypes.c_char_p
     lib.ti_gemm_config_name.argtypes = [_int]
     lib.ti_layernorm_q.restype = _int

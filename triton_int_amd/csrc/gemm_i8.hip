@@ -57,7 +57,6 @@ struct GemmParams {
   int batch, M, N, K;
   const void* bias;
   int bias_kind;
-  int keep;  // gemm_mfma_shortk_kernel: int8 outputs are stored for the next launch to find in the Infinity Cache, else streamed past it
   const float* alpha;
   const float* beta;
   int epilogue, out_dtype, round_mode;
@@ -94,6 +93,7 @@ template <int NORM>
 using RowpiecesParams = typename std::conditional<NORM == NORM_NONE, GemmParams, GemmNormParams>::type;
 
 enum OutClass { OUT8 = 0, OUT32 = 1, OUT16 = 2 };
+constexpr int OUT8_STREAM = 3;  // in a table of kernels only: int8 outputs that pass the caches by
 
 
 // ---- tile -> (m, n) mapping ----------------------------------------------------------------
@@ -661,8 +661,9 @@ constexpr int epi_strip_bytes(int wtn) { return ((wtn / 16) & (wtn / 16 - 1)) ==
 // Cache policy of the stores.  Non-temporal leaves the operand panels in L2 and the Infinity Cache (P.V with fp32 output,
 // 168 MB of probabilities: 192 -> 162 us; every store instruction of a 4-byte output writes two whole 128-byte lines), but the
 // launch that reads the outputs then fetches them from HBM.  Device scope (sc1) writes them through L2 into the
-// Infinity Cache, where that launch finds them: stream_epilogue says which.
+// Infinity Cache, where that launch finds them.  4- and 2-byte outputs stream; int8 ones have a kernel for each, and keep_outputs says which.
 constexpr int STORE_STREAM = 2, STORE_KEEP = 16;
+constexpr int store_default(int outcls) { return outcls == OUT8 ? STORE_KEEP : STORE_STREAM; }
 
 // 2-byte outputs: pairs of neighbouring elements of a row can go out as one aligned dword
 __device__ __forceinline__ bool out16_pairs(const GemmParams& p) {
@@ -670,9 +671,9 @@ __device__ __forceinline__ bool out16_pairs(const GemmParams& p) {
 }
 // LDS_COLS false: `strip` has no room for the column terms; int8 launches with a bias or GELU are not
 // compiled in (the host refuses them for such a kernel).
-template <int TM, int TN, int OUTCLS, bool LDS_COLS, int AUX>
-__device__ __forceinline__ void store_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
-                                               int mw, int nw, char* strip, int lane) {
+template <int TM, int TN, int OUTCLS, int AUX, bool LDS_COLS = true>
+__device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
+                                                int mw, int nw, char* strip, int lane) {
   constexpr int WTN = TN * 32;
   constexpr int ESZ = OUTCLS == OUT8 ? 1 : (OUTCLS == OUT32 ? 4 : 2);
   const int OOB = (int)0x80000000;
@@ -973,18 +974,6 @@ __device__ __forceinline__ void store_epilogue(const GemmParams& p, const EpiCtx
   }
 }
 
-template <int TM, int TN, int OUTCLS, bool LDS_COLS = true>
-__device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCtx& e, v16i (&acc)[TM][TN], int bz,
-                                                int mw, int nw, char* strip, int lane) {
-  // One copy of the code each, except in the kernel for a short K (the one without column terms): a second one cost the launches of a linear set 1 %.
-  // int8 outputs are read by the next launch and a quarter of the bytes: for the cache.  4- and 2-byte ones stream: kept, the output of fc2 gained
-  // its launch nothing, and P.V over 168 MB of probabilities lost 10 %.
-  if constexpr (OUTCLS == OUT8 && LDS_COLS) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_KEEP>(p, e, acc, bz, mw, nw, strip, lane);
-  else if constexpr (OUTCLS != OUT8) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_STREAM>(p, e, acc, bz, mw, nw, strip, lane);
-  else if (p.keep) store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_KEEP>(p, e, acc, bz, mw, nw, strip, lane);
-  else store_epilogue<TM, TN, OUTCLS, LDS_COLS, STORE_STREAM>(p, e, acc, bz, mw, nw, strip, lane);
-}
-
 // ---- persistent ("stream") variant of the fast family --------------------------------------------
 //
 // One workgroup per CU slot walks a list of output tiles, and the global -> LDS pipeline does not
@@ -1010,7 +999,7 @@ __device__ __forceinline__ void stream_epilogue(const GemmParams& p, const EpiCt
 // instruction), 2-byte outputs as dword pairs after a lane exchange where the output's alignment
 // allows, int8 outputs exchange dwords between the two wave halves so that every lane owns 16
 // consecutive bytes of a row and go through a wave-private LDS strip.
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int OCC = 1>
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int OCC = 1, int AUX = store_default(OUTCLS)>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (WAVES_M * WAVES_N * OCC + 3) / 4) void gemm_mfma_stream_kernel(GemmParams p) {
   constexpr int NT = WAVES_M * WAVES_N * 64;
   constexpr int CH = BK / 16;
@@ -1225,8 +1214,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (WAVES_M * WAVES_N * OCC + 3
     }
 
     // ---- epilogue
-    stream_epilogue<TM, TN, OUTCLS>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN,
-                                    lds + NSTAGE * STAGE + wave * (STRIP + COLS), lane);
+    stream_epilogue<TM, TN, OUTCLS, AUX>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN,
+                                         lds + NSTAGE * STAGE + wave * (STRIP + COLS), lane);
   }
   // the trailing (empty-buffer) loads still write zeros into LDS: they must land before the
   // workgroup's LDS is handed to another one
@@ -1252,7 +1241,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, (WAVES_M * WAVES_N * OCC + 3
 // Tried and removed: a ping-pong order (the two waves of a SIMD in opposite order between barriers,
 // one wave's MFMAs under the other's epilogue), 9-16 % slower than this order for every pairing of
 // waves (160 x 2048 x 2048 x 128: 193 us against 209-224 us).
-template <int OUTCLS>
+template <int OUTCLS, int AUX = store_default(OUTCLS)>
 __global__ __launch_bounds__(512) void gemm_mfma_shortk_kernel(GemmParams p) {
   constexpr int BM = 256, BN = 256, BK = 64, WAVES_N = 2, SWZ = 2, KTMAX = 2;
   constexpr int NT = 512, CH = BK / 16;
@@ -1382,7 +1371,7 @@ __global__ __launch_bounds__(512) void gemm_mfma_shortk_kernel(GemmParams p) {
     int bz, m0, n0;
     locate(t, bz, m0, n0);
     const EpiCtx e = make_epi(p, bz);
-    stream_epilogue<TM, TN, OUTCLS, false>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN, lds + 2 * TILE + wave * STRIP, lane);
+    stream_epilogue<TM, TN, OUTCLS, AUX, false>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN, lds + 2 * TILE + wave * STRIP, lane);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
@@ -1471,7 +1460,7 @@ __device__ __forceinline__ bool split_k_settle(const GemmParams& p, v16i (&acc)[
 // BKN: B is [K,N] (V as it comes out of its projection).  A stage holds it as [k][128 n] and the consumers read it
 // with the transposing LDS read.  40 x 1024 x 128 x 1024 14.5 us: 160 of the 256 CUs have a tile, and each takes in its
 // 384 KB at about 33 GB/s.
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int PW, bool BKN = false>
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int SWZ, int NSTAGE, int OUTCLS, int PW, bool BKN = false, int AUX = store_default(OUTCLS)>
 __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_kernel(GemmParams p) {
   constexpr int NWC = WAVES_M * WAVES_N;  // consumer waves
   constexpr int NTP = PW * 64;            // producer threads
@@ -1757,8 +1746,8 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
       if (!split_k_settle<TM, TN, NWC>(p, acc, rank, sp, SPL, wave, lane)) continue;
     }
     if (wave == 0 && it == 0) TI_TL(2);
-    stream_epilogue<TM, TN, OUTCLS>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN,
-                                    lds + NSTAGE * STAGE + wave * (STRIP + COLS), lane);
+    stream_epilogue<TM, TN, OUTCLS, AUX>(p, e, acc, bz, m0 + wm * WTM, n0 + wn * WTN,
+                                         lds + NSTAGE * STAGE + wave * (STRIP + COLS), lane);
     if (wave == 0 && it == 0) TI_TL(3);
   }
   if (wave == 0) TI_TL(4);
@@ -2831,7 +2820,7 @@ typedef void (*NormKernelFn)(GemmNormParams);
 
 struct Config {
   const char* name;
-  KernelFn fn[3];  // by OutClass
+  KernelFn fn[4];  // by OutClass, then OUT8_STREAM (persistent kernels of tiles that many rows take)
   int bm, bn, bk, threads;
   bool fast;       // needs the aligned K-contiguous layout
   bool skinny = false;  // gemm_skinny_kernel: M <= 64, grid over 16-row slabs of B
@@ -2857,18 +2846,22 @@ struct Config {
     "stream_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_s" #SWZ "_p" #NS "_o" #OCC,            \
         {gemm_mfma_stream_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT8, OCC>,                   \
          gemm_mfma_stream_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT32, OCC>,                  \
-         gemm_mfma_stream_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT16, OCC>},                 \
+         gemm_mfma_stream_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT16, OCC>,                  \
+         gemm_mfma_stream_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT8, OCC, STORE_STREAM>},    \
         BM, BN, BK, WM * WN * 64, true, false, OCC                                        \
   }
 
-#define TI_WS(BM, BN, BK, WM, WN, SWZ, NS, PW)                                            \
+#define TI_WS_AS(BM, BN, BK, WM, WN, SWZ, NS, PW, ...)                                    \
   {                                                                                       \
     "ws_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_s" #SWZ "_p" #NS "_l" #PW,                 \
         {gemm_mfma_ws_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT8, PW>,                        \
          gemm_mfma_ws_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT32, PW>,                       \
-         gemm_mfma_ws_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT16, PW>},                      \
+         gemm_mfma_ws_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT16, PW>, __VA_ARGS__},         \
         BM, BN, BK, (WM * WN + PW) * 64, true, false, 1, false, WM * WN                   \
   }
+#define TI_WS(BM, BN, BK, WM, WN, SWZ, NS, PW) \
+  TI_WS_AS(BM, BN, BK, WM, WN, SWZ, NS, PW, gemm_mfma_ws_kernel<BM, BN, BK, WM, WN, SWZ, NS, OUT8, PW, false, STORE_STREAM>)
+#define TI_WS_FEW(BM, BN, BK, WM, WN, SWZ, NS, PW) TI_WS_AS(BM, BN, BK, WM, WN, SWZ, NS, PW, nullptr)  // up to 128 rows: outputs of a few MB
 
 #define TI_ROWPIECES(MT)                                                                  \
   {                                                                                       \
@@ -2888,8 +2881,9 @@ static KernelFn ragged_kn_kernel(int bm, int oc) {
 // gemm_mfma_ws_kernel for a [K,N] operand: 256 x 128 and 128 x 128 tiles
 static KernelFn ws_kn_kernel(int bm, int oc) {
 #define TI_WS_KN(BM, NS) {gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT8, 4, true>, \
-                          gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT32, 4, true>, gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT16, 4, true>}
-  static const KernelFn fns[2][3] = {TI_WS_KN(128, 4), TI_WS_KN(256, 3)};
+                          gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT32, 4, true>, gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT16, 4, true>, \
+                          gemm_mfma_ws_kernel<BM, 128, 128, 2, 2, 1, NS, OUT8, 4, true, STORE_STREAM>}
+  static const KernelFn fns[2][4] = {TI_WS_KN(128, 4), TI_WS_KN(256, 3)};
 #undef TI_WS_KN
   return fns[bm > 128][oc];
 }
@@ -2984,18 +2978,18 @@ static const Config g_configs[] = {
     {"rows4_m16", {gemm_rows4_kernel<OUT8, 8, 3>, gemm_rows4_kernel<OUT32, 8, 3>, gemm_rows4_kernel<OUT16, 8, 3>}, 16, 4, 1024, (R4_NW + 1) * 64, true, false, 0, true},
     TI_WS(256, 160, 128, 4, 1, 1, 3, 4),
     TI_WS(128, 128, 128, 2, 2, 1, 4, 4),
-    {"shortk_256x256x64_w4x2_k128", {gemm_mfma_shortk_kernel<OUT8>, gemm_mfma_shortk_kernel<OUT32>, gemm_mfma_shortk_kernel<OUT16>}, 256, 256, 64, 512,
+    {"shortk_256x256x64_w4x2_k128", {gemm_mfma_shortk_kernel<OUT8>, gemm_mfma_shortk_kernel<OUT32>, gemm_mfma_shortk_kernel<OUT16>, gemm_mfma_shortk_kernel<OUT8, STORE_STREAM>}, 256, 256, 64, 512,
      true, false, 1, false, 0, 128},
-    TI_WS(64, 128, 128, 2, 2, 1, 6, 4),
-    TI_WS(32, 128, 128, 1, 4, 1, 7, 4),
+    TI_WS_FEW(64, 128, 128, 2, 2, 1, 6, 4),
+    TI_WS_FEW(32, 128, 128, 1, 4, 1, 7, 4),
     TI_ROWPIECES(16),
     TI_ROWPIECES(32),
     TI_ROWPIECES(48),
     TI_ROWPIECES(64),
     {"ragged_128x128x64", TI_RAGGED(128, 128, false), 128, 128, 64, 256, false, false, 0, false, 0, 0, false, true},
     {"ragged_64x64x64", TI_RAGGED(64, 64, false), 64, 64, 64, 256, false, false, 0, false, 0, 0, false, true},
-    TI_WS(64, 64, 256, 2, 2, 0, 4, 4),
-    TI_WS(128, 64, 256, 2, 2, 0, 3, 4),
+    TI_WS_FEW(64, 64, 256, 2, 2, 0, 4, 4),
+    TI_WS_FEW(128, 64, 256, 2, 2, 0, 3, 4),
 };
 static const int g_num_configs = (int)(sizeof(g_configs) / sizeof(g_configs[0]));
 
@@ -3409,13 +3403,17 @@ static int pick_group_m(const GemmParams& p, const Config& k) {
   return best;
 }
 
-// Whether int8 scores from gemm_mfma_shortk_kernel stay in the 256 MB Infinity Cache for the launch that reads them: where they, with what this
-// launch reads, take 96 MB of it at most.  us of a launch and its softmax, streamed / kept: 40 x 1024^2 40.0 / 38.8, but 160 x 1024^2 (168 MB
-// of scores) 120 / 123, 40 x 2048^2 with P.V 141 / 155.
-static bool keep_outputs(const GemmParams& p) {
-  const int esz = p.out_dtype == TI_I8 ? 1 : ((p.out_dtype == TI_F16 || p.out_dtype == TI_BF16) ? 2 : 4);
-  const double a = (double)p.M * p.K * (p.sAb ? p.batch : 1), b = (double)p.N * p.K * p.batch, c = (double)p.M * p.N * p.batch * esz;
-  return a + b + c <= 96e6;
+// Whether int8 outputs of the persistent kernels stay in the 256 MB Infinity Cache: where they, with what the launch reads, take 96 MB of it at
+// most, or, where the caller says that the next launch reads them (TI_CONFIG_NEXT_READS), fit it.  Nobody reading them, kept outputs cost nothing up to
+// there, and beyond they push out weights and activations that would be found.  us, streamed / kept: one linear 4096 x 12288 x 2048 (84 MB) 96.2 / 95.9, 4096 x
+// 16384 x 1024 (88 MB) 73.4 / 71.6, but 1536 x 16384 x 4096 (99 MB) 88.2 / 93.6, 2048 x 16384 x 4096 (109 MB) 116.3 / 124.7, 4096 x 16384 x 4096 229 / 243, 8192 x 20480
+// x 5120 734 / 741; decoder layers, 1024 wide 4096 rows 205 / 196, 4096 wide 512 rows 175.2 / 174.3, 4096 rows 953 / 941, 8192 rows 1852 / 1833, 12288 rows (201 MB from
+// fc1) 2729 / 2724, 16384 rows 3633 / 3637.  Scores and the softmax after them, K = 256: 12 x 2048^2 (63 MB) 57.3 / 54.5, 20 (105 MB) 99.4 / 109.4, 60
+// 280 / 286, 96 440 / 454 (but 40 194 / 187); gemm_mfma_shortk_kernel 40 x 1024^2 40.0 / 38.8, 160 x 1024^2 120 / 123, 40 x 2048^2 with P.V 141 / 155.  P.V,
+// V as [K,N], 80 x 2048 x 128 x 2048 75.1 / 75.6.
+static bool keep_outputs(int64_t batch, bool shared_a, int64_t M, int64_t N, int64_t K, bool next_reads) {
+  const double a = (double)M * K * (shared_a ? 1 : batch), b = (double)N * K * batch, c = (double)M * N * batch;
+  return next_reads ? c <= 256e6 : a + b + c <= 96e6;
 }
 
 static int validate(const GemmParams& p) {
@@ -3587,7 +3585,7 @@ struct LaunchPlan {
 };
 
 // `config`: bits 0..7 the configuration (0xff or a negative value: choose), bits 8..15 the number of
-// K splits to use with a wave-specialised configuration (0: choose).
+// K splits to use with a wave-specialised configuration (0: choose), bit 16 (TI_CONFIG_NEXT_READS) see keep_outputs.
 // static_scratch: split-K launches use the fixed device array instead of the allocated workspace, and a
 // launch whose partial sums do not fit it is refused (nothing is allocated or freed on this path).
 // dry: every decision is taken as for a launch (same code), but no device is touched, nothing is
@@ -3598,6 +3596,8 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
                const NormArgs* norm = nullptr) {
   g_last_splits = 1;
   int want_splits = config < 0 ? 0 : (config >> 8) & 0xff;
+  const bool next_reads = config >= 0 && (config & TI_CONFIG_NEXT_READS);
+  const int choose = next_reads ? 0xff | TI_CONFIG_NEXT_READS : -1;
   if (config >= 0) config = (config & 0xff) == 0xff ? -1 : (config & 0xff);
   int rc = validate(p);
   if (rc != TI_OK) return rc;
@@ -3750,7 +3750,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
         return fail(TI_E_SHAPE, "%d K splits of %lld tiles need %zu bytes of partial sums: more than the %zu bytes of static scratch "
                     "(use ti_bmm_i8, which allocates its workspace)", splits, (long long)tiles, (size_t)tiles * splits * item_bytes,
                     SK_STATIC_PARTIAL_BYTES);
-      if (chosen) return run(p, -1, stream, static_scratch, dry, false);
+      if (chosen) return run(p, choose, stream, static_scratch, dry, false);
       sk_shape(kt, 1, splits, p.kt_split);
     }
     if (splits > 1 && static_scratch) {
@@ -3760,7 +3760,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       }
     } else if (splits > 1 && ((size_t)tiles * sk_waves(k) > SK_COUNTER_INTS || (size_t)tiles * splits * item_bytes > SK_MAX_PARTIAL_BYTES)) {
       if (want_splits) return fail(TI_E_SHAPE, "%d splits of %lld tiles exceed the split-K workspace", splits, (long long)tiles);
-      if (chosen) return run(p, -1, stream, static_scratch, dry, false);
+      if (chosen) return run(p, choose, stream, static_scratch, dry, false);
       splits = 1;
     }
     if (splits > 1 && !static_scratch && !dry) {
@@ -3770,7 +3770,7 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       // capturing without a large enough workspace, or no memory for one: an automatic split gives way
       if (!want_splits && (rc == TI_E_COMBO || rc == (int)hipErrorOutOfMemory)) {
         if (rc != TI_E_COMBO) (void)hipGetLastError();  // launch_status below asks for the launch's own
-        if (chosen) return run(p, -1, stream, false, nullptr, false);
+        if (chosen) return run(p, choose, stream, false, nullptr, false);
         splits = 1;
       } else if (rc == TI_E_COMBO) return fail(TI_E_COMBO, "no split-K workspace on this stream and none can be allocated during graph capture");
       else if (rc != TI_OK) return rc;
@@ -3795,8 +3795,8 @@ static int run(GemmParams p, int config, hipStream_t stream, bool static_scratch
       dry->grid_x = (unsigned)g; dry->grid_y = 1;
       return TI_OK;
     }
-    const KernelFn fn = kn ? ws_kn_kernel(k.bm, out_class(p.out_dtype)) : k.fn[out_class(p.out_dtype)];
-    p.keep = keep_outputs(p);
+    const int kind = p.out_dtype == TI_I8 && k.fn[OUT8_STREAM] && !keep_outputs(p.batch, !p.sAb, p.M, p.N, p.K, next_reads) ? OUT8_STREAM : out_class(p.out_dtype);
+    const KernelFn fn = kn ? ws_kn_kernel(k.bm, kind) : k.fn[kind];
     fn<<<dim3((unsigned)g), dim3(k.threads), 0, stream>>>(p);
     return launch_status(k.name);
   }
@@ -3910,6 +3910,10 @@ int ti_bmm_i8_grouped(const int8_t* A, int64_t sAb, int64_t sAm, int64_t sAk, co
   p.kv_k = p.kv_vt = nullptr; p.kv_k_hs = p.kv_k_rs = p.kv_vt_rs = 0; p.kv_D = p.kv_S = 1;
   p.splits = 1; p.kt_split = 0; p.sk_partial = p.sk_counter = nullptr;
   return ti::run(p, config, (hipStream_t)stream);
+}
+
+int ti_gemm_keeps_outputs(int batch, int shared_a, int M, int N, int K, int config) {
+  return ti::keep_outputs(batch, shared_a != 0, M, N, K, config >= 0 && (config & TI_CONFIG_NEXT_READS));
 }
 
 // Whether gemm_rowpieces_kernel can make these activations from their LayerNorm: few rows, whole 16-byte pieces of every row, and

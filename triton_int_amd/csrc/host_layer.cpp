@@ -217,6 +217,7 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
       int32_t* acc = (int32_t*)(base + at[3]);
       float* resid = (float*)(base + at[4]);
       const float* xp = (const float*)ptr(x);
+      const int next_reads = 0xff | TI_CONFIG_NEXT_READS;
       const auto run = [&]() {
         bool appended = false;
         if (few && cached) {
@@ -234,7 +235,7 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
         }
         if (!appended) {
           if ((rc = ti_bmm_i8_grouped(h8, 0, H, 1, (const int8_t*)ptr(w3), H * H, H, 1, qkv, H, 3 * H, 1, 3, M32, H32, H32, b3, TI_BIAS_I8, H, a3, s3, 1,
-                                      TI_EPI_SCALE_I8, TI_I8, TI_ROUND_RNE_CLAMP, -1, c.stream))) return;
+                                      TI_EPI_SCALE_I8, TI_I8, TI_ROUND_RNE_CLAMP, next_reads, c.stream))) return;
           if ((rc = ti_kv_append_i8_seqs(cached ? qkv + H : nullptr, cached ? 3 * H : 0, qkv + 2 * H, 3 * H, k_dst, dst_hs, dst_rs, vd, vt_rs, B32, S32,
                                          (int)heads, (int)D, c.stream))) return;
         }
@@ -250,7 +251,7 @@ PyObject* decoder_layer(PyObject*, PyObject* const* v, Py_ssize_t n) {
           if ((rc = ti_dq_add_layernorm_q(acc, H, in_scale, nullptr, xp, x_rs, ln2.g, ln2.b, ln2.eps, resid, H, h8b, H, nullptr, H, M32, H32, TI_ROUND_RNE_CLAMP,
                                           nullptr, nullptr, c.stream))) return;
           if ((rc = ti_bmm_i8_config(h8b, 0, H, 1, fc1.w, 0, fc1.ldw, 1, f8, 0, fc1.N, 1, 1, M32, F32, H32, fc1.bias, TI_BIAS_F32, fc1.a, fc1.b, TI_EPI_GELU_I8, TI_I8,
-                                     TI_ROUND_RNE_CLAMP, -1, c.stream))) return;
+                                     TI_ROUND_RNE_CLAMP, next_reads, c.stream))) return;
         }
         rc = ti_linear_i8_residual_f32(f8, fc1.N, fc2.w, fc2.ldw, (const float*)fc2.bias, fc2.a, fc2.b, resid, H, (float*)mptr(out), H, M32, H32, F32, c.stream);
       };
