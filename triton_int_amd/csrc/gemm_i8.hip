@@ -1551,9 +1551,10 @@ __global__ __launch_bounds__((WAVES_M * WAVES_N + PW) * 64) void gemm_mfma_ws_ke
     int b_extent = 0, b_n0 = 0;
     // one column of tiles: every byte of A is read exactly once, so it need not stay in the caches
     const bool a_once = p.tiles_n == 1;
-    // Tiles of 64 columns: weights read once (one row tile) of 96 MB and more pass the caches by, 128 x 5120 x 20480 37.3 / 36.2 us, 128 x 16384 x 16384
-    // 65.7 / 61.7; smaller ones may still lie in the Infinity Cache, 64 x 6848 x 10240 16.5 / 19.5
-    const bool b_once = p.tiles_m == 1 && (int64_t)p.N * p.K * p.batch >= 96000000;
+    // Tiles of 64 columns: weights read once (one row tile) that cannot lie in the Infinity Cache (256 MB) pass it by.  us, through the caches / past them: 54 x 16224
+    // x 19776 (321 MB) 68.3 / 67.6, 61 x 16384 x 19472 74.1 / 71.7.  Smaller ones may still lie there, 64 x 6848 x 10240 16.5 / 19.5, 60 x 7680 x 17184 (132 MB) 27.4 /
+    // 35.0, 61 x 15840 x 15760 (250 MB) 43.2 / 57.8; from HBM 34.2 / 33.1, 60.8 / 58.3.
+    const bool b_once = p.tiles_m == 1 && (int64_t)p.N * p.K * p.batch >= 256000000;
     auto aim = [&](int i) {
       kt_left = KT;
       k_issue = 0;
