@@ -5,8 +5,11 @@ import torch
 from tests import gemm_bounds_model as G
 from triton_int_amd import _lib as L
 
-SIZES = [(149, 1000, 1000, 128, "mfma_128x128"), (22, 429, 429, 128, "ragged_64"), (5, 65, 4001, 16, "ragged_64"), (8, 300, 1001, 64, "ragged_64"), (30, 510, 510, 64, "mfma_128x128"),
-         (100, 150, 150, 128, "ragged_64"), (20, 257, 2047, 128, "mfma_128x128"), (150, 90, 90, 128, "ragged_64")]
+SIZES = [(149, 1000, 1000, 128, "mfma_256x256"), (22, 429, 429, 128, "mfma_128x128"), (5, 65, 4001, 16, "ragged_64"), (8, 300, 1001, 64, "ragged_64"), (30, 510, 510, 64, "mfma_128x128"),
+         (100, 150, 150, 128, "ragged_64"), (20, 257, 2047, 128, "mfma_128x128"), (150, 90, 90, 128, "mfma_64x64"),
+         # sizes that rules by padding alone sent to slower tiles
+         (94, 1154, 1154, 64, "mfma_256x256"), (64, 184, 1825, 80, "mfma_256x256"), (37, 504, 504, 128, "mfma_128x128"), (47, 77, 77, 128, "mfma_64x64"), (54, 294, 294, 128, "mfma_128x128"),
+         (84, 165, 165, 64, "ragged_64")]
 
 
 @pytest.mark.parametrize("B,M,N,K,name", SIZES)

@@ -3234,6 +3234,34 @@ static int pick_ragged(const GemmParams& p, int64_t tiles128, int* splits_out) {
   return CFG_RAGGED_64;
 }
 
+// Attention scores that the persistent kernels cannot store (an odd number of keys): the epilogue is most of the launch.  Times fitted to 1050 launches of 5
+// .. 600 heads of 65 .. 2048 rows against 17 .. 2048 keys, K = 16 .. 128: a start, rounds of one workgroup per CU and of as many as a CU holds, a tile's k-steps of
+// 64, the outputs.  The choice is 0.7 % above the fastest on average; the estimate for whole K below 9.7 %, and 128 x 128 tiles or 64 x 64 ones by the share of
+// padding 2.6 %.  us, 256 x 256 / 128 x 128 / 64 x 64 / 64 x 64 of gemm_ragged_kernel: 94 heads x 1154 x 1154, K = 64 86.2 / 101 / 134 / 99.6, 145 x 1023 x 1023 152 / 126 / 164 / 147, 64 x
+// 184 x 1825, K = 80 17.4 / 21.6 / 24.8 / 22.8, 263 x 87 x 87 13.0 / 6.7 / 7.8 / 8.1, 26 x 356 x 552, K = 64 9.0 / 6.5 / 7.8 / 7.1, 47 x 77 x 77 7.9 / 5.9 / 4.3 / 4.8, 84 x 165 x 165, K = 64 7.0 / 5.8 /
+// 5.2 / 5.0.  256 x 128 tiles led nowhere.  Where it loses: 142 x 415 x 415 33.0 / 26.6 / 29.2 / 26.3.
+static int pick_scores(const GemmParams& p) {
+  struct Cost { int cfg, per_cu; double start, round, full_round, kstep, mb, kstep_first; };
+  static const Cost costs[] = {
+      {CFG_TILE_256x256, 1, 3.41, 0.00, 3.34, 0.77, 0.28, 0.39},
+      {CFG_TILE_128x128, 2, 2.65, 0.91, 1.20, 0.25, 0.12, 0.22},
+      {CFG_TILE_64x64, 3, 2.59, 0.59, 0.81, 0.04, 0.04, 0.00},
+      {CFG_RAGGED_64, 4, 2.75, 0.40, 0.58, 0.14, 0.02, 0.18},
+  };
+  const double ksteps = (p.K + 63) / 64, mb = (double)p.M * p.N * p.batch * 1e-6;
+  int best = CFG_TILE_128x128;
+  double best_time = -1.0;
+  for (const Cost& c : costs) {
+    if (c.cfg == CFG_RAGGED_64 && !ragged_eligible(p)) continue;
+    const Config& k = g_configs[c.cfg];
+    const int64_t tiles = (int64_t)((p.M + k.bm - 1) / k.bm) * ((p.N + k.bn - 1) / k.bn) * p.batch, held = 256 * c.per_cu;
+    const double t = c.start + (double)((tiles + 255) / 256) * c.round + (double)((tiles + held - 1) / held) * c.full_round +
+                     (double)tiles / 256 * ksteps * c.kstep + mb * c.mb + ksteps * c.kstep_first;
+    if (best_time < 0 || t < best_time) best_time = t, best = c.cfg;
+  }
+  return best;
+}
+
 // Tile choice: the configuration (and K split) with the lowest estimated run time.  The class
 // efficiencies were measured with weights streamed from HBM.  Outputs the persistent kernels can
 // store (row-major, aligned) go to them; the rest to the one-tile kernels.
@@ -3339,14 +3367,7 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
     const int64_t tm = (p.M + 255) / 256, tn = (p.N + 255) / 256;
     if (tm * tn * p.batch >= 512 && (double)p.M * p.N >= 0.6 * (double)(tm * 256) * (double)(tn * 256)) return CFG_SHORTK_256x256;
   }
-  // Attention scores that the persistent kernels cannot store (an odd number of keys): the epilogue is most of the launch.  128 x 128 tiles, and 64 x 64
-  // of gemm_ragged_kernel where they are a fifth less padding or the larger are few.  us, the 256-row tiles that the estimate took / 128 x 128 / 64 x 64: 149 heads x
-  // 1000 x 1000 95.0 / 90.3 / 123, 40 x 1366 57.5 / 52.0 / 67, 107 x 234 9.8 / 8.8 / 10.8, 30 x 510, K = 64 11.1 / 9.8 / 10.2, 100 x 150 7.5 / 6.2 / 5.9, 90 x 190 9.7 / 7.9 /
-  // 7.2, 141 x 137 8.7 / 10.2 / 8.1, 150 x 90 7.4 / 5.9 / 5.4; 160 x 130 7.5 / 11.1 / 8.4 loses.
-  if (!stream && out_class(p.out_dtype) == OUT8 && p.batch > 4 && p.K <= 128) {
-    const int64_t t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64), t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
-    return (ragged_eligible(p) && (t64 * 5 < t128 * 16 || t128 * p.batch <= 192)) ? CFG_RAGGED_64 : CFG_TILE_128x128;
-  }
+  if (!stream && out_class(p.out_dtype) == OUT8 && p.batch > 4 && p.K <= 128) return pick_scores(p);
   // short K: the epilogue dominates and the larger tile halves the operand traffic per output
   const double big = p.K <= 512 ? 1.20 : 0.92;
   // 256 x 160 tiles: as good as 256 x 128 per unit of work with 2- and 4-byte outputs; with int8 outputs
