@@ -28,6 +28,17 @@ def test_more_query_rows_run_on_the_kernel_that_measures_faster():
         assert rows(heads, S, T) == 16, (heads, S, T)
 
 
+def test_rows_of_vt_at_any_byte_cost_the_groups_more():
+    """us, groups / blocks, V^T rows of 16-byte pieces and others: 32 heads x 387 x 387 13.9 / 20.3 and 29.5 / 21.8."""
+    from triton_int_amd import _lib as L
+
+    rows = lambda heads, S, T, pitch: L.lib().ti_attention_i8_rows(heads, S, T, 128, 128, pitch)
+    for heads, S, T in ((32, 387, 387), (40, 377, 763), (64, 129, 129)):
+        assert rows(heads, S, T, (T + 15) // 16 * 16) == 16 and rows(heads, S, T, T) == 128, (heads, S, T)
+    for heads, S, T in ((40, 207, 207), (48, 229, 229), (80, 115, 243), (8, 19, 1103)):
+        assert rows(heads, S, T, T) == 16, (heads, S, T)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("S", [1, 16, 17])
 @pytest.mark.parametrize("heads,T", [(1024, 33), (1025, 33), (1030, 80), (2600, 17)])

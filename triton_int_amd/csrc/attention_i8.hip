@@ -758,25 +758,27 @@ __global__ __launch_bounds__(NW * 64, 4) void attention_row_i8_kernel(AttnParams
 // rounds of the chip (256 workgroups each) on whichever kernel takes less: a round of groups walks the keys once, 0.2 us per 64 of them and
 // 2.5 us besides, or as long as 4 TB/s take for the caches of the heads in it (up to 256: each is then read again in the
 // next round); two workgroups on a CU fill a last round that is partly empty.  The blocks of 128 rows on attention_i8_kernel, all in one round,
-// 1.8 us per 64 keys and 3 us besides however few their rows.  128-row blocks beyond four rounds.
-// Measured over 170 sizes of 17 .. 600 rows against 17 .. 1950 keys, masked: the estimate's choice is 1.6 % above the better one on
-// average (the one before it, fitted when a workgroup had four chunks of keys a wave at least, 5.3 %).  us, groups / blocks: 40 heads x 205
-// rows x 205 keys 9.1 / 15.2, 80 x 107 x 196 10.6 / 16.2, 32 x 371 x 371 13.7 / 20.3, 8 x 19 x 1103 10.1 / 46.9, 96 x 57 x 755 22.5 / 37.9; but 80 x 377 x 377
-// 28.6 / 20.6, 160 x 232 x 434 58.8 / 32.0.  Where it loses: 80 x 139 x 139 9.4 / 12.2, 32 x 516 x 516 (1056 groups) 20.4 / 25.9.
-// 16 rows and fewer, as many workgroups either way: 1280 x 1 x 2048 156 / 265, 2560 x 16 x 2048 297 / 464, 1056 x 1 x
-// 333 24.8 / 57.8, 20000 x 1 x 304 346 / 707 (20000 x 1 x 64 265 / 242).
-static bool attn_groups_lead(int64_t heads, int S, int T) {
+// 1.8 us per 64 keys and 3 us besides however few their rows.  Rows of V^T of no whole 16-byte pieces: 0.5 us per 64 keys and 2 us, eight tenths of a last round's
+// empty part, against 2.3 and 3.5.  128-row blocks beyond four rounds.
+// Measured over 837 sizes of 17 .. 700 rows against 17 .. 4096 keys, with and without a mask: the choice is 1.1 % above the better kernel on average where rows
+// of V^T are whole pieces (337 sizes; no launch of groups 3 % above the blocks), 0.6 % where they are not (500; by the first estimate 1.0 %).  us, groups / blocks, 40
+// heads x 205 rows x 205 keys 9.1 / 15.2, 80 x 107 x 196 10.6 / 16.2, 32 x 371 x 371 13.7 / 20.3, 8 x 19 x 1103 10.1 / 46.9, 96 x 57 x 755 22.5 / 37.9; but 80 x 377 x 377
+// 28.6 / 20.6, 160 x 232 x 434 58.8 / 32.0; V^T at any byte 40 x 207 x 207 12.4 / 15.8, 32 x 501 x 501 26.0 / 25.0, 40 x 377 x 763 46.4 / 35.5, 64 x 129 x 129 14.1 / 12.4.  Where it
+// loses: 80 x 139 x 139 9.4 / 12.2, 32 x 516 x 516 (1056 groups) 20.4 / 25.9, at any byte 32 x 258 x 258 19.8 / 16.8.
+// 16 rows and fewer, as many workgroups either way: 2560 x 16 x 2048 297 / 464.
+static bool attn_groups_lead(int64_t heads, int S, int T, bool whole_pieces) {
   const int64_t groups = heads * ((S + 15) / 16);
   if (S <= 16) return true;
   if (groups > 1024) return false;
-  const double walk = 2.5 + 0.2 * T / 64, fetch = (double)(heads < 256 ? heads : 256) * T * 2 * AT_D / 4.0e6;
-  const double rounds = groups > 256 ? (double)groups / 256 : 1.0;
-  return rounds * (walk > fetch ? walk : fetch) <= 3.0 + 1.8 * T / 64;
+  const double walk = whole_pieces ? 2.5 + 0.2 * T / 64 : 2.0 + 0.5 * T / 64, fetch = (double)(heads < 256 ? heads : 256) * T * 2 * AT_D / 4.0e6;
+  const double full = groups > 256 ? (double)groups / 256 : 1.0, empty = (double)((groups + 255) / 256) - full;
+  const double rounds = whole_pieces ? full : full + 0.8 * empty;
+  return rounds * (walk > fetch ? walk : fetch) <= (whole_pieces ? 3.0 + 1.8 * T / 64 : 3.5 + 2.3 * T / 64);
 }
 
 static bool attn_few_rows(int64_t heads, int S, int T, int64_t q_row_stride, int64_t k_row_stride, int64_t vt_row_stride) {
   const int64_t lim32 = (int64_t)1 << 31;  // descriptor extents and offsets
-  return attn_groups_lead(heads, S, T) && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 &&
+  return attn_groups_lead(heads, S, T, !(vt_row_stride & 15)) && T <= AD_MAXT && (int64_t)(T + 256) * k_row_stride < lim32 &&
          (int64_t)AT_D * vt_row_stride < lim32 && (int64_t)S * q_row_stride < lim32;
 }
 
