@@ -36,7 +36,8 @@ def test_row_norms(rows, cols):
         assert torch.equal(resid[a:b], r) and torch.equal(z[a:b], q)
 
 
-@pytest.mark.parametrize("rows,cols,causal", [(82000, 2048, 0), (82000, 2048, 2000), (82000, 2047, 0), (49153, 2048, 0), (49152, 2048, 0)])  # beyond 96 Mi scores; the last is on the line (kept)
+@pytest.mark.parametrize("rows,cols,causal", [(82000, 2048, 0), (82000, 2048, 2000), (82000, 2047, 0),
+                                              (32768, 2048, 0), (32769, 2048, 0), (49176, 2047, 0), (49177, 2047, 0)])  # beyond 64 and 96 Mi scores; each line from both sides
 def test_softmax(rows, cols, causal):
     g = torch.Generator(device=DEV).manual_seed(2)
     s = _int8(g, rows, cols)

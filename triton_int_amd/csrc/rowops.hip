@@ -723,9 +723,10 @@ int ti_softmax_q(const int8_t* x, int64_t x_row_stride, float scale, int8_t* y, 
   dim3 grid((unsigned)((rows + ti::SM_WAVES - 1) / ti::SM_WAVES)), block(ti::SM_WAVES * 64);
   const int vpt = (cols + 1023) / 1024;
   const bool aligned = ((((uintptr_t)x) | ((uintptr_t)y) | (uintptr_t)x_row_stride | (uintptr_t)y_row_stride | (uintptr_t)cols) & 15) == 0;
-  // for the Infinity Cache (see LOAD_AUX) up to 100 MB of scores, us, non-temporal / for the cache: 40 x 1024^2 22.0 / 20.3, 80 x 1024^2
-  // 36.3 / 31.4, but 80 x 2048^2 110 / 125, 160 x 2048^2 215 / 248
-  const bool keep = (int64_t)rows * cols <= (int64_t)96 << 20, vec = aligned && scale > 0.0f;
+  // For the Infinity Cache (see LOAD_AUX) up to 64 Mi scores, rows at any byte up to 96 Mi.  us of scores, this and P.V, D = 128, non-temporal / for the cache: 13 x 2048^2 50.5 /
+  // 48.3, 15 54.4 / 52.8, but 17 63.9 / 65.3, 19 67.5 / 76.3, 21 79.0 / 82.4, 24 84.6 / 93.6, 72 x 1024^2 82.3 / 86.3, 96 99.3 / 102.0 (52 x 1280^2 100.1 / 94.8); odd 18 x 1999^2
+  // 112.7 / 109.5, 90 x 1001^2 176.4 / 174.4, 23 x 1999^2 159.2 / 151.8.
+  const bool vec = aligned && scale > 0.0f, keep = (int64_t)rows * cols <= (int64_t)(vec ? 64 : 96) << 20;
   const auto launch = [&](auto vpt_tag, auto keep_tag) {
     constexpr int VPT = decltype(vpt_tag)::value;
     constexpr bool KEEP = decltype(keep_tag)::value;
