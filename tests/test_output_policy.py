@@ -8,12 +8,11 @@ NEXT_READS = 0x100ff  # 0xff | TI_CONFIG_NEXT_READS
 
 
 @pytest.mark.parametrize("batch,shared_a,M,N,K,alone,read_next", [
-    (1, 1, 2048, 4096, 4096, 1, 1),
+    (1, 1, 1500, 2048, 2048, 1, 1),        # 10 MB
+    (1, 1, 2048, 4096, 4096, 0, 1),        # 34 MB: weights and activations would be pushed out for outputs that nobody may read
     (1, 1, 232, 4096, 4096, 0, 1),         # weights are most of the launch
     (1, 1, 1023, 4096, 4096, 0, 1),        # outputs of a quarter of the weights: the line
     (1, 1, 1024, 4096, 4096, 1, 1),
-    (1, 1, 4096, 16384, 1024, 1, 1),       # 88 MB
-    (1, 1, 1536, 16384, 4096, 0, 1),       # 99 MB: weights and activations would be pushed out for outputs that nobody may read
     (1, 1, 2048, 16384, 4096, 0, 1),
     (3, 1, 2048, 5120, 5120, 0, 1),        # 10 + 79 + 31 MB
     (3, 0, 1024, 4096, 4096, 1, 1),        # 13 + 50 + 13 MB

@@ -3425,18 +3425,17 @@ static int pick_group_m(const GemmParams& p, const Config& k) {
   return best;
 }
 
-// Whether int8 outputs of the persistent kernels stay in the 256 MB Infinity Cache: where they, with what the launch reads, take 96 MB of it at
-// most and are a quarter of the weights or more, or, where the caller says that the next launch reads them (TI_CONFIG_NEXT_READS), fit it.  Nobody reading them, kept outputs cost nothing up to
-// there, and beyond they push out weights and activations that would be found.  us, streamed / kept: one linear 4096 x 12288 x 2048 (84 MB) 96.2 / 95.9, 4096 x
-// 16384 x 1024 (88 MB) 73.4 / 71.6, but 1536 x 16384 x 4096 (99 MB) 88.2 / 93.6, 2048 x 16384 x 4096 (109 MB) 116.3 / 124.7, 4096 x 16384 x 4096 229 / 243, 8192 x 20480
-// x 5120 734 / 741; decoder layers, 1024 wide 4096 rows 205 / 196, 4096 wide 512 rows 175.2 / 174.3, 4096 rows 953 / 941, 8192 rows 1852 / 1833, 12288 rows (201 MB from
-// fc1) 2729 / 2724, 16384 rows 3633 / 3637.  Scores and the softmax after them, K = 256: 12 x 2048^2 (63 MB) 57.3 / 54.5, 20 (105 MB) 99.4 / 109.4, 60
-// 280 / 286, 96 440 / 454 (but 40 194 / 187); gemm_mfma_shortk_kernel 40 x 1024^2 40.0 / 38.8, 160 x 1024^2 120 / 123, 40 x 2048^2 with P.V 141 / 155.  P.V,
-// V as [K,N], 80 x 2048 x 128 x 2048 75.1 / 75.6.  Where the weights are most of a launch, a set of six linears, 4096 wide, 150 rows 103.5 / 104.5, 232 rows 111.7 / 113.5, but 1500 x
-// 2048 x 2048 9.83 / 9.66, 2048 x 4096 x 4096 29.9 / 29.7.
+// Whether int8 outputs of the persistent kernels stay in the 256 MB Infinity Cache: where they, with what the launch reads, take 96 MB of it at most (one
+// GEMM: 32 MB) and are a quarter of the weights or more, or, where the caller says that the next launch reads them (TI_CONFIG_NEXT_READS), fit it.
+// Kept for nobody, they push out weights and activations that would be found.  us, streamed / kept: one linear 1500 x 2048 x 2048 (10 MB) 9.83 / 9.66, 1024 x 4096 x
+// 4096 (25 MB) 18.15 / 18.03, 2048 x 4096 x 4096 (34 MB) 29.9 / 29.7 alone, but 381.7 / 385.0 for a set of six 4096 wide with three of it; 1536 x 16384 x 4096 (99 MB) 88.2 /
+// 93.6, 2048 x 16384 x 4096 116.3 / 124.7, 8192 x 20480 x 5120 734 / 741; mostly weights, the set with 150 rows 103.5 / 104.5, 232 rows 111.7 / 113.5.  Scores and the
+// softmax after them, K = 256: 12 x 2048^2 (63 MB) 57.3 / 54.5, 20 (105 MB) 99.4 / 109.4, 60 280 / 286, 96 440 / 454 (but 40 194 / 187); gemm_mfma_shortk_kernel 40 x 1024^2
+// 40.0 / 38.8, 160 x 1024^2 120 / 123, 40 x 2048^2 with P.V 141 / 155.  P.V, V as [K,N], 80 x 2048 x 128 x 2048 75.1 / 75.6.  Decoder layers, whose next launch reads: 1024
+// wide 4096 rows 205 / 196, 4096 wide 512 rows 175.2 / 174.3, 4096 rows 953 / 941, 8192 rows 1852 / 1833, 12288 rows (201 MB from fc1) 2729 / 2724, 16384 rows 3633 / 3637.
 static bool keep_outputs(int64_t batch, bool shared_a, int64_t M, int64_t N, int64_t K, bool next_reads) {
   const double a = (double)M * K * (shared_a ? 1 : batch), b = (double)N * K * batch, c = (double)M * N * batch;
-  return next_reads ? c <= 256e6 : a + b + c <= 96e6 && 4 * c >= b;
+  return next_reads ? c <= 256e6 : a + b + c <= (batch > 1 ? 96e6 : 32e6) && 4 * c >= b;
 }
 
 static int validate(const GemmParams& p) {
