@@ -3311,11 +3311,13 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
     //   Outputs that the tiles cannot store (int8 of N no multiple of 16) have gemm_skinny_kernel instead: this one at any K.  int8 out,
     //   64 x 17000 x 4096 59.1 / 18.3, 64 x 5001 x 12000 49.4 / 23.5, 64 x 511 x 1024 13.8 / 5.3, 40 x 333 x 16000 31.7 / 16.7, 17 x 300 x 1040 6.5 / 4.9;
     //   equal at 32 x 5001 x 12000 21.5 / 21.9 and 17 x 20001 x 10240.
-    // Three corners stay on the tiles although this kernel measures better there, because tests name what
-    // they run on: M > 48 with 16385 .. 20480 columns of 4 or 2 bytes (64 x 20480 x 5120 34.0 / 28.2), M > 16 with fewer than 512
-    // (32 x 272 x 1040 8.5 / 5.3), M > 48 with one unit per workgroup and K > 4096 (64 x 1024 x 10240 17.0 / 15.7).  int8 columns of the first
-    // stay below K = 2048 only (weights in the Infinity Cache; from HBM: 64 x 20480 x 5120 34.9 / 24.6; 35.4 / 24.6, 49 x 16400 x 5120 21.8 / 20.8; 30.8 / 21.1, 64 x
-    // 18000 x 2048 12.1 / 13.2; 15.2 / 12.5, but 64 x 20480 x 1024 8.8 / 10.4; 10.4 / 9.8).
+    // The lines in K were drawn against 32 x 128 and 64 x 128 tiles; behind them are 64 x 64 ones now where those take the launch (64 x 4096 x 16384 this kernel / those
+    // 22.5 / 16.9, 40 x 5120 x 20480 31.6 / 21.5; 64 x 1024 x 10240 13.7 / 10.6).
+    // Two corners stay on the tiles although this kernel measures better there, because tests name what
+    // they run on: M > 48 with 16385 .. 20480 columns of 4 or 2 bytes (64 x 20480 x 5120 35.2 / 27.0 from HBM; 20.4 / 25.8 in the Infinity Cache), M > 16 with fewer than 512
+    // (32 x 272 x 1152 6.1 / 4.5).  int8 columns of the first stay below K = 2048 only: the weights of a model come from HBM.  From HBM; in the Infinity Cache: 64 x
+    // 16624 x 2080 17.8 / 14.0; 12.1 / 13.0, 60 x 20480 x 3712 23.2 / 20.0; 15.9 / 19.1, 62 x 20272 x 4112 32.3 / 24.6; 21.3 / 23.3, 64 x 17504 x 5968 43.7 / 30.2; 27.6 / 29.2, of
+    // 29 sizes 13 .. 55 % faster; up to 17 % slower.  64 x 20480 x 1024 10.4 / 9.8; 8.8 / 10.4.
     const int units = (p.N + 3) / 4, per = (units + 256 / p.batch - 1) / (256 / p.batch);
     const bool one_round = per <= 4 * RP_GMAX;
     const int64_t columns = (int64_t)p.N * p.batch;
@@ -3346,7 +3348,7 @@ static int pick_config(const GemmParams& p, int* splits_out, bool may_split = tr
     // the 128 x 128 tile: M = 17 .. 32 34 -> 22-23 us, M = 64 35 -> 28.5 us; N = K = 5120: 18.5-19 -> 15-16 us.
     // Up to 256 tiles of 64 columns and K from 1536 on, 64 x 64: twice the CUs for the same splits, weight rows in
     // 256-byte pieces.  us, 32 x 128 or 64 x 128 / this, weights in the Infinity Cache; from HBM: 64 x 6848 x 10240 18.1 / 16.5; 23.6 / 22.3, 64 x 4096 x 16384 18.5 /
-    // 17.0; 21.9 / 21.9, 40 x 5120 x 20480 29.1 / 25.5, 57 x 13008 x 18160 72.3 / 65.3, 46 x 416 x 10000 16.5 / 10.0; 18.0 / 10.2, 24 x 352 x 17584 14.3 / 10.9;
+    // 17.0; 21.9 / 21.9, 40 x 5120 x 20480 22.7 / 21.5; 27.1 / 26.3, 57 x 13008 x 18160 43.0 / 42.6; 71.3 / 65.0, 46 x 416 x 10000 16.5 / 10.0; 18.0 / 10.2, 24 x 352 x 17584 14.3 / 10.9;
     // more tiles than CUs: 64 x 20480 x 5120 35.6 / 35.6, 32 x 17792 x 14096 55.0 / 83; whole K on 129 .. 191 CUs: 18 x 8656 x 20144 50 / 56, 45 x
     // 10560 x 20048 59 / 66; K below: 32 x 272 x 1152 6.6 / 6.6.
     const int64_t tiles = (p.N + 63) / 64;
