@@ -384,7 +384,9 @@ constexpr int AD_MAXT = 4096;
 
 // CPW: 16-key chunks per wave (T <= 256 * CPW), in steps of 256 keys up to 1536: chunks past the last key cost their loads' latency, scores and
 // exponentials like any other.  us, 4 chunks at least and then 8 and 16 / these: 32 heads x 64 rows x 64 keys 6.2 / 4.5, x 128 x 128 7.1 / 5.3, x 64 x
-// 1064 12.7 / 11.1, 64 x 140 x 437 27.7 / 19.9, 40 x 7 x 1200 11.5 / 10.1, 8 x 27 x 27 5.5 / 4.1.  DBW: 16-column blocks of the output a workgroup
+// 1064 12.7 / 11.1, 64 x 140 x 437 27.7 / 19.9, 40 x 7 x 1200 11.5 / 10.1, 8 x 27 x 27 5.5 / 4.1.  3, 6 and 12 chunks alone against the
+// next larger: 32 x 256 x 768 17.0 / 15.8, 40 x 16 x 600 7.7 / 7.3; 32 x 256 x 1400 31.4 / 28.0, 40 x 16 x 1400 13.0 / 11.7; 32 x 256 x 2500 49.7 / 47.4, 8 x 16 x 3072 19.7 / 18.5, 40 x 16 x
+// 2500 20.9 / 21.1.  DBW: 16-column blocks of the output a workgroup
 // produces (8: the whole head; fewer: the head is spread over 8 / DBW workgroups, each of which
 // repeats the scores and the softmax and reads only its rows of V^T — a single CU fills its caches at
 // about 30 GB/s, so a head's 512 KB of K and V^T through one CU alone would take 17 us).
